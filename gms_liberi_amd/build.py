@@ -2,9 +2,9 @@
 
     python -m gms_liberi_amd.build            # -> gms_liberi_amd/libliberi_hip.so
 
-The kernels of the 55 integral classes are split over several translation
-units (one per class group) that compile in parallel; the host orchestration
-is one more unit.  Every HIP unit is compiled with packed FP32 disabled
+The kernels of the 55 integral classes are spread over translation units of
+about equal compile time, which compile in parallel; the host orchestration is
+one more unit.  Every HIP unit is compiled with packed FP32 disabled
 (`-target-feature -packed-fp32-ops`).
 """
 from __future__ import annotations
@@ -14,6 +14,8 @@ import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
+
+from .census import CLASS_L
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
@@ -25,8 +27,20 @@ ARCH = "gfx950"
 COMMON = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", str(PKG.parent / "include")]
 
-# class-kernel translation units: LIBERI_CLASS_GROUP selects which classes a unit instantiates
-KERNEL_GROUPS = 8
+
+# units the class kernels are spread over (each carries its own copy of the Rys tables)
+KERNEL_UNITS = 16
+# seconds a class's kernels take to compile, where that is above 5 (the wave-split forms)
+COMPILE_S = {36: 97, 38: 87, 19: 39, 35: 35, 37: 15, 33: 15, 30: 15, 14: 14, 15: 12, 29: 11, 18: 10, 34: 10, 17: 6}
+
+
+def kernel_units() -> list:
+    """Class ids of each unit, the longest compile first onto the unit with the least so far."""
+    cost = {c: COMPILE_S.get(c, 4) for c in range(len(CLASS_L))}
+    units = [[] for _ in range(KERNEL_UNITS)]
+    for c in sorted(cost, key=cost.get, reverse=True):
+        min(units, key=lambda u: sum(cost[x] for x in u)).append(c)
+    return units
 
 
 def _run(cmd):
@@ -39,16 +53,14 @@ def _run(cmd):
 
 def build(verbose: bool = True) -> Path:
     OBJ.mkdir(exist_ok=True)
-    jobs = []
+    kernels = [HIPCC, *COMMON, "-c", str(CSRC / "eri_kernels.hip")]
+    jobs = [[*kernels, "-DLIBERI_UNIT=-3", "-o", str(OBJ / "eri_fused.o")]]
+    for g, classes in enumerate(kernel_units()):
+        entries = " ".join("X(%d, %d, %d, %d, %d)" % (c, *CLASS_L[c]) for c in classes)
+        jobs.append([*kernels, "-DLIBERI_UNIT=1", f"-DLIBERI_UNIT_LIST(X)={entries}", "-o", str(OBJ / f"eri_g{g}.o")])
+    jobs.append([*kernels, "-DLIBERI_UNIT=-1", "-o", str(OBJ / "eri_common.o")])
     jobs.append([HIPCC, *COMMON, "-c", str(CSRC / "api.cpp"), "-o", str(OBJ / "api.o")])
-    jobs.append([HIPCC, *COMMON, "-DLIBERI_CLASS_GROUP=-1", "-c", str(CSRC / "eri_kernels.hip"), "-o",
-                 str(OBJ / "eri_common.o")])
     jobs.append([HIPCC, *COMMON, "-c", str(CSRC / "noalloc.hip"), "-o", str(OBJ / "noalloc.o")])
-    jobs.append([HIPCC, *COMMON, "-DLIBERI_CLASS_GROUP=-3", "-c", str(CSRC / "eri_kernels.hip"), "-o",
-                 str(OBJ / "eri_fused.o")])
-    for g in range(KERNEL_GROUPS):
-        jobs.append([HIPCC, *COMMON, f"-DLIBERI_CLASS_GROUP={g}", f"-DLIBERI_CLASS_GROUPS={KERNEL_GROUPS}", "-c",
-                     str(CSRC / "eri_kernels.hip"), "-o", str(OBJ / f"eri_g{g}.o")])
     nproc = min(len(jobs), int(os.environ.get("MAX_JOBS", os.cpu_count() or 4)))
     with ThreadPoolExecutor(nproc) as ex:
         list(ex.map(_run, jobs))

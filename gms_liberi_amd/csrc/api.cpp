@@ -89,19 +89,17 @@ struct ClassState {
   int64_t nquart = 0, nprimq = 0;
   int32_t nseg = 0;
   int tile = -1;        // row-tile length chosen for the class, index into kTileLens (-1: not yet)
-  DevBuf ket_list, seg_start, seg_bra, seg_ket0;
+  DevBuf seg_start, seg_bra, seg_ket0;
   // the row tiles of this rank's share, for each tile length
-  DevBuf tile_q[kNumTileLens], tile_seg[kNumTileLens];
-  int32_t t_begin[kNumTileLens] = {}, t_end[kNumTileLens] = {};
+  DevBuf tiles[kNumTileLens];
+  int32_t ntile[kNumTileLens] = {};
   ClassDev dev{};
 };
 
 // Point the class's launch arguments at its row tiles of length kTileLens[k].
 static void use_tiles(ClassState &cs_, int k) {
-  cs_.dev.tile_q = (const int64_t *)cs_.tile_q[k].p;
-  cs_.dev.tile_seg = (const int32_t *)cs_.tile_seg[k].p;
-  cs_.dev.t_begin = cs_.t_begin[k];
-  cs_.dev.t_end = cs_.t_end[k];
+  cs_.dev.tiles = (const RowTile *)cs_.tiles[k].p;
+  cs_.dev.ntile = cs_.ntile[k];
 }
 
 struct liberi_ctx {
@@ -118,8 +116,14 @@ struct liberi_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // builds share the handle's workspace (Dp, Jp, Dsq): one on another stream
+  // than the last waits for its end (ev1; last_stream is NULL after a build
+  // under a caller's capture, whose events cannot be waited for)
+  hipStream_t last_stream = nullptr;
   std::vector<DevBuf> owned;
   DevBuf pairs, prims, dens, fock, scratch;
+  PairLayout layout{};      // pair layout of the basis
+  DevBuf dpair, jpair, dsq;  // per build: density and Coulomb sums by pair, square exchange density
   int64_t scratch_per_wg = 0;
   DevBuf col_bf[4];     // compact columns per angular momentum -> basis function
   int32_t ncol[4] = {};
@@ -224,11 +228,10 @@ static void drop_graph(liberi_ctx *h) {
 static void release_device(liberi_ctx *h) {
   drop_graph(h);
   for (auto &c : h->cls) {
-    dev_free(c.ket_list);
     dev_free(c.seg_start);
     dev_free(c.seg_bra);
     dev_free(c.seg_ket0);
-    for (int k = 0; k < kNumTileLens; ++k) dev_free(c.tile_q[k]), dev_free(c.tile_seg[k]);
+    for (int k = 0; k < kNumTileLens; ++k) dev_free(c.tiles[k]);
     c = ClassState{};
   }
   dev_free(h->pairs);
@@ -242,6 +245,9 @@ static void release_device(liberi_ctx *h) {
   dev_free(h->fused_head);
   h->fused_n = 0;
   dev_free(h->tune_F);
+  dev_free(h->dpair);
+  dev_free(h->jpair);
+  dev_free(h->dsq);
   dev_free(h->dens_t);
   dev_free(h->dens_b);
   dev_free(h->fock_b);
@@ -507,7 +513,7 @@ static void append_pair(std::vector<PairRec> &pairs, std::vector<PrimRec> &prims
   r.ABy = A.c[1] - B.c[1];
   r.ABz = A.c[2] - B.c[2];
   r.sameAB = sA == sB;
-  r.shA = sA;
+  r.prim_stride = 1;
   r.cA = rank ? (*rank)[sA] * ncart_host(A.l) : 0;
   r.cB = rank ? (*rank)[sB] * ncart_host(B.l) : 0;
   const double ab2 = r.ABx * r.ABx + r.ABy * r.ABy + r.ABz * r.ABz;
@@ -564,6 +570,60 @@ static int setup_fused(liberi_ctx *h) {
   h->fused_nwg = 12 * ncu;  // three one-wave workgroups per SIMD
   h->fused_n = (int64_t)items.size();
   return LIBERI_OK;
+}
+
+// Row tiles of the quartets [q_begin, q_end) of class c, in launch order: the
+// rows of the fixed pairs with the most primitives first (the kept rows run
+// from few to many), the longest rows first among those.  Consecutive
+// segments of a row whose quartets are shared by the same number of lanes are
+// cut into tiles of `len` quartets at one lane each, fewer at more, or of what
+// one step of the workgroup holds where the class has few tiles.
+static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int64_t primq, int64_t len,
+                                      const std::vector<int64_t> &sstart, const std::vector<int32_t> &sbra,
+                                      const std::vector<int32_t> &sket0, const std::vector<PairRec> &pairs) {
+  std::vector<RowTile> tiles;
+  if (q_begin >= q_end) return tiles;
+  const size_t s0 = (size_t)(std::upper_bound(sstart.begin(), sstart.end(), q_begin) - sstart.begin()) - 1;
+  const size_t s1 = (size_t)(std::lower_bound(sstart.begin(), sstart.end(), q_end) - sstart.begin());
+  // rows [first segment, last) of the share
+  std::vector<std::pair<size_t, size_t>> rows;
+  for (size_t a = s0, b; a < s1; a = b) {
+    for (b = a; b < s1 && sbra[b] == sbra[a];) ++b;
+    rows.push_back({a, b});
+  }
+  const int64_t hold = class_row_quartets(c);
+  if (q_end - q_begin <= hold * kRowSteps) len = std::min(len, hold);
+  const double chain = class_row_chain(c, primq);
+  auto team_of = [&](size_t s) {
+    int32_t t = 1;
+    if (chain > 0.0) {
+      const int nf = pairs[sbra[s]].nprim, nm = pairs[sket0[s]].nprim;
+      while (t < 64 && t < nm && (double)((nm + t - 1) / t) * nf > chain) t *= 2;
+      while (t > 1 && (nm + t / 2 - 1) / (t / 2) == (nm + t - 1) / t) t /= 2;  // no shorter chain
+    }
+    return t;
+  };
+  auto cut_row = [&](size_t a, size_t b) {
+    for (size_t s = a, e; s < b; s = e) {
+      const int32_t team = team_of(s);
+      for (e = s + 1; e < b && team_of(e) == team;) ++e;
+      const int64_t cap = std::max<int64_t>(1, len / team);
+      size_t sg = s;
+      const int64_t q1 = std::min(sstart[e], q_end);
+      for (int64_t q = std::max(sstart[s], q_begin); q < q1; q += cap) {
+        while (sstart[sg + 1] <= q) ++sg;
+        tiles.push_back(RowTile{q, (int32_t)std::min(cap, q1 - q), (int32_t)sg, team, 0});
+      }
+    }
+  };
+  for (size_t hi = rows.size(); hi > 0;) {
+    size_t lo = hi - 1;
+    auto np = [&](size_t r) { return pairs[sbra[rows[r].first]].nprim; };
+    while (lo > 0 && np(lo - 1) == np(hi - 1)) --lo;
+    for (size_t r = lo; r < hi; ++r) cut_row(rows[r].first, rows[r].second);
+    hi = lo;
+  }
+  return tiles;
 }
 
 // Setup proper, on a handle whose device data is released; the caller
@@ -687,6 +747,63 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     h->stats.prim_pairs_dropped = (int64_t)(prims.size() - kept.size());
     prims.swap(kept);
   }
+  // ---- device order.  Pairs of one class sorted by (kept primitives, Schwarz
+  // value descending, shell order): every class's kept list is then a run of
+  // consecutive pairs per primitive count (its pre-screen keeps the largest
+  // Schwarz values), and so are the kets of a segment.  The k-th primitive
+  // records of the pairs of one run are consecutive as well, so that the lanes
+  // of a row tile read neighbouring 64-byte records (207 G records/s against
+  // 103 G for scattered ones).
+  {
+    std::vector<PairRec> sorted;
+    std::vector<double> sorted_x;
+    std::vector<PrimRec> laid;
+    sorted.reserve(pairs.size());
+    sorted_x.reserve(pairs.size());
+    laid.reserve(prims.size());
+    // (a Schwarz value that is not a number is never kept: last)
+    auto key = [&](int32_t p) { return pair_x[p] == pair_x[p] ? pair_x[p] : -INFINITY; };
+    for (auto &list : class_pairs) {
+      std::sort(list.begin(), list.end(), [&](int32_t a, int32_t b) {
+        if (pairs[a].nprim != pairs[b].nprim) return pairs[a].nprim < pairs[b].nprim;
+        if (key(a) != key(b)) return key(a) > key(b);
+        return a < b;
+      });
+      for (size_t g0 = 0, g1; g0 < list.size(); g0 = g1) {
+        const int np = pairs[list[g0]].nprim;
+        for (g1 = g0; g1 < list.size() && pairs[list[g1]].nprim == np;) ++g1;
+        const int32_t off = (int32_t)laid.size(), n = (int32_t)(g1 - g0);
+        for (int k = 0; k < np; ++k)
+          for (size_t j = g0; j < g1; ++j) laid.push_back(prims[pairs[list[j]].prim_off + k]);
+        for (int32_t j = 0; j < n; ++j) {
+          const int32_t p = list[g0 + j];
+          sorted.push_back(pairs[p]);
+          sorted.back().prim_off = off + j;
+          sorted.back().prim_stride = n;
+          sorted_x.push_back(pair_x[p]);
+          list[g0 + j] = (int32_t)sorted.size() - 1;
+        }
+      }
+    }
+    pairs.swap(sorted);
+    pair_x.swap(sorted_x);
+    prims.swap(laid);
+    PairLayout &pl = h->layout = PairLayout{};
+    int64_t off = 0;
+    int32_t first = 0;
+    for (int pc = 0; pc < kNumPairClasses; ++pc) {
+      pl.off[pc] = off;
+      pl.first[pc] = first;
+      pl.n[pc] = (int32_t)class_pairs[pc].size();
+      const int64_t comps = (int64_t)ncart_host(kPairL[pc][0]) * ncart_host(kPairL[pc][1]);
+      off += pl.n[pc] * comps;
+      first += pl.n[pc];
+      // workgroups of 256 pairs each per component (fewer for the largest bases)
+      pl.chunks[pc] = (int32_t)std::min<int64_t>((pl.n[pc] + 255) / 256, 4096);
+      pl.block[pc + 1] = pl.block[pc] + (int32_t)(pl.chunks[pc] * comps);
+    }
+    pl.off[kNumPairClasses] = off;
+  }
   h->stats.prim_pairs = (int64_t)prims.size();
 
   int rc;
@@ -698,6 +815,10 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
   if (int e = launch_fill_zero((double *)h->aux.p, 2, h->stream))
     return fail(LIBERI_EDEVICE, std::string("zero aux: ") + hipGetErrorString((hipError_t)e));
   if ((rc = dev_alloc(h, h->fock, ntri * sizeof(double)))) return rc;
+  const size_t npl = (size_t)h->layout.off[kNumPairClasses];
+  if ((rc = dev_alloc(h, h->dpair, npl * sizeof(double))) || (rc = dev_alloc(h, h->jpair, npl * sizeof(double))) ||
+      (rc = dev_alloc(h, h->dsq, (size_t)num_bas * num_bas * sizeof(double))))
+    return rc;
 
   // ---- per class: pair pre-screen (host), quartet segments (device)
   std::vector<DevBuf> tmp;
@@ -725,16 +846,11 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     const double sk = def.ps == PS_CROSS ? cut / mb : cut / mk;
     const bool diag = def.bra == def.ket;
     auto group_key = [&](int32_t p) { return (int64_t)pairs[p].nprim; };
+    // (the lists are in device order: by primitive count, Schwarz value descending)
     auto keep = [&](const std::vector<int32_t> &l, double thr) {
       std::vector<int32_t> out;
       for (int32_t p : l)
         if (pair_x[p] >= thr) out.push_back(p);
-      // sort by (group key, Schwarz value descending, pair index)
-      std::sort(out.begin(), out.end(), [&](int32_t a, int32_t b) {
-        if (group_key(a) != group_key(b)) return group_key(a) < group_key(b);
-        if (pair_x[a] != pair_x[b]) return pair_x[a] > pair_x[b];
-        return a < b;
-      });
       return out;
     };
     std::vector<int32_t> kb = keep(lb, sb);
@@ -801,48 +917,32 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     cleanup_tmp();
     if (e != hipSuccess)
       return fail(LIBERI_EDEVICE, std::string("segment generation: ") + hipGetErrorString((hipError_t)e));
-    std::vector<int64_t> sstart, tq[kNumTileLens];
-    std::vector<int32_t> sbra, sket0, tseg[kNumTileLens];
+    std::vector<int64_t> sstart;
+    std::vector<int32_t> sbra, sket0;
     int64_t total = 0, primq = 0;
     for (size_t i = 0; i < kb.size(); ++i) {
-      const int64_t row0 = total;
-      const size_t sfirst = sstart.size();
       for (int g = 0; g < ng; ++g) {
         const int64_t L = len[i * ng + g];
         if (L <= 0) continue;
         sstart.push_back(total);
         sbra.push_back(kb[i]);
-        sket0.push_back(gbeg[g]);
+        sket0.push_back(kk[gbeg[g]]);
         total += L;
         primq += L * (int64_t)pairs[kb[i]].nprim * pairs[kk[gbeg[g]]].nprim;
       }
-      // row tiles: the row's quartets in runs of at most kTileLens[k]
-      for (int k = 0; k < kNumTileLens; ++k) {
-        size_t sg = sfirst;
-        for (int64_t t0 = row0; t0 < total; t0 += kTileLens[k]) {
-          while (sg + 1 < sstart.size() && sstart[sg + 1] <= t0) ++sg;
-          tq[k].push_back(t0);
-          tseg[k].push_back((int32_t)sg);
-        }
-      }
     }
     sstart.push_back(total);
-    for (auto &t : tq) t.push_back(total);
     cs_.nquart = total;
     cs_.nprimq = primq;
     if (total == 0) continue;
-    if (sbra.size() >= (size_t)INT32_MAX || tq[0].size() >= (size_t)INT32_MAX)
+    if (sbra.size() >= (size_t)INT32_MAX || total / kTileLens[0] + (int64_t)kb.size() >= (int64_t)INT32_MAX)
       return fail(LIBERI_ESIZE, std::string("class ") + def.name + ": too many segments");
     cs_.nseg = (int32_t)sbra.size();
-    if ((rc = dev_upload(h, cs_.ket_list, kk)) || (rc = dev_upload(h, cs_.seg_start, sstart)) ||
+    if ((rc = dev_upload(h, cs_.seg_start, sstart)) ||
         (rc = dev_upload(h, cs_.seg_bra, sbra)) || (rc = dev_upload(h, cs_.seg_ket0, sket0)))
       return rc;
-    for (int k = 0; k < kNumTileLens; ++k)
-      if ((rc = dev_upload(h, cs_.tile_q[k], tq[k])) || (rc = dev_upload(h, cs_.tile_seg[k], tseg[k]))) return rc;
     cs_.active = true;
     ClassDev &d = cs_.dev;
-    d.bra_list = nullptr;
-    d.ket_list = (const int32_t *)cs_.ket_list.p;
     d.seg_start = (const int64_t *)cs_.seg_start.p;
     d.seg_bra = (const int32_t *)cs_.seg_bra.p;
     d.seg_ket0 = (const int32_t *)cs_.seg_ket0.p;
@@ -865,7 +965,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
       const size_t ns = sbra.size();
       std::vector<double> cum(ns + 1, 0.0), unit(ns);
       for (size_t k = 0; k < ns; ++k) {
-        unit[k] = (double)pairs[sbra[k]].nprim * pairs[kk[sket0[k]]].nprim + kQuartetCost;
+        unit[k] = (double)pairs[sbra[k]].nprim * pairs[sket0[k]].nprim + kQuartetCost;
         cum[k + 1] = cum[k] + unit[k] * (double)(sstart[k + 1] - sstart[k]);
       }
       // first quartet at or past cost b
@@ -884,22 +984,27 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
       int64_t pq = 0;
       for (size_t k = 0; k < sbra.size(); ++k) {
         const int64_t a = std::max(sstart[k], d.q_begin), b = std::min(sstart[k + 1], d.q_end);
-        if (b > a) pq += (b - a) * (int64_t)pairs[sbra[k]].nprim * pairs[kk[sket0[k]]].nprim;
+        if (b > a) pq += (b - a) * (int64_t)pairs[sbra[k]].nprim * pairs[sket0[k]].nprim;
       }
       primq = pq;
     }
-    // tiles overlapping [q_begin, q_end): tq is strictly increasing, tq.back() = total
     for (int k = 0; k < kNumTileLens; ++k) {
-      const std::vector<int64_t> &t = tq[k];
-      const int32_t ntile = (int32_t)t.size() - 1;
-      int32_t b = (int32_t)(std::upper_bound(t.begin(), t.end(), d.q_begin) - t.begin()) - 1;
-      int32_t e = (int32_t)(std::lower_bound(t.begin(), t.end(), d.q_end) - t.begin());
-      cs_.t_begin[k] = b = std::max<int32_t>(0, std::min(b, ntile));
-      cs_.t_end[k] = std::max(b, std::min(e, ntile));
+      std::vector<RowTile> tiles;
+      if (cs_.row_ok) tiles = row_tiles(c, d.q_begin, d.q_end, primq, kTileLens[k], sstart, sbra, sket0, pairs);
+      cs_.ntile[k] = (int32_t)tiles.size();
+      if ((rc = dev_upload(h, cs_.tiles[k], tiles))) return rc;
     }
     use_tiles(cs_, kDefaultTile);
     d.row_mode = 0;
     d.transposed = transposed;
+    {
+      const PairLayout &pl = h->layout;
+      const int pf = transposed ? def.ket : def.bra, pm = transposed ? def.bra : def.ket;
+      d.fix_base = pl.off[pf] - pl.first[pf];
+      d.mov_base = pl.off[pm] - pl.first[pm];
+      d.fix_n = pl.n[pf];
+      d.mov_n = pl.n[pm];
+    }
     d.xswitch = h->exact_large_t ? class_rys_xmax(c) : reference_switch(c);
     h->stats.quartets[c] = d.q_end - d.q_begin;
     h->stats.prim_quartets[c] = primq;
@@ -987,7 +1092,7 @@ static void forget_tuned_choices() {
 // Whether class c runs its row-tiled kernel in this build.
 static bool class_row_mode(const liberi_ctx *h, int c) {
   const ClassState &cs_ = h->cls[c];
-  return cs_.row_ok && cs_.dev.t_end > cs_.dev.t_begin &&
+  return cs_.row_ok && cs_.dev.ntile > 0 &&
          (h->row_tiles == 2 || (h->row_tiles == 1 && cs_.variant == 1));
 }
 
@@ -1029,7 +1134,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
       // group class with a cooperative form (variant 3), and with a
       // wave-split row form (variant 1) where it has one: one launch of each
       // is cheap at any size, so they are timed without a size threshold
-      const bool row = cs_.row_ok && cs_.dev.t_end > cs_.dev.t_begin && h->row_tiles != 0;
+      const bool row = cs_.row_ok && cs_.dev.ntile > 0 && h->row_tiles != 0;
       cs_.variant = (dflt == 1 && h->row_tiles != 0) || h->row_tiles == 2 ? 1 : 0;
       cs_.dev.coop = 0;
       if (!h->autotune || h->row_tiles == 2 || (h->only_class >= 0 && c != h->only_class)) continue;
@@ -1055,7 +1160,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
       set_tuned_choice(c, nq, -3.0, cs_.variant);
       continue;
     }
-    if (!h->autotune || h->row_tiles != 1 || !cs_.row_ok || nq < kTuneMinQuartets || cs_.dev.t_end <= cs_.dev.t_begin ||
+    if (!h->autotune || h->row_tiles != 1 || !cs_.row_ok || nq < kTuneMinQuartets || cs_.dev.ntile <= 0 ||
         (h->only_class >= 0 && c != h->only_class)) {
       cs_.variant = dflt;
       continue;
@@ -1097,7 +1202,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     for (int k = 0; k < kNumTileLens; ++k) best[k] = 1e30f;
     for (int rep = 0; rep < 2; ++rep)
       for (int k = 0; k < kNumTileLens; ++k) {
-        if (cs_.t_end[k] <= cs_.t_begin[k]) continue;
+        if (cs_.ntile[k] <= 0) continue;
         use_tiles(cs_, k);
         float ms = 0.f;
         if (int rc = time_class(h, ba, st, c, true, false, ms)) return rc;
@@ -1163,11 +1268,10 @@ static int enqueue_dmax(liberi_ctx *h, const double *dD, hipStream_t st) {
 // Zero F (and find max |D| for the mixed form), then every class's kernel.
 // With ns > 1 the classes are spread over the side streams, longest first
 // onto the least-loaded stream, forked from and joined back into st.
-static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, double *dF, hipStream_t st, int ns) {
-  const int64_t ntri = (int64_t)h->num_bas * (h->num_bas + 1) / 2;
+static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, hipStream_t st, int ns) {
   // fock = 0 (src/liberi_driver.F90:64)
-  if (int e = launch_fill_zero(dF, ntri, st))
-    return fail(LIBERI_EDEVICE, std::string("zero F: ") + hipGetErrorString((hipError_t)e));
+  if (int e = launch_build_begin(ba, h->layout, (double *)h->dpair.p, (double *)h->dsq.p, st))
+    return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
   // the fused group launch, where on: its classes leave the per-class launches
@@ -1240,6 +1344,8 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, d
       HIP_TRY(hipEventRecord(h->join_ev[k], h->side[k]));
       HIP_TRY(hipStreamWaitEvent(st, h->join_ev[k], 0));
     }
+  if (int e = launch_build_end(ba, h->layout, st))
+    return fail(LIBERI_EDEVICE, std::string("end of the build: ") + hipGetErrorString((hipError_t)e));
   return LIBERI_OK;
 }
 
@@ -1253,6 +1359,9 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   ba.D = dD;
   ba.DK = dK ? dK : dD;
   ba.k_scale = k_scale;
+  ba.Dp = (const double *)h->dpair.p;
+  ba.Dsq = (const double *)h->dsq.p;
+  ba.Jp = (double *)h->jpair.p;
   ba.F = dF;
   ba.value_cut = h->value_cut;
   ba.scratch = (double *)h->scratch.p;
@@ -1265,10 +1374,25 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     ba.col_bf[l] = (const int32_t *)h->col_bf[l].p;
     ba.ncol[l] = h->ncol[l];
   }
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  if (cap == hipStreamCaptureStatusNone && h->last_stream && h->last_stream != st)
+    HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
   // the autotuner's timed launches see this build's max |D| (mixed form)
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
-  if (int rc = choose_variants(h, ba, st)) return rc;
+  // (they also run before any build: Dp and Dsq from this build's density)
+  const bool choose = [&] {
+    for (const ClassState &c : h->cls)
+      if (c.active && (c.variant < 0 || c.tile < 0 || c.ms < 0.f || (h->fp32_tau > 0.0 && c.fp32 < 0)))
+        return true;
+    return false;
+  }();
+  if (choose) {
+    if (int e = launch_build_begin(ba, h->layout, (double *)h->dpair.p, (double *)h->dsq.p, st))
+      return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
+    if (int rc = choose_variants(h, ba, st)) return rc;
+  }
   // the batched form: capture once (per D, F), replay afterwards.  Per-class
   // timing and single-class diagnostics run eagerly on st.
   const bool graph = h->use_graph && !h->class_timing && h->only_class < 0 && ba.DK == dD && k_scale == 1.0;
@@ -1281,7 +1405,7 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     if (!h->fork_ev) HIP_TRY(hipEventCreateWithFlags(&h->fork_ev, hipEventDisableTiming));
     HIP_TRY(hipStreamSynchronize(h->stream));
     HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_build(h, ba, dD, dF, h->stream, kSideStreams);
+    int rc = enqueue_build(h, ba, dD, h->stream, kSideStreams);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(h->stream, &g);
     if (rc) {
@@ -1297,10 +1421,11 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   HIP_TRY(hipEventRecord(h->ev0, st));
   if (graph) {
     HIP_TRY(hipGraphLaunch(h->gexec, st));
-  } else if (int rc = enqueue_build(h, ba, dD, dF, st, 1)) {
+  } else if (int rc = enqueue_build(h, ba, dD, st, 1)) {
     return rc;
   }
   HIP_TRY(hipEventRecord(h->ev1, st));
+  h->last_stream = cap == hipStreamCaptureStatusNone ? st : nullptr;
   h->build_pending = true;
   h->fp32_pending = h->fp32_tau > 0.0;
   if (!h->fp32_pending) h->stats.fp32_quartets = 0;

@@ -24,6 +24,10 @@
 
 #include "liberi_internal.hpp"
 
+#ifndef LIBERI_UNIT
+#define LIBERI_UNIT -2
+#endif
+
 #define RYS_CONST static __device__ const
 #include "rys_table.inc"
 // host copy of the end of the tabulated range per root count
@@ -113,14 +117,14 @@ __device__ __forceinline__ uint32_t tri(uint32_t i, uint32_t j) {
 // result within a few ulp of the correctly rounded value (the IEEE divide
 // and square root sequences cost about twice as many instructions).
 __device__ __forceinline__ double nr_rcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return fma(fma(-x, r, 1.0), r, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 __device__ __forceinline__ double nr_rsqrt(double x) {
-  double r = __builtin_amdgcn_rsq(x);
-  r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
-  return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * r, r, 1.0);
+  return fma(r * e, fma(e, 0.375, 0.5), r);
 }
 __device__ __forceinline__ float nr_rcp(float x) {
   const float r = __builtin_amdgcn_rcpf(x);
@@ -234,7 +238,7 @@ __device__ __forceinline__ int find_segment(const ClassDev &cd, int64_t q, int l
 __device__ __forceinline__ void quartet_of_segment(const ClassDev &cd, int s, int64_t q, int32_t &bra,
                                                    int32_t &ket) {
   const int32_t row = cd.seg_bra[s];
-  const int32_t col = cd.ket_list[cd.seg_ket0[s] + (int32_t)(q - cd.seg_start[s])];
+  const int32_t col = cd.seg_ket0[s] + (int32_t)(q - cd.seg_start[s]);
   bra = cd.transposed ? col : row;
   ket = cd.transposed ? row : col;
 }
@@ -264,6 +268,13 @@ typedef __attribute__((address_space(4))) const PrimRec ConstPrimRec;
 typedef __attribute__((address_space(4))) const PairRec ConstPairRec;
 __device__ __forceinline__ ConstPrimRec *const_view(const PrimRec *p) { return (ConstPrimRec *)p; }
 __device__ __forceinline__ ConstPairRec *const_view(const PairRec *p) { return (ConstPairRec *)p; }
+typedef __attribute__((address_space(4))) const double ConstDouble;
+__device__ __forceinline__ ConstDouble *const_view(const double *p) { return (ConstDouble *)p; }
+// element at byte offset `off` of the row starting at element `row` (uniform:
+// a scalar base and a 32-bit lane offset, no vector address arithmetic)
+__device__ __forceinline__ double dens_at(const double *d, int64_t row, uint32_t off) {
+  return *(const double *)((const char *)(d + row) + off);
+}
 // record i of a constant view, by value
 __device__ __forceinline__ PrimRec load_rec(ConstPrimRec *v, int64_t i) {
   ConstPrimRec *q = v + i;
@@ -289,7 +300,7 @@ __device__ __forceinline__ PairRec load_rec(ConstPairRec *v, int64_t i) {
   r.ABy = q->ABy;
   r.ABz = q->ABz;
   r.sameAB = q->sameAB;
-  r.shA = q->shA;
+  r.prim_stride = q->prim_stride;
   r.cA = q->cA;
   r.cB = q->cB;
   r.x = q->x;
@@ -410,13 +421,17 @@ __device__ __forceinline__ void count_fp32(const BuildArgs &ba, unsigned n) {
 // v[((a*NB + b)*NC + c)*ND + d], components in internal order.  T is the
 // arithmetic type of the 2-D integrals, the primitive accumulation and the
 // HRR; the Rys argument, roots and weights are always FP64 (they stand where
-// the reference evaluates its Boys function), and so is the result.
+// the reference evaluates its Boys function), and so is the result.  In a row
+// tile `team` adjacent lanes may share the quartet: lane `part` of them takes
+// every team-th primitive of the moving pair, and all end with the whole
+// result.
 template <class T, int LA, int LB, int LC, int LD, bool KET_OUTER = false, bool FIXED_KET = false>
 __device__ __forceinline__ void small_integrals(const PairRec &bra, const PairRec &ket, const PrimRec *prims,
                                                 double xswitch, double cut,
                                                 double (&v)[Small<LA, LB, LC, LD>::NABCD],
                                                 const double *tab = rys_table + rys_offset[Small<LA, LB, LC, LD>::NR],
-                                                int istride = rys_ncoef(Small<LA, LB, LC, LD>::NR)) {
+                                                int istride = rys_ncoef(Small<LA, LB, LC, LD>::NR), int part = 0,
+                                                int team = 1) {
   using S = Small<LA, LB, LC, LD>;
   constexpr int NE = S::NE, NF = S::NF, NR = S::NR, NI = S::LAB + 1, NK = S::LCD + 1;
   constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND;
@@ -458,34 +473,40 @@ __device__ __forceinline__ void small_integrals(const PairRec &bra, const PairRe
           acc[e * NF + f] += gx[re.lx[e]][rf.lx[f]] * gy[re.ly[e]][rf.ly[f]] * gz[re.lz[e]][rf.lz[f]];
     }
   };
-  if constexpr (KET_OUTER) {
-    // the inner loop walks the bra pair's primitives (the pair a row tile
-    // keeps fixed: every lane then reads the same records, through the
-    // scalar cache)
-    ConstPrimRec *cprims = const_view(prims);
-    for (int iq = 0; iq < ket.nprim; ++iq) {
-      const PrimRec Q = prims[ket.prim_off + iq];
-      for (int ip = 0; ip < bra.nprim; ++ip) prim(load_rec(cprims, bra.prim_off + ip), Q);
+  if constexpr (KET_OUTER || FIXED_KET) {
+    // row tiles: the outer loop walks the lane's own (moving) pair, whose
+    // records lie next to those of the neighbouring lanes' pairs, the inner
+    // one the fixed pair's primitives, which every lane reads through the
+    // scalar cache
+    const PairRec &mov = KET_OUTER ? ket : bra, &fix = KET_OUTER ? bra : ket;
+    ConstPrimRec *cf = const_view(prims) + fix.prim_off;
+    const PrimRec *cm = prims + mov.prim_off;
+    for (int im = part; im < mov.nprim; im += team) {
+      const PrimRec M = cm[(int64_t)im * mov.prim_stride];
+      for (int i = 0; i < fix.nprim; ++i) {
+        const PrimRec X = load_rec(cf, (int64_t)i * fix.prim_stride);
+        if constexpr (KET_OUTER)
+          prim(X, M);
+        else
+          prim(M, X);
+      }
     }
+    // the partial sums of a team of lanes (a power of two, within the wave)
+    for (int o = 1; o < team; o <<= 1)
+#pragma unroll
+      for (int k = 0; k < NE * NF; ++k) acc[k] += __shfl_xor(acc[k], o);
   } else {
     for (int ip = 0; ip < bra.nprim; ++ip) {
-      const PrimRec P = prims[bra.prim_off + ip];
+      const PrimRec P = prims[bra.prim_off + ip * bra.prim_stride];
       // (ss|ss): the next ket primitive is loaded one iteration ahead, its
       // latency hidden behind this iteration's arithmetic (in the other
       // classes the extra registers cost more occupancy than the latency it
       // hides)
       constexpr bool ahead = LA + LB + LC + LD == 0;
-      // a row tile's fixed pair is the ket here (uniform: the scalar cache)
-      auto ket_rec = [&](int iq) -> PrimRec {
-        if constexpr (FIXED_KET)
-          return load_rec(const_view(prims), ket.prim_off + iq);
-        else
-          return prims[ket.prim_off + iq];
-      };
-      PrimRec Qn = ket_rec(0);
+      PrimRec Qn = prims[ket.prim_off];
       for (int iq = 0; iq < ket.nprim; ++iq) {
-        const PrimRec Q = ahead ? Qn : ket_rec(iq);
-        if (ahead && iq + 1 < ket.nprim) Qn = ket_rec(iq + 1);
+        const PrimRec Q = ahead ? Qn : prims[ket.prim_off + iq * ket.prim_stride];
+        if (ahead && iq + 1 < ket.nprim) Qn = prims[ket.prim_off + (iq + 1) * ket.prim_stride];
         prim(P, Q);
       }
     }
@@ -800,15 +821,11 @@ constexpr int row_threads() {
 }
 
 template <int LA, int LB, int LC, int LD, bool TR>
-__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kernel(ClassDev cd, BuildArgs ba) {
+__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_kernel(ClassDev cd, BuildArgs ba) {
   using S = Small<LA, LB, LC, LD>;
   using R = RowShape<LA, LB, LC, LD, TR>;
   constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND;
   constexpr int N1 = R::N1, N2 = R::N2, NFIX = R::NFIX, NROW = R::NROW;
-  constexpr Range<LA, LA> ra{};
-  constexpr Range<LB, LB> rb{};
-  constexpr Range<LC, LC> rc{};
-  constexpr Range<LD, LD> rd{};
   constexpr Range<R::L1, R::L1> r1{};
   constexpr Range<R::L2, R::L2> r2{};
   constexpr Range<R::M1, R::M1> rm1{};
@@ -817,6 +834,11 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
   double *jfix_s = lds, *rows = lds + NFIX;
   const int ncols = (int)row_columns<LA, LB, LC, LD, TR>(ba.ncol);
   const int off2 = R::M1 == R::M2 ? 0 : ba.ncol[R::M1];
+  const RowTile tl = cd.tiles[blockIdx.x];
+  const int64_t q0 = tl.q0, q1 = q0 + tl.n;
+  const int seg0 = tl.seg, team = tl.team;
+  const int32_t ifix = cd.seg_bra[seg0];
+  const PairRec fix = load_rec(const_view(ba.pairs), ifix);
   // the class's Rys table below the switch, staged once per workgroup with
   // intervals padded to an odd stride
   double *tab = rows + NROW * ncols;
@@ -827,61 +849,64 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
     for (int i = threadIdx.x; i < ntab; i += blockDim.x) tab[(i / IN) * LS + i % IN] = src[i];
   }
 
-  const int tile = cd.t_begin + (int)blockIdx.x;
-  const int64_t q0 = cd.tile_q[tile] > cd.q_begin ? cd.tile_q[tile] : cd.q_begin;
-  const int64_t q1 = cd.tile_q[tile + 1] < cd.q_end ? cd.tile_q[tile + 1] : cd.q_end;
-  const int seg0 = cd.tile_seg[tile];
-  const int32_t ifix = cd.seg_bra[seg0];
-  const PairRec fix = load_rec(const_view(ba.pairs), ifix);
   for (int i = threadIdx.x; i < NFIX + NROW * ncols; i += blockDim.x) lds[i] = 0.0;
 
-  const double *Dm = ba.D, *Dk = ba.DK;  // Coulomb and exchange densities
-  double *F = ba.F;
-  // the fixed pair's density block and Coulomb partial sums
-  double dfix[NFIX], jfix[NFIX];
+  double jfix[NFIX];  // the fixed pair's Coulomb partial sums
 #pragma unroll
-  for (int i = 0; i < N1; ++i)
-#pragma unroll
-    for (int j = 0; j < N2; ++j) {
-      dfix[i * N2 + j] = Dm[tri(fix.bfA + gamess_pos(r1.lx[i], r1.ly[i], r1.lz[i]),
-                                fix.bfB + gamess_pos(r2.lx[j], r2.ly[j], r2.lz[j]))];
-      jfix[i * N2 + j] = 0.0;
-    }
+  for (int k = 0; k < NFIX; ++k) jfix[k] = 0.0;
   const double sfix = fix.sameAB ? 0.5 : 1.0;
   __syncthreads();
 
   unsigned nlow = 0;  // quartets this lane evaluated in FP32
   int sg = seg0;      // segment of the lane's quartet (its quartets ascend)
-  for (int64_t qb = q0; qb < q1; qb += blockDim.x) {
-    const int64_t q = qb + threadIdx.x;
+  const int part = (int)threadIdx.x & (team - 1);
+  for (int64_t qb = q0; qb < q1; qb += blockDim.x / (unsigned)team) {
+    const int64_t q = qb + threadIdx.x / (unsigned)team;
     if (q >= q1) continue;
     while (sg + 1 < cd.nseg && cd.seg_start[sg + 1] <= q) ++sg;
-    const int32_t imov = cd.ket_list[cd.seg_ket0[sg] + (int32_t)(q - cd.seg_start[sg])];
+    const int32_t imov = cd.seg_ket0[sg] + (int32_t)(q - cd.seg_start[sg]);
     const PairRec mov = ba.pairs[imov];
     const PairRec &bra = TR ? mov : fix;
     const PairRec &ket = TR ? fix : mov;
     double v[S::NABCD];
     if (mixed_wave(cd, ba, bra, ket)) {
-      ++nlow;
+      nlow += part == 0;
       small_integrals<float, LA, LB, LC, LD, !TR, TR>(bra, ket, ba.prims, cd.xswitch, ba.value_cut, v, tab,
-                                             rys_lds_stride(S::NR));
+                                             rys_lds_stride(S::NR), part, team);
     } else {
       small_integrals<double, LA, LB, LC, LD, !TR, TR>(bra, ket, ba.prims, cd.xswitch, ba.value_cut, v, tab,
-                                              rys_lds_stride(S::NR));
+                                              rys_lds_stride(S::NR), part, team);
     }
+    if (part != 0) continue;
 
     double s = sfix;
     if (mov.sameAB) s *= 0.5;
     if (cd.diag && ifix == imov) s *= 0.5;
-    int ga[NA], gb[NB], gc[NC], gd[ND];
+    // byte offsets of the moving pair's functions in a row of the square
+    // exchange density
+    uint32_t mo1[R::NM1], mo2[R::NM2];
 #pragma unroll
-    for (int a = 0; a < NA; ++a) ga[a] = bra.bfA + gamess_pos(ra.lx[a], ra.ly[a], ra.lz[a]);
+    for (int i = 0; i < R::NM1; ++i) mo1[i] = 8u * (mov.bfA + gamess_pos(rm1.lx[i], rm1.ly[i], rm1.lz[i]));
 #pragma unroll
-    for (int b = 0; b < NB; ++b) gb[b] = bra.bfB + gamess_pos(rb.lx[b], rb.ly[b], rb.lz[b]);
+    for (int i = 0; i < R::NM2; ++i) mo2[i] = 8u * (mov.bfB + gamess_pos(rm2.lx[i], rm2.ly[i], rm2.lz[i]));
+    // exchange density of component i of the fixed pair's shell A (B) with
+    // the function at byte offset mo: a uniform row and a lane offset
+    // (the first functions and the address below are made opaque here, so that
+    // the rows' addresses and the density block do not occupy scalar
+    // registers throughout the primitive loops)
+    int32_t fbA = fix.bfA, fbB = fix.bfB;
+    const double *dfix_a = ba.Dp + cd.fix_base + ifix;
+    asm volatile("" : "+s"(fbA), "+s"(fbB), "+s"(dfix_a));
+    ConstDouble *dfix_p = const_view(dfix_a);
+    double dfix[NFIX];  // the fixed pair's Coulomb density block
 #pragma unroll
-    for (int c = 0; c < NC; ++c) gc[c] = ket.bfA + gamess_pos(rc.lx[c], rc.ly[c], rc.lz[c]);
-#pragma unroll
-    for (int d = 0; d < ND; ++d) gd[d] = ket.bfB + gamess_pos(rd.lx[d], rd.ly[d], rd.lz[d]);
+    for (int k = 0; k < NFIX; ++k) dfix[k] = dfix_p[(int64_t)k * cd.fix_n];
+    auto dka = [&](int i, uint32_t mo) -> double {
+      return dens_at(ba.Dsq, (int64_t)(fbA + gamess_pos(r1.lx[i], r1.ly[i], r1.lz[i])) * ba.nbf, mo);
+    };
+    auto dkb = [&](int j, uint32_t mo) -> double {
+      return dens_at(ba.Dsq, (int64_t)(fbB + gamess_pos(r2.lx[j], r2.ly[j], r2.lz[j])) * ba.nbf, mo);
+    };
     // compact columns of the moving pair's functions
     int cm1[R::NM1], cm2[R::NM2];
 #pragma unroll
@@ -895,7 +920,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int d = 0; d < ND; ++d) dcd[c * ND + d] = Dm[tri(gc[c], gd[d])];
+        for (int d = 0; d < ND; ++d) dcd[c * ND + d] = ba.Dp[cd.mov_base + (int64_t)(c * ND + d) * cd.mov_n + imov];
 #pragma unroll
       for (int ab = 0; ab < NA * NB; ++ab) {
         double t = 0.0;
@@ -908,14 +933,14 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
         double t = 0.0;
 #pragma unroll
         for (int ab = 0; ab < NA * NB; ++ab) t += v[ab * NC * ND + k] * dfix[ab];
-        if (t != 0.0) fock_add(F, gc[k / ND], gd[k % ND], 4.0 * s * t);
+        unsafeAtomicAdd(ba.Jp + cd.mov_base + (int64_t)k * cd.mov_n + imov, 4.0 * s * t);
       }
     } else {
       double dab[NA * NB];
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) dab[a * NB + b] = Dm[tri(ga[a], gb[b])];
+        for (int b = 0; b < NB; ++b) dab[a * NB + b] = ba.Dp[cd.mov_base + (int64_t)(a * NB + b) * cd.mov_n + imov];
 #pragma unroll
       for (int k = 0; k < NC * ND; ++k) {
         double t = 0.0;
@@ -928,7 +953,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
         double t = 0.0;
 #pragma unroll
         for (int k = 0; k < NC * ND; ++k) t += v[ab * NC * ND + k] * dfix[k];
-        if (t != 0.0) fock_add(F, ga[ab / NB], gb[ab % NB], 4.0 * s * t);
+        unsafeAtomicAdd(ba.Jp + cd.mov_base + (int64_t)ab * cd.mov_n + imov, 4.0 * s * t);
       }
     }
     const double sk = s * ba.k_scale;
@@ -938,11 +963,11 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int d = 0; d < ND; ++d) dbd[b * ND + d] = Dk[tri(gb[b], gd[d])];
+        for (int d = 0; d < ND; ++d) dbd[b * ND + d] = TR ? dkb(d, mo2[b]) : dkb(b, mo2[d]);
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) dac[a * NC + c] = Dk[tri(ga[a], gc[c])];
+        for (int c = 0; c < NC; ++c) dac[a * NC + c] = TR ? dka(c, mo1[a]) : dka(a, mo1[c]);
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
@@ -952,7 +977,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
           for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int d = 0; d < ND; ++d) t += v[((a * NB + b) * NC + c) * ND + d] * dbd[b * ND + d];
-          if (t != 0.0) lds_add(TR ? &rows[c * ncols + cm1[a]] : &rows[a * ncols + cm1[c]], -sk * t);
+          lds_add(TR ? &rows[c * ncols + cm1[a]] : &rows[a * ncols + cm1[c]], -sk * t);
         }
 #pragma unroll
       for (int b = 0; b < NB; ++b)
@@ -963,7 +988,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
           for (int a = 0; a < NA; ++a)
 #pragma unroll
             for (int c = 0; c < NC; ++c) t += v[((a * NB + b) * NC + c) * ND + d] * dac[a * NC + c];
-          if (t != 0.0) lds_add(TR ? &rows[(NC + d) * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm2[d]], -sk * t);
+          lds_add(TR ? &rows[(NC + d) * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm2[d]], -sk * t);
         }
     }
     // exchange: K(AD) and K(BC)
@@ -972,11 +997,11 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) dbc[b * NC + c] = Dk[tri(gb[b], gc[c])];
+        for (int c = 0; c < NC; ++c) dbc[b * NC + c] = TR ? dka(c, mo2[b]) : dkb(b, mo1[c]);
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int d = 0; d < ND; ++d) dad[a * ND + d] = Dk[tri(ga[a], gd[d])];
+        for (int d = 0; d < ND; ++d) dad[a * ND + d] = TR ? dkb(d, mo1[a]) : dka(a, mo2[d]);
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
@@ -986,7 +1011,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
           for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int c = 0; c < NC; ++c) t += v[((a * NB + b) * NC + c) * ND + d] * dbc[b * NC + c];
-          if (t != 0.0) lds_add(TR ? &rows[(NC + d) * ncols + cm1[a]] : &rows[a * ncols + cm2[d]], -sk * t);
+          lds_add(TR ? &rows[(NC + d) * ncols + cm1[a]] : &rows[a * ncols + cm2[d]], -sk * t);
         }
 #pragma unroll
       for (int b = 0; b < NB; ++b)
@@ -997,7 +1022,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
           for (int a = 0; a < NA; ++a)
 #pragma unroll
             for (int d = 0; d < ND; ++d) t += v[((a * NB + b) * NC + c) * ND + d] * dad[a * ND + d];
-          if (t != 0.0) lds_add(TR ? &rows[c * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm1[c]], -sk * t);
+          lds_add(TR ? &rows[c * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm1[c]], -sk * t);
         }
     }
   }
@@ -1008,7 +1033,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
   __syncthreads();
   for (int i = threadIdx.x; i < NFIX; i += blockDim.x) {
     const double x = jfix_s[i];
-    if (x != 0.0) fock_add(F, fix.bfA + gpos_of(R::L1, i / N2), fix.bfB + gpos_of(R::L2, i % N2), x);
+    if (x != 0.0) unsafeAtomicAdd(ba.Jp + cd.fix_base + (int64_t)i * cd.fix_n + ifix, x);
   }
   for (int i = threadIdx.x; i < NROW * ncols; i += blockDim.x) {
     const double x = rows[i];
@@ -1016,7 +1041,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void eri_row_kerne
     const int r = i / ncols, k = i - r * ncols;
     const int rbf = r < N1 ? fix.bfA + gpos_of(R::L1, r) : fix.bfB + gpos_of(R::L2, r - N1);
     const int cbf = (R::M1 == R::M2 || k < off2) ? ba.col_bf[R::M1][k] : ba.col_bf[R::M2][k - off2];
-    fock_add(F, rbf, cbf, x);
+    fock_add(ba.F, rbf, cbf, x);
   }
 }
 
@@ -1212,13 +1237,13 @@ __device__ __forceinline__ void split_integrals(const PairRec &bra, const PairRe
   ConstPrimRec *cprims = const_view(prims);
   if constexpr (KET_OUTER) {
     for (int iq = 0; iq < ket.nprim; ++iq) {
-      const PrimRec Q = prims[ket.prim_off + iq];
-      for (int ip = 0; ip < bra.nprim; ++ip) prim(load_rec(cprims, bra.prim_off + ip), Q);
+      const PrimRec Q = prims[ket.prim_off + iq * ket.prim_stride];
+      for (int ip = 0; ip < bra.nprim; ++ip) prim(load_rec(cprims, bra.prim_off + ip * bra.prim_stride), Q);
     }
   } else {
     for (int ip = 0; ip < bra.nprim; ++ip) {
-      const PrimRec Pp = prims[bra.prim_off + ip];
-      for (int iq = 0; iq < ket.nprim; ++iq) prim(Pp, load_rec(cprims, ket.prim_off + iq));
+      const PrimRec Pp = prims[bra.prim_off + ip * bra.prim_stride];
+      for (int iq = 0; iq < ket.nprim; ++iq) prim(Pp, load_rec(cprims, ket.prim_off + iq * ket.prim_stride));
     }
   }
 
@@ -1296,8 +1321,9 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
   constexpr Range<R::M2, R::M2> rm2{};
   // this part's share of the fixed pair's Coulomb block
   constexpr int NJ = TR ? NCP * NDP : NAP * NB;
-  const double *Dm = ba.D, *Dk = ba.DK;
-  double *F = ba.F;
+  constexpr Range<R::L1, R::L1> r1{};
+  constexpr Range<R::L2, R::L2> r2{};
+  (void)ra, (void)rb, (void)rc, (void)rd;
   const double sfix = fix.sameAB ? 0.5 : 1.0;
   const int lane = threadIdx.x & 63;
   int sg = seg0;
@@ -1308,7 +1334,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
     for (int k = 0; k < NJ; ++k) jf[k] = 0.0;
     if (q < q1) {
       while (sg + 1 < cd.nseg && cd.seg_start[sg + 1] <= q) ++sg;
-      const int32_t imov = cd.ket_list[cd.seg_ket0[sg] + (int32_t)(q - cd.seg_start[sg])];
+      const int32_t imov = cd.seg_ket0[sg] + (int32_t)(q - cd.seg_start[sg]);
       const PairRec mov = ba.pairs[imov];
       const PairRec &bra = TR ? mov : fix;
       const PairRec &ket = TR ? fix : mov;
@@ -1318,15 +1344,23 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
       double s = sfix;
       if (mov.sameAB) s *= 0.5;
       if (cd.diag && ifix == imov) s *= 0.5;
-      int ga[NAP], gb[NB], gc[NCP], gd[NDP];
+      // byte offsets of the moving pair's functions in a row of the square
+      // exchange density
+      uint32_t mo1[NM1], mo2[NM2];
 #pragma unroll
-      for (int a = 0; a < NAP; ++a) ga[a] = bra.bfA + gamess_pos(ra.lx[A0 + a], ra.ly[A0 + a], ra.lz[A0 + a]);
+      for (int i = 0; i < NM1; ++i)
+        mo1[i] = 8u * (mov.bfA + gamess_pos(rm1.lx[M10 + i], rm1.ly[M10 + i], rm1.lz[M10 + i]));
 #pragma unroll
-      for (int b = 0; b < NB; ++b) gb[b] = bra.bfB + gamess_pos(rb.lx[b], rb.ly[b], rb.lz[b]);
-#pragma unroll
-      for (int c = 0; c < NCP; ++c) gc[c] = ket.bfA + gamess_pos(rc.lx[C0 + c], rc.ly[C0 + c], rc.lz[C0 + c]);
-#pragma unroll
-      for (int d = 0; d < NDP; ++d) gd[d] = ket.bfB + gamess_pos(rd.lx[D0 + d], rd.ly[D0 + d], rd.lz[D0 + d]);
+      for (int i = 0; i < NM2; ++i)
+        mo2[i] = 8u * (mov.bfB + gamess_pos(rm2.lx[M20 + i], rm2.ly[M20 + i], rm2.lz[M20 + i]));
+      // exchange density of component i of the fixed pair's shell A (B) with
+      // the function at byte offset mo: a uniform row and a lane offset
+      auto dka = [&](int i, uint32_t mo) -> double {
+        return dens_at(ba.Dsq, (int64_t)(fix.bfA + gamess_pos(r1.lx[i], r1.ly[i], r1.lz[i])) * ba.nbf, mo);
+      };
+      auto dkb = [&](int j, uint32_t mo) -> double {
+        return dens_at(ba.Dsq, (int64_t)(fix.bfB + gamess_pos(r2.lx[j], r2.ly[j], r2.lz[j])) * ba.nbf, mo);
+      };
       int cm1[NM1], cm2[NM2];
 #pragma unroll
       for (int i = 0; i < NM1; ++i) cm1[i] = mov.cA + gamess_pos(rm1.lx[M10 + i], rm1.ly[M10 + i], rm1.lz[M10 + i]);
@@ -1340,7 +1374,8 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
 #pragma unroll
         for (int c = 0; c < NCP; ++c)
 #pragma unroll
-          for (int d = 0; d < NDP; ++d) dcd[c * NDP + d] = Dm[tri(gc[c], gd[d])];
+          for (int d = 0; d < NDP; ++d) 
+            dcd[c * NDP + d] = ba.Dp[cd.mov_base + (int64_t)((C0 + c) * ND + D0 + d) * cd.mov_n + imov];
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
@@ -1361,14 +1396,15 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
             for (int a = 0; a < NAP; ++a)
 #pragma unroll
               for (int b = 0; b < NB; ++b) t += V(a, b, c, d) * dfix_s[(A0 + a) * NB + b];
-            if (t != 0.0) fock_add(F, gc[c], gd[d], 4.0 * s * t);
+            unsafeAtomicAdd(ba.Jp + cd.mov_base + (int64_t)((C0 + c) * ND + D0 + d) * cd.mov_n + imov, 4.0 * s * t);
           }
       } else {
         double dab[NAP * NB];
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
-          for (int b = 0; b < NB; ++b) dab[a * NB + b] = Dm[tri(ga[a], gb[b])];
+          for (int b = 0; b < NB; ++b) 
+            dab[a * NB + b] = ba.Dp[cd.mov_base + (int64_t)((A0 + a) * NB + b) * cd.mov_n + imov];
 #pragma unroll
         for (int c = 0; c < NCP; ++c)
 #pragma unroll
@@ -1389,7 +1425,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
             for (int c = 0; c < NCP; ++c)
 #pragma unroll
               for (int d = 0; d < NDP; ++d) t += V(a, b, c, d) * dfix_s[(C0 + c) * ND + D0 + d];
-            if (t != 0.0) fock_add(F, ga[a], gb[b], 4.0 * s * t);
+            unsafeAtomicAdd(ba.Jp + cd.mov_base + (int64_t)((A0 + a) * NB + b) * cd.mov_n + imov, 4.0 * s * t);
           }
       }
       const double sk = s * ba.k_scale;
@@ -1399,11 +1435,11 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-          for (int d = 0; d < NDP; ++d) dbd[b * NDP + d] = Dk[tri(gb[b], gd[d])];
+          for (int d = 0; d < NDP; ++d) dbd[b * NDP + d] = TR ? dkb(D0 + d, mo2[b]) : dkb(b, mo2[d]);
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
-          for (int c = 0; c < NCP; ++c) dac[a * NCP + c] = Dk[tri(ga[a], gc[c])];
+          for (int c = 0; c < NCP; ++c) dac[a * NCP + c] = TR ? dka(C0 + c, mo1[a]) : dka(A0 + a, mo1[c]);
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
@@ -1413,8 +1449,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
             for (int b = 0; b < NB; ++b)
 #pragma unroll
               for (int d = 0; d < NDP; ++d) t += V(a, b, c, d) * dbd[b * NDP + d];
-            if (t != 0.0)
-              lds_add(TR ? &rows[(C0 + c) * ncols + cm1[a]] : &rows[(A0 + a) * ncols + cm1[c]], -sk * t);
+            lds_add(TR ? &rows[(C0 + c) * ncols + cm1[a]] : &rows[(A0 + a) * ncols + cm1[c]], -sk * t);
           }
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -1425,7 +1460,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
             for (int a = 0; a < NAP; ++a)
 #pragma unroll
               for (int c = 0; c < NCP; ++c) t += V(a, b, c, d) * dac[a * NCP + c];
-            if (t != 0.0) lds_add(TR ? &rows[(NC + D0 + d) * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm2[d]], -sk * t);
+            lds_add(TR ? &rows[(NC + D0 + d) * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm2[d]], -sk * t);
           }
       }
       // exchange: K(AD) and K(BC)
@@ -1434,11 +1469,11 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-          for (int c = 0; c < NCP; ++c) dbc[b * NCP + c] = Dk[tri(gb[b], gc[c])];
+          for (int c = 0; c < NCP; ++c) dbc[b * NCP + c] = TR ? dka(C0 + c, mo2[b]) : dkb(b, mo1[c]);
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
-          for (int d = 0; d < NDP; ++d) dad[a * NDP + d] = Dk[tri(ga[a], gd[d])];
+          for (int d = 0; d < NDP; ++d) dad[a * NDP + d] = TR ? dkb(D0 + d, mo1[a]) : dka(A0 + a, mo2[d]);
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
@@ -1448,7 +1483,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
             for (int b = 0; b < NB; ++b)
 #pragma unroll
               for (int c = 0; c < NCP; ++c) t += V(a, b, c, d) * dbc[b * NCP + c];
-            if (t != 0.0) lds_add(TR ? &rows[(NC + D0 + d) * ncols + cm1[a]] : &rows[(A0 + a) * ncols + cm2[d]], -sk * t);
+            lds_add(TR ? &rows[(NC + D0 + d) * ncols + cm1[a]] : &rows[(A0 + a) * ncols + cm2[d]], -sk * t);
           }
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -1459,7 +1494,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
             for (int a = 0; a < NAP; ++a)
 #pragma unroll
               for (int d = 0; d < NDP; ++d) t += V(a, b, c, d) * dad[a * NDP + d];
-            if (t != 0.0) lds_add(TR ? &rows[(C0 + c) * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm1[c]], -sk * t);
+            lds_add(TR ? &rows[(C0 + c) * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm1[c]], -sk * t);
           }
       }
     }
@@ -1503,7 +1538,7 @@ template <int LA, int LB, int LC, int LD, bool TR>
 __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_kernel(ClassDev cd, BuildArgs ba) {
   using P = SplitShape<LA, LB, LC, LD>;
   using R = RowShape<LA, LB, LC, LD, TR>;
-  constexpr int N1 = R::N1, N2 = R::N2, NFIX = R::NFIX, NROW = R::NROW;
+  constexpr int N1 = R::N1, NFIX = R::NFIX, NROW = R::NROW;
   extern __shared__ double lds[];
   double *jfix_s = lds, *dfix_s = lds + NFIX, *rows = lds + 2 * NFIX;
   const int ncols = (int)row_columns<LA, LB, LC, LD, TR>(ba.ncol);
@@ -1515,15 +1550,14 @@ __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_ke
     const double *src = rys_table + rys_offset[P::NR];
     for (int i = threadIdx.x; i < ntab; i += blockDim.x) tab[(i / IN) * LS + i % IN] = src[i];
   }
-  const int tile = cd.t_begin + (int)blockIdx.x;
-  const int64_t q0 = cd.tile_q[tile] > cd.q_begin ? cd.tile_q[tile] : cd.q_begin;
-  const int64_t q1 = cd.tile_q[tile + 1] < cd.q_end ? cd.tile_q[tile + 1] : cd.q_end;
-  const int seg0 = cd.tile_seg[tile];
+  const RowTile tl = cd.tiles[blockIdx.x];
+  const int64_t q0 = tl.q0, q1 = q0 + tl.n;
+  const int seg0 = tl.seg;
   const int32_t ifix = cd.seg_bra[seg0];
   const PairRec fix = load_rec(const_view(ba.pairs), ifix);
   for (int i = threadIdx.x; i < NFIX; i += blockDim.x) {
     jfix_s[i] = 0.0;
-    dfix_s[i] = ba.D[tri(fix.bfA + gpos_of(R::L1, i / N2), fix.bfB + gpos_of(R::L2, i % N2))];
+    dfix_s[i] = ba.Dp[cd.fix_base + (int64_t)i * cd.fix_n + ifix];
   }
   for (int i = threadIdx.x; i < NROW * ncols; i += blockDim.x) rows[i] = 0.0;
   __syncthreads();
@@ -1534,10 +1568,9 @@ __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_ke
                                         rows, ncols, off2, tab);
   __syncthreads();
 
-  double *F = ba.F;
   for (int i = threadIdx.x; i < NFIX; i += blockDim.x) {
     const double x = jfix_s[i];
-    if (x != 0.0) fock_add(F, fix.bfA + gpos_of(R::L1, i / N2), fix.bfB + gpos_of(R::L2, i % N2), x);
+    if (x != 0.0) unsafeAtomicAdd(ba.Jp + cd.fix_base + (int64_t)i * cd.fix_n + ifix, x);
   }
   for (int i = threadIdx.x; i < NROW * ncols; i += blockDim.x) {
     const double x = rows[i];
@@ -1545,7 +1578,7 @@ __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_ke
     const int r = i / ncols, k = i - r * ncols;
     const int rbf = r < N1 ? fix.bfA + gpos_of(R::L1, r) : fix.bfB + gpos_of(R::L2, r - N1);
     const int cbf = (R::M1 == R::M2 || k < off2) ? ba.col_bf[R::M1][k] : ba.col_bf[R::M2][k - off2];
-    fock_add(F, rbf, cbf, x);
+    fock_add(ba.F, rbf, cbf, x);
   }
 }
 
@@ -1730,8 +1763,8 @@ __global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT)) void eri_coop_kernel(Cl
     for (int ip = 0; ip < bra.nprim; ++ip) {
       for (int iq = 0; iq < ket.nprim; ++iq) {
         if (t < 3 * NR) {
-          const PrimRec P = ba.prims[bra.prim_off + ip];
-          const PrimRec Q = ba.prims[ket.prim_off + iq];
+          const PrimRec P = ba.prims[bra.prim_off + ip * bra.prim_stride];
+          const PrimRec Q = ba.prims[ket.prim_off + iq * ket.prim_stride];
           const int r = t / 3, dim = t - 3 * (t / 3);
           const double pq = P.p + Q.p, ipq = 1.0 / pq;
           const double pqx = P.Px - Q.Px, pqy = P.Py - Q.Py, pqz = P.Pz - Q.Pz;
@@ -2344,7 +2377,7 @@ __device__ __forceinline__ int gpos_of(int L, int k) {
 // 2 waves without spill.
 template <int LA, int LB, int LC, int LD>
 __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba, int64_t c0, int64_t c1,
-                                        double *lds, int *s_npq, int *s_nk, int *s_boff, int *s_koff) {
+                                        double *lds, int *s_npq, int *s_nk, int *s_boff, int *s_koff, int *s_bst, int *s_kst) {
   using S = Grp<LA, LB, LC, LD>;
   constexpr int G = S::G, NQ = S::NQ, NR = S::NR, NI = S::NI, NK = S::NK, NE = S::NE, NF = S::NF, NKC = S::NKC;
   constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND, NABCD = S::NABCD;
@@ -2420,6 +2453,8 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
       s_nk[slot] = nk;
       s_boff[slot] = bra.prim_off;
       s_koff[slot] = ket.prim_off;
+      s_bst[slot] = bra.prim_stride;
+      s_kst[slot] = ket.prim_stride;
     }
     wave_sync();
     int maxpq = 0;
@@ -2442,8 +2477,8 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
         // t / nka in FP32: both are small integers, the quotient's fraction
         // stays >= 0.5/nka away from an integer, far above the rounding error
         const int ip = (int)(((float)t + 0.5f) * __builtin_amdgcn_rcpf((float)nka)), iq = t - ip * nka;
-        const PrimRec P = ba.prims[s_boff[sa] + ip];
-        const PrimRec Q = ba.prims[s_koff[sa] + iq];
+        const PrimRec P = ba.prims[s_boff[sa] + ip * s_bst[sa]];
+        const PrimRec Q = ba.prims[s_koff[sa] + iq * s_kst[sa]];
         const double rs = nr_rsqrt(P.p + Q.p), ipq = rs * rs;
         const double pqx = P.Px - Q.Px, pqy = P.Py - Q.Py, pqz = P.Pz - Q.Pz;
         const double X = P.p * Q.p * ipq * (pqx * pqx + pqy * pqy + pqz * pqz);
@@ -2949,7 +2984,7 @@ __global__ __launch_bounds__(64) void eri_group_kernel(ClassDev cd, BuildArgs ba
   using S = Grp<LA, LB, LC, LD>;
   constexpr int NQ = S::NQ;
   __shared__ double lds[NQ * S::SLOT];
-  __shared__ int s_npq[NQ], s_nk[NQ], s_boff[NQ], s_koff[NQ];
+  __shared__ int s_npq[NQ], s_nk[NQ], s_boff[NQ], s_koff[NQ], s_bst[NQ], s_kst[NQ];
   // a contiguous chunk of the class's quartets per workgroup (a multiple of
   // NQ).  Workgroups resident at the same time take chunks spread over the
   // whole quartet range (chunk = workgroup x chunk_stride(grid) mod grid, a
@@ -2958,11 +2993,11 @@ __global__ __launch_bounds__(64) void eri_group_kernel(ClassDev cd, BuildArgs ba
   const int64_t per = ((nq + gridDim.x - 1) / gridDim.x + NQ - 1) / NQ * NQ;
   const int64_t chunk = (int64_t)blockIdx.x * cd.chunk_stride % gridDim.x;
   const int64_t c0 = chunk * per, c1 = c0 + per < nq ? c0 + per : nq;
-  grp_run<LA, LB, LC, LD>(cd, ba, c0, c1, lds, s_npq, s_nk, s_boff, s_koff);
+  grp_run<LA, LB, LC, LD>(cd, ba, c0, c1, lds, s_npq, s_nk, s_boff, s_koff, s_bst, s_kst);
 }
 
 // ----------------------------------------------------- segment lengths
-#if !defined(LIBERI_CLASS_GROUP) || LIBERI_CLASS_GROUP == -1 || LIBERI_CLASS_GROUP == -2
+#if LIBERI_UNIT == -1 || LIBERI_UNIT == -2
 __global__ void segment_lengths_kernel(const double *bra_x, const int32_t *bra_group, const int32_t *bra_pos,
                                        int32_t nbra, const double *ket_x, const int32_t *gbeg, const int32_t *gend,
                                        int32_t ngroup, int32_t diag, int32_t cmp, double cut, int64_t *seg_len) {
@@ -3121,7 +3156,69 @@ int launch_schwarz(int la, int lb, const PairRec *pairs, const PrimRec *prims, c
   }
 }
 
-// F = 0 as a kernel (not a memset node) so that a build can be captured in a graph
+// Calls f(element, pair, a, b) for this thread's elements of the pair layout:
+// workgroup blk covers a run of pairs of one class and one component (a, b),
+// so nothing of the decoding is per lane.
+template <class Body>
+__device__ __forceinline__ void for_pair_layout(const PairLayout &pl, int blk, Body f) {
+  int c = 0;
+  while (blk >= pl.block[c + 1]) ++c;
+  const int comp = (blk - pl.block[c]) / pl.chunks[c], chunk = (blk - pl.block[c]) - comp * pl.chunks[c];
+  const int lb = kPairL[c][0], nb = (lb + 1) * (lb + 2) / 2, a = comp / nb, b = comp - a * nb;
+  for (int i = chunk * 256 + (int)threadIdx.x; i < pl.n[c]; i += pl.chunks[c] * 256)
+    f(pl.off[c] + (int64_t)comp * pl.n[c] + i, pl.first[c] + i, c, a, b);
+}
+
+// Start of a build: F and the Coulomb sums by pair zeroed, the Coulomb
+// density by pair and the square exchange density filled from the packed
+// ones.  A kernel (not memset nodes), so that a build can be captured in a
+// graph.  The first nbf workgroups take a row of F and of the square density
+// each, the others the pair layout.
+__global__ __launch_bounds__(256) void build_begin_kernel(const PairRec *pairs, PairLayout pl, const double *D,
+                                                          const double *DK, int32_t nbf, double *F, double *Jp,
+                                                          double *Dp, double *Dsq) {
+  if ((int)blockIdx.x < nbf) {
+    const uint32_t r = blockIdx.x;
+    const int64_t row = (int64_t)r * (r + 1) / 2;
+    for (uint32_t k = threadIdx.x; k <= r; k += 256) F[row + k] = 0.0;
+    for (uint32_t k = threadIdx.x; k < (uint32_t)nbf; k += 256) Dsq[(int64_t)r * nbf + k] = DK[tri(r, k)];
+    return;
+  }
+  for_pair_layout(pl, (int)blockIdx.x - nbf, [&](int64_t e, int p, int c, int a, int b) {
+    Dp[e] = D[tri(pairs[p].bfA + gpos_rt(kPairL[c][1], a), pairs[p].bfB + gpos_rt(kPairL[c][0], b))];
+    Jp[e] = 0.0;
+  });
+}
+
+// End of a build: the Coulomb sums by pair added to F.  Every element of F
+// belongs to one shell pair; a pair of one shell holds (a, b) and (b, a),
+// both added by the thread of a >= b.
+__global__ __launch_bounds__(256) void build_end_kernel(const PairRec *pairs, PairLayout pl, const double *Jp,
+                                                        double *F) {
+  for_pair_layout(pl, (int)blockIdx.x, [&](int64_t e, int p, int c, int a, int b) {
+    double x = Jp[e];
+    if (pairs[p].sameAB) {
+      const int nb = (kPairL[c][0] + 1) * (kPairL[c][0] + 2) / 2;
+      if (a < b) return;
+      if (a > b) x += Jp[e + (int64_t)(b * nb + a - (a * nb + b)) * pl.n[c]];
+    }
+    F[tri(pairs[p].bfA + gpos_rt(kPairL[c][1], a), pairs[p].bfB + gpos_rt(kPairL[c][0], b))] += x;
+  });
+}
+
+int launch_build_begin(const BuildArgs &ba, const PairLayout &pl, double *Dp, double *Dsq, void *stream) {
+  hipLaunchKernelGGL(build_begin_kernel, dim3((unsigned)(ba.nbf + pl.block[kNumPairClasses])), dim3(256), 0,
+                     (hipStream_t)stream, ba.pairs, pl, ba.D, ba.DK, ba.nbf, ba.F, ba.Jp, Dp, Dsq);
+  return hipGetLastError();
+}
+
+int launch_build_end(const BuildArgs &ba, const PairLayout &pl, void *stream) {
+  hipLaunchKernelGGL(build_end_kernel, dim3((unsigned)pl.block[kNumPairClasses]), dim3(256), 0, (hipStream_t)stream,
+                     ba.pairs, pl, ba.Jp, ba.F);
+  return hipGetLastError();
+}
+
+// p = 0 as a kernel (not a memset node) so that it can be captured in a graph
 __global__ void fill_zero_kernel(double *p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     p[i] = 0.0;
@@ -3233,8 +3330,8 @@ constexpr bool has_coop_alt() {
 template <int LA, int LB, int LC, int LD, bool TR>
 static int launch_row(const ClassDev &cd, const BuildArgs &ba, hipStream_t st) {
   const int64_t lds = row_lds<LA, LB, LC, LD, TR>(ba.ncol, cd.xswitch);
-  if (lds < 0 || cd.t_end <= cd.t_begin) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(cd.t_end - cd.t_begin));
+  if (lds < 0 || cd.ntile <= 0) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)cd.ntile);
   if constexpr (!RowShape<LA, LB, LC, LD, TR>::exists) {
     return hipErrorInvalidValue;
   } else if constexpr (use_small<LA, LB, LC, LD>() && !SplitShape<LA, LB, LC, LD>::exists) {
@@ -3331,20 +3428,11 @@ static int64_t scratch_one() {
   X(46, 3, 2, 3, 1) X(47, 3, 2, 3, 2) X(48, 3, 3, 0, 0) X(49, 3, 3, 1, 0) X(50, 3, 3, 1, 1)               \
   X(51, 3, 3, 2, 0) X(52, 3, 3, 2, 1) X(53, 3, 3, 2, 2) X(54, 3, 3, 3, 2)
 
-// The 55 instantiations are spread over LIBERI_CLASS_GROUPS translation units
-// (class id modulo the group count) so they compile in parallel; the unit
-// built with LIBERI_CLASS_GROUP=-1 holds the dispatcher and the common
-// kernels, the one built with -3 the fused group launch; without the macro
-// one unit holds everything.
-#define LIBERI_CLASS_LIST_G0(X) X(0, 0, 0, 0, 0) X(8, 1, 0, 2, 0) X(16, 2, 1, 2, 0) X(24, 0, 0, 3, 2) X(32, 3, 1, 1, 0) X(40, 3, 3, 3, 1) X(48, 3, 3, 0, 0)
-#define LIBERI_CLASS_LIST_G1(X) X(1, 0, 0, 1, 0) X(9, 1, 0, 2, 1) X(17, 2, 1, 1, 1) X(25, 1, 0, 3, 0) X(33, 3, 1, 1, 1) X(41, 3, 2, 1, 1) X(49, 3, 3, 1, 0)
-#define LIBERI_CLASS_LIST_G2(X) X(2, 0, 0, 1, 1) X(10, 0, 0, 2, 2) X(18, 2, 2, 2, 0) X(26, 3, 3, 3, 0) X(34, 3, 1, 2, 0) X(42, 3, 2, 2, 0) X(50, 3, 3, 1, 1)
-#define LIBERI_CLASS_LIST_G3(X) X(3, 1, 0, 1, 1) X(11, 1, 0, 2, 2) X(19, 2, 2, 2, 1) X(27, 3, 0, 1, 1) X(35, 3, 1, 2, 1) X(43, 3, 2, 2, 1) X(51, 3, 3, 2, 0)
-#define LIBERI_CLASS_LIST_G4(X) X(4, 1, 0, 1, 0) X(12, 1, 1, 2, 0) X(20, 2, 2, 2, 2) X(28, 3, 0, 2, 0) X(36, 2, 2, 3, 1) X(44, 3, 2, 2, 2) X(52, 3, 3, 2, 1)
-#define LIBERI_CLASS_LIST_G5(X) X(5, 1, 1, 1, 1) X(13, 2, 0, 2, 0) X(21, 3, 3, 3, 3) X(29, 2, 1, 3, 0) X(37, 3, 1, 3, 0) X(45, 3, 2, 3, 0) X(53, 3, 3, 2, 2)
-#define LIBERI_CLASS_LIST_G6(X) X(6, 0, 0, 2, 0) X(14, 2, 2, 1, 1) X(22, 0, 0, 3, 0) X(30, 2, 2, 3, 0) X(38, 3, 1, 3, 1) X(46, 3, 2, 3, 1) X(54, 3, 3, 3, 2)
-#define LIBERI_CLASS_LIST_G7(X) X(7, 0, 0, 2, 1) X(15, 2, 1, 2, 1) X(23, 0, 0, 3, 1) X(31, 3, 0, 3, 0) X(39, 3, 2, 1, 0) X(47, 3, 2, 3, 2)
-
+// The 55 instantiations are spread over several translation units that
+// compile in parallel: a unit built with LIBERI_UNIT=1 instantiates the
+// classes of the list it is given (LIBERI_UNIT_LIST, entries as above), the
+// unit -1 holds the dispatcher and the common kernels, the unit -3 the fused
+// group launch; without the macro (-2) one unit holds everything.
 #define DECL_CLASS(id, a, b, cc, d)                                                       \
   int launch_class_##id(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, int nwg); \
   int64_t scratch_class_##id();                                                            \
@@ -3359,32 +3447,20 @@ LIBERI_CLASS_LIST(DECL_CLASS)
   int64_t scratch_class_##id() { return scratch_one<a, b, cc, d>(); }                      \
   int prepare_class_##id() { return prepare_one<a, b, cc, d>(); }
 
-#ifndef LIBERI_CLASS_GROUP
-#define LIBERI_CLASS_GROUP -2
-#endif
-#if LIBERI_CLASS_GROUP == 0 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G0(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 1 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G1(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 2 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G2(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 3 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G3(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 4 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G4(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 5 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G5(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 6 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G6(DEF_CLASS)
-#endif
-#if LIBERI_CLASS_GROUP == 7 || LIBERI_CLASS_GROUP == -2
-LIBERI_CLASS_LIST_G7(DEF_CLASS)
+#if LIBERI_UNIT == -2
+LIBERI_CLASS_LIST(DEF_CLASS)
+#elif LIBERI_UNIT > 0
+constexpr bool class_is(int a, int b, int c, int d, int e) {
+#define X(id, la, lb, lc, ld) \
+  if (a == id) return b == la && c == lb && d == lc && e == ld;
+  LIBERI_CLASS_LIST(X)
+#undef X
+  return false;
+}
+#define X(id, la, lb, lc, ld) static_assert(class_is(id, la, lb, lc, ld), "angular momenta of the class");
+LIBERI_UNIT_LIST(X)
+#undef X
+LIBERI_UNIT_LIST(DEF_CLASS)
 #endif
 #undef DEF_CLASS
 
@@ -3398,7 +3474,7 @@ LIBERI_CLASS_LIST_G7(DEF_CLASS)
 #define LIBERI_FUSED_LIST(X) \
   X(11, 1, 0, 2, 2) X(14, 2, 2, 1, 1) X(15, 2, 1, 2, 1) X(16, 2, 1, 2, 0) X(17, 2, 1, 1, 1) X(18, 2, 2, 2, 0) X(19, 2, 2, 2, 1)
 
-#if LIBERI_CLASS_GROUP == -3 || LIBERI_CLASS_GROUP == -2
+#if LIBERI_UNIT == -3 || LIBERI_UNIT == -2
 constexpr int fused_lds_doubles() {
   int m = 0;
 #define X(id, a, b, cc, d) m = Grp<a, b, cc, d>::NQ * Grp<a, b, cc, d>::SLOT > m ? Grp<a, b, cc, d>::NQ * Grp<a, b, cc, d>::SLOT : m;
@@ -3424,14 +3500,14 @@ LIBERI_FUSED_LIST(X)
 // own register allocation instead of one allocation over all of them
 template <int LA, int LB, int LC, int LD>
 __device__ __noinline__ void grp_run_item(const ClassDev &cd, const BuildArgs &ba, int64_t c0, int64_t c1,
-                                          double *lds, int *s_npq, int *s_nk, int *s_boff, int *s_koff) {
-  grp_run<LA, LB, LC, LD>(cd, ba, c0, c1, lds, s_npq, s_nk, s_boff, s_koff);
+                                          double *lds, int *s_npq, int *s_nk, int *s_boff, int *s_koff, int *s_bst, int *s_kst) {
+  grp_run<LA, LB, LC, LD>(cd, ba, c0, c1, lds, s_npq, s_nk, s_boff, s_koff, s_bst, s_kst);
 }
 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void eri_group_fused_kernel(
     const ClassDev *cds, BuildArgs ba, const FusedItem *items, int64_t nitems, unsigned long long *head) {
   __shared__ double lds[fused_lds_doubles()];
-  __shared__ int s_npq[fused_nq()], s_nk[fused_nq()], s_boff[fused_nq()], s_koff[fused_nq()];
+  __shared__ int s_npq[fused_nq()], s_nk[fused_nq()], s_boff[fused_nq()], s_koff[fused_nq()], s_bst[fused_nq()], s_kst[fused_nq()];
   for (;;) {
     unsigned long long it = 0;
     if (threadIdx.x == 0) it = atomicAdd(head, 1ull);
@@ -3441,7 +3517,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     switch (w.cls) {
 #define X(id, a, b, cc, d)                                                                 \
   case id:                                                                                 \
-    grp_run_item<a, b, cc, d>(cds[id], ba, w.c0, w.c1, lds, s_npq, s_nk, s_boff, s_koff); \
+    grp_run_item<a, b, cc, d>(cds[id], ba, w.c0, w.c1, lds, s_npq, s_nk, s_boff, s_koff, s_bst, s_kst); \
     break;
       LIBERI_FUSED_LIST(X)
 #undef X
@@ -3473,7 +3549,7 @@ int class_fused_nq(int c) {
 }
 #endif
 
-#if LIBERI_CLASS_GROUP == -1 || LIBERI_CLASS_GROUP == -2
+#if LIBERI_UNIT == -1 || LIBERI_UNIT == -2
 int launch_class(int c, const ClassDev &cd, const BuildArgs &ba, void *stream, int nwg) {
   hipStream_t st = (hipStream_t)stream;
   if (!(cd.xswitch <= class_rys_xmax(c))) return hipErrorInvalidValue;
@@ -3545,6 +3621,47 @@ int64_t class_row_lds(int c, int transposed, const int32_t *ncol, double xswitch
 #undef X
     default:
       return -1;
+  }
+}
+
+template <int LA, int LB, int LC, int LD>
+static int row_quartets() {
+  using P = SplitShape<LA, LB, LC, LD>;
+  return P::exists ? 64 * P::NBAT : row_threads<LA, LB, LC, LD>();
+}
+
+// Instruction counts of a primitive quartet and of the rest of a quartet (with
+// the latency of its loads), which set when lanes share a quartet
+template <int LA, int LB, int LC, int LD>
+static double row_chain(int64_t primq) {
+  using S = Small<LA, LB, LC, LD>;
+  if (SplitShape<LA, LB, LC, LD>::exists || !use_small<LA, LB, LC, LD>()) return 0.0;
+  const double d = (1850.0 + 18.0 * S::NABCD + 15.0 * S::NE * S::NF) / (40.0 + S::NR * (14.0 + 2.0 * S::NE * S::NF));
+  const double c = 1.5 * sqrt((double)primq * d / (64.0 * kRowWaves));
+  return c > 0.5 * d ? c : 0.5 * d;
+}
+
+int class_row_quartets(int c) {
+  switch (c) {
+#define X(id, a, b, cc, d) \
+  case id:                 \
+    return row_quartets<a, b, cc, d>();
+    LIBERI_CLASS_LIST(X)
+#undef X
+    default:
+      return 0;
+  }
+}
+
+double class_row_chain(int c, int64_t primq) {
+  switch (c) {
+#define X(id, a, b, cc, d) \
+  case id:                 \
+    return row_chain<a, b, cc, d>(primq);
+    LIBERI_CLASS_LIST(X)
+#undef X
+    default:
+      return 0.0;
   }
 }
 

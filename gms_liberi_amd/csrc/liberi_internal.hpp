@@ -47,12 +47,12 @@ extern const ClassDef kClasses[kNumClasses];
 
 // One shell pair, A = the shell of higher angular momentum (A first for equal L).
 struct PairRec {
-  int32_t prim_off;  // first primitive pair record
+  int32_t prim_off;  // first primitive pair record (the k-th is prim_stride k further on)
   int32_t nprim;
   int32_t bfA, bfB;  // first basis function (0-based) of A and B
   double ABx, ABy, ABz;
   int32_t sameAB;    // A and B are one shell
-  int32_t shA;       // shell index of A (0-based)
+  int32_t prim_stride;  // primitive record k is prims[prim_off + k * prim_stride]
   int32_t cA, cB;    // compact column of A's / B's first function among all
                      // functions of that angular momentum (shell rank * ncart)
   double x;          // Schwarz value of the pair
@@ -67,33 +67,42 @@ struct alignas(64) PrimRec {
   double p, Px, Py, Pz, PAx, PAy, PAz, K;
 };
 
+// One workgroup of a row-tiled kernel: the quartets [q0, q0 + n) of one row,
+// starting in segment seg; in the lane-per-quartet kernels `team` adjacent
+// lanes share a quartet (a power of two up to 64).
+struct RowTile {
+  int64_t q0;
+  int32_t n, seg, team, pad;
+};
+
 // Device view of one class's quartet enumeration.  Kept pair lists are sorted
 // by (primitive count, Schwarz value descending); a segment is one kept bra
 // row against one primitive-count group of kets, and its surviving kets are a
 // prefix of that group (the quartet test is monotone in the ket's Schwarz
 // value).  Quartet q of the class lies in segment s with
-// seg_start[s] <= q < seg_start[s+1], ket = ket_list[seg_ket0[s] + q - seg_start[s]].
+// seg_start[s] <= q < seg_start[s+1], ket = seg_ket0[s] + q - seg_start[s]: the
+// PairRec array itself is in that order, so that the kets of a segment, and
+// their k-th primitive records, are neighbours in memory.
 struct ClassDev {
-  const int32_t *bra_list;  // pair indices (into the PairRec array)
-  const int32_t *ket_list;
   const int64_t *seg_start;  // nseg + 1
   const int32_t *seg_bra;    // bra pair index of the segment
-  const int32_t *seg_ket0;   // position in ket_list of the segment's first ket
+  const int32_t *seg_ket0;   // ket pair index of the segment's first quartet
   int32_t nseg;
   int32_t diag;
   int64_t q_begin, q_end;    // this rank's share of the class's quartets
   double xswitch;            // Rys argument from which the asymptotic rule is used
-  // Row tiles: runs of at most the class's tile length (kTileLens) of one row.  Tile t
-  // covers [tile_q[t], tile_q[t+1]) and starts in segment tile_seg[t]; this
-  // rank's tiles are [t_begin, t_end).  row_mode selects the row-tiled kernel.
-  const int64_t *tile_q;     // ntile + 1
-  const int32_t *tile_seg;   // ntile
-  int32_t t_begin, t_end;
+  // this rank's row tiles in launch order; row_mode selects the row-tiled kernel
+  const RowTile *tiles;
+  int32_t ntile;
   int32_t row_mode;
   // 0: rows run over the class's bra pairs, segments over its kets (as
-  // above); 1: the roles are swapped -- seg_bra holds ket pairs and ket_list
+  // above); 1: the roles are swapped -- seg_bra holds ket pairs and seg_ket0
   // bra pairs -- so that a row tile fixes the ket pair (non-diagonal classes)
   int32_t transposed;
+  // the fixed (rows) and the moving pairs' classes in the pair layout: element
+  // of component k of pair p is base + k * n + p
+  int64_t fix_base, mov_base;
+  int32_t fix_n, mov_n;
   // group kernels: chunk_stride(grid) of the launch (set at launch)
   int64_t chunk_stride;
   // 1: the mixed form may evaluate this class's quartets in FP32 (chosen per
@@ -103,11 +112,30 @@ struct ClassDev {
   int32_t coop;
 };
 
+// Pair layout: quantities with one value per (shell pair, component pair) of
+// every pair class, class after class, component-major over the class's pairs
+// in device order, components a * nb + b in internal order.  The element of
+// component k of pair p of class c is off[c] + k * n[c] + (p - first[c]), so
+// consecutive pairs are neighbours in memory: the Coulomb sums of a row
+// tile's moving pairs are added there instead of to F, 64 lanes to 64
+// consecutive doubles (measured 187 G atomic adds/s against 23.7 G to
+// scattered ones).
+struct PairLayout {
+  int64_t off[kNumPairClasses + 1];
+  int32_t n[kNumPairClasses], first[kNumPairClasses];
+  // workgroups of the kernels over it: those of class c are [block[c],
+  // block[c + 1]), chunks[c] per component
+  int32_t chunks[kNumPairClasses], block[kNumPairClasses + 1];
+};
+
 struct BuildArgs {
   const PairRec *pairs;
   const PrimRec *prims;
-  const double *D;   // density of the Coulomb blocks
-  const double *DK;  // density of the exchange blocks (= D for RHF)
+  const double *D;   // density of the Coulomb blocks (packed)
+  const double *DK;  // density of the exchange blocks (= D for RHF, packed)
+  const double *Dp;  // D in the pair layout
+  const double *Dsq;  // DK as a full nbf x nbf matrix
+  double *Jp;        // Coulomb sums in the pair layout, added to F at the end
   double k_scale;    // exchange weight (1 for RHF: F = J[D] - K[D]/2; 2 for a UHF spin: J[Da+Db] - K[Ds])
   double *F;
   double value_cut;
@@ -142,6 +170,11 @@ double class_rys_xmax(int c);
 // angular momentum and the Rys switch (the kernel stages the table below it);
 // -1 when the class has no such kernel
 int64_t class_row_lds(int c, int transposed, const int32_t *ncol, double xswitch);
+// quartets a workgroup of the class's row-tiled kernel holds at one lane each
+int class_row_quartets(int c);
+// longest chain of primitive quartets a lane of class c is left with in a
+// share of primq primitive quartets (0: the class's kernel has no teams)
+double class_row_chain(int c, int64_t primq);
 // kernel shape of class c: 0 lane per quartet, 1 workgroup group per
 // quartet, 2 cooperative workgroup per quartet
 int class_kernel_kind(int c);
@@ -167,6 +200,24 @@ int launch_group_fused(const ClassDev *cds, const BuildArgs &ba, const FusedItem
 constexpr int kNumTileLens = 4;
 constexpr int64_t kTileLens[kNumTileLens] = {512, 1024, 4096, 16384};
 constexpr int kDefaultTile = 2;
+// Spreading a class over the chip.  A lane evaluates a quartet's primitive
+// quartets one after the other, up to 1296 in (ss|ss), 0.1 to 2 us each, so a
+// class of few quartets is bound by its longest chain (water's (ss|ss): 406
+// quartets, 0.30 ms).  `team` lanes then share a quartet: each takes every
+// team-th primitive of the moving pair.  A team costs the wave its fixed work
+// (records, the sum over the team, the digestion, which one lane does) for
+// 64 / team quartets, d primitive quartets' worth; with C the longest chain
+// left to a lane, a class of p primitive quartets on the waves the chip runs
+// at once takes about (p / C) d / (64 kRowWaves) + C, least at
+// C = sqrt(p d / (64 kRowWaves)).  Measured on 12 atoms of the cage: (ss|ss)
+// 0.39 -> 0.10 ms, (ss|ps) 0.28 -> 0.11; on water 0.30 -> 0.02, 0.20 -> 0.02.
+constexpr double kRowWaves = 1740;  // 1024 SIMDs, 1.7 waves each
+// a class of at most this many workgroup steps runs one step per tile: its
+// tiles then still fit the chip a few times over, and the flush of a tile's
+// exchange rows costs less than the idle compute units (more steps: the timed
+// tile length; C60's (dd|dp), 9100 steps on 1830 rows, 5.1 ms in whole rows,
+// 6.1 cut to steps)
+constexpr int64_t kRowSteps = 1024;
 // LDS the row-tiled kernel may take per workgroup
 constexpr int64_t kRowLdsBytes = 64 * 1024;
 // workgroups the cooperative kernels use
@@ -224,6 +275,11 @@ int schwarz_enqueue(const SchwarzStage &s, PairRec *dp, PrimRec *dq, int32_t *dl
 void schwarz_scatter(const SchwarzStage &s, const double *out, double *schwrz_int);
 // records the message of liberi_c_last_error and returns code
 int set_last_error(int code, const std::string &msg);
+
+// start of a build (F and Jp zeroed, Dp and Dsq filled from D and DK) and its
+// end (Jp added to F)
+int launch_build_begin(const BuildArgs &ba, const PairLayout &pl, double *Dp, double *Dsq, void *stream);
+int launch_build_end(const BuildArgs &ba, const PairLayout &pl, void *stream);
 
 // p[0..n) = 0 on the stream (a kernel, so it may sit in a captured graph)
 int launch_fill_zero(double *p, int64_t n, void *stream);

@@ -94,7 +94,11 @@ int liberi_c_fock_build(liberi_ctx *ctx, const double *density, double *fock, in
 /* Same build on device-resident arrays (hipMalloc'd, n doubles each) on the
  * given hipStream_t (NULL = the handle's stream).  Asynchronous: returns after
  * enqueueing.  No counterpart in the reference (which maps D/F per call,
- * src/liberi_driver.F90:66,163); for callers that keep D and F in HBM. */
+ * src/liberi_driver.F90:66,163); for callers that keep D and F in HBM.
+ * Builds of one handle share its device workspace: one enqueued on another
+ * stream than the last waits for it (a build that the caller has captured
+ * into a graph of its own must not be replayed beside another build of the
+ * same handle; other handles are independent). */
 int liberi_c_fock_build_device(liberi_ctx *ctx, const double *d_density, double *d_fock, int64_t n,
                                void *stream);
 

@@ -1057,6 +1057,7 @@ int liberi_c_setup(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_bas, 
 // atomics), direct digestion for the workgroup classes (whose occupancy the
 // LDS accumulators would cut).
 constexpr int64_t kTuneMinQuartets = 20000;
+constexpr float kTileGain = 0.06f;
 constexpr int kSideStreams = 4;
 
 // Choices made so far in this process: later handles (a request loop sets up
@@ -1208,8 +1209,13 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
         if (int rc = time_class(h, ba, st, c, true, false, ms)) return rc;
         best[k] = std::min(best[k], ms);
       }
-    for (int k = 0; k < kNumTileLens; ++k)
-      if (best[k] < best[cs_.tile]) cs_.tile = k;
+    // the longest one unless a shorter is clearly faster: alone, short tiles
+    // fill the tail of a class, but in a build the other classes do that, and
+    // each tile costs a flush (one of 8 rank shares of C60: 4096 for every
+    // class 10.6 ms, 512 12.2, the fastest of each class alone 10.7)
+    cs_.tile = kNumTileLens - 1;
+    for (int k = kNumTileLens - 2; k >= 0; --k)
+      if (best[k] < (1.f - kTileGain) * best[cs_.tile]) cs_.tile = k;
     use_tiles(cs_, cs_.tile);
     cs_.ms = best[cs_.tile];
     set_tuned_choice(c, nq, -2.0, cs_.tile);

@@ -121,10 +121,11 @@ struct liberi_ctx {
   // under a caller's capture, whose events cannot be waited for)
   hipStream_t last_stream = nullptr;
   std::vector<DevBuf> owned;
-  DevBuf pairs, prims, dens, fock, scratch;
+  DevBuf pairs, prims, dens, fock;
   PairLayout layout{};      // pair layout of the basis
-  DevBuf dpair, jpair, dsq;  // per build: density and Coulomb sums by pair, square exchange density
-  int64_t scratch_per_wg = 0;
+  // per build: density and Coulomb sums by pair (component- then pair-major),
+  // square exchange density and exchange sums
+  DevBuf dpair, jpair, dsq, ksq;
   DevBuf col_bf[4];     // compact columns per angular momentum -> basis function
   int32_t ncol[4] = {};
   DevBuf aux;           // per build: max |D|, FP32 quartet count
@@ -238,7 +239,6 @@ static void release_device(liberi_ctx *h) {
   dev_free(h->prims);
   dev_free(h->dens);
   dev_free(h->fock);
-  dev_free(h->scratch);
   dev_free(h->aux);
   dev_free(h->fused_items);
   dev_free(h->fused_cds);
@@ -248,6 +248,7 @@ static void release_device(liberi_ctx *h) {
   dev_free(h->dpair);
   dev_free(h->jpair);
   dev_free(h->dsq);
+  dev_free(h->ksq);
   dev_free(h->dens_t);
   dev_free(h->dens_b);
   dev_free(h->fock_b);
@@ -816,8 +817,10 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     return fail(LIBERI_EDEVICE, std::string("zero aux: ") + hipGetErrorString((hipError_t)e));
   if ((rc = dev_alloc(h, h->fock, ntri * sizeof(double)))) return rc;
   const size_t npl = (size_t)h->layout.off[kNumPairClasses];
-  if ((rc = dev_alloc(h, h->dpair, npl * sizeof(double))) || (rc = dev_alloc(h, h->jpair, npl * sizeof(double))) ||
-      (rc = dev_alloc(h, h->dsq, (size_t)num_bas * num_bas * sizeof(double))))
+  const size_t nsq = (size_t)num_bas * num_bas;
+  if ((rc = dev_alloc(h, h->dpair, 2 * npl * sizeof(double))) ||
+      (rc = dev_alloc(h, h->jpair, 2 * npl * sizeof(double))) || (rc = dev_alloc(h, h->dsq, nsq * sizeof(double))) ||
+      (rc = dev_alloc(h, h->ksq, nsq * sizeof(double))))
     return rc;
 
   // ---- per class: pair pre-screen (host), quartet segments (device)
@@ -826,7 +829,6 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     for (auto &b : tmp) dev_free(b);
     tmp.clear();
   };
-  int64_t max_scratch = 0;
   for (int c = 0; c < kNumClasses; ++c) {
     const ClassDef &def = kClasses[c];
     ClassState &cs_ = h->cls[c];
@@ -1004,16 +1006,17 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
       d.mov_base = pl.off[pm] - pl.first[pm];
       d.fix_n = pl.n[pf];
       d.mov_n = pl.n[pm];
+      auto pair_major = [&](int pc) {
+        return pl.off[pc] - (int64_t)pl.first[pc] * ncart_host(kPairL[pc][0]) * ncart_host(kPairL[pc][1]);
+      };
+      d.bra_q = pair_major(def.bra);
+      d.ket_q = pair_major(def.ket);
     }
     d.xswitch = h->exact_large_t ? class_rys_xmax(c) : reference_switch(c);
     h->stats.quartets[c] = d.q_end - d.q_begin;
     h->stats.prim_quartets[c] = primq;
     h->stats.total_quartets += d.q_end - d.q_begin;
-    max_scratch = std::max(max_scratch, class_scratch_doubles(c));
   }
-  h->scratch_per_wg = max_scratch;
-  if (max_scratch > 0)
-    if ((rc = dev_alloc(h, h->scratch, (size_t)max_scratch * kCoopWorkgroups * sizeof(double)))) return rc;
   if ((rc = setup_fused(h))) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   h->initialized = true;
@@ -1271,12 +1274,17 @@ static int enqueue_dmax(liberi_ctx *h, const double *dD, hipStream_t st) {
   return LIBERI_OK;
 }
 
+static BuildWork build_work(const liberi_ctx *h) {
+  double *dp = (double *)h->dpair.p;
+  return BuildWork{dp, dp + h->layout.off[kNumPairClasses], (double *)h->dsq.p};
+}
+
 // Zero F (and find max |D| for the mixed form), then every class's kernel.
 // With ns > 1 the classes are spread over the side streams, longest first
 // onto the least-loaded stream, forked from and joined back into st.
 static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, hipStream_t st, int ns) {
   // fock = 0 (src/liberi_driver.F90:64)
-  if (int e = launch_build_begin(ba, h->layout, (double *)h->dpair.p, (double *)h->dsq.p, st))
+  if (int e = launch_build_begin(ba, h->layout, build_work(h), st))
     return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
@@ -1307,7 +1315,7 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
   }
   if (fused) {
     // one persistent launch for the fused classes, first onto the least-loaded
-    // stream (the cooperative classes keep side stream 0 to themselves)
+    // stream
     for (int c = 0; c < kNumClasses; ++c)
       if (h->cls[c].active && class_fused_nq(c) > 0) fused_cost += cost(c);
     int k = 0;
@@ -1326,9 +1334,7 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
   for (int c : order) {
     hipStream_t cs = st;
     if (ns > 1) {
-      // the cooperative kernels share one per-workgroup scratch buffer: their
-      // classes all go to side stream 0, which runs them one after another
-      const int k = class_scratch_doubles(c) > 0 ? 0 : (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
       load[k] += cost(c);
       cs = h->side[k];
     }
@@ -1365,13 +1371,15 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   ba.D = dD;
   ba.DK = dK ? dK : dD;
   ba.k_scale = k_scale;
-  ba.Dp = (const double *)h->dpair.p;
-  ba.Dsq = (const double *)h->dsq.p;
+  const BuildWork w = build_work(h);
+  ba.Dp = w.Dp;
+  ba.Dq = w.Dq;
+  ba.Dsq = w.Dsq;
   ba.Jp = (double *)h->jpair.p;
+  ba.Jq = ba.Jp + h->layout.off[kNumPairClasses];
+  ba.Ksq = (double *)h->ksq.p;
   ba.F = dF;
   ba.value_cut = h->value_cut;
-  ba.scratch = (double *)h->scratch.p;
-  ba.scratch_per_wg = h->scratch_per_wg;
   ba.nbf = h->num_bas;
   ba.fp32_tau = h->fp32_tau;
   ba.dmax = (const double *)h->aux.p;
@@ -1395,7 +1403,7 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     return false;
   }();
   if (choose) {
-    if (int e = launch_build_begin(ba, h->layout, (double *)h->dpair.p, (double *)h->dsq.p, st))
+    if (int e = launch_build_begin(ba, h->layout, build_work(h), st))
       return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
     if (int rc = choose_variants(h, ba, st)) return rc;
   }

@@ -9,17 +9,20 @@
 // reference's three kernel families (rotated-axis, ERIC, Rys; src/rhf/) with
 // one engine specialised per class at compile time.
 //
-// Two execution shapes:
-//  * lane-per-quartet (small classes): one lane owns one contracted quartet,
-//    all intermediates in registers, loops fully unrolled per class;
-//  * workgroup-per-quartet (large classes): the (e0|f0) accumulators are
-//    spread over the workgroup's lanes, the 2-D Rys tables of each primitive
-//    quartet are staged in LDS, the HRR runs on a per-workgroup scratch area.
+// Execution shapes:
+//  * lane-per-quartet (small classes): one lane (or a team) owns one contracted
+//    quartet, all intermediates in registers, loops fully unrolled per class;
+//  * wave-split rows: slices of a quartet's (e0|f0) in several waves' registers;
+//  * group-per-quartet: (e0|f0) spread over a group of lanes, the 2-D tables
+//    and the HRR in LDS;
+//  * cooperative (large classes): a lane per row (ab| of the block, which is
+//    formed directly from 2-D tables in LDS, without (e0|f0).
 //
 // Digestion (the reference's DIRFCK_RHF, e.g. src/rhf/rot_axis/int0000.F90:241-311)
-// contracts each shell block with the six density blocks and adds the result
-// to the packed Fock matrix with one hardware FP64 atomic per Fock element of
-// the block (not one per integral).
+// contracts each shell block with the six density blocks; the results are
+// added with one hardware FP64 atomic per element of a block (not one per
+// integral) to Coulomb sums by shell pair and a square matrix of exchange
+// sums, which the end of the build folds into the packed Fock matrix.
 #include <hip/hip_runtime.h>
 
 #include "liberi_internal.hpp"
@@ -258,6 +261,15 @@ __device__ __forceinline__ void decode_quartet(const ClassDev &cd, int64_t q, in
 
 __device__ __forceinline__ void fock_add(double *F, uint32_t i, uint32_t j, double v) {
   unsafeAtomicAdd(F + tri(i, j), v);
+}
+
+// element of the exchange sums (of the square exchange density) at row i of
+// the bra pair's functions and column j
+__device__ __forceinline__ double *exch_at(const BuildArgs &ba, int i, int j) {
+  return ba.Ksq + (int64_t)i * ba.nbf + j;
+}
+__device__ __forceinline__ const double *dens_exch(const BuildArgs &ba, int i, int j) {
+  return ba.Dsq + (int64_t)i * ba.nbf + j;
 }
 
 // Read-only views of the pair and primitive records in the constant address
@@ -1041,7 +1053,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_ke
     const int r = i / ncols, k = i - r * ncols;
     const int rbf = r < N1 ? fix.bfA + gpos_of(R::L1, r) : fix.bfB + gpos_of(R::L2, r - N1);
     const int cbf = (R::M1 == R::M2 || k < off2) ? ba.col_bf[R::M1][k] : ba.col_bf[R::M2][k - off2];
-    fock_add(ba.F, rbf, cbf, x);
+    unsafeAtomicAdd(ba.Ksq + (int64_t)rbf * ba.nbf + cbf, x);
   }
 }
 
@@ -1578,7 +1590,7 @@ __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_ke
     const int r = i / ncols, k = i - r * ncols;
     const int rbf = r < N1 ? fix.bfA + gpos_of(R::L1, r) : fix.bfB + gpos_of(R::L2, r - N1);
     const int cbf = (R::M1 == R::M2 || k < off2) ? ba.col_bf[R::M1][k] : ba.col_bf[R::M2][k - off2];
-    fock_add(ba.F, rbf, cbf, x);
+    unsafeAtomicAdd(ba.Ksq + (int64_t)rbf * ba.nbf + cbf, x);
   }
 }
 
@@ -1616,300 +1628,431 @@ __device__ __forceinline__ double scale_rt(int L, int k) {
   return 1.0;
 }
 
-// Workgroup-per-quartet path for the classes whose group slot exceeds the
-// LDS (the f classes).  One workgroup of NT lanes evaluates one quartet at a
-// time: 3 NR lanes make the 2-D tables of a primitive quartet, every lane
-// accumulates its components of (e0|f0); the HRR levels, the cartesian
-// scales and the digestion then run over all lanes.  The HRR buffers live in
-// LDS wherever the class's two buffers, tables, density blocks and step
-// tables fit kCoopLds (gfx950: 160 KB per workgroup), else in a per-workgroup
-// HBM scratch.  Each HRR level reads a per-row step table (source rows and
-// direction, made once per workgroup), so an item costs two reads, one FMA
-// and one write; the digestion reads the six density blocks from LDS with
-// compile-time strides.
-constexpr int kCoopLds = 160 * 1024;
+// The group kernels run one wave per workgroup.  A wave's LDS operations
+// complete in program order, so between the LDS phases of such a kernel a
+// compiler-level fence at wavefront scope is enough: no s_barrier and no
+// drain of the wave's outstanding memory operations.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
+// Cooperative path for the classes with many components: one workgroup of W
+// waves evaluates Q quartets at a time and forms the integrals directly from
+// 2-D tables, without (e0|f0) and a contracted HRR.  For every primitive
+// quartet 3 NR lanes (one root and direction each) run the 2-D recursion and
+// its transfer to shells A and B in registers and write H(a, b, k) to LDS.  A
+// lane owns one row (ab| of the block: per root it reads the three rows of H
+// of its exponents, transfers them to shells C and D in registers, and adds
+// the products to all |cd) columns (one half of shell C's components per
+// wave where there are more than 64).  No intermediate of the block's size is
+// stored: with one or few primitive quartets per quartet, as d and f shells
+// have, the (e0|f0) block, its HRR levels and their barriers cost several
+// times the products.  The digestion works from the registers; sums over the
+// rows go through LDS.
+//
+// What bounds it: the FP64 products (2 per integral and root) at two waves
+// per SIMD, then the digestion.
 template <int LA, int LB, int LC, int LD>
 struct Coop {
   static constexpr int LAB = LA + LB, LCD = LC + LD;
   static constexpr int NR = (LAB + LCD) / 2 + 1;
   static constexpr int NI = LAB + 1, NK = LCD + 1;
-  static constexpr int NE = nrange(LA, LAB), NF = nrange(LC, LCD);
   static constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-  static constexpr int NABCD = NA * NB * NC * ND;
   static constexpr int NAB = NA * NB, NCD = NC * ND, NAC = NA * NC, NBD = NB * ND, NAD = NA * ND, NBC = NB * NC;
   static constexpr int DB = NAB + NCD + NAC + NBD + NAD + NBC;
-  static constexpr int GT = 3 * NR * NI * NK;  // 2-D tables of one primitive quartet
-  static constexpr int64_t buf_doubles() { return hrr_max_buffer(LA, LB, LC, LD); }
-  // step-table entries: bra levels 1..LB (rows a, b), then ket levels 1..LD (c, d)
-  static constexpr int bra_rows(int j) { return nrange(LA, LAB - j) * ncart(j); }
-  static constexpr int ket_rows(int j) { return nrange(LC, LCD - j) * ncart(j); }
-  static constexpr int tab_off(int lev) {  // lev 0..LB-1 bra, LB..LB+LD-1 ket
-    int o = 0;
-    for (int i = 0; i < lev; ++i) o += i < LB ? bra_rows(i + 1) : ket_rows(i - LB + 1);
-    return o;
+  // column slices: halves of shell C's components when |cd) has more than 64
+  static constexpr int CS = NCD > 64 && NC % 2 == 0 ? 2 : 1;
+  static constexpr int NCS = NC / CS, NV = NCS * ND;
+  // quartets per wave where several blocks' rows fit its lanes; waves over the rows
+  static constexpr int Q = NAB <= 32 ? 64 / NAB : 1;
+  static constexpr int WR = (NAB + 63) / 64, RW = (NAB + WR - 1) / WR;
+  static constexpr int W = WR * CS, NT = 64 * W;
+  // H of one root and direction: rows (a, b) of NK values, odd stride
+  static constexpr int HK = NK | 1, HT = (LA + 1) * (LB + 1) * HK, H = 3 * NR * HT;
+  // primitive quartets per pass of the table lanes
+  static constexpr int KT0 = NT / (3 * NR * Q), KT1 = 1400 / (H * Q);
+  static constexpr int KT = KT1 < 1 ? 1 : (KT0 < KT1 ? KT0 : KT1);
+  static_assert(KT0 >= 1, "table lanes");
+  // partial sums of the digestion: two exchange blocks' columns per row, then
+  // the J(CD) columns (one quartet per wave: JCH of them at a time)
+  static constexpr int P1 = (2 * NCS) | 1, P2 = (2 * ND) | 1, PJ = NCD | 1, JCH = 15;
+  static constexpr int part() {
+    const int a = Q * CS * NAB * (P1 > P2 ? P1 : P2), b = Q > 1 ? Q * NAB * PJ : W * 64 * JCH;
+    return a > b ? a : b;
   }
-  static constexpr int NTAB = tab_off(LB + LD);
-  static constexpr int fixed_doubles() { return GT + DB + (NTAB + 1) / 2; }
-  static constexpr bool IN_LDS = (int64_t)8 * (fixed_doubles() + 2 * buf_doubles()) <= kCoopLds;
-  static constexpr int LDS_DOUBLES = fixed_doubles() + (IN_LDS ? 2 * (int)buf_doubles() : 0);
-  static constexpr int NT = IN_LDS || NE * NF > 2048 ? 512 : (NE * NF > 512 ? 128 : 64);
-  static constexpr int NKC = (NE * NF + NT - 1) / NT;  // accumulators per lane
-  static constexpr int64_t scratch() { return IN_LDS ? 0 : 2 * buf_doubles(); }
+  static constexpr int UNI = KT * Q * H > part() ? KT * Q * H : part();
+  static constexpr int LDS_DOUBLES = UNI + Q * DB;
+  static_assert(LDS_DOUBLES * 8 <= 64 * 1024, "LDS of the cooperative form");
 };
 
-template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT)) void eri_coop_kernel(ClassDev cd, BuildArgs ba) {
-  using S = Coop<LA, LB, LC, LD>;
-  constexpr int NT = S::NT, NR = S::NR, NI = S::NI, NK = S::NK, NE = S::NE, NF = S::NF, NKC = S::NKC;
-  constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND;
-  constexpr int NAB = S::NAB, NCD = S::NCD, NAC = S::NAC, NBD = S::NBD, NAD = S::NAD, NBC = S::NBC;
-  constexpr int GSZ = NI * NK;
-  __shared__ double lds[S::LDS_DOUBLES];
-  double *Gt = lds;                   // [3][NR][GSZ]
-  double *Dab = Gt + S::GT, *Dcd = Dab + NAB, *Dbd = Dcd + NCD, *Dac = Dbd + NBD, *Dbc = Dac + NAC, *Dad = Dbc + NBC;
-  int *tab = (int *)(Dad + NAD);      // HRR step tables
-  double *buf0 = S::IN_LDS ? lds + S::fixed_doubles() : ba.scratch + (int64_t)blockIdx.x * ba.scratch_per_wg;
-  double *buf1 = buf0 + S::buf_doubles();
-
-  const int t = threadIdx.x;
-  // step tables: output row -> source rows s1 (shifted) and s2, direction
-  for (int i = t; i < S::NTAB; i += NT) {
-    int lev = 0;
-    while (lev + 1 < LB + LD && S::tab_off(lev + 1) <= i) ++lev;
-    const int r = i - S::tab_off(lev);
-    int s1, s2, dir;
-    if (lev < LB) {  // bra level j: row (a in range(LA, LAB-j), b in cart(j))
-      const int j = lev + 1, nb = ncart(j), nbm = ncart(j - 1), a = r / nb, b = r % nb;
-      int bx, by, bz, La, ax, ay, az;
-      cart_decode(j, b, bx, by, bz);
-      range_decode(LA, a, La, ax, ay, az);
-      dir = bx ? 0 : (by ? 1 : 2);
-      const int bmi = cidx(bx - (dir == 0), by - (dir == 1), bz - (dir == 2));
-      s1 = range_index(LA, ax + (dir == 0), ay + (dir == 1), az + (dir == 2)) * nbm + bmi;
-      s2 = a * nbm + bmi;
-    } else {  // ket level j: column (c in range(LC, LCD-j), d in cart(j))
-      const int j = lev - LB + 1, nd = ncart(j), ndm = ncart(j - 1), c = r / nd, d = r % nd;
-      int dx, dy, dz, Lc, cx, cy, cz;
-      cart_decode(j, d, dx, dy, dz);
-      range_decode(LC, c, Lc, cx, cy, cz);
-      dir = dx ? 0 : (dy ? 1 : 2);
-      const int dmi = cidx(dx - (dir == 0), dy - (dir == 1), dz - (dir == 2));
-      s1 = range_index(LC, cx + (dir == 0), cy + (dir == 1), cz + (dir == 2)) * ndm + dmi;
-      s2 = c * ndm + dmi;
-    }
-    tab[i] = s1 | (s2 << 14) | (dir << 28);
-  }
-
-  // per-lane component offsets into the G tables (fixed for the kernel)
-  int offx[NKC], offy[NKC], offz[NKC];
-#pragma unroll
-  for (int k = 0; k < NKC; ++k) {
-    const int c = t + NT * k;
-    if (c < NE * NF) {
-      int Le, ex, ey, ez, Lf, fx, fy, fz;
-      range_decode(LA, c / NF, Le, ex, ey, ez);
-      range_decode(LC, c % NF, Lf, fx, fy, fz);
-      offx[k] = ex * NK + fx;
-      offy[k] = ey * NK + fy;
-      offz[k] = ez * NK + fz;
-    } else {
-      offx[k] = offy[k] = offz[k] = 0;
-    }
-  }
-  const double *Dm = ba.D, *Dk = ba.DK;
-  double *F = ba.F;
-  const double ks = ba.k_scale;
-
-  // a contiguous chunk of the class's quartets per workgroup: the segment is
-  // searched once and then followed, and consecutive quartets share the bra
-  // pair (the cached bra records)
-  const int64_t nq = cd.q_end - cd.q_begin;
-  const int64_t per = (nq + gridDim.x - 1) / gridDim.x;
-  const int64_t q0 = cd.q_begin + (int64_t)blockIdx.x * per;
-  const int64_t q1 = q0 + per < cd.q_end ? q0 + per : cd.q_end;
-  int sg = q0 < q1 ? find_segment(cd, q0, 0, cd.nseg) : 0;
-  for (int64_t q = q0; q < q1; ++q) {
-    while (sg + 1 < cd.nseg && cd.seg_start[sg + 1] <= q) ++sg;
-    int32_t ib, ik;
-    quartet_of_segment(cd, sg, q, ib, ik);
-    const PairRec bra = ba.pairs[ib];
-    const PairRec ket = ba.pairs[ik];
-    // the six density blocks of the digestion (Coulomb: D(ab), D(cd); exchange: the rest)
-    for (int i = t; i < S::DB; i += NT) {
-      int k = i;
-      const double *src = Dm;
-      uint32_t r0, r1;
-      if (k < NAB) {
-        r0 = bra.bfA + gpos_rt(LA, k / NB), r1 = bra.bfB + gpos_rt(LB, k % NB);
-      } else if ((k -= NAB) < NCD) {
-        r0 = ket.bfA + gpos_rt(LC, k / ND), r1 = ket.bfB + gpos_rt(LD, k % ND);
-      } else if (src = Dk, (k -= NCD) < NBD) {
-        r0 = bra.bfB + gpos_rt(LB, k / ND), r1 = ket.bfB + gpos_rt(LD, k % ND);
-      } else if ((k -= NBD) < NAC) {
-        r0 = bra.bfA + gpos_rt(LA, k / NC), r1 = ket.bfA + gpos_rt(LC, k % NC);
-      } else if ((k -= NAC) < NBC) {
-        r0 = bra.bfB + gpos_rt(LB, k / NC), r1 = ket.bfA + gpos_rt(LC, k % NC);
-      } else {
-        k -= NBC;
-        r0 = bra.bfA + gpos_rt(LA, k / ND), r1 = ket.bfB + gpos_rt(LD, k % ND);
-      }
-      Dab[i] = src[tri(r0, r1)];
-    }
-    double acc[NKC];
-#pragma unroll
-    for (int k = 0; k < NKC; ++k) acc[k] = 0.0;
-
-    for (int ip = 0; ip < bra.nprim; ++ip) {
-      for (int iq = 0; iq < ket.nprim; ++iq) {
-        if (t < 3 * NR) {
-          const PrimRec P = ba.prims[bra.prim_off + ip * bra.prim_stride];
-          const PrimRec Q = ba.prims[ket.prim_off + iq * ket.prim_stride];
-          const int r = t / 3, dim = t - 3 * (t / 3);
-          const double pq = P.p + Q.p, ipq = 1.0 / pq;
-          const double pqx = P.Px - Q.Px, pqy = P.Py - Q.Py, pqz = P.Pz - Q.Pz;
-          const double rho = P.p * Q.p * ipq;
-          const double X = rho * (pqx * pqx + pqy * pqy + pqz * pqz);
-          double t2, wr;
-          rys_root<NR>(X, cd.xswitch, r, t2, wr);
-          const double hp = 0.5 / P.p, hq = 0.5 / Q.p;
-          const double b00 = 0.5 * t2 * ipq;
-          const double b10 = hp - hp * Q.p * t2 * ipq;
-          const double b01 = hq - hq * P.p * t2 * ipq;
-          const double fa = Q.p * ipq * t2, fc = P.p * ipq * t2;
-          const double pqd = dim == 0 ? pqx : (dim == 1 ? pqy : pqz);
-          const double pa = dim == 0 ? P.PAx : (dim == 1 ? P.PAy : P.PAz);
-          const double qc = dim == 0 ? Q.PAx : (dim == 1 ? Q.PAy : Q.PAz);
-          const double g00 = dim == 2 ? wr * kTwoPi52 * P.K * Q.K * sqrt(ipq) : 1.0;
-          double g[NI][NK];
-          rys_2d<NI, NK>(g, pa - fa * pqd, qc + fc * pqd, b10, b01, b00, g00);
-#pragma unroll
-          for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int k = 0; k < NK; ++k) Gt[(dim * NR + r) * GSZ + i * NK + k] = g[i][k];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < NKC; ++k) {
-          double v = 0.0;
-#pragma unroll
-          for (int r = 0; r < NR; ++r)
-            v += Gt[r * GSZ + offx[k]] * Gt[(NR + r) * GSZ + offy[k]] * Gt[(2 * NR + r) * GSZ + offz[k]];
-          acc[k] += v;
-        }
-        __syncthreads();
-      }
-    }
-    // cartesian scales and the value cutoff, applied by the last write of the
-    // HRR (whose output index is v's [a][b][c][d])
-    auto final_value = [&](int it, double x) -> double {
-      const int d = it % ND, c = (it / ND) % NC, b = (it / NCD) % NB, a = it / (NB * NCD);
-      const double v = x * scale_rt(LA, a) * scale_rt(LB, b) * scale_rt(LC, c) * scale_rt(LD, d);
-      return fabs(v) < ba.value_cut ? 0.0 : v;
-    };
-#pragma unroll
-    for (int k = 0; k < NKC; ++k) {
-      const int c = t + NT * k;
-      if (c < NE * NF) buf0[c] = LB == 0 && LD == 0 ? final_value(c, acc[k]) : acc[k];
-    }
+// barrier between the LDS phases of a workgroup of W waves
+template <int W>
+__device__ __forceinline__ void coop_sync() {
+  if constexpr (W == 1)
+    wave_sync();
+  else
     __syncthreads();
+}
 
-    // bra HRR: level j out[a in range(LA, LAB-j)][b in cart(j)][f] from level j-1
-    double *in = buf0, *out = buf1;
+// Columns of slice SL of the lane's row: the primitive quartet's tables h
+// (rows of the lane's exponents at hx, hy, hz) added to v
+template <int LA, int LB, int LC, int LD, int SL>
+__device__ __forceinline__ void coop_accumulate(const double *h, int hx, int hy, int hz, double cdx, double cdy,
+                                                double cdz, double (&v)[Coop<LA, LB, LC, LD>::NV]) {
+  using S = Coop<LA, LB, LC, LD>;
+  constexpr Range<LC, LC> rc{};
+  constexpr Range<LD, LD> rd{};
+  constexpr int RD = S::NR * S::HT;  // tables of one direction
+#pragma unroll 1
+  for (int r = 0; r < S::NR; ++r) {
+    double x[LD + 1][S::NK], y[LD + 1][S::NK], z[LD + 1][S::NK];  // [d][c]
+    const double *p = h + r * S::HT;
 #pragma unroll
-    for (int j = 1; j <= LB; ++j) {
-      const int *tj = tab + S::tab_off(j - 1);
-      const int items = S::bra_rows(j) * NF;
-      for (int it = t; it < items; it += NT) {
-        const int row = it / NF, f = it - row * NF;
-        const int e = tj[row], dir = e >> 28;
-        const double abv = dir == 0 ? bra.ABx : (dir == 1 ? bra.ABy : bra.ABz);
-        const double x = in[(e & 16383) * NF + f] + abv * in[((e >> 14) & 16383) * NF + f];
-        out[it] = j == LB && LD == 0 ? final_value(it, x) : x;
-      }
-      __syncthreads();
-      double *tmp = in;
-      in = out;
-      out = tmp;
+    for (int k = 0; k < S::NK; ++k) {
+      x[0][k] = p[hx + k];
+      y[0][k] = p[RD + hy + k];
+      z[0][k] = p[2 * RD + hz + k];
     }
-    // ket HRR on the inner index: out[ab][c in range(LC, LCD-j)][d in cart(j)]
 #pragma unroll
-    for (int j = 1; j <= LD; ++j) {
-      const int *tj = tab + S::tab_off(LB + j - 1);
-      const int nin = S::ket_rows(j - 1), nout = S::ket_rows(j);
-      for (int it = t; it < NAB * nout; it += NT) {
-        const int ab = it / nout, cdi = it - ab * nout;
-        const int e = tj[cdi], dir = e >> 28;
-        const double cdv = dir == 0 ? ket.ABx : (dir == 1 ? ket.ABy : ket.ABz);
-        const double x = in[ab * nin + (e & 16383)] + cdv * in[ab * nin + ((e >> 14) & 16383)];
-        out[it] = j == LD ? final_value(it, x) : x;
+    for (int d = 1; d <= LD; ++d)
+#pragma unroll
+      for (int c = 0; c + d < S::NK; ++c) {
+        x[d][c] = fma(cdx, x[d - 1][c], x[d - 1][c + 1]);
+        y[d][c] = fma(cdy, y[d - 1][c], y[d - 1][c + 1]);
+        z[d][c] = fma(cdz, z[d - 1][c], z[d - 1][c + 1]);
       }
-      __syncthreads();
-      double *tmp = in;
-      in = out;
-      out = tmp;
+#pragma unroll
+    for (int c = 0; c < S::NCS; ++c)
+#pragma unroll
+      for (int d = 0; d < S::ND; ++d) {
+        const int cc = SL * S::NCS + c;
+        v[c * S::ND + d] += x[rd.lx[d]][rc.lx[cc]] * y[rd.ly[d]][rc.ly[cc]] * z[rd.lz[d]][rc.lz[cc]];
+      }
+  }
+}
+
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT), 2) void eri_coop_kernel(ClassDev cd, BuildArgs ba) {
+  using S = Coop<LA, LB, LC, LD>;
+  constexpr int NR = S::NR, NI = S::NI, NK = S::NK, NT = S::NT, Q = S::Q, KT = S::KT, W = S::W, CS = S::CS;
+  constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND, NCS = S::NCS, NV = S::NV;
+  constexpr int NAB = S::NAB, NCD = S::NCD, NAC = S::NAC, NBD = S::NBD, NAD = S::NAD;
+  __shared__ double lds[S::LDS_DOUBLES];
+  double *uni = lds, *dens = lds + S::UNI;
+
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int slice = CS == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave / S::WR);
+  // the lane's quartet slot and row
+  const int slot = Q > 1 ? lane / NAB : 0;
+  const int row = Q > 1 ? lane - slot * NAB : (wave % S::WR) * S::RW + lane;
+  const bool on = Q > 1 ? slot < Q : (lane < S::RW && row < NAB);
+  const int a = row / NB, b = row - a * NB;
+  int hx = 0, hy = 0, hz = 0;
+  double sab = 0.0;
+  if (on) {
+    int ax, ay, az, bx, by, bz;
+    cart_decode(LA, a, ax, ay, az);
+    cart_decode(LB, b, bx, by, bz);
+    hx = (ax * (LB + 1) + bx) * S::HK;
+    hy = (ay * (LB + 1) + by) * S::HK;
+    hz = (az * (LB + 1) + bz) * S::HK;
+    sab = scale_rt(LA, a) * scale_rt(LB, b);
+  }
+  // the lane's table task: slot ts, primitive quartet tk of the pass, root, direction
+  const int tdim = t % 3, tr = t / 3 % NR, tk = t / (3 * NR) % KT, ts = t / (3 * NR * KT);
+  const bool table = ts < Q;
+
+  // a contiguous chunk of the class's quartets per workgroup (consecutive
+  // quartets share the row's pair); the workgroups resident together work on
+  // distant chunks
+  const int64_t nq = cd.q_end - cd.q_begin;
+  const int64_t per = ((nq + gridDim.x - 1) / gridDim.x + Q - 1) / Q * Q;
+  const int64_t chunk = (int64_t)blockIdx.x * cd.chunk_stride % gridDim.x;
+  const int64_t c0 = cd.q_begin + chunk * per, c1 = c0 + per < cd.q_end ? c0 + per : cd.q_end;
+  int sg = c0 < c1 ? find_segment(cd, c0, 0, cd.nseg) : 0;
+
+  double jab = 0.0;  // the row's J(AB) element over a run of quartets of one bra pair
+  int32_t jab_pair = -1;
+  auto flush_jab = [&]() {
+    if (jab_pair >= 0 && on && jab != 0.0) unsafeAtomicAdd(ba.Jq + cd.bra_q + (int64_t)jab_pair * NAB + row, jab);
+    jab = 0.0;
+  };
+
+  for (int64_t q = c0; q < c1; q += Q) {
+    const int64_t mine = q + slot;
+    const bool valid = slot < Q && mine < c1;
+    int32_t ib = -1, ik = -1;
+    if (valid) {
+      while (sg + 1 < cd.nseg && cd.seg_start[sg + 1] <= mine) ++sg;
+      quartet_of_segment(cd, sg, mine, ib, ik);
+    }
+    if constexpr (Q == 1) ib = __builtin_amdgcn_readfirstlane(ib), ik = __builtin_amdgcn_readfirstlane(ik);
+    PairRec bra{}, ket{};
+    if (valid) {
+      bra = ba.pairs[ib];
+      ket = ba.pairs[ik];
+    }
+    // slot s's pairs
+    auto bra_of = [&](int s) { return Q > 1 ? __shfl(ib, s * NAB) : ib; };
+    auto ket_of = [&](int s) { return Q > 1 ? __shfl(ik, s * NAB) : ik; };
+    const int npq = bra.nprim * ket.nprim;
+    int maxpq = npq;
+    if constexpr (Q > 1) {
+      maxpq = 0;
+#pragma unroll
+      for (int s = 0; s < Q; ++s) maxpq = max(maxpq, __shfl(npq, s * NAB));
+    }
+    // the six density blocks of each slot
+#pragma unroll
+    for (int s = 0; s < Q; ++s) {
+      const int32_t jb = bra_of(s), jk = ket_of(s);
+      if (jb < 0) continue;
+      const int bA = ba.pairs[jb].bfA, bB = ba.pairs[jb].bfB, kA = ba.pairs[jk].bfA, kB = ba.pairs[jk].bfB;
+      double *d = dens + s * S::DB;
+      for (int i = t; i < NAB; i += NT) d[i] = ba.Dq[cd.bra_q + (int64_t)jb * NAB + i];
+      d += NAB;
+      for (int i = t; i < NCD; i += NT) d[i] = ba.Dq[cd.ket_q + (int64_t)jk * NCD + i];
+      d += NCD;
+      for (int i = t; i < NAC; i += NT) d[i] = *dens_exch(ba, bA + gpos_rt(LA, i / NC), kA + gpos_rt(LC, i % NC));
+      d += NAC;
+      for (int i = t; i < NBD; i += NT) d[i] = *dens_exch(ba, bB + gpos_rt(LB, i / ND), kB + gpos_rt(LD, i % ND));
+      d += NBD;
+      for (int i = t; i < NAD; i += NT) d[i] = *dens_exch(ba, bA + gpos_rt(LA, i / ND), kB + gpos_rt(LD, i % ND));
+      d += NAD;
+      for (int i = t; i < S::NBC; i += NT) d[i] = *dens_exch(ba, bB + gpos_rt(LB, i / NC), kA + gpos_rt(LC, i % NC));
     }
 
+    double v[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = 0.0;
+    // the table task's pairs
+    PairRec tb{}, tq{};
+    {
+      const int s = table ? ts : 0;
+      const int32_t jb = bra_of(s), jk = ket_of(s);
+      if (table && jb >= 0) tb = ba.pairs[jb], tq = ba.pairs[jk];
+    }
+    const int tnpq = tb.nprim * tq.nprim;
+    for (int t0 = 0; t0 < maxpq; t0 += KT) {
+      if (table && t0 + tk < tnpq) {
+        // (as in the group kernel: a quotient of small integers in FP32)
+        const int pq = t0 + tk, ip = (int)(((float)pq + 0.5f) * __builtin_amdgcn_rcpf((float)tq.nprim)),
+                  iq = pq - ip * tq.nprim;
+        const PrimRec P = ba.prims[tb.prim_off + ip * tb.prim_stride];
+        const PrimRec R = ba.prims[tq.prim_off + iq * tq.prim_stride];
+        const double rs = nr_rsqrt(P.p + R.p), ipq = rs * rs;
+        const double pqx = P.Px - R.Px, pqy = P.Py - R.Py, pqz = P.Pz - R.Pz;
+        const double X = P.p * R.p * ipq * (pqx * pqx + pqy * pqy + pqz * pqz);
+        double u, w;
+        rys_root<NR>(X, cd.xswitch, tr, u, w);
+        const double fa = R.p * ipq * u, fc = P.p * ipq * u;
+        const double hp = 0.5 * nr_rcp(P.p), hq = 0.5 * nr_rcp(R.p);
+        const double b00 = 0.5 * u * ipq, b10 = hp - hp * fa, b01 = hq - hq * fc;
+        const double pqd = tdim == 0 ? pqx : (tdim == 1 ? pqy : pqz);
+        const double pa = tdim == 0 ? P.PAx : (tdim == 1 ? P.PAy : P.PAz);
+        const double qc = tdim == 0 ? R.PAx : (tdim == 1 ? R.PAy : R.PAz);
+        const double ab = tdim == 0 ? tb.ABx : (tdim == 1 ? tb.ABy : tb.ABz);
+        const double g00 = tdim == 2 ? w * kTwoPi52 * P.K * R.K * rs : 1.0;
+        double g[NI][NK];
+        rys_2d<NI, NK>(g, pa - fa * pqd, qc + fc * pqd, b10, b01, b00, g00);
+        double *dst = uni + (ts * KT + tk) * S::H + (tdim * NR + tr) * S::HT;
+#pragma unroll
+        for (int lb = 0; lb <= LB; ++lb) {
+#pragma unroll
+          for (int la = 0; la <= LA; ++la)
+#pragma unroll
+            for (int k = 0; k < NK; ++k) dst[(la * (LB + 1) + lb) * S::HK + k] = g[la][k];
+          // to one unit more on B
+          if (lb < LB) {
+#pragma unroll
+            for (int i = 0; i + lb + 1 < NI; ++i)
+#pragma unroll
+              for (int k = 0; k < NK; ++k) g[i][k] = fma(ab, g[i][k], g[i + 1][k]);
+          }
+        }
+      }
+      coop_sync<W>();
+#pragma unroll 1
+      for (int k = 0; k < KT; ++k) {
+        if (!(on && t0 + k < npq)) continue;
+        const double *h = uni + (slot * KT + k) * S::H;
+        if (CS == 1 || slice == 0)
+          coop_accumulate<LA, LB, LC, LD, 0>(h, hx, hy, hz, ket.ABx, ket.ABy, ket.ABz, v);
+        else
+          coop_accumulate<LA, LB, LC, LD, CS - 1>(h, hx, hy, hz, ket.ABx, ket.ABy, ket.ABz, v);
+      }
+      coop_sync<W>();
+    }
+    if (maxpq == 0) coop_sync<W>();  // the density blocks
+
+    // cartesian scales and the value cutoff
+    const int cs0 = slice * NCS;  // first component of C of the slice
+#pragma unroll
+    for (int c = 0; c < NCS; ++c) {
+      const double sc = sab * scale_rt(LC, cs0 + c);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        constexpr Range<LD, LD> rd{};
+        const double x = v[c * ND + d] * (sc * cart_scale(rd.lx[d], rd.ly[d], rd.lz[d]));
+        v[c * ND + d] = fabs(x) < ba.value_cut ? 0.0 : x;
+      }
+    }
     double s = 1.0;
     if (bra.sameAB) s *= 0.5;
     if (ket.sameAB) s *= 0.5;
     if (cd.diag && ib == ik) s *= 0.5;
-    const double *v = in;
-    // six contracted blocks, one output element per lane iteration; the sums
-    // run over compile-time strides from the output's base
-    constexpr int n1 = NAB, n2 = n1 + NCD, n3 = n2 + NAC, n4 = n3 + NBD, n5 = n4 + NAD, n6 = n5 + NBC;
-    for (int it = t; it < n6; it += NT) {
-      double acc2 = 0.0, fac;
-      uint32_t fi, fj;
-      if (it < n1) {  // F[ab] += 4s sum_cd v D[cd]
-        const int a = it / NB, b = it % NB;
-        const double *vb = v + it * NCD;
-#pragma unroll 4
-        for (int k = 0; k < NCD; ++k) acc2 += vb[k] * Dcd[k];
-        fi = bra.bfA + gpos_rt(LA, a), fj = bra.bfB + gpos_rt(LB, b), fac = 4.0 * s;
-      } else if (it < n2) {  // F[cd] += 4s sum_ab v D[ab]
-        const int k0 = it - n1, c = k0 / ND, d = k0 % ND;
-        const double *vb = v + k0;
-#pragma unroll 4
-        for (int k = 0; k < NAB; ++k) acc2 += vb[k * NCD] * Dab[k];
-        fi = ket.bfA + gpos_rt(LC, c), fj = ket.bfB + gpos_rt(LD, d), fac = 4.0 * s;
-      } else if (it < n3) {  // F[ac] -= s sum_bd v D[bd]
-        const int k0 = it - n2, a = k0 / NC, c = k0 % NC;
-        const double *vb = v + a * NB * NCD + c * ND;
-#pragma unroll 4
-        for (int b = 0; b < NB; ++b)
-#pragma unroll 4
-          for (int d = 0; d < ND; ++d) acc2 += vb[b * NCD + d] * Dbd[b * ND + d];
-        fi = bra.bfA + gpos_rt(LA, a), fj = ket.bfA + gpos_rt(LC, c), fac = -s * ks;
-      } else if (it < n4) {  // F[bd] -= s sum_ac v D[ac]
-        const int k0 = it - n3, b = k0 / ND, d = k0 % ND;
-        const double *vb = v + b * NCD + d;
-#pragma unroll 4
-        for (int a = 0; a < NA; ++a)
-#pragma unroll 4
-          for (int c = 0; c < NC; ++c) acc2 += vb[a * NB * NCD + c * ND] * Dac[a * NC + c];
-        fi = bra.bfB + gpos_rt(LB, b), fj = ket.bfB + gpos_rt(LD, d), fac = -s * ks;
-      } else if (it < n5) {  // F[ad] -= s sum_bc v D[bc]
-        const int k0 = it - n4, a = k0 / ND, d = k0 % ND;
-        const double *vb = v + a * NB * NCD + d;
-#pragma unroll 4
-        for (int b = 0; b < NB; ++b)
-#pragma unroll 4
-          for (int c = 0; c < NC; ++c) acc2 += vb[b * NCD + c * ND] * Dbc[b * NC + c];
-        fi = bra.bfA + gpos_rt(LA, a), fj = ket.bfB + gpos_rt(LD, d), fac = -s * ks;
-      } else {  // F[bc] -= s sum_ad v D[ad]
-        const int k0 = it - n5, b = k0 / NC, c = k0 % NC;
-        const double *vb = v + b * NCD + c * ND;
-#pragma unroll 4
-        for (int a = 0; a < NA; ++a)
-#pragma unroll 4
-          for (int d = 0; d < ND; ++d) acc2 += vb[a * NB * NCD + d] * Dad[a * ND + d];
-        fi = bra.bfB + gpos_rt(LB, b), fj = ket.bfA + gpos_rt(LC, c), fac = -s * ks;
-      }
-      if (acc2 != 0.0) fock_add(F, fi, fj, fac * acc2);
+    const double sk = s * ba.k_scale;
+    const double *dab = dens + (on ? slot : 0) * S::DB, *dcd = dab + NAB, *dac = dcd + NCD, *dbd = dac + NAC,
+                 *dad = dbd + NBD, *dbc = dad + NAD;
+    const bool live = on && valid;
+
+    // J(AB): the row's element, over the bra pair's run
+    if (valid && jab_pair != ib) {
+      flush_jab();
+      jab_pair = ib;
     }
-    __syncthreads();  // buffers and density blocks are reused by the next quartet
+    if (live) {
+      double x = 0.0;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) x += v[k] * dcd[cs0 * ND + k];
+      jab += 4.0 * s * x;
+    }
+    // exchange blocks with C: the row's share per component, then the sums over b (a)
+    if (live) {
+      double *p = uni + ((slot * CS + slice) * NAB + row) * S::P1;
+      double eb[ND], ea[ND];
+#pragma unroll
+      for (int d = 0; d < ND; ++d) eb[d] = dbd[b * ND + d], ea[d] = dad[a * ND + d];
+#pragma unroll
+      for (int c = 0; c < NCS; ++c) {
+        double x = 0.0, y = 0.0;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) x += v[c * ND + d] * eb[d], y += v[c * ND + d] * ea[d];
+        p[c] = x;
+        p[NCS + c] = y;
+      }
+    }
+    coop_sync<W>();
+#pragma unroll
+    for (int sl = 0; sl < Q; ++sl) {
+      const int32_t jb = bra_of(sl), jk = ket_of(sl);
+      const double f = Q > 1 ? __shfl(sk, sl * NAB) : sk;
+      if (jb < 0) continue;
+      const int bA = ba.pairs[jb].bfA, bB = ba.pairs[jb].bfB, kA = ba.pairs[jk].bfA;
+      for (int i = t; i < NAC + S::NBC; i += NT) {
+        const bool first = i < NAC;
+        const int k = first ? i : i - NAC, e = k / NC, c = k - e * NC, cs = c / NCS;
+        const double *p = uni + (sl * CS + cs) * NAB * S::P1 + (c - cs * NCS);
+        double x = 0.0;
+        if (first) {
+          p += e * NB * S::P1;
+#pragma unroll
+          for (int j = 0; j < NB; ++j) x += p[j * S::P1];
+        } else {
+          p += e * S::P1 + NCS;
+#pragma unroll
+          for (int j = 0; j < NA; ++j) x += p[j * NB * S::P1];
+        }
+        if (x != 0.0)
+          unsafeAtomicAdd(exch_at(ba, first ? bA + gpos_rt(LA, e) : bB + gpos_rt(LB, e), kA + gpos_rt(LC, c)), -f * x);
+      }
+    }
+    coop_sync<W>();
+    // exchange blocks with D
+    if (live) {
+      double *p = uni + ((slot * CS + slice) * NAB + row) * S::P2;
+      double x[ND], y[ND];
+#pragma unroll
+      for (int d = 0; d < ND; ++d) x[d] = y[d] = 0.0;
+#pragma unroll
+      for (int c = 0; c < NCS; ++c) {
+        const double eb = dbc[b * NC + cs0 + c], ea = dac[a * NC + cs0 + c];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) x[d] += v[c * ND + d] * eb, y[d] += v[c * ND + d] * ea;
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d) p[d] = x[d], p[ND + d] = y[d];
+    }
+    coop_sync<W>();
+#pragma unroll
+    for (int sl = 0; sl < Q; ++sl) {
+      const int32_t jb = bra_of(sl), jk = ket_of(sl);
+      const double f = Q > 1 ? __shfl(sk, sl * NAB) : sk;
+      if (jb < 0) continue;
+      const int bA = ba.pairs[jb].bfA, bB = ba.pairs[jb].bfB, kB = ba.pairs[jk].bfB;
+      for (int i = t; i < NAD + NBD; i += NT) {
+        const bool first = i < NAD;
+        const int k = first ? i : i - NAD, e = k / ND, d = k - e * ND;
+        double x = 0.0;
+#pragma unroll
+        for (int cs = 0; cs < CS; ++cs) {
+          const double *p = uni + (sl * CS + cs) * NAB * S::P2 + d;
+          if (first) {
+            p += e * NB * S::P2;
+#pragma unroll
+            for (int j = 0; j < NB; ++j) x += p[j * S::P2];
+          } else {
+            p += e * S::P2 + ND;
+#pragma unroll
+            for (int j = 0; j < NA; ++j) x += p[j * NB * S::P2];
+          }
+        }
+        if (x != 0.0)
+          unsafeAtomicAdd(exch_at(ba, first ? bA + gpos_rt(LA, e) : bB + gpos_rt(LB, e), kB + gpos_rt(LD, d)), -f * x);
+      }
+    }
+    coop_sync<W>();
+    // J(CD): the columns' sums over the rows
+    const double da = live ? dab[row] : 0.0;
+    if constexpr (Q > 1) {
+      if (live) {
+        double *p = uni + (slot * NAB + row) * S::PJ;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) p[k] = v[k] * da;
+      }
+      wave_sync();
+#pragma unroll
+      for (int sl = 0; sl < Q; ++sl) {
+        const int32_t jk = ket_of(sl);
+        const double f = 4.0 * __shfl(s, sl * NAB);
+        if (jk < 0) continue;
+        for (int i = lane; i < NCD; i += 64) {
+          const double *p = uni + sl * NAB * S::PJ + i;
+          double x = 0.0;
+#pragma unroll
+          for (int j = 0; j < NAB; ++j) x += p[j * S::PJ];
+          if (x != 0.0) unsafeAtomicAdd(ba.Jq + cd.ket_q + (int64_t)jk * NCD + i, f * x);
+        }
+      }
+    } else {
+      // JCH columns at a time, each summed by four lanes over a quarter of the wave's rows
+      constexpr int JCH = S::JCH, RQ = (S::RW + 3) / 4;
+      double *p = uni + wave * 64 * JCH;
+      const int col = lane % JCH, quarter = lane / JCH;
+#pragma unroll
+      for (int k0 = 0; k0 < NV; k0 += JCH) {
+#pragma unroll
+        for (int j = 0; j < JCH; ++j)
+          if (k0 + j < NV) p[lane * JCH + j] = v[k0 + j] * da;
+        wave_sync();
+        double x = 0.0;
+        if (quarter < 4 && k0 + col < NV) {
+#pragma unroll
+          for (int j = 0; j < RQ; ++j)
+            if (4 * RQ <= 64 || quarter * RQ + j < 64) x += p[(quarter * RQ + j) * JCH + col];
+        }
+        x += __shfl(x, lane + 2 * JCH, 64);
+        x += __shfl(x, lane + JCH, 64);
+        if (lane < JCH && k0 + lane < NV && x != 0.0)
+          unsafeAtomicAdd(ba.Jq + cd.ket_q + (int64_t)ik * NCD + cs0 * ND + k0 + lane, 4.0 * s * x);
+        wave_sync();
+      }
+    }
+    coop_sync<W>();  // the tables and density blocks are overwritten by the next round
   }
+  flush_jab();
 }
 
 // =================================================== group-per-quartet path
@@ -2329,16 +2472,6 @@ struct Grp {
   static constexpr int RT = RT1 / KT * KT;
 };
 
-// The group kernels run one wave per workgroup.  A wave's LDS operations
-// complete in program order, so between the LDS phases of such a kernel a
-// compiler-level fence at wavefront scope is enough: no s_barrier and no
-// drain of the wave's outstanding memory operations.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Lanes per output of a digestion block of `no` outputs on a slot of g
 // lanes, splitting a summed index of extent x: the largest power of two
 // that keeps no x split <= g and the split <= x
@@ -2427,14 +2560,14 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
   double jab[NJL];
 #pragma unroll
   for (int k = 0; k < NJL; ++k) jab[k] = 0.0;
-  int32_t jab_pair = -1, jab_a = 0, jab_b = 0;
+  int32_t jab_pair = -1;
   auto flush_jab = [&]() {
     if (jab_pair < 0) return;
 #pragma unroll
     for (int k = 0; k < NJL; ++k) {
       const int i = gl + k * G;
       if (i < S::NAB && jab[k] != 0.0)
-        fock_add(ba.F, jab_a + gpos_rt(LA, i / S::NB), jab_b + gpos_rt(LB, i % S::NB), jab[k]);
+        unsafeAtomicAdd(ba.Jq + cd.bra_q + (int64_t)jab_pair * S::NAB + i, jab[k]);
       jab[k] = 0.0;
     }
   };
@@ -2620,13 +2753,12 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
       double *DAB = Gt + S::UNI, *DCD = DAB + NAB, *DAC = DCD + NCD, *DBD = DAC + S::NAC, *DAD = DBD + S::NBD,
              *DBC = DAD + S::NAD;
       if (valid) {
-        const double *Dm = ba.D, *Dk = ba.DK;  // Coulomb and exchange densities
-        for (int i = gl; i < NAB; i += G) DAB[i] = Dm[tri(bra.bfA + gpos_rt(LA, i / NB), bra.bfB + gpos_rt(LB, i % NB))];
-        for (int i = gl; i < NCD; i += G) DCD[i] = Dm[tri(ket.bfA + gpos_rt(LC, i / ND), ket.bfB + gpos_rt(LD, i % ND))];
-        for (int i = gl; i < S::NAC; i += G) DAC[i] = Dk[tri(bra.bfA + gpos_rt(LA, i / NC), ket.bfA + gpos_rt(LC, i % NC))];
-        for (int i = gl; i < S::NBD; i += G) DBD[i] = Dk[tri(bra.bfB + gpos_rt(LB, i / ND), ket.bfB + gpos_rt(LD, i % ND))];
-        for (int i = gl; i < S::NAD; i += G) DAD[i] = Dk[tri(bra.bfA + gpos_rt(LA, i / ND), ket.bfB + gpos_rt(LD, i % ND))];
-        for (int i = gl; i < S::NBC; i += G) DBC[i] = Dk[tri(bra.bfB + gpos_rt(LB, i / NC), ket.bfA + gpos_rt(LC, i % NC))];
+        for (int i = gl; i < NAB; i += G) DAB[i] = ba.Dq[cd.bra_q + (int64_t)ib * S::NAB + i];
+        for (int i = gl; i < NCD; i += G) DCD[i] = ba.Dq[cd.ket_q + (int64_t)ik * S::NCD + i];
+        for (int i = gl; i < S::NAC; i += G) DAC[i] = *dens_exch(ba, bra.bfA + gpos_rt(LA, i / NC), ket.bfA + gpos_rt(LC, i % NC));
+        for (int i = gl; i < S::NBD; i += G) DBD[i] = *dens_exch(ba, bra.bfB + gpos_rt(LB, i / ND), ket.bfB + gpos_rt(LD, i % ND));
+        for (int i = gl; i < S::NAD; i += G) DAD[i] = *dens_exch(ba, bra.bfA + gpos_rt(LA, i / ND), ket.bfB + gpos_rt(LD, i % ND));
+        for (int i = gl; i < S::NBC; i += G) DBC[i] = *dens_exch(ba, bra.bfB + gpos_rt(LB, i / NC), ket.bfA + gpos_rt(LC, i % NC));
       }
       // bra HRR: one column f per lane, in registers; (ab|f) to [ab][f]
       double *bufT = Gt + NE * NF;
@@ -2675,8 +2807,6 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
       if (valid && jab_pair != ib) {
         flush_jab();
         jab_pair = ib;
-        jab_a = bra.bfA;
-        jab_b = bra.bfB;
       }
 #pragma unroll
       for (int k = 0; k < NJ; ++k) {
@@ -2716,44 +2846,43 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
       }
       wave_sync();
       if (valid) {
-        double *F = ba.F;
         const double sk = s * ba.k_scale;
-        auto put = [&](int64_t fi, int64_t fj, double x) {
-          if (x != 0.0) fock_add(F, fi, fj, x);
-        };
+        auto put = [&](double *dst, double x) {
+        if (x != 0.0) unsafeAtomicAdd(dst, x);
+      };
         for (int i = gl; i < NCD; i += G) {
           double t = 0.0;
 #pragma unroll
           for (int ab = 0; ab < NAB; ++ab) t += JC[ab * JS + i];
-          put(ket.bfA + gpos_rt(LC, i / ND), ket.bfB + gpos_rt(LD, i % ND), 4.0 * s * t);
+          put(ba.Jq + cd.ket_q + (int64_t)ik * S::NCD + i, 4.0 * s * t);
         }
         for (int i = gl; i < NA * NC; i += G) {
           const int a = i / NC, c = i - a * NC;
           double t = 0.0;
 #pragma unroll
           for (int b = 0; b < NB; ++b) t += KAC[(a * NB + b) * NC + c];
-          put(bra.bfA + gpos_rt(LA, a), ket.bfA + gpos_rt(LC, c), -sk * t);
+          put(exch_at(ba, bra.bfA + gpos_rt(LA, a), ket.bfA + gpos_rt(LC, c)), -sk * t);
         }
         for (int i = gl; i < NB * ND; i += G) {
           const int b = i / ND, d = i - b * ND;
           double t = 0.0;
 #pragma unroll
           for (int a = 0; a < NA; ++a) t += KBD[(b * NA + a) * ND + d];
-          put(bra.bfB + gpos_rt(LB, b), ket.bfB + gpos_rt(LD, d), -sk * t);
+          put(exch_at(ba, bra.bfB + gpos_rt(LB, b), ket.bfB + gpos_rt(LD, d)), -sk * t);
         }
         for (int i = gl; i < NA * ND; i += G) {
           const int a = i / ND, d = i - a * ND;
           double t = 0.0;
 #pragma unroll
           for (int b = 0; b < NB; ++b) t += KAD[(a * NB + b) * ND + d];
-          put(bra.bfA + gpos_rt(LA, a), ket.bfB + gpos_rt(LD, d), -sk * t);
+          put(exch_at(ba, bra.bfA + gpos_rt(LA, a), ket.bfB + gpos_rt(LD, d)), -sk * t);
         }
         for (int i = gl; i < NB * NC; i += G) {
           const int b = i / NC, c = i - b * NC;
           double t = 0.0;
 #pragma unroll
           for (int a = 0; a < NA; ++a) t += KBC[(b * NA + a) * NC + c];
-          put(bra.bfB + gpos_rt(LB, b), ket.bfA + gpos_rt(LC, c), -sk * t);
+          put(exch_at(ba, bra.bfB + gpos_rt(LB, b), ket.bfA + gpos_rt(LC, c)), -sk * t);
         }
       }
     } else {
@@ -2831,13 +2960,12 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
             row[c * ND + d] = fabs(x) < ba.value_cut ? 0.0 : x;
           }
       }
-      const double *Dm = ba.D, *Dk = ba.DK;  // Coulomb and exchange densities
-      for (int i = gl; i < S::NAB; i += G) DAB[i] = Dm[tri(bra.bfA + gpos_rt(LA, i / NB), bra.bfB + gpos_rt(LB, i % NB))];
-      for (int i = gl; i < NCD; i += G) DCD[i] = Dm[tri(ket.bfA + gpos_rt(LC, i / ND), ket.bfB + gpos_rt(LD, i % ND))];
-      for (int i = gl; i < S::NAC; i += G) DAC[i] = Dk[tri(bra.bfA + gpos_rt(LA, i / NC), ket.bfA + gpos_rt(LC, i % NC))];
-      for (int i = gl; i < S::NBD; i += G) DBD[i] = Dk[tri(bra.bfB + gpos_rt(LB, i / ND), ket.bfB + gpos_rt(LD, i % ND))];
-      for (int i = gl; i < S::NAD; i += G) DAD[i] = Dk[tri(bra.bfA + gpos_rt(LA, i / ND), ket.bfB + gpos_rt(LD, i % ND))];
-      for (int i = gl; i < S::NBC; i += G) DBC[i] = Dk[tri(bra.bfB + gpos_rt(LB, i / NC), ket.bfA + gpos_rt(LC, i % NC))];
+      for (int i = gl; i < S::NAB; i += G) DAB[i] = ba.Dq[cd.bra_q + (int64_t)ib * S::NAB + i];
+      for (int i = gl; i < NCD; i += G) DCD[i] = ba.Dq[cd.ket_q + (int64_t)ik * S::NCD + i];
+      for (int i = gl; i < S::NAC; i += G) DAC[i] = *dens_exch(ba, bra.bfA + gpos_rt(LA, i / NC), ket.bfA + gpos_rt(LC, i % NC));
+      for (int i = gl; i < S::NBD; i += G) DBD[i] = *dens_exch(ba, bra.bfB + gpos_rt(LB, i / ND), ket.bfB + gpos_rt(LD, i % ND));
+      for (int i = gl; i < S::NAD; i += G) DAD[i] = *dens_exch(ba, bra.bfA + gpos_rt(LA, i / ND), ket.bfB + gpos_rt(LD, i % ND));
+      for (int i = gl; i < S::NBC; i += G) DBC[i] = *dens_exch(ba, bra.bfB + gpos_rt(LB, i / NC), ket.bfA + gpos_rt(LC, i % NC));
     }
     wave_sync();
     if (valid) {
@@ -2846,17 +2974,14 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
       if (ket.sameAB) s *= 0.5;
       if (cd.diag && ib == ik) s *= 0.5;
       const double *__restrict__ v = in;
-      double *F = ba.F;
-      auto put = [&](int64_t fi, int64_t fj, double x) {
-        if (x != 0.0) fock_add(F, fi, fj, x);
+      auto put = [&](double *dst, double x) {
+        if (x != 0.0) unsafeAtomicAdd(dst, x);
       };
       // J(AB): F[ab] += 4s sum_cd v D[cd], summed in registers while the
       // slot's bra pair stays the same
       if (jab_pair != ib) {
         flush_jab();
         jab_pair = ib;
-        jab_a = bra.bfA;
-        jab_b = bra.bfB;
       }
 #pragma unroll
       for (int k = 0; k < NJL; ++k) {
@@ -2884,7 +3009,7 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
           for (int k = 0; k * SP < S::NAB; ++k)
             if (S::NAB % SP == 0 || p + k * SP < S::NAB) t += vb[k * SP * KS] * db[k * SP];
           t = part_sum<SP>(t);
-          if (p == 0) put(ket.bfA + gpos_rt(LC, c), ket.bfB + gpos_rt(LD, d), 4.0 * s * t);
+          if (p == 0) put(ba.Jq + cd.ket_q + (int64_t)ik * S::NCD + i, 4.0 * s * t);
         }
       }
       // K(AC): F[ac] -= s sum_bd v D[bd], b split
@@ -2900,7 +3025,7 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
 #pragma unroll
               for (int d = 0; d < ND; ++d) t += vb[k * SP * KS + d] * db[k * SP * ND + d];
           t = part_sum<SP>(t);
-          if (p == 0) put(bra.bfA + gpos_rt(LA, a), ket.bfA + gpos_rt(LC, c), -s * ba.k_scale * t);
+          if (p == 0) put(exch_at(ba, bra.bfA + gpos_rt(LA, a), ket.bfA + gpos_rt(LC, c)), -s * ba.k_scale * t);
         }
       }
       // K(BD): F[bd] -= s sum_ac v D[ac], a split
@@ -2916,7 +3041,7 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
 #pragma unroll
               for (int c = 0; c < NC; ++c) t += vb[k * SP * NB * KS + c * ND] * db[k * SP * NC + c];
           t = part_sum<SP>(t);
-          if (p == 0) put(bra.bfB + gpos_rt(LB, b), ket.bfB + gpos_rt(LD, d), -s * ba.k_scale * t);
+          if (p == 0) put(exch_at(ba, bra.bfB + gpos_rt(LB, b), ket.bfB + gpos_rt(LD, d)), -s * ba.k_scale * t);
         }
       }
       // K(AD): F[ad] -= s sum_bc v D[bc], b split
@@ -2932,7 +3057,7 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
 #pragma unroll
               for (int c = 0; c < NC; ++c) t += vb[k * SP * KS + c * ND] * db[k * SP * NC + c];
           t = part_sum<SP>(t);
-          if (p == 0) put(bra.bfA + gpos_rt(LA, a), ket.bfB + gpos_rt(LD, d), -s * ba.k_scale * t);
+          if (p == 0) put(exch_at(ba, bra.bfA + gpos_rt(LA, a), ket.bfB + gpos_rt(LD, d)), -s * ba.k_scale * t);
         }
       }
       // K(BC): F[bc] -= s sum_ad v D[ad], a split
@@ -2948,7 +3073,7 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
 #pragma unroll
               for (int d = 0; d < ND; ++d) t += vb[k * SP * NB * KS + d] * db[k * SP * ND + d];
           t = part_sum<SP>(t);
-          if (p == 0) put(bra.bfB + gpos_rt(LB, b), ket.bfA + gpos_rt(LC, c), -s * ba.k_scale * t);
+          if (p == 0) put(exch_at(ba, bra.bfB + gpos_rt(LB, b), ket.bfA + gpos_rt(LC, c)), -s * ba.k_scale * t);
         }
       }
     }
@@ -3156,8 +3281,8 @@ int launch_schwarz(int la, int lb, const PairRec *pairs, const PrimRec *prims, c
   }
 }
 
-// Calls f(element, pair, a, b) for this thread's elements of the pair layout:
-// workgroup blk covers a run of pairs of one class and one component (a, b),
+// Calls f(element, element in pair-major order, pair, class, a, b) for this
+// thread's elements of the pair layout: workgroup blk covers a run of pairs of one class and one component (a, b),
 // so nothing of the decoding is per lane.
 template <class Body>
 __device__ __forceinline__ void for_pair_layout(const PairLayout &pl, int blk, Body f) {
@@ -3165,56 +3290,72 @@ __device__ __forceinline__ void for_pair_layout(const PairLayout &pl, int blk, B
   while (blk >= pl.block[c + 1]) ++c;
   const int comp = (blk - pl.block[c]) / pl.chunks[c], chunk = (blk - pl.block[c]) - comp * pl.chunks[c];
   const int lb = kPairL[c][0], nb = (lb + 1) * (lb + 2) / 2, a = comp / nb, b = comp - a * nb;
+  const int ncomp = nb * (kPairL[c][1] + 1) * (kPairL[c][1] + 2) / 2;
   for (int i = chunk * 256 + (int)threadIdx.x; i < pl.n[c]; i += pl.chunks[c] * 256)
-    f(pl.off[c] + (int64_t)comp * pl.n[c] + i, pl.first[c] + i, c, a, b);
+    f(pl.off[c] + (int64_t)comp * pl.n[c] + i, pl.off[c] + (int64_t)i * ncomp + comp, pl.first[c] + i, c, a, b);
 }
 
-// Start of a build: F and the Coulomb sums by pair zeroed, the Coulomb
+// Start of a build: F and the Coulomb and exchange sums zeroed, the Coulomb
 // density by pair and the square exchange density filled from the packed
 // ones.  A kernel (not memset nodes), so that a build can be captured in a
-// graph.  The first nbf workgroups take a row of F and of the square density
+// graph.  The first nbf workgroups take a row of F and of the square matrices
 // each, the others the pair layout.
-__global__ __launch_bounds__(256) void build_begin_kernel(const PairRec *pairs, PairLayout pl, const double *D,
-                                                          const double *DK, int32_t nbf, double *F, double *Jp,
-                                                          double *Dp, double *Dsq) {
-  if ((int)blockIdx.x < nbf) {
-    const uint32_t r = blockIdx.x;
-    const int64_t row = (int64_t)r * (r + 1) / 2;
-    for (uint32_t k = threadIdx.x; k <= r; k += 256) F[row + k] = 0.0;
-    for (uint32_t k = threadIdx.x; k < (uint32_t)nbf; k += 256) Dsq[(int64_t)r * nbf + k] = DK[tri(r, k)];
+__global__ __launch_bounds__(256) void build_begin_kernel(PairLayout pl, BuildArgs ba, BuildWork w) {
+  if ((int)blockIdx.x < ba.nbf) {
+    const uint32_t r = blockIdx.x, nbf = ba.nbf;
+    const int64_t row = (int64_t)r * (r + 1) / 2, sq = (int64_t)r * nbf;
+    for (uint32_t k = threadIdx.x; k <= r; k += 256) ba.F[row + k] = 0.0;
+    for (uint32_t k = threadIdx.x; k < nbf; k += 256) {
+      w.Dsq[sq + k] = ba.DK[tri(r, k)];
+      ba.Ksq[sq + k] = 0.0;
+    }
     return;
   }
-  for_pair_layout(pl, (int)blockIdx.x - nbf, [&](int64_t e, int p, int c, int a, int b) {
-    Dp[e] = D[tri(pairs[p].bfA + gpos_rt(kPairL[c][1], a), pairs[p].bfB + gpos_rt(kPairL[c][0], b))];
-    Jp[e] = 0.0;
+  for_pair_layout(pl, (int)blockIdx.x - ba.nbf, [&](int64_t e, int64_t q, int p, int c, int a, int b) {
+    const double d = ba.D[tri(ba.pairs[p].bfA + gpos_rt(kPairL[c][1], a), ba.pairs[p].bfB + gpos_rt(kPairL[c][0], b))];
+    w.Dp[e] = d;
+    w.Dq[q] = d;
+    ba.Jp[e] = 0.0;
+    ba.Jq[q] = 0.0;
   });
 }
 
-// End of a build: the Coulomb sums by pair added to F.  Every element of F
+// End of a build: the exchange sums (both triangles) and the Coulomb sums by
+// pair added to F, which may hold direct contributions.  Every element of F
 // belongs to one shell pair; a pair of one shell holds (a, b) and (b, a),
-// both added by the thread of a >= b.
-__global__ __launch_bounds__(256) void build_end_kernel(const PairRec *pairs, PairLayout pl, const double *Jp,
-                                                        double *F) {
-  for_pair_layout(pl, (int)blockIdx.x, [&](int64_t e, int p, int c, int a, int b) {
-    double x = Jp[e];
-    if (pairs[p].sameAB) {
-      const int nb = (kPairL[c][0] + 1) * (kPairL[c][0] + 2) / 2;
-      if (a < b) return;
-      if (a > b) x += Jp[e + (int64_t)(b * nb + a - (a * nb + b)) * pl.n[c]];
+// both added by the thread of a >= b.  The two parts of an element are added
+// atomically: the workgroups of a row and of a pair run side by side.
+__global__ __launch_bounds__(256) void build_end_kernel(PairLayout pl, BuildArgs ba) {
+  if ((int)blockIdx.x < ba.nbf) {
+    const uint32_t r = blockIdx.x, nbf = ba.nbf;
+    const int64_t row = (int64_t)r * (r + 1) / 2;
+    for (uint32_t k = threadIdx.x; k <= r; k += 256) {
+      const double x = ba.Ksq[(int64_t)r * nbf + k] + (k < r ? ba.Ksq[(int64_t)k * nbf + r] : 0.0);
+      if (x != 0.0) unsafeAtomicAdd(ba.F + row + k, x);
     }
-    F[tri(pairs[p].bfA + gpos_rt(kPairL[c][1], a), pairs[p].bfB + gpos_rt(kPairL[c][0], b))] += x;
+    return;
+  }
+  for_pair_layout(pl, (int)blockIdx.x - ba.nbf, [&](int64_t e, int64_t q, int p, int c, int a, int b) {
+    double x = ba.Jp[e] + ba.Jq[q];
+    if (ba.pairs[p].sameAB) {
+      const int nb = (kPairL[c][0] + 1) * (kPairL[c][0] + 2) / 2, o = b * nb + a - (a * nb + b);
+      if (a < b) return;
+      if (a > b) x += ba.Jp[e + (int64_t)o * pl.n[c]] + ba.Jq[q + o];
+    }
+    if (x != 0.0)
+      fock_add(ba.F, ba.pairs[p].bfA + gpos_rt(kPairL[c][1], a), ba.pairs[p].bfB + gpos_rt(kPairL[c][0], b), x);
   });
 }
 
-int launch_build_begin(const BuildArgs &ba, const PairLayout &pl, double *Dp, double *Dsq, void *stream) {
+int launch_build_begin(const BuildArgs &ba, const PairLayout &pl, const BuildWork &w, void *stream) {
   hipLaunchKernelGGL(build_begin_kernel, dim3((unsigned)(ba.nbf + pl.block[kNumPairClasses])), dim3(256), 0,
-                     (hipStream_t)stream, ba.pairs, pl, ba.D, ba.DK, ba.nbf, ba.F, ba.Jp, Dp, Dsq);
+                     (hipStream_t)stream, pl, ba, w);
   return hipGetLastError();
 }
 
 int launch_build_end(const BuildArgs &ba, const PairLayout &pl, void *stream) {
-  hipLaunchKernelGGL(build_end_kernel, dim3((unsigned)pl.block[kNumPairClasses]), dim3(256), 0, (hipStream_t)stream,
-                     ba.pairs, pl, ba.Jp, ba.F);
+  hipLaunchKernelGGL(build_end_kernel, dim3((unsigned)(ba.nbf + pl.block[kNumPairClasses])), dim3(256), 0,
+                     (hipStream_t)stream, pl, ba);
   return hipGetLastError();
 }
 
@@ -3319,12 +3460,15 @@ int64_t row_lds(const int32_t *ncol, double xswitch) {
   }
 }
 
-// group classes with an f shell also get the cooperative form when its
-// buffers fit the LDS; which one runs is timed per class
+// (dd|dd) and the group classes with an f shell also have the cooperative
+// form; which one runs is timed per class (on the 20-atom C-N chain it takes
+// (fd|dd) 1.29 -> 0.53 ms, (fd|fd) 1.08 -> 0.39, (ff|dp) 1.40 -> 0.49; on C60
+// (dd|dd) 2.92 -> 2.61).  The other d classes run faster wave-split or grouped
+// wherever they are large: (dd|dp) 5.1 ms, (dp|dp) 4.4 on C60.
 template <int LA, int LB, int LC, int LD>
 constexpr bool has_coop_alt() {
-  return !use_small<LA, LB, LC, LD>() && Grp<LA, LB, LC, LD>::fits && Coop<LA, LB, LC, LD>::IN_LDS &&
-         (LA == 3 || LB == 3 || LC == 3 || LD == 3);
+  return !use_small<LA, LB, LC, LD>() && Grp<LA, LB, LC, LD>::fits &&
+         (LA == 3 || LB == 3 || LC == 3 || LD == 3 || LA + LB + LC + LD == 8);
 }
 
 template <int LA, int LB, int LC, int LD, bool TR>
@@ -3344,6 +3488,16 @@ static int launch_row(const ClassDev &cd, const BuildArgs &ba, hipStream_t st) {
   } else {
     return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+template <int LA, int LB, int LC, int LD>
+static int launch_coop(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, int nwg) {
+  using S = Coop<LA, LB, LC, LD>;
+  const int64_t need = (cd.q_end - cd.q_begin + S::Q - 1) / S::Q, g = need < nwg ? need : nwg;
+  ClassDev cg = cd;
+  cg.chunk_stride = chunk_stride(g);
+  hipLaunchKernelGGL((eri_coop_kernel<LA, LB, LC, LD>), dim3((unsigned)g), dim3(S::NT), 0, st, cg, ba);
   return hipGetLastError();
 }
 
@@ -3369,10 +3523,7 @@ static int launch_one(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, i
     }
     if (cd.coop) {
       if constexpr (has_coop_alt<LA, LB, LC, LD>()) {
-        using S = Coop<LA, LB, LC, LD>;
-        const int64_t g = n < nwg ? n : nwg;
-        hipLaunchKernelGGL((eri_coop_kernel<LA, LB, LC, LD>), dim3((unsigned)g), dim3(S::NT), 0, st, cd, ba);
-        return hipGetLastError();
+        return launch_coop<LA, LB, LC, LD>(cd, ba, st, nwg);
       } else {
         return hipErrorInvalidValue;
       }
@@ -3384,9 +3535,7 @@ static int launch_one(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, i
     cg.chunk_stride = chunk_stride(g);
     hipLaunchKernelGGL((eri_group_kernel<LA, LB, LC, LD>), dim3((unsigned)g), dim3(64), 0, st, cg, ba);
   } else {
-    using S = Coop<LA, LB, LC, LD>;
-    const int64_t g = n < nwg ? n : nwg;
-    hipLaunchKernelGGL((eri_coop_kernel<LA, LB, LC, LD>), dim3((unsigned)g), dim3(S::NT), 0, st, cd, ba);
+    return launch_coop<LA, LB, LC, LD>(cd, ba, st, nwg);
   }
   return hipGetLastError();
 }
@@ -3404,14 +3553,6 @@ static int prepare_one() {
     return e;
   }
   return hipSuccess;
-}
-
-template <int LA, int LB, int LC, int LD>
-static int64_t scratch_one() {
-  if constexpr (use_small<LA, LB, LC, LD>() || Grp<LA, LB, LC, LD>::fits)
-    return 0;
-  else
-    return Coop<LA, LB, LC, LD>::scratch();
 }
 
 // class c -> angular momenta (A >= B within a pair: the higher-L shell first)
@@ -3435,7 +3576,6 @@ static int64_t scratch_one() {
 // group launch; without the macro (-2) one unit holds everything.
 #define DECL_CLASS(id, a, b, cc, d)                                                       \
   int launch_class_##id(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, int nwg); \
-  int64_t scratch_class_##id();                                                            \
   int prepare_class_##id();
 LIBERI_CLASS_LIST(DECL_CLASS)
 #undef DECL_CLASS
@@ -3444,7 +3584,6 @@ LIBERI_CLASS_LIST(DECL_CLASS)
   int launch_class_##id(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, int nwg) { \
     return launch_one<a, b, cc, d>(cd, ba, st, nwg);                                        \
   }                                                                                         \
-  int64_t scratch_class_##id() { return scratch_one<a, b, cc, d>(); }                      \
   int prepare_class_##id() { return prepare_one<a, b, cc, d>(); }
 
 #if LIBERI_UNIT == -2
@@ -3689,17 +3828,6 @@ int prepare_class(int c) {
   }
 }
 
-int64_t class_scratch_doubles(int c) {
-  switch (c) {
-#define X(id, a, b, cc, d) \
-  case id:                 \
-    return scratch_class_##id();
-    LIBERI_CLASS_LIST(X)
-#undef X
-    default:
-      return 0;
-  }
-}
 #endif
 
 }  // namespace liberi

@@ -103,7 +103,10 @@ struct ClassDev {
   // of component k of pair p is base + k * n + p
   int64_t fix_base, mov_base;
   int32_t fix_n, mov_n;
-  // group kernels: chunk_stride(grid) of the launch (set at launch)
+  // the bra and the ket pairs' classes in the pair-major form: element of
+  // component k of pair p is bra_q + p * components + k
+  int64_t bra_q, ket_q;
+  // group and cooperative kernels: chunk_stride(grid) of the launch (set at launch)
   int64_t chunk_stride;
   // 1: the mixed form may evaluate this class's quartets in FP32 (chosen per
   // class at the first build under a given switch tau)
@@ -119,7 +122,8 @@ struct ClassDev {
 // consecutive pairs are neighbours in memory: the Coulomb sums of a row
 // tile's moving pairs are added there instead of to F, 64 lanes to 64
 // consecutive doubles (measured 187 G atomic adds/s against 23.7 G to
-// scattered ones).
+// scattered ones).  The pair-major form has component k of pair p at
+// off[c] + (p - first[c]) * components + k.
 struct PairLayout {
   int64_t off[kNumPairClasses + 1];
   int32_t n[kNumPairClasses], first[kNumPairClasses];
@@ -128,19 +132,27 @@ struct PairLayout {
   int32_t chunks[kNumPairClasses], block[kNumPairClasses + 1];
 };
 
+// the densities of BuildArgs the start of a build fills
+struct BuildWork {
+  double *Dp, *Dq, *Dsq;
+};
+
 struct BuildArgs {
   const PairRec *pairs;
   const PrimRec *prims;
   const double *D;   // density of the Coulomb blocks (packed)
   const double *DK;  // density of the exchange blocks (= D for RHF, packed)
-  const double *Dp;  // D in the pair layout
+  const double *Dp, *Dq;  // D in the pair layout, component- and pair-major
   const double *Dsq;  // DK as a full nbf x nbf matrix
-  double *Jp;        // Coulomb sums in the pair layout, added to F at the end
+  // sums that the end of the build adds to F: Coulomb blocks in the pair
+  // layout, component-major (kernels with a pair per lane) and pair-major
+  // (kernels with a pair's components over the lanes), and exchange blocks as a
+  // full matrix, rows the functions of one pair and columns those of the
+  // other, so that a block's rows are runs of consecutive elements
+  double *Jp, *Jq, *Ksq;
   double k_scale;    // exchange weight (1 for RHF: F = J[D] - K[D]/2; 2 for a UHF spin: J[Da+Db] - K[Ds])
   double *F;
   double value_cut;
-  double *scratch;       // per-workgroup scratch for the cooperative kernels
-  int64_t scratch_per_wg;  // doubles
   int32_t nbf;           // basis functions
   // compact columns of the row-tiled accumulators: the functions of angular
   // momentum L in shell order, col_bf[L][k] = basis function of column k
@@ -160,8 +172,6 @@ int class_has_split(int c);
 // dynamic LDS above 64 KB), on the current device; called at setup, outside
 // any stream capture.  Returns hipError_t.
 int prepare_class(int c);
-// doubles of scratch the cooperative kernel of class c needs per workgroup (0 if none)
-int64_t class_scratch_doubles(int c);
 // Rys roots of class c and the end of its tabulated range
 int class_nroots(int c);
 double class_rys_xmax(int c);
@@ -178,8 +188,8 @@ double class_row_chain(int c, int64_t primq);
 // kernel shape of class c: 0 lane per quartet, 1 workgroup group per
 // quartet, 2 cooperative workgroup per quartet
 int class_kernel_kind(int c);
-// 1 when group class c also has the cooperative workgroup-per-quartet form
-// with its buffers in LDS (classes with an f shell), selected by ClassDev::coop
+// 1 when group class c also has the cooperative form ((dd|dd) and the classes
+// with an f shell), selected by ClassDev::coop
 int class_has_coop(int c);
 
 // Fused group launch: one work item = quartets [c0, c1) of class cls (relative
@@ -220,8 +230,8 @@ constexpr double kRowWaves = 1740;  // 1024 SIMDs, 1.7 waves each
 constexpr int64_t kRowSteps = 1024;
 // LDS the row-tiled kernel may take per workgroup
 constexpr int64_t kRowLdsBytes = 64 * 1024;
-// workgroups the cooperative kernels use
-constexpr int kCoopWorkgroups = 2048;
+// workgroups the cooperative kernels use at most
+constexpr int kCoopWorkgroups = 8192;
 // one-wave workgroups the group-per-quartet kernels use at most (persistent loop)
 constexpr int kGroupWorkgroups = 65536;
 
@@ -276,9 +286,9 @@ void schwarz_scatter(const SchwarzStage &s, const double *out, double *schwrz_in
 // records the message of liberi_c_last_error and returns code
 int set_last_error(int code, const std::string &msg);
 
-// start of a build (F and Jp zeroed, Dp and Dsq filled from D and DK) and its
-// end (Jp added to F)
-int launch_build_begin(const BuildArgs &ba, const PairLayout &pl, double *Dp, double *Dsq, void *stream);
+// start of a build (F and the sums zeroed, Dp, Dq and Dsq filled from D and
+// DK) and its end (the sums added to F)
+int launch_build_begin(const BuildArgs &ba, const PairLayout &pl, const BuildWork &w, void *stream);
 int launch_build_end(const BuildArgs &ba, const PairLayout &pl, void *stream);
 
 // p[0..n) = 0 on the stream (a kernel, so it may sit in a captured graph)

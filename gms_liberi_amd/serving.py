@@ -71,10 +71,11 @@ def estimate_device_bytes(basis: Basis) -> int:
     # few segments (16 B) and tiles (12 B); a pair class serves as the rows of at
     # most ~10 classes
     tables = sum(10 * 60 * n for n in pcount.values())
-    # the density and the Coulomb sums by shell pair, the square density
+    # the density and the Coulomb sums by shell pair (twice each), the square
+    # density and exchange sums
     ncart = [1, 3, 6, 10]
     by_pair = sum(n * ncart[a] * ncart[b] for (a, b), n in pcount.items())
-    return int(64 * (npairs + nprim) + 8 * (3 * ntri + 2 * by_pair + basis.num_bas ** 2) + tables + 4 * basis.num_bas
+    return int(64 * (npairs + nprim) + 8 * (3 * ntri + 4 * by_pair + 2 * basis.num_bas ** 2) + tables + 4 * basis.num_bas
                + (1 << 20))
 
 

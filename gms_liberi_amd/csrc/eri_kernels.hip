@@ -174,6 +174,49 @@ __device__ __forceinline__ void rys_rule(double X, double xswitch, double (&u)[N
   }
 }
 
+// The rule of a primitive quartet and the reciprocal square root it goes with.
+// With s = p + q and t = p q |P - Q|^2 (X = t / s): below the switch r = 1/sqrt(s)
+// and u, w from the table; above it r = 1/sqrt(t) and u, w the constants of
+// the asymptotic rule, u/X and w/sqrt(X).  Either way u r^2 is u/(p+q) and
+// w r is w/sqrt(p+q), all that the integrals take from them, so the lanes
+// above the switch need no second reciprocal square root and no division: a
+// wave with lanes on both sides, most of them in a large molecule, evaluates
+// one.
+template <int N>
+__device__ __forceinline__ void rys_pair(double p, double q, double r2, double xswitch, double &r, double (&u)[N],
+                                         double (&w)[N], const double *tab, int istride) {
+  const double s = p + q, t = p * q * r2;
+  // (the margin covers the rounding of x: below the switch x never leaves the
+  // intervals of the table)
+  const bool below = t < xswitch * (1.0 - 4e-15) * s;
+  r = nr_rsqrt(below ? s : t);
+  if (below) {
+    constexpr int DG = rys_deg(N);
+    constexpr double IH = rys_inv_h(N);
+    const double x = t * (r * r);
+    const int j = (int)(x * IH);
+    const double y = x * (2.0 * IH) - (double)(2 * j + 1);
+    const double *c = tab + __mul24(j, istride);
+#pragma unroll
+    for (int k = 0; k < 2 * N; ++k) {
+      const double *ck = c + k * (DG + 1);
+      double acc = ck[DG];
+#pragma unroll
+      for (int i = DG - 1; i >= 0; --i) acc = fma(acc, y, ck[i]);
+      if (k < N)
+        u[k] = acc;
+      else
+        w[k - N] = acc;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      u[k] = rys_herm_u[N][k];
+      w[k] = rys_herm_w[N][k];
+    }
+  }
+}
+
 // one root of the rule (used by the cooperative kernels: one lane per root)
 template <int N>
 __device__ __forceinline__ void rys_root(double X, double xswitch, int r, double &u, double &w) {
@@ -457,23 +500,20 @@ __device__ __forceinline__ void small_integrals(const PairRec &bra, const PairRe
 
   // one primitive quartet into acc
   auto prim = [&](const PrimRec &P, const PrimRec &Q) {
-    const double rs = nr_rsqrt(P.p + Q.p), ipq = rs * rs;  // 1/sqrt(p+q), 1/(p+q)
     const double pqx = P.Px - Q.Px, pqy = P.Py - Q.Py, pqz = P.Pz - Q.Pz;
-    const double rho = P.p * Q.p * ipq;
-    const double X = rho * (pqx * pqx + pqy * pqy + pqz * pqz);
-    const double pref = kTwoPi52 * P.K * Q.K * rs;
-    double u[NR], w[NR];
-    rys_rule<NR>(X, xswitch, u, w, tab, istride);
-    const T tp = (T)P.p, tq = (T)Q.p, tipq = (T)ipq;
+    double rs, u[NR], w[NR];
+    rys_pair<NR>(P.p, Q.p, pqx * pqx + pqy * pqy + pqz * pqz, xswitch, rs, u, w, tab, istride);
+    const double rs2 = rs * rs;
+    // (the factors of the outer loop's record first)
+    const double pref = (KET_OUTER ? kTwoPi52 * Q.K * P.K : kTwoPi52 * P.K * Q.K) * rs;
+    const T tp = (T)P.p, tq = (T)Q.p;
     const T hp = (T)0.5 * nr_rcp(tp), hq = (T)0.5 * nr_rcp(tq);
     const T tpqx = (T)pqx, tpqy = (T)pqy, tpqz = (T)pqz;
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-      const T t2 = (T)u[r];
-      const T b00 = (T)0.5 * t2 * tipq;
-      const T b10 = hp - hp * tq * t2 * tipq;
-      const T b01 = hq - hq * tp * t2 * tipq;
-      const T fa = tq * tipq * t2, fc = tp * tipq * t2;
+      const T t2 = (T)(u[r] * rs2);  // u/(p+q)
+      const T fa = tq * t2, fc = tp * t2;
+      const T b00 = (T)0.5 * t2, b10 = hp - hp * fa, b01 = hq - hq * fc;
       T gx[NI][NK], gy[NI][NK], gz[NI][NK];
       rys_2d<NI, NK>(gx, (T)P.PAx - fa * tpqx, (T)Q.PAx + fc * tpqx, b10, b01, b00, (T)1);
       rys_2d<NI, NK>(gy, (T)P.PAy - fa * tpqy, (T)Q.PAy + fc * tpqy, b10, b01, b00, (T)1);
@@ -735,6 +775,29 @@ __host__ __device__ inline int64_t rys_table_used(int n, double xswitch) {
   return rys_table_intervals(n, xswitch) * rys_lds_stride(n);
 }
 
+// The N-root table below xswitch copied into LDS by the workgroup, intervals
+// at their odd stride; eight loads in flight per lane (a loop of single loads
+// took 4 to 10 us per workgroup, most of a small tile)
+template <int N>
+__device__ __forceinline__ void stage_rys_table(double *tab, double xswitch) {
+  constexpr int IN = rys_ncoef(N), LS = rys_lds_stride(N), U = 8;
+  const int ntab = (int)rys_table_intervals(N, xswitch) * IN, nt = (int)blockDim.x;
+  const double *src = rys_table + rys_offset[N];
+  for (int i0 = threadIdx.x; i0 < ntab; i0 += U * nt) {
+    double r[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int i = i0 + k * nt;
+      r[k] = src[i < ntab ? i : ntab - 1];
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int i = i0 + k * nt;
+      if (i < ntab) tab[(i / IN) * LS + i % IN] = r[k];
+    }
+  }
+}
+
 // Shape of a row tile of class (LA LB | LC LD).  The tile fixes one shell
 // pair (the bra pair, or with TR the ket pair): its shells give the rows of
 // the on-chip Fock accumulators.  The other ("moving") pair varies per
@@ -854,12 +917,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_ke
   // the class's Rys table below the switch, staged once per workgroup with
   // intervals padded to an odd stride
   double *tab = rows + NROW * ncols;
-  {
-    constexpr int IN = rys_ncoef(S::NR), LS = rys_lds_stride(S::NR);
-    const int ntab = (int)rys_table_intervals(S::NR, cd.xswitch) * IN;
-    const double *src = rys_table + rys_offset[S::NR];
-    for (int i = threadIdx.x; i < ntab; i += blockDim.x) tab[(i / IN) * LS + i % IN] = src[i];
-  }
+  stage_rys_table<S::NR>(tab, cd.xswitch);
 
   for (int i = threadIdx.x; i < NFIX + NROW * ncols; i += blockDim.x) lds[i] = 0.0;
 
@@ -1218,6 +1276,8 @@ __device__ __forceinline__ void split_integrals(const PairRec &bra, const PairRe
   for (int i = 0; i < NEP * NFP; ++i) acc[i] = 0.0;
 
   auto prim = [&](const PrimRec &Pp, const PrimRec &Q) {
+    // (the one-square-root rule of rys_pair holds more of its values at once
+    // and spills here: (dd|ds) 2.85 -> 3.73 ms, (dd|dp) 5.13 -> 5.91 on C60)
     const double rs = nr_rsqrt(Pp.p + Q.p), ipq = rs * rs;
     const double pqx = Pp.Px - Q.Px, pqy = Pp.Py - Q.Py, pqz = Pp.Pz - Q.Pz;
     const double X = Pp.p * Q.p * ipq * (pqx * pqx + pqy * pqy + pqz * pqz);
@@ -1556,12 +1616,7 @@ __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_ke
   const int ncols = (int)row_columns<LA, LB, LC, LD, TR>(ba.ncol);
   const int off2 = R::M1 == R::M2 ? 0 : ba.ncol[R::M1];
   double *tab = rows + NROW * ncols;
-  {
-    constexpr int IN = rys_ncoef(P::NR), LS = rys_lds_stride(P::NR);
-    const int ntab = (int)rys_table_intervals(P::NR, cd.xswitch) * IN;
-    const double *src = rys_table + rys_offset[P::NR];
-    for (int i = threadIdx.x; i < ntab; i += blockDim.x) tab[(i / IN) * LS + i % IN] = src[i];
-  }
+  stage_rys_table<P::NR>(tab, cd.xswitch);
   const RowTile tl = cd.tiles[blockIdx.x];
   const int64_t q0 = tl.q0, q1 = q0 + tl.n;
   const int seg0 = tl.seg;
@@ -1665,8 +1720,9 @@ struct Coop {
   // column slices: halves of shell C's components when |cd) has more than 64
   static constexpr int CS = NCD > 64 && NC % 2 == 0 ? 2 : 1;
   static constexpr int NCS = NC / CS, NV = NCS * ND;
-  // quartets per wave where several blocks' rows fit its lanes; waves over the rows
-  static constexpr int Q = NAB <= 32 ? 64 / NAB : 1;
+  // quartets per wave where several blocks' rows (and table lanes) fit its
+  // lanes; waves over the rows
+  static constexpr int Q = NAB > 32 ? 1 : (64 / NAB < 64 / (3 * NR) ? 64 / NAB : 64 / (3 * NR));
   static constexpr int WR = (NAB + 63) / 64, RW = (NAB + WR - 1) / WR;
   static constexpr int W = WR * CS, NT = 64 * W;
   // H of one root and direction: rows (a, b) of NK values, odd stride
@@ -3460,15 +3516,18 @@ int64_t row_lds(const int32_t *ncol, double xswitch) {
   }
 }
 
-// (dd|dd) and the group classes with an f shell also have the cooperative
-// form; which one runs is timed per class (on the 20-atom C-N chain it takes
+// (dd|dd), (fs|fs) and the group classes with an f shell also have the
+// cooperative form; which one runs is timed per class (on the 20-atom C-N chain it takes
 // (fd|dd) 1.29 -> 0.53 ms, (fd|fd) 1.08 -> 0.39, (ff|dp) 1.40 -> 0.49; on C60
 // (dd|dd) 2.92 -> 2.61).  The other d classes run faster wave-split or grouped
 // wherever they are large: (dd|dp) 5.1 ms, (dp|dp) 4.4 on C60.
 template <int LA, int LB, int LC, int LD>
 constexpr bool has_coop_alt() {
-  return !use_small<LA, LB, LC, LD>() && Grp<LA, LB, LC, LD>::fits &&
-         (LA == 3 || LB == 3 || LC == 3 || LD == 3 || LA + LB + LC + LD == 8);
+  // (fs|fs) is the one lane class that spills its whole block and whose rows
+  // and table exceed the LDS of the row-tiled form: 3-atom chain 0.28 -> 0.06
+  // ms, 20-atom chain 0.54 -> 0.40
+  if (use_small<LA, LB, LC, LD>()) return LA + LB + LC + LD >= 6;
+  return Grp<LA, LB, LC, LD>::fits && (LA == 3 || LB == 3 || LC == 3 || LD == 3 || LA + LB + LC + LD == 8);
 }
 
 template <int LA, int LB, int LC, int LD, bool TR>
@@ -3509,6 +3568,11 @@ static int launch_one(const ClassDev &cd, const BuildArgs &ba, hipStream_t st, i
     const int tpb = 256;
     if (cd.row_mode) {
       return cd.transposed ? launch_row<LA, LB, LC, LD, true>(cd, ba, st) : launch_row<LA, LB, LC, LD, false>(cd, ba, st);
+    } else if (cd.coop) {
+      if constexpr (has_coop_alt<LA, LB, LC, LD>())
+        return launch_coop<LA, LB, LC, LD>(cd, ba, st, nwg);
+      else
+        return hipErrorInvalidValue;
     } else {
       hipLaunchKernelGGL((eri_small_kernel<LA, LB, LC, LD>), dim3((unsigned)((n + tpb - 1) / tpb)), dim3(tpb), 0,
                          st, cd, ba);

@@ -111,7 +111,7 @@ struct ClassDev {
   // 1: the mixed form may evaluate this class's quartets in FP32 (chosen per
   // class at the first build under a given switch tau)
   int32_t fp32;
-  // 1: a group class with a cooperative form (class_has_coop) runs that form
+  // 1: a class with a cooperative form (class_has_coop) runs that form
   int32_t coop;
 };
 
@@ -188,8 +188,8 @@ double class_row_chain(int c, int64_t primq);
 // kernel shape of class c: 0 lane per quartet, 1 workgroup group per
 // quartet, 2 cooperative workgroup per quartet
 int class_kernel_kind(int c);
-// 1 when group class c also has the cooperative form ((dd|dd) and the classes
-// with an f shell), selected by ClassDev::coop
+// 1 when class c also has the cooperative form ((dd|dd), (fs|fs) and the group
+// classes with an f shell), selected by ClassDev::coop
 int class_has_coop(int c);
 
 // Fused group launch: one work item = quartets [c0, c1) of class cls (relative

@@ -1088,9 +1088,26 @@ static void set_tuned_choice(int c, int64_t nq, double tau, int v) {
   g_tuned[{c, size_bucket(nq), tau}] = v;
 }
 
+// Measured time of a class's launch and its primitive quartets, by class and
+// size as above: later handles scale it to theirs.
+static std::map<std::pair<int, int>, std::pair<float, int64_t>> g_class_ms;
+
+static float scaled_class_ms(int c, int64_t nq, int64_t primq) {
+  std::lock_guard<std::mutex> lk(g_tune_mu);
+  auto it = g_class_ms.find({c, size_bucket(nq)});
+  if (it == g_class_ms.end()) return -1.f;
+  return it->second.first * (float)((double)std::max<int64_t>(primq, 1) / (double)std::max<int64_t>(it->second.second, 1));
+}
+
+static void set_class_ms(int c, int64_t nq, int64_t primq, float ms) {
+  std::lock_guard<std::mutex> lk(g_tune_mu);
+  g_class_ms[{c, size_bucket(nq)}] = {ms, primq};
+}
+
 static void forget_tuned_choices() {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tuned.clear();
+  g_class_ms.clear();
 }
 
 // Whether class c runs its row-tiled kernel in this build.
@@ -1254,12 +1271,21 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     cs_.fp32 = best[1] < (1.f - kFp32Gain) * best[0] ? 1 : 0;
     set_tuned_choice(c, nq, h->fp32_tau, cs_.fp32);
   }
-  // one timed launch of every class not timed above: the measured times
-  // order the classes over the side streams
+  // the time of every class not timed above, which spreads the classes over
+  // the side streams: from an earlier handle, or the second of two launches
+  // (the first one of a kernel in the process loads its code, up to
+  // milliseconds)
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
-    if (!cs_.active || cs_.ms >= 0.f || (h->only_class >= 0 && c != h->only_class)) continue;
-    if (int rc = time_class(h, ba, st, c, class_row_mode(h, c), cs_.fp32 == 1, cs_.ms)) return rc;
+    if (!cs_.active || (h->only_class >= 0 && c != h->only_class)) continue;
+    const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin, primq = h->stats.prim_quartets[c];
+    if (cs_.ms < 0.f && (cs_.ms = scaled_class_ms(c, nq, primq)) >= 0.f) continue;
+    for (int rep = 0; cs_.ms < 0.f && rep < 2; ++rep) {
+      float ms = 0.f;
+      if (int rc = time_class(h, ba, st, c, class_row_mode(h, c), cs_.fp32 == 1, ms)) return rc;
+      if (rep == 1) cs_.ms = ms;
+    }
+    set_class_ms(c, nq, primq, cs_.ms);
   }
   return LIBERI_OK;
 }

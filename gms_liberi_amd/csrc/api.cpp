@@ -503,7 +503,7 @@ static int ncart_host(int l) { return (l + 1) * (l + 2) / 2; }
 // (the per-primitive-pair quantities of src/liberi_shell_pair.F90:416-459);
 // rank[s] = position of shell s among the shells of its angular momentum.
 static void append_pair(std::vector<PairRec> &pairs, std::vector<PrimRec> &prims, const std::vector<HostShell> &sh,
-                        const std::vector<int> *rank, int sA, int sB) {
+                        const std::vector<int> &rank, int sA, int sB) {
   const HostShell &A = sh[sA], &B = sh[sB];
   PairRec r{};
   r.prim_off = (int32_t)prims.size();
@@ -515,8 +515,8 @@ static void append_pair(std::vector<PairRec> &pairs, std::vector<PrimRec> &prims
   r.ABz = A.c[2] - B.c[2];
   r.sameAB = sA == sB;
   r.prim_stride = 1;
-  r.cA = rank ? (*rank)[sA] * ncart_host(A.l) : 0;
-  r.cB = rank ? (*rank)[sB] * ncart_host(B.l) : 0;
+  r.cA = rank[sA] * ncart_host(A.l);
+  r.cB = rank[sB] * ncart_host(B.l);
   const double ab2 = r.ABx * r.ABx + r.ABy * r.ABy + r.ABz * r.ABz;
   for (int i = 0; i < A.k; ++i)
     for (int j = 0; j < B.k; ++j) {
@@ -664,7 +664,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     const int hi = std::max(sA, sB), lo = std::min(sA, sB);
     pair_x.push_back(schwrz[(int64_t)hi * (hi + 1) / 2 + lo]);
     class_pairs[pc].push_back((int32_t)pairs.size());
-    append_pair(pairs, prims, sh, &rank, sA, sB);
+    append_pair(pairs, prims, sh, rank, sA, sB);
     pairs.back().x = pair_x.back();
   };
   for (int pc = 0; pc < kNumPairClasses; ++pc) {
@@ -1593,24 +1593,18 @@ int liberi_c_schwarz(int32_t nsh, int32_t natoms, int32_t num_bas, int32_t mxgto
                              atom_num, atom_loc, exponents, cs, cp, cd, cf, coords, s))
     return rc;
   if (int rc = schwarz_check_device("liberi_c_schwarz")) return rc;
-  void *dp = nullptr, *dq = nullptr, *dl = nullptr, *dout = nullptr;
+  void *buf = nullptr;
   hipStream_t st = nullptr;
-  auto release = [&]() {
-    if (st) (void)hipStreamDestroy(st);
-    for (void *p : {dp, dq, dl, dout})
-      if (p) (void)hipFree(p);
-  };
-  std::vector<double> out(s.list.size());
+  std::vector<unsigned char> host;
+  std::vector<double> out(s.pairs.size());
   hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&dp, s.pairs.size() * sizeof(PairRec));
-  if (e == hipSuccess) e = hipMalloc(&dq, s.prims.size() * sizeof(PrimRec));
-  if (e == hipSuccess) e = hipMalloc(&dl, s.list.size() * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc(&dout, s.list.size() * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&buf, s.bytes);
+  if (e == hipSuccess) e = (hipError_t)schwarz_enqueue(s, (unsigned char *)buf, host, st);
   if (e == hipSuccess)
-    e = (hipError_t)schwarz_enqueue(s, (PairRec *)dp, (PrimRec *)dq, (int32_t *)dl, (double *)dout, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(out.data(), dout, out.size() * sizeof(double), hipMemcpyDeviceToHost, st);
+    e = hipMemcpyAsync(out.data(), (unsigned char *)buf + s.o_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
-  release();
+  if (st) (void)hipStreamDestroy(st);
+  if (buf) (void)hipFree(buf);
   if (e != hipSuccess)
     return fail(e == hipErrorOutOfMemory ? LIBERI_ENOMEM : LIBERI_EDEVICE,
                 std::string("liberi_c_schwarz: ") + hipGetErrorString(e));
@@ -1632,26 +1626,48 @@ int schwarz_stage(const char *who, int32_t nsh, int32_t natoms, int32_t num_bas,
   if (int rc = read_shells(who, nsh, natoms, num_bas, mxgtot, ang_mom, contr_num, sh_loc, atom_num, atom_loc,
                            exponents, cs, cp, cd, cf, coords, sh))
     return rc;
+  s = SchwarzStage{};
+  s.shells.resize(nsh);
+  std::vector<double> coef;
+  for (int i = 0; i < nsh; ++i) {
+    s.shells[i] = SchwarzShell{sh[i].c[0], sh[i].c[1], sh[i].c[2], (int32_t)s.ew.size(), sh[i].k};
+    s.ew.insert(s.ew.end(), sh[i].e, sh[i].e + sh[i].k);
+    coef.insert(coef.end(), sh[i].w, sh[i].w + sh[i].k);
+  }
+  s.ew.insert(s.ew.end(), coef.begin(), coef.end());
   // every shell pair i >= j, A = the shell of higher angular momentum, grouped by (la, lb)
-  std::vector<int32_t> by_l[16];
-  s.pairs.clear();
-  s.prims.clear();
-  s.where.clear();
-  s.list.clear();
+  const size_t np = (size_t)nsh * (nsh + 1) / 2;
+  size_t count[17] = {};
+  int64_t nprims = 0;
   for (int i = 0; i < nsh; ++i)
     for (int j = 0; j <= i; ++j) {
-      const int sA = sh[i].l >= sh[j].l ? i : j, sB = sA == i ? j : i;
-      by_l[sh[sA].l * 4 + sh[sB].l].push_back((int32_t)s.pairs.size());
-      s.where.push_back((int64_t)i * (i + 1) / 2 + j);
-      append_pair(s.pairs, s.prims, sh, nullptr, sA, sB);
+      ++count[std::max(sh[i].l, sh[j].l) * 4 + std::min(sh[i].l, sh[j].l) + 1];
+      nprims += (int64_t)sh[i].k * sh[j].k;
     }
-  if (s.prims.size() > (size_t)INT32_MAX || s.pairs.size() > (size_t)INT32_MAX)
+  if (nprims > (int64_t)INT32_MAX || np > (size_t)INT32_MAX)
     return fail(LIBERI_EARG, std::string(who) + ": basis too large for 32-bit pair indices");
-  for (int k = 0; k < 16; ++k) {
-    s.off[k] = s.list.size();
-    s.list.insert(s.list.end(), by_l[k].begin(), by_l[k].end());
-  }
-  s.off[16] = s.list.size();
+  for (int k = 0; k < 16; ++k) count[k + 1] += count[k];
+  std::copy(count, count + 17, s.off);
+  s.pairs.resize(np);
+  s.where.resize(np);
+  s.nprims = nprims;
+  int64_t at = 0, prim = 0;
+  for (int i = 0; i < nsh; ++i)
+    for (int j = 0; j <= i; ++j, ++at) {
+      const int sA = sh[i].l >= sh[j].l ? i : j, sB = sA == i ? j : i, g = sh[sA].l * 4 + sh[sB].l;
+      const int32_t n = sh[sA].k * sh[sB].k;
+      s.longest[g] = std::max(s.longest[g], n);
+      s.where[count[g]] = at;
+      s.pairs[count[g]++] = SchwarzPair{sA, sB, (int32_t)prim, n};
+      prim += n;
+    }
+  auto align256 = [](size_t n) { return (n + 255) / 256 * 256; };
+  s.o_shells = np * sizeof(SchwarzPair);
+  s.o_ew = s.o_shells + nsh * sizeof(SchwarzShell);
+  s.upload = s.o_ew + s.ew.size() * sizeof(double);
+  s.o_prims = align256(s.upload);
+  s.o_out = s.o_prims + align256((size_t)nprims * sizeof(PrimRec));
+  s.bytes = s.o_out + np * sizeof(double);
   return LIBERI_OK;
 }
 
@@ -1666,22 +1682,30 @@ int schwarz_check_device(const char *who) {
   return LIBERI_OK;
 }
 
-int schwarz_enqueue(const SchwarzStage &s, PairRec *dp, PrimRec *dq, int32_t *dl, double *dout, void *stream) {
+int schwarz_enqueue(const SchwarzStage &s, unsigned char *buf, std::vector<unsigned char> &host, void *stream) {
   hipStream_t st = (hipStream_t)stream;
-  hipError_t e = hipMemcpyAsync(dp, s.pairs.data(), s.pairs.size() * sizeof(PairRec), hipMemcpyHostToDevice, st);
+  host.resize(s.upload);
+  std::memcpy(host.data(), s.pairs.data(), s.pairs.size() * sizeof(SchwarzPair));
+  std::memcpy(host.data() + s.o_shells, s.shells.data(), s.shells.size() * sizeof(SchwarzShell));
+  std::memcpy(host.data() + s.o_ew, s.ew.data(), s.ew.size() * sizeof(double));
+  const auto *pairs = (const SchwarzPair *)buf;
+  const auto *shells = (const SchwarzShell *)(buf + s.o_shells);
+  auto *prims = (PrimRec *)(buf + s.o_prims);
+  auto *out = (double *)(buf + s.o_out);
+  hipError_t e = hipMemcpyAsync(buf, host.data(), s.upload, hipMemcpyHostToDevice, st);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(dq, s.prims.data(), s.prims.size() * sizeof(PrimRec), hipMemcpyHostToDevice, st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dl, s.list.data(), s.list.size() * sizeof(int32_t), hipMemcpyHostToDevice, st);
+    e = (hipError_t)launch_schwarz_records(pairs, (int32_t)s.pairs.size(), shells, (const double *)(buf + s.o_ew),
+                                           (int32_t)(s.ew.size() / 2), prims, st);
   for (int k = 0; k < 16 && e == hipSuccess; ++k) {
     const int32_t n = (int32_t)(s.off[k + 1] - s.off[k]);
-    if (n > 0) e = (hipError_t)launch_schwarz(k / 4, k % 4, dp, dq, dl + s.off[k], n, dout + s.off[k], st);
+    if (n > 0)
+      e = (hipError_t)launch_schwarz(k / 4, k % 4, pairs + s.off[k], shells, prims, n, s.longest[k], out + s.off[k], st);
   }
   return (int)e;
 }
 
 void schwarz_scatter(const SchwarzStage &s, const double *out, double *schwrz_int) {
-  for (size_t k = 0; k < s.list.size(); ++k) schwrz_int[s.where[s.list[k]]] = out[k];
+  for (size_t k = 0; k < s.pairs.size(); ++k) schwrz_int[s.where[k]] = out[k];
 }
 
 int set_last_error(int code, const std::string &msg) { return fail(code, msg); }

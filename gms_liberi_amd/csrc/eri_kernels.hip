@@ -3218,7 +3218,12 @@ __global__ void segment_lengths_kernel(const double *bra_x, const int32_t *bra_g
 // ------------------------------------------------------ Schwarz integrals
 // Schwarz value of a shell pair: sqrt(max over components |(ab|ab)|) of the
 // normalised cartesian components, the quantity the reference takes as
-// schwrz_int (src/interface/liberi_interface.F90:128).  One lane per pair;
+// schwrz_int (src/interface/liberi_interface.F90:128).  `team` adjacent lanes
+// (a power of two) share a pair, each taking every team-th of its primitive
+// quartets; (ij|kl) and (kl|ij) of the one pair are equal, so that only those
+// with ij >= kl are formed, the others counted twice.  A lane alone walked up
+// to 1296 quartets: 20-atom C-N chain, (ss| 566 -> 27 us, all groups 1190 ->
+// 197 us;
 // the 2-D Rys integrals G(i, k) of each root (i on A, k on C = A) are moved
 // to the diagonal (a b | a b) in one step with the binomial form of the
 // transfer relation, I(a,b,a,b) = sum_t sum_u C(b,t) C(b,u) AB^(2b-t-u)
@@ -3249,26 +3254,30 @@ __device__ __forceinline__ void diag_transfer(const double (&g)[NI][NI], double 
 }
 
 template <int LA, int LB>
-__global__ __launch_bounds__(64) void schwarz_kernel(const PairRec *pairs, const PrimRec *prims, const int32_t *list,
-                                                     int32_t n, double xswitch, double *out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64) void schwarz_kernel(const SchwarzPair *pairs, const SchwarzShell *shells,
+                                                     const PrimRec *prims, int32_t n, int team, double xswitch,
+                                                     double *out) {
+  const int i = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) / (unsigned)team);
+  const int part = (int)threadIdx.x & (team - 1);
   if (i >= n) return;
   constexpr int L = LA + LB, NR = L + 1, NI = L + 1;
   constexpr int NA = ncart(LA), NB = ncart(LB);
   constexpr Range<LA, LA> ra{};
   constexpr Range<LB, LB> rb{};
-  const PairRec pr = pairs[list[i]];
+  const SchwarzPair pr = pairs[i];
+  const SchwarzShell sa = shells[pr.a], sb = shells[pr.b];
+  const double abx = sa.x - sb.x, aby = sa.y - sb.y, abz = sa.z - sb.z;
   double acc[NA * NB];
 #pragma unroll
   for (int k = 0; k < NA * NB; ++k) acc[k] = 0.0;
-  for (int ip = 0; ip < pr.nprim; ++ip) {
+  for (int ip = 0, iq = part; ip < pr.nprim; ++ip) {
     const PrimRec P = prims[pr.prim_off + ip];
-    for (int iq = 0; iq < pr.nprim; ++iq) {
+    for (; iq <= ip; iq += team) {
       const PrimRec Q = prims[pr.prim_off + iq];
       const double pq = P.p + Q.p, ipq = 1.0 / pq;
       const double pqx = P.Px - Q.Px, pqy = P.Py - Q.Py, pqz = P.Pz - Q.Pz;
       const double X = P.p * Q.p * ipq * (pqx * pqx + pqy * pqy + pqz * pqz);
-      const double pref = kTwoPi52 * P.K * Q.K * sqrt(ipq);
+      const double pref = (iq < ip ? 2.0 : 1.0) * kTwoPi52 * P.K * Q.K * sqrt(ipq);
       double u[NR], w[NR];
       rys_rule<NR>(X, xswitch, u, w);
       const double hp = 0.5 / P.p, hq = 0.5 / Q.p;
@@ -3283,11 +3292,11 @@ __global__ __launch_bounds__(64) void schwarz_kernel(const PairRec *pairs, const
         {
           double g[NI][NI];
           rys_2d<NI, NI>(g, P.PAx - fa * pqx, Q.PAx + fc * pqx, b10, b01, b00, 1.0);
-          diag_transfer<LA, LB, NI>(g, pr.ABx, h[0]);
+          diag_transfer<LA, LB, NI>(g, abx, h[0]);
           rys_2d<NI, NI>(g, P.PAy - fa * pqy, Q.PAy + fc * pqy, b10, b01, b00, 1.0);
-          diag_transfer<LA, LB, NI>(g, pr.ABy, h[1]);
+          diag_transfer<LA, LB, NI>(g, aby, h[1]);
           rys_2d<NI, NI>(g, P.PAz - fa * pqz, Q.PAz + fc * pqz, b10, b01, b00, w[r] * pref);
-          diag_transfer<LA, LB, NI>(g, pr.ABz, h[2]);
+          diag_transfer<LA, LB, NI>(g, abz, h[2]);
         }
 #pragma unroll
         for (int a = 0; a < NA; ++a)
@@ -3296,7 +3305,11 @@ __global__ __launch_bounds__(64) void schwarz_kernel(const PairRec *pairs, const
             acc[a * NB + b] += h[0][ra.lx[a]][rb.lx[b]] * h[1][ra.ly[a]][rb.ly[b]] * h[2][ra.lz[a]][rb.lz[b]];
       }
     }
+    iq -= ip + 1;  // the team's next quartets, in the next row of the triangle
   }
+  for (int o = 1; o < team; o <<= 1)
+#pragma unroll
+    for (int k = 0; k < NA * NB; ++k) acc[k] += __shfl_xor(acc[k], o);
   double mx = 0.0;
 #pragma unroll
   for (int a = 0; a < NA; ++a)
@@ -3306,33 +3319,74 @@ __global__ __launch_bounds__(64) void schwarz_kernel(const PairRec *pairs, const
       const double v = fabs(acc[a * NB + b]) * sc * sc;
       mx = v > mx ? v : mx;
     }
-  out[i] = sqrt(mx);
+  if (part == 0) out[i] = sqrt(mx);
 }
 
-template <int LA, int LB>
-static int launch_schwarz_t(const PairRec *pairs, const PrimRec *prims, const int32_t *list, int32_t n, double *out,
-                            hipStream_t st) {
-  const int tpb = 64;
-  hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3((unsigned)((n + tpb - 1) / tpb)), dim3(tpb), 0, st, pairs,
-                     prims, list, n, rys_xmax_host[LA + LB + 1], out);
+// Primitive-pair records of the Schwarz pairs (the quantities of
+// src/liberi_shell_pair.F90:416-459): sixteen lanes a pair.  Forming them here
+// leaves 16 bytes a pair to copy in place of 64 a primitive pair.
+__global__ __launch_bounds__(256) void schwarz_records_kernel(const SchwarzPair *pairs, int32_t n,
+                                                              const SchwarzShell *shells, const double *e,
+                                                              const double *w, PrimRec *prims) {
+  const int i = (int)(blockIdx.x * 16u + threadIdx.x / 16u);
+  if (i >= n) return;
+  const SchwarzPair pr = pairs[i];
+  const SchwarzShell A = shells[pr.a], B = shells[pr.b];
+  const double abx = A.x - B.x, aby = A.y - B.y, abz = A.z - B.z;
+  const double ab2 = abx * abx + aby * aby + abz * abz;
+  for (int k = (int)threadIdx.x % 16; k < pr.nprim; k += 16) {
+    const int ia = k / B.k, ib = k - ia * B.k;
+    const double a = e[A.first + ia], b = e[B.first + ib], p = a + b;
+    PrimRec r;
+    r.p = p;
+    r.Px = (a * A.x + b * B.x) / p;
+    r.Py = (a * A.y + b * B.y) / p;
+    r.Pz = (a * A.z + b * B.z) / p;
+    r.PAx = r.Px - A.x;
+    r.PAy = r.Py - A.y;
+    r.PAz = r.Pz - A.z;
+    r.K = w[A.first + ia] * w[B.first + ib] * exp(-a * b / p * ab2) / p;
+    prims[pr.prim_off + k] = r;
+  }
+}
+
+int launch_schwarz_records(const SchwarzPair *pairs, int32_t n, const SchwarzShell *shells, const double *ew,
+                           int32_t nprim_total, PrimRec *prims, void *stream) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(schwarz_records_kernel, dim3(((unsigned)n + 15) / 16), dim3(256), 0, (hipStream_t)stream, pairs,
+                     n, shells, ew, ew + nprim_total, prims);
   return hipGetLastError();
 }
 
-int launch_schwarz(int la, int lb, const PairRec *pairs, const PrimRec *prims, const int32_t *list, int32_t n,
-                   double *out, void *stream) {
+template <int LA, int LB>
+static int launch_schwarz_t(const SchwarzPair *pairs, const SchwarzShell *shells, const PrimRec *prims, int32_t n,
+                            int32_t longest, double *out, hipStream_t st) {
+  // lanes for each primitive quartet of the longest pair, while the group's
+  // waves are at most eight per SIMD of the chip
+  const int64_t quartets = (int64_t)longest * (longest + 1) / 2;
+  int team = 1;
+  while (team < 64 && team < quartets && (int64_t)n * team * 2 <= 64 * 8192) team *= 2;
+  const unsigned per = 64u / (unsigned)team;
+  hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3(((unsigned)n + per - 1) / per), dim3(64), 0, st, pairs, shells,
+                     prims, n, team, rys_xmax_host[LA + LB + 1], out);
+  return hipGetLastError();
+}
+
+int launch_schwarz(int la, int lb, const SchwarzPair *pairs, const SchwarzShell *shells, const PrimRec *prims,
+                   int32_t n, int32_t longest, double *out, void *stream) {
   if (n <= 0) return hipSuccess;
   hipStream_t st = (hipStream_t)stream;
   switch (la * 4 + lb) {
-    case 0: return launch_schwarz_t<0, 0>(pairs, prims, list, n, out, st);
-    case 4: return launch_schwarz_t<1, 0>(pairs, prims, list, n, out, st);
-    case 5: return launch_schwarz_t<1, 1>(pairs, prims, list, n, out, st);
-    case 8: return launch_schwarz_t<2, 0>(pairs, prims, list, n, out, st);
-    case 9: return launch_schwarz_t<2, 1>(pairs, prims, list, n, out, st);
-    case 10: return launch_schwarz_t<2, 2>(pairs, prims, list, n, out, st);
-    case 12: return launch_schwarz_t<3, 0>(pairs, prims, list, n, out, st);
-    case 13: return launch_schwarz_t<3, 1>(pairs, prims, list, n, out, st);
-    case 14: return launch_schwarz_t<3, 2>(pairs, prims, list, n, out, st);
-    case 15: return launch_schwarz_t<3, 3>(pairs, prims, list, n, out, st);
+    case 0: return launch_schwarz_t<0, 0>(pairs, shells, prims, n, longest, out, st);
+    case 4: return launch_schwarz_t<1, 0>(pairs, shells, prims, n, longest, out, st);
+    case 5: return launch_schwarz_t<1, 1>(pairs, shells, prims, n, longest, out, st);
+    case 8: return launch_schwarz_t<2, 0>(pairs, shells, prims, n, longest, out, st);
+    case 9: return launch_schwarz_t<2, 1>(pairs, shells, prims, n, longest, out, st);
+    case 10: return launch_schwarz_t<2, 2>(pairs, shells, prims, n, longest, out, st);
+    case 12: return launch_schwarz_t<3, 0>(pairs, shells, prims, n, longest, out, st);
+    case 13: return launch_schwarz_t<3, 1>(pairs, shells, prims, n, longest, out, st);
+    case 14: return launch_schwarz_t<3, 2>(pairs, shells, prims, n, longest, out, st);
+    case 15: return launch_schwarz_t<3, 3>(pairs, shells, prims, n, longest, out, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -255,22 +255,41 @@ constexpr int64_t chunk_stride(int64_t grid) {
   }
 }
 
-// Schwarz values sqrt(max |(ab|ab)|) of the n shell pairs list[0..n) whose
-// shells have angular momenta la >= lb (A the la shell); out[i] for list[i].
-int launch_schwarz(int la, int lb, const PairRec *pairs, const PrimRec *prims, const int32_t *list, int32_t n,
-                   double *out, void *stream);
-
-// Schwarz integrals of a whole basis, host side (api.cpp): every shell pair
-// i >= j with its primitive pairs (A = the shell of higher angular momentum),
-// the pairs grouped by (la, lb) in `list` (group la*4+lb is
-// list[off[k] .. off[k+1])), and per pair its packed index i(i+1)/2 + j.
-struct SchwarzStage {
-  std::vector<PairRec> pairs;
-  std::vector<PrimRec> prims;
-  std::vector<int64_t> where;
-  std::vector<int32_t> list;
-  size_t off[17];
+// Schwarz integrals of a whole basis.  The host stages the shells and the
+// list of shell pairs; the primitive-pair records are formed on the device.
+struct SchwarzShell {
+  double x, y, z;
+  int32_t first, k;  // its exponents and coefficients in SchwarzStage::ew
 };
+// one shell pair, A the shell of higher angular momentum
+struct SchwarzPair {
+  int32_t a, b;            // shells
+  int32_t prim_off, nprim;  // its primitive records
+};
+// every shell pair i >= j, grouped by (la, lb) (group la*4+lb is
+// pairs[off[k] .. off[k+1])), per pair its packed index i(i+1)/2 + j, and the
+// longest primitive list of each group
+struct SchwarzStage {
+  std::vector<SchwarzShell> shells;
+  std::vector<double> ew;  // exponents of all shells, then their coefficients
+  std::vector<SchwarzPair> pairs;
+  std::vector<int64_t> where;
+  int64_t nprims = 0;
+  size_t off[17];
+  int32_t longest[16];
+  // byte offsets of the parts of the device buffer -- the stage (`upload`
+  // bytes in one copy: pairs | shells | ew), primitive records, results -- and
+  // its size
+  size_t o_shells, o_ew, upload, o_prims, o_out, bytes;
+};
+// the primitive-pair records of the staged pairs
+int launch_schwarz_records(const SchwarzPair *pairs, int32_t n, const SchwarzShell *shells, const double *ew,
+                           int32_t nprim_total, PrimRec *prims, void *stream);
+// Schwarz values sqrt(max |(ab|ab)|) of the n shell pairs `pairs`, whose
+// shells have angular momenta la >= lb and at most `longest` primitive pairs;
+// out[i] for pairs[i].
+int launch_schwarz(int la, int lb, const SchwarzPair *pairs, const SchwarzShell *shells, const PrimRec *prims,
+                   int32_t n, int32_t longest, double *out, void *stream);
 // checked basis -> stage (LIBERI_OK or a status with the message set)
 int schwarz_stage(const char *who, int32_t nsh, int32_t natoms, int32_t num_bas, int32_t mxgtot,
                   const int32_t *ang_mom, const int32_t *contr_num, const int32_t *sh_loc, const int32_t *atom_num,
@@ -278,10 +297,12 @@ int schwarz_stage(const char *who, int32_t nsh, int32_t natoms, int32_t num_bas,
                   const double *cd, const double *cf, const double *coords, SchwarzStage &s);
 // a gfx950 device is current (LIBERI_OK or LIBERI_EDEVICE with the message set)
 int schwarz_check_device(const char *who);
-// records and list uploaded into the given device buffers, one kernel per
-// (la, lb) group writing out[list position]; returns a hipError_t
-int schwarz_enqueue(const SchwarzStage &s, PairRec *dp, PrimRec *dq, int32_t *dl, double *dout, void *stream);
-// out (list order) -> schwrz_int (packed by shell pair)
+// the stage uploaded to the device buffer `buf` (s.bytes, 256-byte aligned) and
+// the kernels that leave the results at s.o_out (pair order); `host` receives
+// the upload and has to live until the stream has been waited for; returns a
+// hipError_t
+int schwarz_enqueue(const SchwarzStage &s, unsigned char *buf, std::vector<unsigned char> &host, void *stream);
+// out (pair order) -> schwrz_int (packed by shell pair)
 void schwarz_scatter(const SchwarzStage &s, const double *out, double *schwrz_int);
 // records the message of liberi_c_last_error and returns code
 int set_last_error(int code, const std::string &msg);

@@ -1,8 +1,7 @@
 // Schwarz integrals without any device allocation: liberi_c_schwarz_noalloc.
 //
-// liberi_c_schwarz allocates four device buffers (pair records, primitive-pair
-// records, the pair list, the results) and a stream per call, and frees them
-// again; hipFree synchronises the whole device, which stalls every other
+// liberi_c_schwarz allocates a device buffer (pair list, shells, primitive-pair
+// records, results) and a stream per call, and frees them again; hipFree synchronises the whole device, which stalls every other
 // build in flight, and neither call is allowed under HIP graph capture.  This
 // variant stages the same data in one library-owned device array, `scratch`,
 // and runs on the caller's stream.
@@ -23,7 +22,13 @@
 
 using namespace liberi;
 
-static __device__ __align__(256) unsigned char scratch[LIBERI_SCHWARZ_SCRATCH_BYTES];
+// The staged form takes less than the records the limit counts (16 bytes a
+// pair and 32 a shell against 68 a pair) but for the exponents and
+// coefficients, 16 bytes a primitive; K primitives make at least K^2/2
+// primitive pairs of 64 bytes, so at the limit of 64 MiB they take at most 16
+// sqrt(2^26/32) = 23 KB.
+constexpr size_t kScratchBytes = (size_t)LIBERI_SCHWARZ_SCRATCH_BYTES + (32 << 10);
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
 
@@ -65,16 +70,15 @@ extern "C" int liberi_c_schwarz_noalloc(int32_t nsh, int32_t natoms, int32_t num
   if (int rc = schwarz_stage(who, nsh, natoms, num_bas, mxgtot, ang_mom, contr_num, sh_loc, atom_num, atom_loc,
                              exponents, cs, cp, cd, cf, coords, s))
     return rc;
-  // layout of the staging area: pair records | primitive records | list | results
-  const size_t o_pairs = 0;
-  const size_t o_prims = o_pairs + align256(s.pairs.size() * sizeof(PairRec));
-  const size_t o_list = o_prims + align256(s.prims.size() * sizeof(PrimRec));
-  const size_t o_out = o_list + align256(s.list.size() * sizeof(int32_t));
-  const size_t need = o_out + s.list.size() * sizeof(double);
+  // the accepted bases are those whose whole records fit: 64 bytes per shell
+  // pair and per primitive pair, 12 for its index and result
+  const size_t np = s.pairs.size();
+  const size_t need = align256(np * sizeof(PairRec)) + align256((size_t)s.nprims * sizeof(PrimRec)) +
+                      align256(np * sizeof(int32_t)) + np * sizeof(double);
   if (need > (size_t)LIBERI_SCHWARZ_SCRATCH_BYTES)
     return set_last_error(LIBERI_ESIZE, std::string(who) + ": the basis needs " + std::to_string(need) +
                                             " bytes of staging (" + std::to_string(s.pairs.size()) +
-                                            " shell pairs, " + std::to_string(s.prims.size()) +
+                                            " shell pairs, " + std::to_string(s.nprims) +
                                             " primitive pairs), above the fixed " +
                                             std::to_string((long long)LIBERI_SCHWARZ_SCRATCH_BYTES) +
                                             " bytes; use liberi_c_schwarz");
@@ -82,12 +86,13 @@ extern "C" int liberi_c_schwarz_noalloc(int32_t nsh, int32_t natoms, int32_t num
   void *base = nullptr;
   if (int rc = scratch_address(who, &base)) return rc;
   unsigned char *b = (unsigned char *)base;
+  if (s.bytes > kScratchBytes)
+    return set_last_error(LIBERI_ESIZE, std::string(who) + ": staging area");  // (cannot happen, see kScratchBytes)
   hipStream_t st = (hipStream_t)stream;
-  std::vector<double> out(s.list.size());
-  hipError_t e = (hipError_t)schwarz_enqueue(s, (PairRec *)(b + o_pairs), (PrimRec *)(b + o_prims),
-                                             (int32_t *)(b + o_list), (double *)(b + o_out), st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(out.data(), b + o_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, st);
+  std::vector<unsigned char> host;
+  std::vector<double> out(np);
+  hipError_t e = (hipError_t)schwarz_enqueue(s, b, host, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(out.data(), b + s.o_out, np * sizeof(double), hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return set_last_error(LIBERI_EDEVICE, std::string(who) + ": " + hipGetErrorString(e));
   schwarz_scatter(s, out.data(), schwrz_int);

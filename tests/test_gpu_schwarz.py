@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from gms_liberi_amd import liberi
-from gms_liberi_amd.caseio import Case
+from gms_liberi_amd.caseio import Basis, Case
 
 GOLD = Path(__file__).resolve().parent / "golden"
 # The device engine moves the (e0|f0) integrals to (ab|ab) with the transfer
@@ -81,3 +81,30 @@ def test_schwarz_rejects_bad_basis():
     with pytest.raises(liberi.LiberiError) as e:
         liberi.schwarz(dataclasses.replace(b, exponents=bad))
     assert e.value.code == 1
+
+
+def _chain_basis(natoms, l, contr):
+    """One shell of angular momentum l per atom, contr[i mod len] primitives each."""
+    rng = np.random.default_rng([7, natoms, l])
+    k = np.array([contr[i % len(contr)] for i in range(natoms)])
+    nc, mx, one = (l + 1) * (l + 2) // 2, int(k.max()), np.arange(natoms) + 1
+    n, loc = int(k.sum()), np.concatenate([[0], np.cumsum(k)[:-1]]) + 1
+    coef = np.zeros((4, mx * natoms))
+    coef[l, :n] = rng.uniform(0.2, 1.0, n)
+    expo = np.ones(mx * natoms)
+    expo[:n] = np.exp(rng.uniform(np.log(0.2), np.log(40.0), n))
+    xyz = np.cumsum(rng.uniform(0.4, 0.9, (natoms, 3)), axis=0)
+    first = (one - 1) * nc + 1
+    return Basis(natoms, natoms, natoms * nc, mx, np.full(natoms, l + 1), k, loc, one, first, first, first + nc - 1, expo,
+                 *coef, xyz.ravel(), np.zeros(natoms * (natoms + 1) // 2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("natoms,l,contr", [(1, 0, [1]), (3, 0, [1, 2]), (5, 1, [1, 3]), (7, 0, [12, 1]), (4, 2, [2, 1]),
+                                            (2, 3, [1, 4]), (180, 0, [3, 1])])
+def test_schwarz_lanes_sharing_a_pair(natoms, l, contr, oracle):
+    """1 to 64 lanes share a pair, by the longest primitive list of the group
+    (1 to 144 here) and the number of pairs (180 atoms: fewer lanes than the
+    list asks for), pairs shorter than the lanes among them."""
+    b = _chain_basis(natoms, l, contr)
+    assert _close(liberi.schwarz(b), oracle.schwarz(b))

@@ -30,6 +30,8 @@ COMMON = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno
 
 # units the class kernels are spread over (each carries its own copy of the Rys tables)
 KERNEL_UNITS = 16
+# launches shared by several small classes, a unit each
+SHARED_LAUNCHES = 6
 # seconds a class's kernels take to compile, where that is above 5 (the wave-split forms)
 COMPILE_S = {36: 97, 38: 87, 19: 39, 35: 35, 37: 15, 33: 15, 30: 15, 14: 14, 15: 12, 29: 11, 18: 10, 34: 10, 17: 6}
 
@@ -55,6 +57,8 @@ def build(verbose: bool = True) -> Path:
     OBJ.mkdir(exist_ok=True)
     kernels = [HIPCC, *COMMON, "-c", str(CSRC / "eri_kernels.hip")]
     jobs = [[*kernels, "-DLIBERI_UNIT=-3", "-o", str(OBJ / "eri_fused.o")]]
+    for k in range(SHARED_LAUNCHES):
+        jobs.append([*kernels, f"-DLIBERI_UNIT={-10 - k}", "-o", str(OBJ / f"eri_shared{k}.o")])
     for g, classes in enumerate(kernel_units()):
         entries = " ".join("X(%d, %d, %d, %d, %d)" % (c, *CLASS_L[c]) for c in classes)
         jobs.append([*kernels, "-DLIBERI_UNIT=1", f"-DLIBERI_UNIT_LIST(X)={entries}", "-o", str(OBJ / f"eri_g{g}.o")])

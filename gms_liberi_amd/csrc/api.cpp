@@ -94,6 +94,11 @@ struct ClassState {
   DevBuf tiles[kNumTileLens];
   int32_t ntile[kNumTileLens] = {};
   ClassDev dev{};
+  // shared launch the class runs in (-1: none), its workgroups there and, in a
+  // row-tiled one, its tiles
+  int shared = -1;
+  int32_t shared_groups = 0;
+  DevBuf shared_tiles;
 };
 
 // Point the class's launch arguments at its row tiles of length kTileLens[k].
@@ -133,6 +138,9 @@ struct liberi_ctx {
   DevBuf fused_items, fused_cds, fused_head;
   int64_t fused_n = 0;
   int fused_nwg = 0;
+  // shared launches of small classes and the ClassDev of every class in them
+  SharedArgs shared[kSharedLaunches];
+  DevBuf shared_cds;
   bool fused = false;      // LIBERI_OPT_FUSED
   int row_orient = 0;      // LIBERI_OPT_ROW_ORIENT
   int tile_len = -1;       // LIBERI_OPT_TILE_LEN as an index into kTileLens; -1 chosen per class
@@ -233,6 +241,7 @@ static void release_device(liberi_ctx *h) {
     dev_free(c.seg_bra);
     dev_free(c.seg_ket0);
     for (int k = 0; k < kNumTileLens; ++k) dev_free(c.tiles[k]);
+    dev_free(c.shared_tiles);
     c = ClassState{};
   }
   dev_free(h->pairs);
@@ -240,6 +249,8 @@ static void release_device(liberi_ctx *h) {
   dev_free(h->dens);
   dev_free(h->fock);
   dev_free(h->aux);
+  for (auto &sa : h->shared) sa = SharedArgs{};
+  dev_free(h->shared_cds);
   dev_free(h->fused_items);
   dev_free(h->fused_cds);
   dev_free(h->fused_head);
@@ -543,6 +554,14 @@ static void append_pair(std::vector<PairRec> &pairs, std::vector<PrimRec> &prims
 // meet few common Fock rows.
 constexpr int64_t kFusedRounds = 32;
 
+// Classes of at most this many workgroups run in a shared launch: row tiles
+// of 256 lanes, and waves of the group and cooperative forms.  Larger classes
+// fill the chip by themselves, and in a shared launch they would run at the
+// registers of its largest class (12 atoms of the cage: 1024 / 4096 1.08 ms,
+// 2048 / 4096 1.10, 8192 / 32768 1.24; unrestricted 17-atom cluster 1.06, 0.97,
+// 0.98 ms; 41-atom cluster 5.24, 5.31, 5.40).
+constexpr int64_t kSharedRowGroups = 2048, kSharedWaveGroups = 4096;
+
 static int setup_fused(liberi_ctx *h) {
   std::vector<int> cls;
   for (int c = 0; c < kNumClasses; ++c)
@@ -573,13 +592,56 @@ static int setup_fused(liberi_ctx *h) {
   return LIBERI_OK;
 }
 
+// Proxy for the device time of class c (ms): primitive quartets x Rys roots x
+// sqrt(cartesian components).
+static double class_cost_proxy(const liberi_ctx *h, int c) {
+  const int la = kPairL[kClasses[c].bra][1], lb = kPairL[kClasses[c].bra][0];
+  const int lc = kPairL[kClasses[c].ket][1], ld = kPairL[kClasses[c].ket][0];
+  const double ncomp = (double)ncart_host(la) * ncart_host(lb) * ncart_host(lc) * ncart_host(ld);
+  return 1e-9 * (double)h->cls[c].nprimq * class_nroots(c) * std::sqrt(ncomp);
+}
+
+// The shared launches: of the classes with a place in one, those that do not
+// have it to themselves; the class with the longest workgroups first.
+static int setup_shared(liberi_ctx *h) {
+  std::vector<ClassDev> cds(kNumClasses);
+  for (int k = 0; k < kSharedLaunches; ++k) {
+    SharedArgs &sa = h->shared[k] = SharedArgs{};
+    std::vector<int> cls;
+    for (int c = 0; c < kNumClasses; ++c)
+      if (h->cls[c].shared == k) cls.push_back(c);
+    if (cls.size() < 2) {
+      for (int c : cls) h->cls[c].shared = -1;
+      continue;
+    }
+    auto per_group = [&](int c) { return class_cost_proxy(h, c) / h->cls[c].shared_groups; };
+    std::stable_sort(cls.begin(), cls.end(), [&](int a, int b) { return per_group(a) > per_group(b); });
+    int64_t at = 0;
+    for (int c : cls) {
+      ClassState &cs_ = h->cls[c];
+      ClassDev &d = cds[c] = cs_.dev;
+      d.tiles = (const RowTile *)cs_.shared_tiles.p;
+      d.ntile = cs_.shared_groups;
+      d.chunk_stride = chunk_stride(cs_.shared_groups);
+      d.fp32 = 0;
+      if (k < kSharedRowLaunches)
+        sa.lds = std::max(sa.lds, (int32_t)class_row_lds(c, d.transposed, h->ncol, d.xswitch));
+      sa.cls[sa.n] = c;
+      sa.first[sa.n++] = (int32_t)at;
+      at += cs_.shared_groups;
+      sa.first[sa.n] = (int32_t)at;
+    }
+  }
+  return dev_upload(h, h->shared_cds, cds);
+}
+
 // Row tiles of the quartets [q_begin, q_end) of class c, in launch order: the
 // rows of the fixed pairs with the most primitives first (the kept rows run
 // from few to many), the longest rows first among those.  Consecutive
 // segments of a row whose quartets are shared by the same number of lanes are
 // cut into tiles of `len` quartets at one lane each, fewer at more, or of what
-// one step of the workgroup holds where the class has few tiles.
-static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int64_t primq, int64_t len,
+// one step of the workgroup (`hold`) holds where the class has few tiles.
+static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int64_t primq, int64_t len, int64_t hold,
                                       const std::vector<int64_t> &sstart, const std::vector<int32_t> &sbra,
                                       const std::vector<int32_t> &sket0, const std::vector<PairRec> &pairs) {
   std::vector<RowTile> tiles;
@@ -592,7 +654,6 @@ static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int
     for (b = a; b < s1 && sbra[b] == sbra[a];) ++b;
     rows.push_back({a, b});
   }
-  const int64_t hold = class_row_quartets(c);
   if (q_end - q_begin <= hold * kRowSteps) len = std::min(len, hold);
   const double chain = class_row_chain(c, primq);
   auto team_of = [&](size_t s) {
@@ -992,7 +1053,8 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     }
     for (int k = 0; k < kNumTileLens; ++k) {
       std::vector<RowTile> tiles;
-      if (cs_.row_ok) tiles = row_tiles(c, d.q_begin, d.q_end, primq, kTileLens[k], sstart, sbra, sket0, pairs);
+      if (cs_.row_ok) tiles = row_tiles(c, d.q_begin, d.q_end, primq, kTileLens[k], class_row_quartets(c), sstart, sbra,
+                                        sket0, pairs);
       cs_.ntile[k] = (int32_t)tiles.size();
       if ((rc = dev_upload(h, cs_.tiles[k], tiles))) return rc;
     }
@@ -1016,8 +1078,28 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     h->stats.quartets[c] = d.q_end - d.q_begin;
     h->stats.prim_quartets[c] = primq;
     h->stats.total_quartets += d.q_end - d.q_begin;
+    // a place in a shared launch, where the class is small
+    const int sl = class_shared_launch(c, transposed);
+    const int64_t nq = d.q_end - d.q_begin;
+    if (sl >= 0 && nq > 0) {
+      int64_t groups = 0;
+      if (sl < kSharedRowLaunches) {
+        if (cs_.row_ok && nq <= kSharedRowThreads * kSharedRowGroups) {
+          const std::vector<RowTile> tiles =
+              row_tiles(c, d.q_begin, d.q_end, primq, kSharedRowThreads, kSharedRowThreads, sstart, sbra, sket0, pairs);
+          groups = (int64_t)tiles.size();
+          if (groups <= kSharedRowGroups && (rc = dev_upload(h, cs_.shared_tiles, tiles))) return rc;
+        }
+      } else {
+        groups = (nq + class_round_quartets(c) - 1) / class_round_quartets(c);
+      }
+      if (groups > 0 && groups <= (sl < kSharedRowLaunches ? kSharedRowGroups : kSharedWaveGroups)) {
+        cs_.shared = sl;
+        cs_.shared_groups = (int32_t)groups;
+      }
+    }
   }
-  if ((rc = setup_fused(h))) return rc;
+  if ((rc = setup_fused(h)) || (rc = setup_shared(h))) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   h->initialized = true;
   return LIBERI_OK;
@@ -1062,6 +1144,9 @@ int liberi_c_setup(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_bas, 
 constexpr int64_t kTuneMinQuartets = 20000;
 constexpr float kTileGain = 0.06f;
 constexpr int kSideStreams = 4;
+// latency of each shared launch, with few quartets in its classes (measured on
+// ethane and the 3-atom C-N chain, ms)
+constexpr double kSharedMs[kSharedLaunches] = {0.03, 0.06, 0.1, 0.05, 0.1, 0.08};
 
 // Choices made so far in this process: later handles (a request loop sets up
 // one per molecule) reuse them instead of timing again, but only for a class
@@ -1140,10 +1225,23 @@ static int time_class(liberi_ctx *h, const BuildArgs &ba, hipStream_t st, int c,
   return LIBERI_OK;
 }
 
+// Whether class c runs in its shared launch in this build: unless a form, a
+// tile length, the mixed form or a diagnostic is asked for, which the
+// launches of one class have.
+static bool class_shared(const liberi_ctx *h, int c) {
+  return h->cls[c].shared >= 0 && h->autotune && h->row_tiles == 1 && h->tile_len < 0 && !(h->fp32_tau > 0.0) &&
+         !h->fused && !h->class_timing && h->only_class < 0;
+}
+
 static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
     if (!cs_.active || cs_.variant >= 0) continue;
+    if (class_shared(h, c)) {  // the form of its shared launch
+      cs_.dev.coop = cs_.shared > kSharedGroupLaunch && class_has_coop(c);
+      cs_.variant = cs_.shared < kSharedRowLaunches ? 1 : cs_.dev.coop ? 3 : 0;
+      continue;
+    }
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
     // untimed choice: row tiles for the lane classes, and for the group
     // classes with a wave-split form unless the class is too small to time
@@ -1209,7 +1307,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     if (!cs_.active || cs_.tile >= 0) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
     cs_.tile = h->tile_len >= 0 ? h->tile_len : kDefaultTile;
-    if (h->tile_len >= 0 || !h->autotune || !class_row_mode(h, c) || nq < kTuneMinQuartets ||
+    if (h->tile_len >= 0 || !h->autotune || !class_row_mode(h, c) || nq < kTuneMinQuartets || class_shared(h, c) ||
         (h->only_class >= 0 && c != h->only_class)) {
       use_tiles(cs_, cs_.tile);
       continue;
@@ -1277,7 +1375,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
   // milliseconds)
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
-    if (!cs_.active || (h->only_class >= 0 && c != h->only_class)) continue;
+    if (!cs_.active || class_shared(h, c) || (h->only_class >= 0 && c != h->only_class)) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin, primq = h->stats.prim_quartets[c];
     if (cs_.ms < 0.f && (cs_.ms = scaled_class_ms(c, nq, primq)) >= 0.f) continue;
     for (int rep = 0; cs_.ms < 0.f && rep < 2; ++rep) {
@@ -1317,25 +1415,25 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
   // the fused group launch, where on: its classes leave the per-class launches
   const bool fused = h->fused && h->fused_n > 0 && !h->class_timing && h->only_class < 0;
   h->last_fused = fused;
-  std::vector<int> order;
+  // launches of the build, by cost (ms): a class (its measured time, else the
+  // proxy), or kNumClasses + k for shared launch k
+  auto cost = [&](int c) { return h->cls[c].ms >= 0.f ? (double)h->cls[c].ms : class_cost_proxy(h, c); };
+  std::vector<std::pair<double, int>> order;
+  double shared_cost[kSharedLaunches] = {};
   double fused_cost = 0.0;
   for (int c = 0; c < kNumClasses; ++c)
     if (h->cls[c].active && (h->only_class < 0 || c == h->only_class)) {
       if (fused && class_fused_nq(c) > 0) continue;
-      order.push_back(c);
+      if (class_shared(h, c))
+        shared_cost[h->cls[c].shared] += class_cost_proxy(h, c);
+      else
+        order.push_back({cost(c), c});
     }
+  for (int k = 0; k < kSharedLaunches; ++k)
+    if (shared_cost[k] > 0.0) order.push_back({kSharedMs[k] + shared_cost[k], kNumClasses + k});
   std::vector<double> load(ns, 0.0);
-  // cost: the class's measured time (first build), else a proxy scaled to
-  // milliseconds: primitive quartets x Rys roots x sqrt(cartesian components)
-  auto cost = [&](int c) {
-    if (h->cls[c].ms >= 0.f) return (double)h->cls[c].ms;
-    const int la = kPairL[kClasses[c].bra][1], lb = kPairL[kClasses[c].bra][0];
-    const int lc = kPairL[kClasses[c].ket][1], ld = kPairL[kClasses[c].ket][0];
-    const double ncomp = (double)ncart_host(la) * ncart_host(lb) * ncart_host(lc) * ncart_host(ld);
-    return 1e-9 * (double)h->cls[c].nprimq * class_nroots(c) * std::sqrt(ncomp);
-  };
   if (ns > 1) {
-    std::sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
+    std::sort(order.begin(), order.end(), std::greater<>());
     HIP_TRY(hipEventRecord(h->fork_ev, st));
     for (int k = 0; k < ns; ++k) HIP_TRY(hipStreamWaitEvent(h->side[k], h->fork_ev, 0));
   }
@@ -1357,12 +1455,17 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
     if (e != hipSuccess)
       return fail(LIBERI_EDEVICE, std::string("fused group launch: ") + hipGetErrorString((hipError_t)e));
   }
-  for (int c : order) {
+  for (const auto &[ms, c] : order) {
     hipStream_t cs = st;
     if (ns > 1) {
       const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-      load[k] += cost(c);
+      load[k] += ms;
       cs = h->side[k];
+    }
+    if (c >= kNumClasses) {
+      if (int e = launch_shared(c - kNumClasses, h->shared[c - kNumClasses], (const ClassDev *)h->shared_cds.p, ba, cs))
+        return fail(LIBERI_EDEVICE, std::string("shared launch: ") + hipGetErrorString((hipError_t)e));
+      continue;
     }
     if (h->class_timing && ns == 1) {
       if (!h->cev0[c]) HIP_TRY(hipEventCreate(&h->cev0[c]));
@@ -1423,9 +1526,12 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
   // (they also run before any build: Dp and Dsq from this build's density)
   const bool choose = [&] {
-    for (const ClassState &c : h->cls)
-      if (c.active && (c.variant < 0 || c.tile < 0 || c.ms < 0.f || (h->fp32_tau > 0.0 && c.fp32 < 0)))
+    for (int k = 0; k < kNumClasses; ++k) {
+      const ClassState &c = h->cls[k];
+      if (c.active && (c.variant < 0 || c.tile < 0 || (c.ms < 0.f && !class_shared(h, k)) ||
+                       (h->fp32_tau > 0.0 && c.fp32 < 0)))
         return true;
+    }
     return false;
   }();
   if (choose) {

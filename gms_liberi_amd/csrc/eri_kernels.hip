@@ -344,6 +344,33 @@ __device__ __forceinline__ PrimRec load_rec(ConstPrimRec *v, int64_t i) {
   r.K = q->K;
   return r;
 }
+typedef const ClassDev __attribute__((address_space(4))) ConstClassDev;
+__device__ __forceinline__ ClassDev load_rec(const ClassDev *v, int64_t i) {
+  ConstClassDev *q = (ConstClassDev *)v + i;
+  ClassDev c;
+  c.seg_start = q->seg_start;
+  c.seg_bra = q->seg_bra;
+  c.seg_ket0 = q->seg_ket0;
+  c.nseg = q->nseg;
+  c.diag = q->diag;
+  c.q_begin = q->q_begin;
+  c.q_end = q->q_end;
+  c.xswitch = q->xswitch;
+  c.tiles = q->tiles;
+  c.ntile = q->ntile;
+  c.row_mode = q->row_mode;
+  c.transposed = q->transposed;
+  c.fix_base = q->fix_base;
+  c.mov_base = q->mov_base;
+  c.fix_n = q->fix_n;
+  c.mov_n = q->mov_n;
+  c.bra_q = q->bra_q;
+  c.ket_q = q->ket_q;
+  c.chunk_stride = q->chunk_stride;
+  c.fp32 = q->fp32;
+  c.coop = q->coop;
+  return c;
+}
 __device__ __forceinline__ PairRec load_rec(ConstPairRec *v, int64_t i) {
   ConstPairRec *q = v + i;
   PairRec r;
@@ -895,8 +922,8 @@ constexpr int row_threads() {
   return 256;
 }
 
-template <int LA, int LB, int LC, int LD, bool TR>
-__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_kernel(ClassDev cd, BuildArgs ba) {
+template <int LA, int LB, int LC, int LD, bool TR, bool MIXED>
+__device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba, int tile, double *lds) {
   using S = Small<LA, LB, LC, LD>;
   using R = RowShape<LA, LB, LC, LD, TR>;
   constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND;
@@ -905,11 +932,11 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_ke
   constexpr Range<R::L2, R::L2> r2{};
   constexpr Range<R::M1, R::M1> rm1{};
   constexpr Range<R::M2, R::M2> rm2{};
-  extern __shared__ double lds[];  // jfix[NFIX], rows[NROW][ncols], then the Rys table
+  // lds: jfix[NFIX], rows[NROW][ncols], then the Rys table
   double *jfix_s = lds, *rows = lds + NFIX;
   const int ncols = (int)row_columns<LA, LB, LC, LD, TR>(ba.ncol);
   const int off2 = R::M1 == R::M2 ? 0 : ba.ncol[R::M1];
-  const RowTile tl = cd.tiles[blockIdx.x];
+  const RowTile tl = cd.tiles[tile];
   const int64_t q0 = tl.q0, q1 = q0 + tl.n;
   const int seg0 = tl.seg, team = tl.team;
   const int32_t ifix = cd.seg_bra[seg0];
@@ -939,7 +966,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_ke
     const PairRec &bra = TR ? mov : fix;
     const PairRec &ket = TR ? fix : mov;
     double v[S::NABCD];
-    if (mixed_wave(cd, ba, bra, ket)) {
+    if (MIXED && mixed_wave(cd, ba, bra, ket)) {
       nlow += part == 0;
       small_integrals<float, LA, LB, LC, LD, !TR, TR>(bra, ket, ba.prims, cd.xswitch, ba.value_cut, v, tab,
                                              rys_lds_stride(S::NR), part, team);
@@ -1097,7 +1124,7 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_ke
     }
   }
 
-  count_fp32(ba, nlow);
+  if constexpr (MIXED) count_fp32(ba, nlow);
   // the fixed pair's Coulomb block: reduce over each wave, then over the waves
   wave_sum_to_lds<NFIX>(jfix, jfix_s, [](int k) { return k; });
   __syncthreads();
@@ -1113,6 +1140,12 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_ke
     const int cbf = (R::M1 == R::M2 || k < off2) ? ba.col_bf[R::M1][k] : ba.col_bf[R::M2][k - off2];
     unsafeAtomicAdd(ba.Ksq + (int64_t)rbf * ba.nbf + cbf, x);
   }
+}
+
+template <int LA, int LB, int LC, int LD, bool TR>
+__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_kernel(ClassDev cd, BuildArgs ba) {
+  extern __shared__ double lds[];
+  row_run<LA, LB, LC, LD, TR, true>(cd, ba, (int)blockIdx.x, lds);
 }
 
 // ====================================================== wave-split row path
@@ -1789,13 +1822,13 @@ __device__ __forceinline__ void coop_accumulate(const double *h, int hx, int hy,
   }
 }
 
+// the quartets of workgroup blk of the nblk of the class
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT), 2) void eri_coop_kernel(ClassDev cd, BuildArgs ba) {
+__device__ __forceinline__ void coop_run(const ClassDev &cd, const BuildArgs &ba, int blk, int nblk, double *lds) {
   using S = Coop<LA, LB, LC, LD>;
   constexpr int NR = S::NR, NI = S::NI, NK = S::NK, NT = S::NT, Q = S::Q, KT = S::KT, W = S::W, CS = S::CS;
   constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND, NCS = S::NCS, NV = S::NV;
   constexpr int NAB = S::NAB, NCD = S::NCD, NAC = S::NAC, NBD = S::NBD, NAD = S::NAD;
-  __shared__ double lds[S::LDS_DOUBLES];
   double *uni = lds, *dens = lds + S::UNI;
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1824,8 +1857,8 @@ __global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT), 2) void eri_coop_kernel
   // quartets share the row's pair); the workgroups resident together work on
   // distant chunks
   const int64_t nq = cd.q_end - cd.q_begin;
-  const int64_t per = ((nq + gridDim.x - 1) / gridDim.x + Q - 1) / Q * Q;
-  const int64_t chunk = (int64_t)blockIdx.x * cd.chunk_stride % gridDim.x;
+  const int64_t per = ((nq + nblk - 1) / nblk + Q - 1) / Q * Q;
+  const int64_t chunk = (int64_t)blk * cd.chunk_stride % nblk;
   const int64_t c0 = cd.q_begin + chunk * per, c1 = c0 + per < cd.q_end ? c0 + per : cd.q_end;
   int sg = c0 < c1 ? find_segment(cd, c0, 0, cd.nseg) : 0;
 
@@ -2109,6 +2142,12 @@ __global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT), 2) void eri_coop_kernel
     coop_sync<W>();  // the tables and density blocks are overwritten by the next round
   }
   flush_jab();
+}
+
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__((Coop<LA, LB, LC, LD>::NT), 2) void eri_coop_kernel(ClassDev cd, BuildArgs ba) {
+  __shared__ double lds[Coop<LA, LB, LC, LD>::LDS_DOUBLES];
+  coop_run<LA, LB, LC, LD>(cd, ba, (int)blockIdx.x, (int)gridDim.x, lds);
 }
 
 // =================================================== group-per-quartet path
@@ -3800,6 +3839,215 @@ int class_fused_nq(int c) {
     return Grp<a, b, cc, d>::NQ;
     LIBERI_FUSED_LIST(X)
 #undef X
+    default:
+      return 0;
+  }
+}
+#endif
+
+// ------------------------------------------------------ shared launches
+// Small classes run together: one launch takes the workgroups of several
+// classes, each workgroup running its class's body.  A launch costs about 9 us
+// between its neighbours on a stream, and a class of few quartets 10 to 60 us
+// of latency (its code and tables read for the first time, one primitive chain,
+// one digestion) on an idle chip: 57 launches on four streams took 516 us for
+// the 3-atom C-N chain, 22 took 209 us for ethane.  The classes of a launch
+// have one form (its workgroup size) and about the same registers, since all
+// its workgroups get the registers of the largest.
+//
+// Entries (class, angular momenta, rows over the ket pairs) per launch.
+#define LIBERI_SHARED_0(X)                                                                                     \
+  X(0, 0, 0, 0, 0, false) X(1, 0, 0, 1, 0, true) X(2, 0, 0, 1, 1, true) X(3, 1, 0, 1, 1, true)                  \
+  X(4, 1, 0, 1, 0, false) X(6, 0, 0, 2, 0, true) X(7, 0, 0, 2, 1, true) X(8, 1, 0, 2, 0, true)                  \
+  X(22, 0, 0, 3, 0, true)
+#define LIBERI_SHARED_1(X)                                                                                     \
+  X(5, 1, 1, 1, 1, false) X(9, 1, 0, 2, 1, true) X(10, 0, 0, 2, 2, true) X(12, 1, 1, 2, 0, false)               \
+  X(13, 2, 0, 2, 0, false)
+#define LIBERI_SHARED_2(X)                                                                                     \
+  X(23, 0, 0, 3, 1, true) X(24, 0, 0, 3, 2, true) X(25, 1, 0, 3, 0, true) X(27, 3, 0, 1, 1, false)              \
+  X(28, 3, 0, 2, 0, false) X(32, 3, 1, 1, 0, false)
+#define LIBERI_SHARED_3(X)                                                                                     \
+  X(11, 1, 0, 2, 2) X(14, 2, 2, 1, 1) X(15, 2, 1, 2, 1) X(16, 2, 1, 2, 0) X(17, 2, 1, 1, 1) X(18, 2, 2, 2, 0)   \
+  X(19, 2, 2, 2, 1)
+#define LIBERI_SHARED_4(X)                                                                                     \
+  X(20, 2, 2, 2, 2) X(29, 2, 1, 3, 0) X(30, 2, 2, 3, 0) X(31, 3, 0, 3, 0) X(33, 3, 1, 1, 1) X(34, 3, 1, 2, 0)   \
+  X(35, 3, 1, 2, 1) X(36, 2, 2, 3, 1) X(37, 3, 1, 3, 0) X(38, 3, 1, 3, 1) X(39, 3, 2, 1, 0) X(41, 3, 2, 1, 1)   \
+  X(42, 3, 2, 2, 0) X(43, 3, 2, 2, 1) X(44, 3, 2, 2, 2) X(45, 3, 2, 3, 0) X(46, 3, 2, 3, 1) X(47, 3, 2, 3, 2)
+#define LIBERI_SHARED_5(X)                                                                                     \
+  X(26, 3, 3, 3, 0) X(40, 3, 3, 3, 1) X(48, 3, 3, 0, 0) X(49, 3, 3, 1, 0) X(50, 3, 3, 1, 1) X(51, 3, 3, 2, 0)   \
+  X(52, 3, 3, 2, 1) X(53, 3, 3, 2, 2) X(54, 3, 3, 3, 2)
+
+// the class of this workgroup and its place among the class's
+__device__ __forceinline__ int shared_entry(const SharedArgs &sa) {
+  int k = 0;
+  while (k + 1 < sa.n && (int)blockIdx.x >= sa.first[k + 1]) ++k;
+  return k;
+}
+
+#define DEF_SHARED_ROWS(N, WAVES)                                                                                 \
+  __global__ __launch_bounds__(256, WAVES) void eri_shared_##N##_kernel(SharedArgs sa, const ClassDev *cds, BuildArgs ba) { \
+    extern __shared__ double lds[];                                                                               \
+    const int k = shared_entry(sa), blk = (int)blockIdx.x - sa.first[k];                                          \
+    const ClassDev cd = load_rec(cds, sa.cls[k]);                                                                 \
+    switch (sa.cls[k]) { LIBERI_SHARED_##N(SHARED_ROW_CASE) default: break; }                                     \
+  }                                                                                                               \
+  int launch_shared_##N(const SharedArgs &sa, const ClassDev *cds, const BuildArgs &ba, hipStream_t st) {         \
+    hipLaunchKernelGGL(eri_shared_##N##_kernel, dim3((unsigned)sa.first[sa.n]), dim3(256), (unsigned)sa.lds, st, sa, \
+                       cds, ba);                                                                                  \
+    return hipGetLastError();                                                                                     \
+  }
+#define SHARED_ROW_CASE(id, a, b, cc, d, tr)             \
+  case id:                                               \
+    row_run<a, b, cc, d, tr, false>(cd, ba, blk, lds);   \
+    break;
+
+#define DEF_SHARED_COOP(N, NTHREADS)                                                                              \
+  constexpr int shared_lds_##N() {                                                                                \
+    int m = 0;                                                                                                    \
+    LIBERI_SHARED_##N(SHARED_COOP_LDS) return m;                                                                  \
+  }                                                                                                               \
+  __global__ __launch_bounds__(NTHREADS, 2) void eri_shared_##N##_kernel(SharedArgs sa, const ClassDev *cds, BuildArgs ba) { \
+    __shared__ double lds[shared_lds_##N()];                                                                      \
+    const int k = shared_entry(sa), blk = (int)blockIdx.x - sa.first[k], nblk = sa.first[k + 1] - sa.first[k];    \
+    const ClassDev cd = load_rec(cds, sa.cls[k]);                                                                 \
+    switch (sa.cls[k]) { LIBERI_SHARED_##N(SHARED_COOP_CASE) default: break; }                                    \
+  }                                                                                                               \
+  int launch_shared_##N(const SharedArgs &sa, const ClassDev *cds, const BuildArgs &ba, hipStream_t st) {         \
+    hipLaunchKernelGGL(eri_shared_##N##_kernel, dim3((unsigned)sa.first[sa.n]), dim3(NTHREADS), 0, st, sa, cds, ba); \
+    return hipGetLastError();                                                                                     \
+  }
+#define SHARED_COOP_LDS(id, a, b, cc, d) \
+  m = Coop<a, b, cc, d>::LDS_DOUBLES > m ? Coop<a, b, cc, d>::LDS_DOUBLES : m;
+#define SHARED_COOP_CASE(id, a, b, cc, d)                                                   \
+  case id:                                                                                  \
+    static_assert(Coop<a, b, cc, d>::NT == SHARED_COOP_NT, "threads of the shared launch"); \
+    coop_run<a, b, cc, d>(cd, ba, blk, nblk, lds);                                          \
+    break;
+
+#define SHARED_GROUP_LDS(id, a, b, cc, d) \
+  m = Grp<a, b, cc, d>::NQ * Grp<a, b, cc, d>::SLOT > m ? Grp<a, b, cc, d>::NQ * Grp<a, b, cc, d>::SLOT : m;
+#define SHARED_GROUP_NQ(id, a, b, cc, d) m = Grp<a, b, cc, d>::NQ > m ? Grp<a, b, cc, d>::NQ : m;
+#define SHARED_GROUP_CASE(id, a, b, cc, d)                                                                      \
+  case id: {                                                                                                    \
+    constexpr int NQ = Grp<a, b, cc, d>::NQ;                                                                    \
+    const int64_t per = ((nq + nblk - 1) / nblk + NQ - 1) / NQ * NQ, c0 = chunk * per;                          \
+    grp_run<a, b, cc, d>(cd, ba, c0, c0 + per < nq ? c0 + per : nq, lds, s_npq, s_nk, s_boff, s_koff, s_bst, s_kst); \
+    break;                                                                                                      \
+  }
+
+#if LIBERI_UNIT == -2 || LIBERI_UNIT == -10
+DEF_SHARED_ROWS(0, 4)
+#endif
+#if LIBERI_UNIT == -2 || LIBERI_UNIT == -11
+DEF_SHARED_ROWS(1, 2)
+#endif
+#if LIBERI_UNIT == -2 || LIBERI_UNIT == -12
+DEF_SHARED_ROWS(2, 2)
+#endif
+#if LIBERI_UNIT == -2 || LIBERI_UNIT == -13
+constexpr int shared_group_lds() {
+  int m = 0;
+  LIBERI_SHARED_3(SHARED_GROUP_LDS)
+  return m;
+}
+constexpr int shared_group_nq() {
+  int m = 0;
+  LIBERI_SHARED_3(SHARED_GROUP_NQ)
+  return m;
+}
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void eri_shared_3_kernel(
+    SharedArgs sa, const ClassDev *cds, BuildArgs ba) {
+  __shared__ double lds[shared_group_lds()];
+  __shared__ int s_npq[shared_group_nq()], s_nk[shared_group_nq()], s_boff[shared_group_nq()], s_koff[shared_group_nq()],
+      s_bst[shared_group_nq()], s_kst[shared_group_nq()];
+  const int k = shared_entry(sa), blk = (int)blockIdx.x - sa.first[k], nblk = sa.first[k + 1] - sa.first[k];
+  const ClassDev cd = load_rec(cds, sa.cls[k]);
+  // (chunks of the class's quartets, as in eri_group_kernel)
+  const int64_t nq = cd.q_end - cd.q_begin, chunk = (int64_t)blk * cd.chunk_stride % nblk;
+  switch (sa.cls[k]) {
+    LIBERI_SHARED_3(SHARED_GROUP_CASE)
+    default:
+      break;
+  }
+}
+int launch_shared_3(const SharedArgs &sa, const ClassDev *cds, const BuildArgs &ba, hipStream_t st) {
+  hipLaunchKernelGGL(eri_shared_3_kernel, dim3((unsigned)sa.first[sa.n]), dim3(64), 0, st, sa, cds, ba);
+  return hipGetLastError();
+}
+#endif
+#define SHARED_COOP_NT 64
+#if LIBERI_UNIT == -2 || LIBERI_UNIT == -14
+DEF_SHARED_COOP(4, 64)
+#endif
+#undef SHARED_COOP_NT
+#define SHARED_COOP_NT 128
+#if LIBERI_UNIT == -2 || LIBERI_UNIT == -15
+DEF_SHARED_COOP(5, 128)
+#endif
+
+#if LIBERI_UNIT == -1 || LIBERI_UNIT == -2
+#define DECL_SHARED(N) int launch_shared_##N(const SharedArgs &, const ClassDev *, const BuildArgs &, hipStream_t);
+DECL_SHARED(0) DECL_SHARED(1) DECL_SHARED(2) DECL_SHARED(3) DECL_SHARED(4) DECL_SHARED(5)
+int launch_shared(int launch, const SharedArgs &sa, const ClassDev *cds, const BuildArgs &ba, void *stream) {
+  hipStream_t st = (hipStream_t)stream;
+  if (sa.n <= 0) return hipSuccess;
+  switch (launch) {
+#define X(N) \
+  case N:    \
+    return launch_shared_##N(sa, cds, ba, st);
+    X(0) X(1) X(2) X(3) X(4) X(5)
+#undef X
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+int class_shared_launch(int c, int transposed) {
+  switch (c) {
+#define X(N, id, tr) \
+  case id:           \
+    return tr == transposed ? N : -1;
+#define X0(id, a, b, cc, d, tr) X(0, id, tr)
+#define X1(id, a, b, cc, d, tr) X(1, id, tr)
+#define X2(id, a, b, cc, d, tr) X(2, id, tr)
+    LIBERI_SHARED_0(X0)
+    LIBERI_SHARED_1(X1)
+    LIBERI_SHARED_2(X2)
+#undef X
+#define X(N, id) \
+  case id:       \
+    return N;
+#define X3(id, a, b, cc, d) X(3, id)
+#define X4(id, a, b, cc, d) X(4, id)
+#define X5(id, a, b, cc, d) X(5, id)
+    LIBERI_SHARED_3(X3)
+    LIBERI_SHARED_4(X4)
+    LIBERI_SHARED_5(X5)
+#undef X
+#undef X0
+#undef X1
+#undef X2
+#undef X3
+#undef X4
+#undef X5
+    default:
+      return -1;
+  }
+}
+
+int class_round_quartets(int c) {
+  switch (c) {
+#define XC(id, a, b, cc, d) \
+  case id:                  \
+    return Coop<a, b, cc, d>::Q;
+#define XG(id, a, b, cc, d) \
+  case id:                  \
+    return Grp<a, b, cc, d>::NQ;
+    LIBERI_SHARED_3(XG)
+    LIBERI_SHARED_4(XC)
+    LIBERI_SHARED_5(XC)
+#undef XC
+#undef XG
     default:
       return 0;
   }

@@ -204,6 +204,23 @@ int class_fused_nq(int c);
 // (zero before the launch); cds: ClassDev of every class by class index
 int launch_group_fused(const ClassDev *cds, const BuildArgs &ba, const FusedItem *items, int64_t nitems,
                        unsigned long long *head, int nwg, void *stream);
+// Shared launches: the workgroups of several small classes in one launch.
+// Entry k is class cls[k] with the workgroups [first[k], first[k + 1]).
+constexpr int kSharedLaunches = 6;
+struct SharedArgs {
+  int32_t n = 0, lds = 0;  // entries; dynamic LDS bytes (row-tiled launches)
+  int32_t cls[18], first[19];
+};
+// shared launch that has a body of class c (in that orientation of its rows),
+// or -1; launches below kSharedRowLaunches run the row-tiled form with
+// kSharedRowThreads threads, the group launch the group form, the others the
+// cooperative one
+constexpr int kSharedRowLaunches = 3, kSharedGroupLaunch = 3, kSharedRowThreads = 256;
+int class_shared_launch(int c, int transposed);
+// quartets per round of a workgroup of class c in its (group or cooperative) shared launch
+int class_round_quartets(int c);
+int launch_shared(int launch, const SharedArgs &sa, const ClassDev *cds, const BuildArgs &ba, void *stream);
+
 // longest row tile, quartets
 // row-tile lengths (quartets of one row per workgroup) the autotuner times
 // per row-tiled class; kDefaultTile where it does not time

@@ -462,3 +462,40 @@ def test_untimed_first_build_captured_in_a_graph():
     assert all(variants[names.index(k)] in (1, 2) for k in SPLIT_CLASSES if counts[names.index(k)] > 0)
     h.destroy()
     s.destroy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mol,natoms,ranks", [("water", 3, 1), ("ethane", 8, 1), ("cn_chain", 2, 1), ("cn_chain", 3, 3),
+                                              ("cn_chain", 5, 1), ("cluster", 9, 4), ("cage", 7, 1), ("cage", 12, 8)])
+def test_shared_launches_match_launches_per_class(mol, natoms, ranks):
+    """Small classes run several to a launch, each workgroup its class's body:
+    the same F as launches of one class (no tuning: none is shared), replayed
+    from a graph and launched eagerly, for classes from one quartet to those
+    that no longer share, and for shares of a build.  The forms differ in the
+    order of the FP64 additions: 1e-12 of the largest element."""
+    from gms_liberi_amd import configs
+
+    case = {"water": lambda: configs.water(3), "ethane": lambda: configs.ethane(4),
+            "cn_chain": lambda: configs.cn_chain(5, natoms), "cluster": lambda: configs.cluster(natoms, 6),
+            "cage": lambda: configs.c60_fragment(natoms, 7)}[mol]()
+    b = case.basis.with_schwarz(liberi.schwarz(case.basis))
+    total = {}
+    for rank in range(ranks):
+        h = liberi.Handle()
+        h.setup(b, rank, ranks)
+        got = [("shared", h.fock_build(case.density).copy()), ("shared", h.fock_build(case.density).copy())]
+        h.set_option(liberi.OPT_GRAPH, 0)
+        got.append(("shared", h.fock_build(case.density).copy()))
+        h.set_option(liberi.OPT_AUTOTUNE, 0)
+        got.append(("single", h.fock_build(case.density).copy()))
+        h.destroy()
+        scale = max(1.0, float(np.max(np.abs(got[-1][1]))))
+        for _, f in got:
+            assert np.max(np.abs(f - got[-1][1])) <= 1e-12 * scale
+        total["shared"] = total.get("shared", 0) + got[0][1]
+    h = liberi.Handle()
+    h.setup(b)
+    h.set_option(liberi.OPT_AUTOTUNE, 0)
+    whole = h.fock_build(case.density)
+    h.destroy()
+    assert np.max(np.abs(total["shared"] - whole)) <= 1e-12 * max(1.0, float(np.max(np.abs(whole))))

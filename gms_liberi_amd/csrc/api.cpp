@@ -12,6 +12,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -89,21 +90,20 @@ struct ClassState {
   int64_t nquart = 0, nprimq = 0;
   int32_t nseg = 0;
   int tile = -1;        // row-tile length chosen for the class, index into kTileLens (-1: not yet)
-  DevBuf seg_start, seg_bra, seg_ket0;
   // the row tiles of this rank's share, for each tile length
-  DevBuf tiles[kNumTileLens];
+  const RowTile *tiles[kNumTileLens] = {};
   int32_t ntile[kNumTileLens] = {};
   ClassDev dev{};
   // shared launch the class runs in (-1: none), its workgroups there and, in a
   // row-tiled one, its tiles
   int shared = -1;
   int32_t shared_groups = 0;
-  DevBuf shared_tiles;
+  const RowTile *shared_tiles = nullptr;
 };
 
 // Point the class's launch arguments at its row tiles of length kTileLens[k].
 static void use_tiles(ClassState &cs_, int k) {
-  cs_.dev.tiles = (const RowTile *)cs_.tiles[k].p;
+  cs_.dev.tiles = cs_.tiles[k];
   cs_.dev.ntile = cs_.ntile[k];
 }
 
@@ -127,6 +127,7 @@ struct liberi_ctx {
   hipStream_t last_stream = nullptr;
   std::vector<DevBuf> owned;
   DevBuf pairs, prims, dens, fock;
+  DevBuf tables;  // segments and row tiles of every class
   PairLayout layout{};      // pair layout of the basis
   // per build: density and Coulomb sums by pair (component- then pair-major),
   // square exchange density and exchange sums
@@ -148,11 +149,9 @@ struct liberi_ctx {
   DevBuf tune_F;        // autotuner's scratch Fock matrix
   DevBuf dens_t, dens_b, fock_b;  // UHF: Da + Db, and the beta density / Fock of the host entry point
   hipEvent_t tev[2] = {};
-  // batched form: the build's class launches spread over kSide streams and
-  // captured once into a graph, replayed by later builds on the same D and F
+  // batched form: the build's class launches spread over the branches of a
+  // graph, captured once and replayed by later builds on the same D and F
   bool use_graph = true;
-  hipStream_t side[4] = {};
-  hipEvent_t fork_ev = nullptr, join_ev[4] = {};
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   const double *g_dD = nullptr;
@@ -191,24 +190,37 @@ static void collect_timing(liberi_ctx *h) {
   h->timing_pending = false;
 }
 
-static int dev_alloc(liberi_ctx *h, DevBuf &b, size_t bytes) {
-  b.bytes = bytes;
-  if (bytes == 0) {
-    b.p = nullptr;
-    return LIBERI_OK;
-  }
-  if (h->max_device_bytes > 0.0 && (double)h->stats.device_bytes + (double)bytes > h->max_device_bytes) {
-    b.bytes = 0;
+// bytes of HBM counted as held by the handle, within its budget
+static int charge(liberi_ctx *h, size_t bytes) {
+  if (h->max_device_bytes > 0.0 && (double)h->stats.device_bytes + (double)bytes > h->max_device_bytes)
     return fail(LIBERI_ENOMEM, "device budget of the handle (LIBERI_OPT_MAX_DEVICE_BYTES = " +
                                    std::to_string((int64_t)h->max_device_bytes) + ") exceeded by an allocation of " +
                                    std::to_string(bytes) + " bytes");
-  }
-  hipError_t e = hipMalloc(&b.p, bytes);
-  if (e != hipSuccess)
-    return fail(e == hipErrorOutOfMemory ? LIBERI_ENOMEM : LIBERI_EDEVICE,
-                "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
   h->stats.device_bytes += (int64_t)bytes;
   return LIBERI_OK;
+}
+
+// an allocation whose bytes are already charged
+static int dev_alloc_charged(DevBuf &b, size_t bytes) {
+  b = DevBuf{};
+  if (bytes == 0) return LIBERI_OK;
+  const hipError_t e = hipMalloc(&b.p, bytes);
+  if (e != hipSuccess) {
+    b.p = nullptr;
+    return fail(e == hipErrorOutOfMemory ? LIBERI_ENOMEM : LIBERI_EDEVICE,
+                "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
+  }
+  b.bytes = bytes;
+  return LIBERI_OK;
+}
+
+static int dev_alloc(liberi_ctx *h, DevBuf &b, size_t bytes) {
+  b = DevBuf{};
+  if (bytes == 0) return LIBERI_OK;
+  if (int rc = charge(h, bytes)) return rc;
+  const int rc = dev_alloc_charged(b, bytes);
+  if (rc) h->stats.device_bytes -= (int64_t)bytes;
+  return rc;
 }
 
 template <class T>
@@ -237,13 +249,9 @@ static void drop_graph(liberi_ctx *h) {
 static void release_device(liberi_ctx *h) {
   drop_graph(h);
   for (auto &c : h->cls) {
-    dev_free(c.seg_start);
-    dev_free(c.seg_bra);
-    dev_free(c.seg_ket0);
-    for (int k = 0; k < kNumTileLens; ++k) dev_free(c.tiles[k]);
-    dev_free(c.shared_tiles);
     c = ClassState{};
   }
+  dev_free(h->tables);
   dev_free(h->pairs);
   dev_free(h->prims);
   dev_free(h->dens);
@@ -334,11 +342,6 @@ int liberi_c_destroy(liberi_ctx **ctx) {
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   for (hipEvent_t e : h->tev)
     if (e) (void)hipEventDestroy(e);
-  for (hipEvent_t e : h->join_ev)
-    if (e) (void)hipEventDestroy(e);
-  if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
-  for (hipStream_t s2 : h->side)
-    if (s2) (void)hipStreamDestroy(s2);
   for (int c = 0; c < kNumClasses; ++c) {
     if (h->cev0[c]) (void)hipEventDestroy(h->cev0[c]);
     if (h->cev1[c]) (void)hipEventDestroy(h->cev1[c]);
@@ -620,7 +623,7 @@ static int setup_shared(liberi_ctx *h) {
     for (int c : cls) {
       ClassState &cs_ = h->cls[c];
       ClassDev &d = cds[c] = cs_.dev;
-      d.tiles = (const RowTile *)cs_.shared_tiles.p;
+      d.tiles = cs_.shared_tiles;
       d.ntile = cs_.shared_groups;
       d.chunk_stride = chunk_stride(cs_.shared_groups);
       d.fp32 = 0;
@@ -884,11 +887,179 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
       (rc = dev_alloc(h, h->ksq, nsq * sizeof(double))))
     return rc;
 
-  // ---- per class: pair pre-screen (host), quartet segments (device)
-  std::vector<DevBuf> tmp;
-  auto cleanup_tmp = [&]() {
-    for (auto &b : tmp) dev_free(b);
-    tmp.clear();
+  // ---- per class: pair pre-screen (host), quartet segments (device, the
+  // classes of a batch in one launch), row tiles (host).  One upload and one
+  // launch a batch, one buffer for all tables: as twenty allocations a class
+  // they took most of a small molecule's setup.
+  struct Plan {
+    int c;
+    bool transposed, diag;
+    std::vector<int32_t> kb, kk, gbeg;
+    int64_t len0;  // the class's first segment length in the batch
+  };
+  std::vector<Plan> plans;
+  std::vector<SegJob> jobs;
+  std::vector<unsigned char> up, tab;  // uploads of the batch; the tables of all classes
+  int64_t nlen = 0, nblock = 0;
+  auto put = [](std::vector<unsigned char> &to, const auto &v) {
+    to.resize((to.size() + 15) / 16 * 16);
+    const size_t at = to.size();
+    to.resize(at + v.size() * sizeof(v[0]));
+    if (!v.empty()) std::memcpy(to.data() + at, v.data(), v.size() * sizeof(v[0]));
+    return at;
+  };
+  // (pointers into the tables are offsets until they are uploaded)
+  auto put_table = [&](const auto &v, auto *&p) -> int {
+    if (int e = charge(h, v.size() * sizeof(v[0]))) return e;
+    p = (std::remove_reference_t<decltype(p)>)put(tab, v);
+    return LIBERI_OK;
+  };
+  // segments, share and tiles of a class from its segment lengths
+  auto finish_class = [&](const Plan &p, const int32_t *len) -> int {
+    const int c = p.c, ng = (int)p.gbeg.size();
+    const ClassDef &def = kClasses[c];
+    ClassState &cs_ = h->cls[c];
+    int rc;
+    std::vector<int64_t> sstart;
+    std::vector<int32_t> sbra, sket0;
+    int64_t total = 0, primq = 0;
+    for (size_t i = 0; i < p.kb.size(); ++i) {
+      for (int g = 0; g < ng; ++g) {
+        const int64_t L = len[i * ng + g];
+        if (L <= 0) continue;
+        sstart.push_back(total);
+        sbra.push_back(p.kb[i]);
+        sket0.push_back(p.kk[p.gbeg[g]]);
+        total += L;
+        primq += L * (int64_t)pairs[p.kb[i]].nprim * pairs[p.kk[p.gbeg[g]]].nprim;
+      }
+    }
+    sstart.push_back(total);
+    cs_.nquart = total;
+    cs_.nprimq = primq;
+    if (total == 0) return LIBERI_OK;
+    if (sbra.size() >= (size_t)INT32_MAX || total / kTileLens[0] + (int64_t)p.kb.size() >= (int64_t)INT32_MAX)
+      return fail(LIBERI_ESIZE, std::string("class ") + def.name + ": too many segments");
+    cs_.nseg = (int32_t)sbra.size();
+    ClassDev &d = cs_.dev;
+    if ((rc = put_table(sstart, d.seg_start)) || (rc = put_table(sbra, d.seg_bra)) ||
+        (rc = put_table(sket0, d.seg_ket0)))
+      return rc;
+    cs_.active = true;
+    d.nseg = cs_.nseg;
+    d.diag = p.diag;
+    // this rank's contiguous share of the class.  The reference splits each
+    // class's index range into equal counts (e.g.
+    // src/rhf/rot_axis/int0001.F90:100-104; LIBERI_OPT_RANK_SPLIT = 1);
+    // by default the shares are equal in estimated cost instead: a quartet
+    // costs its primitive quartets plus kQuartetCost for its HRR and
+    // digestion, and the kept lists run from few to many primitives, so equal
+    // counts leave the last ranks the most work (C60 in 8 shares, time of the
+    // slowest over the mean: equal counts 1.39; kQuartetCost 4: 1.26,
+    // 8: 1.08, 16: 1.08, 32: 1.16).
+    if (h->rank_split == 1 || num_procs == 1) {
+      d.q_begin = total * my_rank / num_procs;
+      d.q_end = total * (my_rank + 1) / num_procs;
+    } else {
+      constexpr double kQuartetCost = 12.0;
+      const size_t ns = sbra.size();
+      std::vector<double> cum(ns + 1, 0.0), unit(ns);
+      for (size_t k = 0; k < ns; ++k) {
+        unit[k] = (double)pairs[sbra[k]].nprim * pairs[sket0[k]].nprim + kQuartetCost;
+        cum[k + 1] = cum[k] + unit[k] * (double)(sstart[k + 1] - sstart[k]);
+      }
+      // first quartet at or past cost b
+      auto q_at = [&](double b) -> int64_t {
+        if (b <= 0.0) return 0;
+        if (b >= cum[ns]) return total;
+        const size_t k = (size_t)(std::upper_bound(cum.begin(), cum.end(), b) - cum.begin()) - 1;
+        const int64_t q = sstart[k] + (int64_t)std::ceil((b - cum[k]) / unit[k]);
+        return std::min(q, sstart[k + 1]);
+      };
+      d.q_begin = q_at(cum[ns] * my_rank / num_procs);
+      d.q_end = my_rank + 1 == num_procs ? total : q_at(cum[ns] * (my_rank + 1) / num_procs);
+    }
+    // this share's primitive quartets
+    {
+      int64_t pq = 0;
+      for (size_t k = 0; k < sbra.size(); ++k) {
+        const int64_t a = std::max(sstart[k], d.q_begin), b = std::min(sstart[k + 1], d.q_end);
+        if (b > a) pq += (b - a) * (int64_t)pairs[sbra[k]].nprim * pairs[sket0[k]].nprim;
+      }
+      primq = pq;
+    }
+    for (int k = 0; k < kNumTileLens; ++k) {
+      std::vector<RowTile> tiles;
+      if (cs_.row_ok) tiles = row_tiles(c, d.q_begin, d.q_end, primq, kTileLens[k], class_row_quartets(c), sstart, sbra,
+                                        sket0, pairs);
+      cs_.ntile[k] = (int32_t)tiles.size();
+      if ((rc = put_table(tiles, cs_.tiles[k]))) return rc;
+    }
+    d.row_mode = 0;
+    d.transposed = p.transposed;
+    {
+      const PairLayout &pl = h->layout;
+      const int pf = p.transposed ? def.ket : def.bra, pm = p.transposed ? def.bra : def.ket;
+      d.fix_base = pl.off[pf] - pl.first[pf];
+      d.mov_base = pl.off[pm] - pl.first[pm];
+      d.fix_n = pl.n[pf];
+      d.mov_n = pl.n[pm];
+      auto pair_major = [&](int pc) {
+        return pl.off[pc] - (int64_t)pl.first[pc] * ncart_host(kPairL[pc][0]) * ncart_host(kPairL[pc][1]);
+      };
+      d.bra_q = pair_major(def.bra);
+      d.ket_q = pair_major(def.ket);
+    }
+    d.xswitch = h->exact_large_t ? class_rys_xmax(c) : reference_switch(c);
+    h->stats.quartets[c] = d.q_end - d.q_begin;
+    h->stats.prim_quartets[c] = primq;
+    h->stats.total_quartets += d.q_end - d.q_begin;
+    // a place in a shared launch, where the class is small
+    const int sl = class_shared_launch(c, p.transposed);
+    const int64_t nq = d.q_end - d.q_begin;
+    if (sl >= 0 && nq > 0) {
+      int64_t groups = 0;
+      if (sl < kSharedRowLaunches) {
+        if (cs_.row_ok && nq <= kSharedRowThreads * kSharedRowGroups) {
+          const std::vector<RowTile> tiles =
+              row_tiles(c, d.q_begin, d.q_end, primq, kSharedRowThreads, kSharedRowThreads, sstart, sbra, sket0, pairs);
+          groups = (int64_t)tiles.size();
+          if (groups <= kSharedRowGroups && (rc = put_table(tiles, cs_.shared_tiles))) return rc;
+        }
+      } else {
+        groups = (nq + class_round_quartets(c) - 1) / class_round_quartets(c);
+      }
+      if (groups > 0 && groups <= (sl < kSharedRowLaunches ? kSharedRowGroups : kSharedWaveGroups)) {
+        cs_.shared = sl;
+        cs_.shared_groups = (int32_t)groups;
+      }
+    }
+    return LIBERI_OK;
+  };
+  auto finish_batch = [&]() -> int {
+    if (plans.empty()) return LIBERI_OK;
+    const size_t o_jobs = put(up, jobs), o_len = (up.size() + 15) / 16 * 16;
+    std::vector<int32_t> len(nlen);
+    DevBuf buf;
+    if (int r = dev_alloc_charged(buf, o_len + nlen * sizeof(int32_t))) return r;
+    auto *base = (unsigned char *)buf.p;
+    hipError_t e = hipMemcpyAsync(base, up.data(), up.size(), hipMemcpyHostToDevice, h->stream);
+    if (e == hipSuccess)
+      e = (hipError_t)launch_segment_lengths(base, (const SegJob *)(base + o_jobs), (int32_t)jobs.size(), nblock,
+                                             h->schwarz_cut, (int32_t *)(base + o_len), h->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(len.data(), base + o_len, nlen * sizeof(int32_t), hipMemcpyDeviceToHost, h->stream);
+    const hipError_t es = hipStreamSynchronize(h->stream);
+    dev_free(buf);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return fail(LIBERI_EDEVICE, std::string("segment generation: ") + hipGetErrorString(e));
+    for (const Plan &p : plans)
+      if (int r = finish_class(p, len.data() + p.len0)) return r;
+    plans.clear();
+    jobs.clear();
+    up.clear();
+    nlen = nblock = 0;
+    return LIBERI_OK;
   };
   for (int c = 0; c < kNumClasses; ++c) {
     const ClassDef &def = kClasses[c];
@@ -949,155 +1120,50 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     gend.push_back((int32_t)kk.size());
     const int ng = (int)gbeg.size();
     std::vector<double> bx(kb.size()), kx(kk.size());
-    std::vector<int32_t> bgroup(kb.size()), bpos(kb.size());
+    std::vector<int32_t> bgroup(diag ? kb.size() : 0);
     for (size_t i = 0; i < kb.size(); ++i) {
       bx[i] = pair_x[kb[i]];
-      bgroup[i] = diag ? kgroup[i] : 0;
-      bpos[i] = (int32_t)i;
+      if (diag) bgroup[i] = kgroup[i];
     }
     for (size_t j = 0; j < kk.size(); ++j) kx[j] = pair_x[kk[j]];
-    DevBuf d_bx, d_bg, d_bp, d_kx, d_gb, d_ge, d_len;
-    if ((rc = dev_upload(h, d_bx, bx)) || (rc = dev_upload(h, d_bg, bgroup)) || (rc = dev_upload(h, d_bp, bpos)) ||
-        (rc = dev_upload(h, d_kx, kx)) || (rc = dev_upload(h, d_gb, gbeg)) || (rc = dev_upload(h, d_ge, gend))) {
-      cleanup_tmp();
-      return rc;
-    }
-    tmp = {d_bx, d_bg, d_bp, d_kx, d_gb, d_ge};
     const int64_t nsegc = (int64_t)kb.size() * ng;
-    if ((rc = dev_alloc(h, d_len, nsegc * sizeof(int64_t)))) {
-      cleanup_tmp();
-      return rc;
-    }
-    tmp.push_back(d_len);
-    int e = launch_segment_lengths((const double *)d_bx.p, (const int32_t *)d_bg.p, (const int32_t *)d_bp.p,
-                                   (int32_t)kb.size(), (const double *)d_kx.p, (const int32_t *)d_gb.p,
-                                   (const int32_t *)d_ge.p, ng, diag, def.cmp, cut, (int64_t *)d_len.p, h->stream);
-    std::vector<int64_t> len(nsegc);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(len.data(), d_len.p, nsegc * sizeof(int64_t), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    for (auto &b : tmp) h->stats.device_bytes -= (int64_t)b.bytes;
-    cleanup_tmp();
-    if (e != hipSuccess)
-      return fail(LIBERI_EDEVICE, std::string("segment generation: ") + hipGetErrorString((hipError_t)e));
-    std::vector<int64_t> sstart;
-    std::vector<int32_t> sbra, sket0;
-    int64_t total = 0, primq = 0;
-    for (size_t i = 0; i < kb.size(); ++i) {
-      for (int g = 0; g < ng; ++g) {
-        const int64_t L = len[i * ng + g];
-        if (L <= 0) continue;
-        sstart.push_back(total);
-        sbra.push_back(kb[i]);
-        sket0.push_back(kk[gbeg[g]]);
-        total += L;
-        primq += L * (int64_t)pairs[kb[i]].nprim * pairs[kk[gbeg[g]]].nprim;
-      }
-    }
-    sstart.push_back(total);
-    cs_.nquart = total;
-    cs_.nprimq = primq;
-    if (total == 0) continue;
-    if (sbra.size() >= (size_t)INT32_MAX || total / kTileLens[0] + (int64_t)kb.size() >= (int64_t)INT32_MAX)
-      return fail(LIBERI_ESIZE, std::string("class ") + def.name + ": too many segments");
-    cs_.nseg = (int32_t)sbra.size();
-    if ((rc = dev_upload(h, cs_.seg_start, sstart)) ||
-        (rc = dev_upload(h, cs_.seg_bra, sbra)) || (rc = dev_upload(h, cs_.seg_ket0, sket0)))
-      return rc;
-    cs_.active = true;
-    ClassDev &d = cs_.dev;
-    d.seg_start = (const int64_t *)cs_.seg_start.p;
-    d.seg_bra = (const int32_t *)cs_.seg_bra.p;
-    d.seg_ket0 = (const int32_t *)cs_.seg_ket0.p;
-    d.nseg = cs_.nseg;
-    d.diag = diag;
-    // this rank's contiguous share of the class.  The reference splits each
-    // class's index range into equal counts (e.g.
-    // src/rhf/rot_axis/int0001.F90:100-104; LIBERI_OPT_RANK_SPLIT = 1);
-    // by default the shares are equal in estimated cost instead: a quartet
-    // costs its primitive quartets plus kQuartetCost for its HRR and
-    // digestion, and the kept lists run from few to many primitives, so equal
-    // counts leave the last ranks the most work (C60 in 8 shares, time of the
-    // slowest over the mean: equal counts 1.39; kQuartetCost 4: 1.26,
-    // 8: 1.08, 16: 1.08, 32: 1.16).
-    if (h->rank_split == 1 || num_procs == 1) {
-      d.q_begin = total * my_rank / num_procs;
-      d.q_end = total * (my_rank + 1) / num_procs;
-    } else {
-      constexpr double kQuartetCost = 12.0;
-      const size_t ns = sbra.size();
-      std::vector<double> cum(ns + 1, 0.0), unit(ns);
-      for (size_t k = 0; k < ns; ++k) {
-        unit[k] = (double)pairs[sbra[k]].nprim * pairs[sket0[k]].nprim + kQuartetCost;
-        cum[k + 1] = cum[k] + unit[k] * (double)(sstart[k + 1] - sstart[k]);
-      }
-      // first quartet at or past cost b
-      auto q_at = [&](double b) -> int64_t {
-        if (b <= 0.0) return 0;
-        if (b >= cum[ns]) return total;
-        const size_t k = (size_t)(std::upper_bound(cum.begin(), cum.end(), b) - cum.begin()) - 1;
-        const int64_t q = sstart[k] + (int64_t)std::ceil((b - cum[k]) / unit[k]);
-        return std::min(q, sstart[k + 1]);
-      };
-      d.q_begin = q_at(cum[ns] * my_rank / num_procs);
-      d.q_end = my_rank + 1 == num_procs ? total : q_at(cum[ns] * (my_rank + 1) / num_procs);
-    }
-    // this share's primitive quartets
-    {
-      int64_t pq = 0;
-      for (size_t k = 0; k < sbra.size(); ++k) {
-        const int64_t a = std::max(sstart[k], d.q_begin), b = std::min(sstart[k + 1], d.q_end);
-        if (b > a) pq += (b - a) * (int64_t)pairs[sbra[k]].nprim * pairs[sket0[k]].nprim;
-      }
-      primq = pq;
-    }
-    for (int k = 0; k < kNumTileLens; ++k) {
-      std::vector<RowTile> tiles;
-      if (cs_.row_ok) tiles = row_tiles(c, d.q_begin, d.q_end, primq, kTileLens[k], class_row_quartets(c), sstart, sbra,
-                                        sket0, pairs);
-      cs_.ntile[k] = (int32_t)tiles.size();
-      if ((rc = dev_upload(h, cs_.tiles[k], tiles))) return rc;
-    }
+    // the class's working memory counts against the budget, one class at a time
+    const size_t work = kb.size() * (sizeof(double) + 2 * sizeof(int32_t)) + kk.size() * sizeof(double) +
+                        2 * ng * sizeof(int32_t) + nsegc * sizeof(int64_t);
+    if ((rc = charge(h, work))) return rc;
+    h->stats.device_bytes -= (int64_t)work;
+    SegJob j;
+    j.bra_x = (int64_t)put(up, bx);
+    j.bra_group = (int64_t)put(up, bgroup);
+    j.ket_x = (int64_t)put(up, kx);
+    j.group_begin = (int64_t)put(up, gbeg);
+    j.group_end = (int64_t)put(up, gend);
+    j.len0 = nlen;
+    j.block0 = nblock;
+    j.nbra = (int32_t)kb.size();
+    j.ngroup = ng;
+    j.diag = diag;
+    j.cmp = def.cmp;
+    jobs.push_back(j);
+    plans.push_back(Plan{c, transposed, diag, std::move(kb), std::move(kk), std::move(gbeg), nlen});
+    nlen += nsegc;
+    nblock += (nsegc + kSegThreads - 1) / kSegThreads;
+    // (a batch holds at most about 64 MB, or one class)
+    if (up.size() + nlen * sizeof(int32_t) > (size_t)64 << 20)
+      if ((rc = finish_batch())) return rc;
+  }
+  if ((rc = finish_batch())) return rc;
+  if ((rc = dev_alloc_charged(h->tables, tab.size()))) return rc;
+  if (!tab.empty()) HIP_TRY(hipMemcpy(h->tables.p, tab.data(), tab.size(), hipMemcpyHostToDevice));
+  for (ClassState &cs_ : h->cls) {
+    if (!cs_.active) continue;
+    auto at = [&](auto *&p) { p = (std::remove_reference_t<decltype(p)>)((unsigned char *)h->tables.p + (size_t)p); };
+    at(cs_.dev.seg_start);
+    at(cs_.dev.seg_bra);
+    at(cs_.dev.seg_ket0);
+    for (auto &t : cs_.tiles) at(t);
+    at(cs_.shared_tiles);
     use_tiles(cs_, kDefaultTile);
-    d.row_mode = 0;
-    d.transposed = transposed;
-    {
-      const PairLayout &pl = h->layout;
-      const int pf = transposed ? def.ket : def.bra, pm = transposed ? def.bra : def.ket;
-      d.fix_base = pl.off[pf] - pl.first[pf];
-      d.mov_base = pl.off[pm] - pl.first[pm];
-      d.fix_n = pl.n[pf];
-      d.mov_n = pl.n[pm];
-      auto pair_major = [&](int pc) {
-        return pl.off[pc] - (int64_t)pl.first[pc] * ncart_host(kPairL[pc][0]) * ncart_host(kPairL[pc][1]);
-      };
-      d.bra_q = pair_major(def.bra);
-      d.ket_q = pair_major(def.ket);
-    }
-    d.xswitch = h->exact_large_t ? class_rys_xmax(c) : reference_switch(c);
-    h->stats.quartets[c] = d.q_end - d.q_begin;
-    h->stats.prim_quartets[c] = primq;
-    h->stats.total_quartets += d.q_end - d.q_begin;
-    // a place in a shared launch, where the class is small
-    const int sl = class_shared_launch(c, transposed);
-    const int64_t nq = d.q_end - d.q_begin;
-    if (sl >= 0 && nq > 0) {
-      int64_t groups = 0;
-      if (sl < kSharedRowLaunches) {
-        if (cs_.row_ok && nq <= kSharedRowThreads * kSharedRowGroups) {
-          const std::vector<RowTile> tiles =
-              row_tiles(c, d.q_begin, d.q_end, primq, kSharedRowThreads, kSharedRowThreads, sstart, sbra, sket0, pairs);
-          groups = (int64_t)tiles.size();
-          if (groups <= kSharedRowGroups && (rc = dev_upload(h, cs_.shared_tiles, tiles))) return rc;
-        }
-      } else {
-        groups = (nq + class_round_quartets(c) - 1) / class_round_quartets(c);
-      }
-      if (groups > 0 && groups <= (sl < kSharedRowLaunches ? kSharedRowGroups : kSharedWaveGroups)) {
-        cs_.shared = sl;
-        cs_.shared_groups = (int32_t)groups;
-      }
-    }
   }
   if ((rc = setup_fused(h)) || (rc = setup_shared(h))) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
@@ -1143,7 +1209,7 @@ int liberi_c_setup(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_bas, 
 // LDS accumulators would cut).
 constexpr int64_t kTuneMinQuartets = 20000;
 constexpr float kTileGain = 0.06f;
-constexpr int kSideStreams = 4;
+constexpr int kBranches = 4;  // of the batched form (one hardware queue each)
 // latency of each shared launch, with few quartets in its classes (measured on
 // ethane and the 3-atom C-N chain, ms)
 constexpr double kSharedMs[kSharedLaunches] = {0.03, 0.06, 0.1, 0.05, 0.1, 0.08};
@@ -1370,7 +1436,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     set_tuned_choice(c, nq, h->fp32_tau, cs_.fp32);
   }
   // the time of every class not timed above, which spreads the classes over
-  // the side streams: from an earlier handle, or the second of two launches
+  // the branches: from an earlier handle, or the second of two launches
   // (the first one of a kernel in the process loads its code, up to
   // milliseconds)
   for (int c = 0; c < kNumClasses; ++c) {
@@ -1404,8 +1470,10 @@ static BuildWork build_work(const liberi_ctx *h) {
 }
 
 // Zero F (and find max |D| for the mixed form), then every class's kernel.
-// With ns > 1 the classes are spread over the side streams, longest first
-// onto the least-loaded stream, forked from and joined back into st.
+// With ns > 1, under capture on st, the classes are spread over ns branches of
+// the graph, longest first onto the least-loaded branch: a launch is captured
+// behind the last one of its branch.  (One stream captures them all; a stream
+// per branch took 0.5 ms to create and destroy, most of a request's teardown.)
 static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, hipStream_t st, int ns) {
   // fock = 0 (src/liberi_driver.F90:64)
   if (int e = launch_build_begin(ba, h->layout, build_work(h), st))
@@ -1432,10 +1500,24 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
   for (int k = 0; k < kSharedLaunches; ++k)
     if (shared_cost[k] > 0.0) order.push_back({kSharedMs[k] + shared_cost[k], kNumClasses + k});
   std::vector<double> load(ns, 0.0);
+  if (ns > 1) std::sort(order.begin(), order.end(), std::greater<>());
+  // captured nodes the next launch on st depends on, and the last of each branch
+  using Nodes = std::vector<hipGraphNode_t>;
+  auto captured = [&](Nodes &v) -> hipError_t {
+    hipStreamCaptureStatus cap;
+    const hipGraphNode_t *deps = nullptr;
+    size_t n = 0;
+    const hipError_t e = hipStreamGetCaptureInfo_v2(st, &cap, nullptr, nullptr, &deps, &n);
+    if (e == hipSuccess) v.assign(deps, deps + n);
+    return e;
+  };
+  auto depend_on = [&](Nodes &v) -> hipError_t {
+    return hipStreamUpdateCaptureDependencies(st, v.data(), v.size(), hipStreamSetCaptureDependencies);
+  };
+  std::vector<Nodes> branch(ns);
   if (ns > 1) {
-    std::sort(order.begin(), order.end(), std::greater<>());
-    HIP_TRY(hipEventRecord(h->fork_ev, st));
-    for (int k = 0; k < ns; ++k) HIP_TRY(hipStreamWaitEvent(h->side[k], h->fork_ev, 0));
+    HIP_TRY(captured(branch[0]));
+    for (int k = 1; k < ns; ++k) branch[k] = branch[0];
   }
   if (fused) {
     // one persistent launch for the fused classes, first onto the least-loaded
@@ -1447,44 +1529,45 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
       k = ns > 1 ? 1 : 0;
       load[k] += fused_cost;
     }
-    hipStream_t fs = ns > 1 ? h->side[k] : st;
-    int e = launch_fill_zero((double *)h->fused_head.p, 1, fs);
+    if (ns > 1) HIP_TRY(depend_on(branch[k]));
+    int e = launch_fill_zero((double *)h->fused_head.p, 1, st);
     if (e == hipSuccess)
       e = launch_group_fused((const ClassDev *)h->fused_cds.p, ba, (const FusedItem *)h->fused_items.p, h->fused_n,
-                             (unsigned long long *)h->fused_head.p, h->fused_nwg, fs);
+                             (unsigned long long *)h->fused_head.p, h->fused_nwg, st);
     if (e != hipSuccess)
       return fail(LIBERI_EDEVICE, std::string("fused group launch: ") + hipGetErrorString((hipError_t)e));
+    if (ns > 1) HIP_TRY(captured(branch[k]));
   }
   for (const auto &[ms, c] : order) {
-    hipStream_t cs = st;
-    if (ns > 1) {
-      const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-      load[k] += ms;
-      cs = h->side[k];
-    }
+    const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    load[k] += ms;
+    if (ns > 1) HIP_TRY(depend_on(branch[k]));
     if (c >= kNumClasses) {
-      if (int e = launch_shared(c - kNumClasses, h->shared[c - kNumClasses], (const ClassDev *)h->shared_cds.p, ba, cs))
+      if (int e = launch_shared(c - kNumClasses, h->shared[c - kNumClasses], (const ClassDev *)h->shared_cds.p, ba, st))
         return fail(LIBERI_EDEVICE, std::string("shared launch: ") + hipGetErrorString((hipError_t)e));
-      continue;
+    } else {
+      if (h->class_timing && ns == 1) {
+        if (!h->cev0[c]) HIP_TRY(hipEventCreate(&h->cev0[c]));
+        if (!h->cev1[c]) HIP_TRY(hipEventCreate(&h->cev1[c]));
+        HIP_TRY(hipEventRecord(h->cev0[c], st));
+      }
+      ClassDev cd = h->cls[c].dev;
+      cd.row_mode = class_row_mode(h, c);
+      cd.fp32 = h->cls[c].fp32 == 1;
+      int e = launch_class(c, cd, ba, st, kCoopWorkgroups);
+      if (e != hipSuccess)
+        return fail(LIBERI_EDEVICE, std::string("launch ") + kClasses[c].name + ": " + hipGetErrorString((hipError_t)e));
+      if (h->class_timing && ns == 1) HIP_TRY(hipEventRecord(h->cev1[c], st));
     }
-    if (h->class_timing && ns == 1) {
-      if (!h->cev0[c]) HIP_TRY(hipEventCreate(&h->cev0[c]));
-      if (!h->cev1[c]) HIP_TRY(hipEventCreate(&h->cev1[c]));
-      HIP_TRY(hipEventRecord(h->cev0[c], cs));
-    }
-    ClassDev cd = h->cls[c].dev;
-    cd.row_mode = class_row_mode(h, c);
-    cd.fp32 = h->cls[c].fp32 == 1;
-    int e = launch_class(c, cd, ba, cs, kCoopWorkgroups);
-    if (e != hipSuccess)
-      return fail(LIBERI_EDEVICE, std::string("launch ") + kClasses[c].name + ": " + hipGetErrorString((hipError_t)e));
-    if (h->class_timing && ns == 1) HIP_TRY(hipEventRecord(h->cev1[c], cs));
+    if (ns > 1) HIP_TRY(captured(branch[k]));
   }
-  if (ns > 1)
-    for (int k = 0; k < ns; ++k) {
-      HIP_TRY(hipEventRecord(h->join_ev[k], h->side[k]));
-      HIP_TRY(hipStreamWaitEvent(st, h->join_ev[k], 0));
-    }
+  if (ns > 1) {
+    Nodes all;
+    for (const Nodes &v : branch)
+      for (hipGraphNode_t n : v)
+        if (std::find(all.begin(), all.end(), n) == all.end()) all.push_back(n);
+    HIP_TRY(depend_on(all));
+  }
   if (int e = launch_build_end(ba, h->layout, st))
     return fail(LIBERI_EDEVICE, std::string("end of the build: ") + hipGetErrorString((hipError_t)e));
   return LIBERI_OK;
@@ -1544,14 +1627,9 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   const bool graph = h->use_graph && !h->class_timing && h->only_class < 0 && ba.DK == dD && k_scale == 1.0;
   if (graph && (!h->gexec || h->g_dD != dD || h->g_dF != dF)) {
     drop_graph(h);
-    for (int k = 0; k < kSideStreams; ++k) {
-      if (!h->side[k]) HIP_TRY(hipStreamCreateWithFlags(&h->side[k], hipStreamNonBlocking));
-      if (!h->join_ev[k]) HIP_TRY(hipEventCreateWithFlags(&h->join_ev[k], hipEventDisableTiming));
-    }
-    if (!h->fork_ev) HIP_TRY(hipEventCreateWithFlags(&h->fork_ev, hipEventDisableTiming));
     HIP_TRY(hipStreamSynchronize(h->stream));
     HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_build(h, ba, dD, h->stream, kSideStreams);
+    int rc = enqueue_build(h, ba, dD, h->stream, kBranches);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(h->stream, &g);
     if (rc) {

@@ -3218,11 +3218,18 @@ __global__ __launch_bounds__(64) void eri_group_kernel(ClassDev cd, BuildArgs ba
 
 // ----------------------------------------------------- segment lengths
 #if LIBERI_UNIT == -1 || LIBERI_UNIT == -2
-__global__ void segment_lengths_kernel(const double *bra_x, const int32_t *bra_group, const int32_t *bra_pos,
-                                       int32_t nbra, const double *ket_x, const int32_t *gbeg, const int32_t *gend,
-                                       int32_t ngroup, int32_t diag, int32_t cmp, double cut, int64_t *seg_len) {
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (int64_t)nbra * ngroup) return;
+__global__ __launch_bounds__(kSegThreads) void segment_lengths_kernel(const unsigned char *base, const SegJob *jobs,
+                                                                      int32_t njob, double cut, int32_t *seg_len) {
+  int k = 0;
+  while (k + 1 < njob && (int64_t)blockIdx.x >= jobs[k + 1].block0) ++k;
+  const SegJob j = jobs[k];
+  const int64_t id = ((int64_t)blockIdx.x - j.block0) * kSegThreads + threadIdx.x;
+  if (id >= (int64_t)j.nbra * j.ngroup) return;
+  const double *bra_x = (const double *)(base + j.bra_x), *ket_x = (const double *)(base + j.ket_x);
+  const int32_t *bra_group = (const int32_t *)(base + j.bra_group);
+  const int32_t *gbeg = (const int32_t *)(base + j.group_begin), *gend = (const int32_t *)(base + j.group_end);
+  const int32_t ngroup = j.ngroup, diag = j.diag, cmp = j.cmp;
+  seg_len += j.len0;
   const int i = (int)(id / ngroup), g = (int)(id % ngroup);
   const double xi = bra_x[i];
   int lo = gbeg[g], hi = gend[g];
@@ -3233,7 +3240,7 @@ __global__ void segment_lengths_kernel(const double *bra_x, const int32_t *bra_g
       seg_len[id] = 0;
       return;
     }
-    if (g == gi) limit = bra_pos[i] + 1;  // kets up to and including the bra itself
+    if (g == gi) limit = i + 1;  // kets up to and including the bra itself
   }
   // first position in [lo, hi) whose product fails the test (x descending)
   int a = lo, b = hi;
@@ -3561,15 +3568,11 @@ int launch_fill_zero(double *p, int64_t n, void *stream) {
   return hipGetLastError();
 }
 
-int launch_segment_lengths(const double *bra_x, const int32_t *bra_group, const int32_t *bra_pos, int32_t nbra,
-                           const double *ket_x, const int32_t *gbeg, const int32_t *gend, int32_t ngroup,
-                           int32_t diag, int32_t cmp, double cut, int64_t *seg_len, void *stream) {
-  const int64_t n = (int64_t)nbra * ngroup;
-  if (n == 0) return hipSuccess;
-  const int tpb = 256;
-  hipLaunchKernelGGL(segment_lengths_kernel, dim3((unsigned)((n + tpb - 1) / tpb)), dim3(tpb), 0,
-                     (hipStream_t)stream, bra_x, bra_group, bra_pos, nbra, ket_x, gbeg, gend, ngroup, diag, cmp,
-                     cut, seg_len);
+int launch_segment_lengths(const unsigned char *base, const SegJob *jobs, int32_t njob, int64_t nblock, double cut,
+                           int32_t *seg_len, void *stream) {
+  if (nblock <= 0) return hipSuccess;
+  hipLaunchKernelGGL(segment_lengths_kernel, dim3((unsigned)nblock), dim3(kSegThreads), 0, (hipStream_t)stream, base,
+                     jobs, njob, cut, seg_len);
   return hipGetLastError();
 }
 #endif

@@ -336,10 +336,17 @@ int launch_add(const double *a, const double *b, double *out, int64_t n, void *s
 // out[0] = max |p[0..n)| (out must be zero on entry)
 int launch_abs_max(const double *p, int64_t n, double *out, void *stream);
 
-// Segment lengths on the device: one thread per (kept bra row, ket group).
-int launch_segment_lengths(const double *bra_x, const int32_t *bra_group, const int32_t *bra_pos_in_group,
-                           int32_t nbra, const double *ket_x, const int32_t *group_begin,
-                           const int32_t *group_end, int32_t ngroup, int32_t diag, int32_t cmp,
-                           double cut, int64_t *seg_len, void *stream);
+// Segment lengths on the device: one thread per (kept bra row, ket group) of
+// every job (a class), job j in the workgroups from block0 on.  The arrays are
+// byte offsets from `base`; bra_group is read in diagonal classes only, whose
+// bras and kets are one list.
+constexpr int kSegThreads = 256;
+struct SegJob {
+  int64_t bra_x, bra_group, ket_x, group_begin, group_end;  // byte offsets
+  int64_t len0, block0;
+  int32_t nbra, ngroup, diag, cmp;
+};
+int launch_segment_lengths(const unsigned char *base, const SegJob *jobs, int32_t njob, int64_t nblock, double cut,
+                           int32_t *seg_len, void *stream);
 
 }  // namespace liberi

@@ -81,12 +81,22 @@ class DeviceArray:
         except Exception:
             pass
 
+    def part(self, first: int, n: int) -> "DeviceArray":
+        """Elements [first, first + n), owned by this array."""
+        d = DeviceArray.__new__(_DevicePart)
+        d.n, d.ptr, d.owner = n, C.c_void_p(self.address + 8 * first), self
+        return d
 
     def copy_from_async(self, host: "PinnedArray", stream: "Stream") -> None:
         _ok(runtime().hipMemcpyAsync(self.ptr, host.ptr, self.n * 8, 1, stream.ptr), "hipMemcpyAsync H2D")
 
     def copy_to_async(self, host: "PinnedArray", stream: "Stream") -> None:
         _ok(runtime().hipMemcpyAsync(host.ptr, self.ptr, self.n * 8, 2, stream.ptr), "hipMemcpyAsync D2H")
+
+
+class _DevicePart(DeviceArray):
+    def free(self) -> None:
+        pass
 
 
 class PinnedArray:
@@ -99,6 +109,13 @@ class PinnedArray:
         _ok(runtime().hipHostMalloc(C.byref(self.ptr), max(1, n) * 8, 0), "hipHostMalloc")
         self.array = np.ctypeslib.as_array(C.cast(self.ptr, C.POINTER(C.c_double)), shape=(n,))
 
+    def part(self, first: int, n: int) -> "PinnedArray":
+        """Elements [first, first + n), owned by this array."""
+        p = PinnedArray.__new__(_PinnedPart)
+        p.n, p.ptr, p.owner = n, C.c_void_p(self.ptr.value + 8 * first), self
+        p.array = self.array[first:first + n]
+        return p
+
     def free(self) -> None:
         if self.ptr:
             self.array = None
@@ -110,6 +127,11 @@ class PinnedArray:
             self.free()
         except Exception:
             pass
+
+
+class _PinnedPart(PinnedArray):
+    def free(self) -> None:
+        self.array = None
 
 
 def device_memory() -> tuple[int, int]:

@@ -101,15 +101,16 @@ class _Slot:
             self.h.set_option(liberi.OPT_FP32_TAU, req.tau)
         self.n = b.ntri
         self.stream = hipmem.Stream()
-        self.D = hipmem.DeviceArray(self.n)
-        self.F = hipmem.DeviceArray(self.n)
-        self.hD = []
-        self.hF = []
-        for d in req.densities:
-            p = hipmem.PinnedArray(self.n)
+        # one allocation on each side: densities and Fock matrices of every
+        # iteration in pinned memory, one of each on the device
+        self.device = hipmem.DeviceArray(2 * self.n)
+        self.D, self.F = self.device.part(0, self.n), self.device.part(self.n, self.n)
+        k = len(req.densities)
+        self.host = hipmem.PinnedArray(2 * k * self.n)
+        self.hD = [self.host.part(i * self.n, self.n) for i in range(k)]
+        self.hF = [self.host.part((k + i) * self.n, self.n) for i in range(k)]
+        for p, d in zip(self.hD, req.densities):
             p.array[:] = d
-            self.hD.append(p)
-            self.hF.append(hipmem.PinnedArray(self.n))
         st = self.h.stats()
         self.quartets = int(st["total_quartets"])
         self.device_bytes = int(st["device_bytes"])
@@ -127,10 +128,10 @@ class _Slot:
         self.h.destroy()
         self.event.destroy()
         self.stream.destroy()
-        self.D.free()
-        self.F.free()
+        self.device.free()
         for p in self.hD + self.hF:
             p.free()
+        self.host.free()
         return focks
 
 

@@ -153,7 +153,7 @@ const char *liberi_c_last_error(void);
                                        wave-split row tiles for the d classes that have them).
                                        Setting it makes the next build decide again. */
 #define LIBERI_OPT_GRAPH 10         /* 1 (default): batched form -- the build's class launches run on
-                                       four side streams (largest first onto the least-loaded
+                                       four branches of a graph (largest first onto the least-loaded
                                        stream), captured once into a HIP graph that later builds on
                                        the same D and F replay; 0: one stream, launched eagerly.
                                        Per-class timing and ONLY_CLASS builds run eagerly.  Read at

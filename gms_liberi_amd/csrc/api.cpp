@@ -156,6 +156,13 @@ struct liberi_ctx {
   hipGraphExec_t gexec = nullptr;
   const double *g_dD = nullptr;
   double *g_dF = nullptr;
+  // the same for the two builds of an unrestricted one: the graph, the arrays
+  // (Da, Db, Fa, Fb) it was captured with and those of the last call, and the
+  // second build's workspace
+  hipGraph_t ugraph = nullptr;
+  hipGraphExec_t uexec = nullptr;
+  const void *ug_arrays[4] = {}, *u_arrays[4] = {};
+  DevBuf uhf_work;
   bool fp32_pending = false;
   ClassState cls[kNumClasses];
   liberi_stats stats{};
@@ -237,7 +244,15 @@ static void dev_free(DevBuf &b) {
   b.bytes = 0;
 }
 
+static void drop_uhf_graph(liberi_ctx *h) {
+  if (h->uexec) (void)hipGraphExecDestroy(h->uexec);
+  if (h->ugraph) (void)hipGraphDestroy(h->ugraph);
+  h->uexec = nullptr;
+  h->ugraph = nullptr;
+}
+
 static void drop_graph(liberi_ctx *h) {
+  drop_uhf_graph(h);
   if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
   if (h->graph) (void)hipGraphDestroy(h->graph);
   h->gexec = nullptr;
@@ -248,6 +263,8 @@ static void drop_graph(liberi_ctx *h) {
 
 static void release_device(liberi_ctx *h) {
   drop_graph(h);
+  std::fill(h->u_arrays, h->u_arrays + 4, nullptr);
+  dev_free(h->uhf_work);
   for (auto &c : h->cls) {
     c = ClassState{};
   }
@@ -1464,9 +1481,8 @@ static int enqueue_dmax(liberi_ctx *h, const double *dD, hipStream_t st) {
   return LIBERI_OK;
 }
 
-static BuildWork build_work(const liberi_ctx *h) {
-  double *dp = (double *)h->dpair.p;
-  return BuildWork{dp, dp + h->layout.off[kNumPairClasses], (double *)h->dsq.p};
+static BuildWork build_work(const BuildArgs &ba) {
+  return BuildWork{const_cast<double *>(ba.Dp), const_cast<double *>(ba.Dq), const_cast<double *>(ba.Dsq)};
 }
 
 // Zero F (and find max |D| for the mixed form), then every class's kernel.
@@ -1474,10 +1490,13 @@ static BuildWork build_work(const liberi_ctx *h) {
 // the graph, longest first onto the least-loaded branch: a launch is captured
 // behind the last one of its branch.  (One stream captures them all; a stream
 // per branch took 0.5 ms to create and destroy, most of a request's teardown.)
-static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, hipStream_t st, int ns) {
+// `spins` builds of one basis (their arguments at bas, each its own
+// workspace) go side by side: the two Fock matrices of an unrestricted build.
+static int enqueue_build(liberi_ctx *h, const BuildArgs *bas, int spins, const double *dD, hipStream_t st, int ns) {
   // fock = 0 (src/liberi_driver.F90:64)
-  if (int e = launch_build_begin(ba, h->layout, build_work(h), st))
-    return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
+  for (int s = 0; s < spins; ++s)
+    if (int e = launch_build_begin(bas[s], h->layout, build_work(bas[s]), st))
+      return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
   // the fused group launch, where on: its classes leave the per-class launches
@@ -1532,35 +1551,38 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
     if (ns > 1) HIP_TRY(depend_on(branch[k]));
     int e = launch_fill_zero((double *)h->fused_head.p, 1, st);
     if (e == hipSuccess)
-      e = launch_group_fused((const ClassDev *)h->fused_cds.p, ba, (const FusedItem *)h->fused_items.p, h->fused_n,
+      e = launch_group_fused((const ClassDev *)h->fused_cds.p, bas[0], (const FusedItem *)h->fused_items.p, h->fused_n,
                              (unsigned long long *)h->fused_head.p, h->fused_nwg, st);
     if (e != hipSuccess)
       return fail(LIBERI_EDEVICE, std::string("fused group launch: ") + hipGetErrorString((hipError_t)e));
     if (ns > 1) HIP_TRY(captured(branch[k]));
   }
-  for (const auto &[ms, c] : order) {
-    const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    load[k] += ms;
-    if (ns > 1) HIP_TRY(depend_on(branch[k]));
-    if (c >= kNumClasses) {
-      if (int e = launch_shared(c - kNumClasses, h->shared[c - kNumClasses], (const ClassDev *)h->shared_cds.p, ba, st))
-        return fail(LIBERI_EDEVICE, std::string("shared launch: ") + hipGetErrorString((hipError_t)e));
-    } else {
-      if (h->class_timing && ns == 1) {
-        if (!h->cev0[c]) HIP_TRY(hipEventCreate(&h->cev0[c]));
-        if (!h->cev1[c]) HIP_TRY(hipEventCreate(&h->cev1[c]));
-        HIP_TRY(hipEventRecord(h->cev0[c], st));
+  for (const auto &[ms, c] : order)
+    for (int s = 0; s < spins; ++s) {
+      const BuildArgs &ba = bas[s];
+      const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      load[k] += ms;
+      if (ns > 1) HIP_TRY(depend_on(branch[k]));
+      if (c >= kNumClasses) {
+        if (int e = launch_shared(c - kNumClasses, h->shared[c - kNumClasses], (const ClassDev *)h->shared_cds.p, ba, st))
+          return fail(LIBERI_EDEVICE, std::string("shared launch: ") + hipGetErrorString((hipError_t)e));
+      } else {
+        if (h->class_timing && ns == 1) {
+          if (!h->cev0[c]) HIP_TRY(hipEventCreate(&h->cev0[c]));
+          if (!h->cev1[c]) HIP_TRY(hipEventCreate(&h->cev1[c]));
+          HIP_TRY(hipEventRecord(h->cev0[c], st));
+        }
+        ClassDev cd = h->cls[c].dev;
+        cd.row_mode = class_row_mode(h, c);
+        cd.fp32 = h->cls[c].fp32 == 1;
+        int e = launch_class(c, cd, ba, st, kCoopWorkgroups);
+        if (e != hipSuccess)
+          return fail(LIBERI_EDEVICE,
+                      std::string("launch ") + kClasses[c].name + ": " + hipGetErrorString((hipError_t)e));
+        if (h->class_timing && ns == 1) HIP_TRY(hipEventRecord(h->cev1[c], st));
       }
-      ClassDev cd = h->cls[c].dev;
-      cd.row_mode = class_row_mode(h, c);
-      cd.fp32 = h->cls[c].fp32 == 1;
-      int e = launch_class(c, cd, ba, st, kCoopWorkgroups);
-      if (e != hipSuccess)
-        return fail(LIBERI_EDEVICE, std::string("launch ") + kClasses[c].name + ": " + hipGetErrorString((hipError_t)e));
-      if (h->class_timing && ns == 1) HIP_TRY(hipEventRecord(h->cev1[c], st));
+      if (ns > 1) HIP_TRY(captured(branch[k]));
     }
-    if (ns > 1) HIP_TRY(captured(branch[k]));
-  }
   if (ns > 1) {
     Nodes all;
     for (const Nodes &v : branch)
@@ -1568,27 +1590,27 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs &ba, const double *dD, h
         if (std::find(all.begin(), all.end(), n) == all.end()) all.push_back(n);
     HIP_TRY(depend_on(all));
   }
-  if (int e = launch_build_end(ba, h->layout, st))
-    return fail(LIBERI_EDEVICE, std::string("end of the build: ") + hipGetErrorString((hipError_t)e));
+  for (int s = 0; s < spins; ++s)
+    if (int e = launch_build_end(bas[s], h->layout, st))
+      return fail(LIBERI_EDEVICE, std::string("end of the build: ") + hipGetErrorString((hipError_t)e));
   return LIBERI_OK;
 }
 
 // RHF: DK = D, k_scale = 1.  A UHF spin component: D = Da + Db, DK = that
 // spin's density, k_scale = 2 (F_s = J[Da+Db] - K[Ds]).
-static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStream_t st, const double *dK = nullptr,
-                           double k_scale = 1.0) {
+static BuildArgs build_args(liberi_ctx *h, const double *dD, const double *dK, double *dF, double k_scale) {
   BuildArgs ba;
   ba.pairs = (const PairRec *)h->pairs.p;
   ba.prims = (const PrimRec *)h->prims.p;
   ba.D = dD;
-  ba.DK = dK ? dK : dD;
+  ba.DK = dK;
   ba.k_scale = k_scale;
-  const BuildWork w = build_work(h);
-  ba.Dp = w.Dp;
-  ba.Dq = w.Dq;
-  ba.Dsq = w.Dsq;
+  const int64_t npl = h->layout.off[kNumPairClasses];
+  ba.Dp = (const double *)h->dpair.p;
+  ba.Dq = ba.Dp + npl;
+  ba.Dsq = (const double *)h->dsq.p;
   ba.Jp = (double *)h->jpair.p;
-  ba.Jq = ba.Jp + h->layout.off[kNumPairClasses];
+  ba.Jq = ba.Jp + npl;
   ba.Ksq = (double *)h->ksq.p;
   ba.F = dF;
   ba.value_cut = h->value_cut;
@@ -1600,6 +1622,40 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     ba.col_bf[l] = (const int32_t *)h->col_bf[l].p;
     ba.ncol[l] = h->ncol[l];
   }
+  return ba;
+}
+
+// whether the next build has to choose forms, tile lengths or times first
+static bool choices_open(const liberi_ctx *h) {
+  for (int k = 0; k < kNumClasses; ++k) {
+    const ClassState &c = h->cls[k];
+    if (c.active && (c.variant < 0 || c.tile < 0 || (c.ms < 0.f && !class_shared(h, k)) ||
+                     (h->fp32_tau > 0.0 && c.fp32 < 0)))
+      return true;
+  }
+  return false;
+}
+
+// The build of bas[0 .. spins) as branches of a graph, captured on the handle's stream.
+static int capture_build(liberi_ctx *h, const BuildArgs *bas, int spins, hipGraph_t *graph, hipGraphExec_t *exec) {
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+  const int rc = enqueue_build(h, bas, spins, bas[0].D, h->stream, kBranches);
+  hipGraph_t g = nullptr;
+  const hipError_t e = hipStreamEndCapture(h->stream, &g);
+  if (rc) {
+    if (g) (void)hipGraphDestroy(g);
+    return rc;
+  }
+  if (e != hipSuccess) return fail(LIBERI_EDEVICE, std::string("graph capture: ") + hipGetErrorString(e));
+  *graph = g;
+  HIP_TRY(hipGraphInstantiate(exec, g, nullptr, nullptr, 0));
+  return LIBERI_OK;
+}
+
+static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStream_t st, const double *dK = nullptr,
+                           double k_scale = 1.0) {
+  const BuildArgs ba = build_args(h, dD, dK ? dK : dD, dF, k_scale);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cap));
   if (cap == hipStreamCaptureStatusNone && h->last_stream && h->last_stream != st)
@@ -1608,17 +1664,8 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
   // (they also run before any build: Dp and Dsq from this build's density)
-  const bool choose = [&] {
-    for (int k = 0; k < kNumClasses; ++k) {
-      const ClassState &c = h->cls[k];
-      if (c.active && (c.variant < 0 || c.tile < 0 || (c.ms < 0.f && !class_shared(h, k)) ||
-                       (h->fp32_tau > 0.0 && c.fp32 < 0)))
-        return true;
-    }
-    return false;
-  }();
-  if (choose) {
-    if (int e = launch_build_begin(ba, h->layout, build_work(h), st))
+  if (choices_open(h)) {
+    if (int e = launch_build_begin(ba, h->layout, build_work(ba), st))
       return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
     if (int rc = choose_variants(h, ba, st)) return rc;
   }
@@ -1627,25 +1674,14 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   const bool graph = h->use_graph && !h->class_timing && h->only_class < 0 && ba.DK == dD && k_scale == 1.0;
   if (graph && (!h->gexec || h->g_dD != dD || h->g_dF != dF)) {
     drop_graph(h);
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_build(h, ba, dD, h->stream, kBranches);
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(h->stream, &g);
-    if (rc) {
-      if (g) (void)hipGraphDestroy(g);
-      return rc;
-    }
-    if (e != hipSuccess) return fail(LIBERI_EDEVICE, std::string("graph capture: ") + hipGetErrorString(e));
-    h->graph = g;
-    HIP_TRY(hipGraphInstantiate(&h->gexec, h->graph, nullptr, nullptr, 0));
+    if (int rc = capture_build(h, &ba, 1, &h->graph, &h->gexec)) return rc;
     h->g_dD = dD;
     h->g_dF = dF;
   }
   HIP_TRY(hipEventRecord(h->ev0, st));
   if (graph) {
     HIP_TRY(hipGraphLaunch(h->gexec, st));
-  } else if (int rc = enqueue_build(h, ba, dD, st, 1)) {
+  } else if (int rc = enqueue_build(h, &ba, 1, dD, st, 1)) {
     return rc;
   }
   HIP_TRY(hipEventRecord(h->ev1, st));
@@ -1687,6 +1723,53 @@ int liberi_c_fock_build_device(liberi_ctx *h, const double *dD, double *dF, int6
 }
 
 // ------------------------------------------------------------------- UHF
+// Both spins' builds side by side in one graph, from the second call on the
+// same four arrays on (one after the other on one stream, the 17-atom
+// cluster's classes leave the chip idle most of the time: 973 -> 832 us).  The
+// second build has a workspace of its own.  Returns 1 when the builds have to
+// run one after the other, 0 when done, else an error.
+static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, const double *dDb, double *dFa,
+                           double *dFb, hipStream_t st, int *rc) {
+  *rc = LIBERI_OK;
+  const void *arrays[4] = {dDa, dDb, dFa, dFb};
+  const bool again = std::equal(arrays, arrays + 4, h->u_arrays);
+  std::copy(arrays, arrays + 4, h->u_arrays);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (!again || !h->use_graph || h->class_timing || h->only_class >= 0 || h->fused || h->fp32_tau > 0.0 ||
+      choices_open(h) || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+    return 1;
+  if (!h->uexec || !std::equal(arrays, arrays + 4, h->ug_arrays)) {
+    drop_uhf_graph(h);
+    const size_t npl = (size_t)h->layout.off[kNumPairClasses], nsq = (size_t)h->num_bas * h->num_bas;
+    if (!h->uhf_work.p && dev_alloc(h, h->uhf_work, (4 * npl + 2 * nsq) * sizeof(double)) != LIBERI_OK) return 1;
+    BuildArgs bas[2] = {build_args(h, dt, dDa, dFa, 2.0), build_args(h, dt, dDb, dFb, 2.0)};
+    double *w = (double *)h->uhf_work.p;
+    bas[1].Dp = w;
+    bas[1].Dq = w + npl;
+    bas[1].Jp = w + 2 * npl;
+    bas[1].Jq = w + 3 * npl;
+    bas[1].Dsq = w + 4 * npl;
+    bas[1].Ksq = w + 4 * npl + nsq;
+    if ((*rc = capture_build(h, bas, 2, &h->ugraph, &h->uexec))) return 0;
+    std::copy(arrays, arrays + 4, h->ug_arrays);
+  }
+  hipError_t e = h->last_stream && h->last_stream != st ? hipStreamWaitEvent(st, h->ev1, 0) : hipSuccess;
+  if (e == hipSuccess) e = (hipError_t)launch_add(dDa, dDb, const_cast<double *>(dt), (int64_t)h->num_bas * (h->num_bas + 1) / 2, st);
+  if (e == hipSuccess) e = hipEventRecord(h->ev0, st);
+  if (e == hipSuccess) e = hipGraphLaunch(h->uexec, st);
+  if (e == hipSuccess) e = hipEventRecord(h->ev1, st);
+  if (e != hipSuccess) {
+    *rc = fail(LIBERI_EDEVICE, std::string("UHF build: ") + hipGetErrorString(e));
+    return 0;
+  }
+  h->last_stream = st;
+  h->build_pending = true;
+  h->fp32_pending = h->timing_pending = false;
+  h->stats.fp32_quartets = 0;
+  for (double &v : h->stats.class_ms) v = 0.0;
+  return 0;
+}
+
 int liberi_c_fock_build_uhf_device(liberi_ctx *h, const double *dDa, const double *dDb, double *dFa, double *dFb,
                                    int64_t n, void *stream) {
   if (!h) return fail(LIBERI_EARG, "liberi_c_fock_build_uhf_device: NULL handle");
@@ -1699,6 +1782,8 @@ int liberi_c_fock_build_uhf_device(liberi_ctx *h, const double *dDa, const doubl
   if (!h->dens_t.p)
     if (int rc = dev_alloc(h, h->dens_t, ntri * sizeof(double))) return rc;
   double *dt = (double *)h->dens_t.p;
+  int rcu = LIBERI_OK;
+  if (!build_uhf_graph(h, dt, dDa, dDb, dFa, dFb, st, &rcu)) return rcu;
   if (int e = launch_add(dDa, dDb, dt, ntri, st))
     return fail(LIBERI_EDEVICE, std::string("Da + Db: ") + hipGetErrorString((hipError_t)e));
   if (int rc = build_on_device(h, dt, dFa, st, dDa, 2.0)) return rc;

@@ -72,3 +72,33 @@ def test_uhf_reduces_to_rhf(name):
     scale = max(1.0, float(np.max(np.abs(f))))
     for g in (fa, fb, f2):
         assert np.max(np.abs(g - f)) <= 1e-11 * scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["cfg_water.npz", "cfg_ethane.npz"])
+def test_uhf_graph_matches_builds_one_after_the_other(name):
+    """From the second call on the same arrays both spins' builds run side by
+    side from one graph: every replay equals the eager builds to summation
+    order (1e-12 of the largest element), with other densities in the arrays,
+    with restricted builds in between, on other arrays, and after a return to
+    eager builds."""
+    case = Case.load_npz(GOLD / name)
+    rng = np.random.default_rng(5)
+    b = case.basis
+    pairs = [(0.5 * case.density, 0.5 * rng.permutation(case.density)), (0.7 * case.density, 0.1 * case.density)]
+    h = liberi.Handle()
+    h.setup(b)
+    h.set_option(liberi.OPT_GRAPH, 0)
+    want = [[f.copy() for f in h.fock_build_uhf(*p)] for p in pairs]
+    rhf = h.fock_build(case.density).copy()
+    h.set_option(liberi.OPT_GRAPH, 1)
+    for call in range(6):
+        got = h.fock_build_uhf(*pairs[call % 2])
+        for g, w in zip(got, want[call % 2]):
+            assert np.max(np.abs(g - w)) <= 1e-12 * max(1.0, float(np.max(np.abs(w))))
+        if call == 3:
+            assert np.max(np.abs(h.fock_build(case.density) - rhf)) <= 1e-12 * max(1.0, float(np.max(np.abs(rhf))))
+    h.setup(b)  # a new setup drops the graph
+    got = h.fock_build_uhf(*pairs[1])
+    assert np.max(np.abs(got[0] - want[1][0])) <= 1e-12 * max(1.0, float(np.max(np.abs(want[1][0]))))
+    h.destroy()

@@ -694,7 +694,10 @@ static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int
       const int64_t q1 = std::min(sstart[e], q_end);
       for (int64_t q = std::max(sstart[s], q_begin); q < q1; q += cap) {
         while (sstart[sg + 1] <= q) ++sg;
-        tiles.push_back(RowTile{q, (int32_t)std::min(cap, q1 - q), (int32_t)sg, team, 0});
+        const int64_t n = std::min(cap, q1 - q);
+        size_t last = sg;
+        while (sstart[last + 1] < q + n) ++last;
+        tiles.push_back(RowTile{q, (int32_t)n, (int32_t)sg, team, (int32_t)last});
       }
     }
   };
@@ -1013,6 +1016,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
       if ((rc = put_table(tiles, cs_.tiles[k]))) return rc;
     }
     d.row_mode = 0;
+    d.threads = kRowThreads[0];
     d.transposed = p.transposed;
     {
       const PairLayout &pl = h->layout;
@@ -1225,7 +1229,7 @@ int liberi_c_setup(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_bas, 
 // atomics), direct digestion for the workgroup classes (whose occupancy the
 // LDS accumulators would cut).
 constexpr int64_t kTuneMinQuartets = 20000;
-constexpr float kTileGain = 0.06f;
+constexpr float kTileGain = 0.06f, kThreadsGain = 0.02f;
 constexpr int kBranches = 4;  // of the batched form (one hardware queue each)
 // latency of each shared launch, with few quartets in its classes (measured on
 // ethane and the 3-atom C-N chain, ms)
@@ -1390,6 +1394,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     if (!cs_.active || cs_.tile >= 0) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
     cs_.tile = h->tile_len >= 0 ? h->tile_len : kDefaultTile;
+    cs_.dev.threads = kRowThreads[0];
     if (h->tile_len >= 0 || !h->autotune || !class_row_mode(h, c) || nq < kTuneMinQuartets || class_shared(h, c) ||
         (h->only_class >= 0 && c != h->only_class)) {
       use_tiles(cs_, cs_.tile);
@@ -1398,6 +1403,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     if (const int prev = tuned_choice(c, nq, -2.0); prev >= 0) {
       cs_.tile = prev;
       use_tiles(cs_, cs_.tile);
+      if (tuned_choice(c, nq, -4.0) == 1) cs_.dev.threads = kRowThreads[1];
       continue;
     }
     float best[kNumTileLens];
@@ -1419,6 +1425,20 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
       if (best[k] < (1.f - kTileGain) * best[cs_.tile]) cs_.tile = k;
     use_tiles(cs_, cs_.tile);
     cs_.ms = best[cs_.tile];
+    // workgroup size of the lane classes, with those tiles
+    if (class_kernel_kind(c) == 0) {
+      cs_.dev.threads = kRowThreads[1];
+      float b = 1e30f;
+      for (int rep = 0; rep < 2; ++rep) {
+        float ms = 0.f;
+        if (int rc = time_class(h, ba, st, c, true, false, ms)) return rc;
+        b = std::min(b, ms);
+      }
+      const bool wide = b < (1.f - kThreadsGain) * cs_.ms;
+      if (wide) cs_.ms = b;
+      cs_.dev.threads = kRowThreads[wide];
+      set_tuned_choice(c, nq, -4.0, wide);
+    }
     set_tuned_choice(c, nq, -2.0, cs_.tile);
   }
   // mixed form: FP32 stays on only in the classes where it is measured

@@ -359,6 +359,7 @@ __device__ __forceinline__ ClassDev load_rec(const ClassDev *v, int64_t i) {
   c.tiles = q->tiles;
   c.ntile = q->ntile;
   c.row_mode = q->row_mode;
+  c.threads = q->threads;
   c.transposed = q->transposed;
   c.fix_base = q->fix_base;
   c.mov_base = q->mov_base;
@@ -909,19 +910,13 @@ __device__ __forceinline__ void wave_sum_to_lds(const double (&x)[K], double *ds
 // added to F once per tile.  The Coulomb block of the fixed pair is summed in
 // registers over the tile and reduced across the workgroup at the end.  Only
 // the Coulomb block of the moving pair goes to F per quartet.
-// Threads of a row-tiled lane-per-quartet workgroup: one copy of the
-// tile's LDS rows and Rys table serves all of them, so larger workgroups
-// hold more waves per CU where the LDS limits them.  Measured on C60 (256 ->
-// 512 / 1024 threads): (pp|ds) 4.61 -> 4.18 ms, (pp|pp) 2.18 -> 1.97, (ps|ps)
-// 6.09 -> 5.83 (1024); the other lane classes are as fast or faster at 256.
-template <int LA, int LB, int LC, int LD>
-constexpr int row_threads() {
-  if constexpr (LA == 1 && LB == 1 && LC == 2 && LD == 0) return 512;
-  if constexpr (LA == 1 && LB == 1 && LC == 1 && LD == 1) return 512;
-  if constexpr (LA == 1 && LB == 0 && LC == 1 && LD == 0) return 1024;
-  return 256;
-}
-
+// A workgroup of the kernel has 256 or 512 threads, timed per class
+// (ClassDev::threads): one copy of the tile's LDS rows and Rys table serves all
+// of them, so that 512 hold more waves per CU where the LDS limits them or the
+// class has few tiles, and 256 leave fewer lanes without quartets.  256 / 512:
+// one of 8 rank shares of C60 (ps|dp) 0.94 / 0.62 ms, (ds|ds) 0.52 / 0.35;
+// 41-atom cluster (ps|ds) 0.35 / 0.46, (ss|ps) 0.42 / 0.54; C60 (ps|ps) 3.42 /
+// 3.26, (ss|dp) 1.83 / 2.11.
 template <int LA, int LB, int LC, int LD, bool TR, bool MIXED>
 __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba, int tile, double *lds) {
   using S = Small<LA, LB, LC, LD>;
@@ -932,21 +927,23 @@ __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba,
   constexpr Range<R::L2, R::L2> r2{};
   constexpr Range<R::M1, R::M1> rm1{};
   constexpr Range<R::M2, R::M2> rm2{};
-  // lds: jfix[NFIX], rows[NROW][ncols], then the Rys table
-  double *jfix_s = lds, *rows = lds + NFIX;
+  // lds: the run counter, jfix[NFIX], rows[NROW][ncols], then the Rys table
+  int *next_run = (int *)lds;
+  double *jfix_s = lds + 1, *rows = jfix_s + NFIX;
   const int ncols = (int)row_columns<LA, LB, LC, LD, TR>(ba.ncol);
   const int off2 = R::M1 == R::M2 ? 0 : ba.ncol[R::M1];
   const RowTile tl = cd.tiles[tile];
   const int64_t q0 = tl.q0, q1 = q0 + tl.n;
-  const int seg0 = tl.seg, team = tl.team;
-  const int32_t ifix = cd.seg_bra[seg0];
+  const int team = tl.team;
+  const int32_t ifix = cd.seg_bra[tl.seg];
   const PairRec fix = load_rec(const_view(ba.pairs), ifix);
   // the class's Rys table below the switch, staged once per workgroup with
   // intervals padded to an odd stride
   double *tab = rows + NROW * ncols;
   stage_rys_table<S::NR>(tab, cd.xswitch);
 
-  for (int i = threadIdx.x; i < NFIX + NROW * ncols; i += blockDim.x) lds[i] = 0.0;
+  for (int i = threadIdx.x; i < NFIX + NROW * ncols; i += blockDim.x) jfix_s[i] = 0.0;
+  if (threadIdx.x == 0) *next_run = 0;
 
   double jfix[NFIX];  // the fixed pair's Coulomb partial sums
 #pragma unroll
@@ -955,12 +952,10 @@ __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba,
   __syncthreads();
 
   unsigned nlow = 0;  // quartets this lane evaluated in FP32
-  int sg = seg0;      // segment of the lane's quartet (its quartets ascend)
-  const int part = (int)threadIdx.x & (team - 1);
-  for (int64_t qb = q0; qb < q1; qb += blockDim.x / (unsigned)team) {
-    const int64_t q = qb + threadIdx.x / (unsigned)team;
-    if (q >= q1) continue;
-    while (sg + 1 < cd.nseg && cd.seg_start[sg + 1] <= q) ++sg;
+  int sg = tl.last;   // segment of the lane's quartet (its runs descend)
+  const int lane = (int)__lane_id(), part = lane & (team - 1);
+  auto quartet = [&](int64_t q) {
+    while (cd.seg_start[sg] > q) --sg;
     const int32_t imov = cd.seg_ket0[sg] + (int32_t)(q - cd.seg_start[sg]);
     const PairRec mov = ba.pairs[imov];
     const PairRec &bra = TR ? mov : fix;
@@ -974,7 +969,7 @@ __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba,
       small_integrals<double, LA, LB, LC, LD, !TR, TR>(bra, ket, ba.prims, cd.xswitch, ba.value_cut, v, tab,
                                               rys_lds_stride(S::NR), part, team);
     }
-    if (part != 0) continue;
+    if (part != 0) return;
 
     double s = sfix;
     if (mov.sameAB) s *= 0.5;
@@ -1122,6 +1117,20 @@ __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba,
           lds_add(TR ? &rows[c * ncols + cm2[b]] : &rows[(NA + b) * ncols + cm1[c]], -sk * t);
         }
     }
+  };
+  // a wave takes the next run of 64 lanes' quartets when it is done with one,
+  // from the end of the tile (the most primitives) to its start: with runs
+  // dealt out in turn the waves of a tile end up to a run of the longest
+  // quartets apart (1024-thread (ps|ps): C60 4.08 -> 3.63 ms, 41-atom cluster
+  // 0.47 -> 0.40; C60 build 67.0 -> 64.7)
+  const int per = 64 / team;
+  for (;;) {
+    int r = 0;
+    if (lane == 0) r = __hip_atomic_fetch_add(next_run, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    r = __builtin_amdgcn_readfirstlane(r);
+    const int64_t end = q1 - (int64_t)r * per, q = end - per + lane / team;
+    if (end <= q0) break;
+    if (q >= q0) quartet(q);
   }
 
   if constexpr (MIXED) count_fp32(ba, nlow);
@@ -1143,7 +1152,7 @@ __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba,
 }
 
 template <int LA, int LB, int LC, int LD, bool TR>
-__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>()), 2) void eri_row_kernel(ClassDev cd, BuildArgs ba) {
+__global__ __launch_bounds__(kRowThreads[1], 2) void eri_row_kernel(ClassDev cd, BuildArgs ba) {
   extern __shared__ double lds[];
   row_run<LA, LB, LC, LD, TR, true>(cd, ba, (int)blockIdx.x, lds);
 }
@@ -3589,7 +3598,7 @@ constexpr bool use_small() {
 template <int LA, int LB, int LC, int LD, bool TR>
 int64_t row_acc_bytes(const int32_t *ncol) {
   using R = RowShape<LA, LB, LC, LD, TR>;
-  return (int64_t)sizeof(double) * (R::NFIX + R::NROW * row_columns<LA, LB, LC, LD, TR>(ncol));
+  return (int64_t)sizeof(double) * (1 + R::NFIX + R::NROW * row_columns<LA, LB, LC, LD, TR>(ncol));
 }
 
 // LDS bytes of the row-tiled form of the class in orientation TR (the lane
@@ -3634,8 +3643,8 @@ static int launch_row(const ClassDev &cd, const BuildArgs &ba, hipStream_t st) {
   if constexpr (!RowShape<LA, LB, LC, LD, TR>::exists) {
     return hipErrorInvalidValue;
   } else if constexpr (use_small<LA, LB, LC, LD>() && !SplitShape<LA, LB, LC, LD>::exists) {
-    hipLaunchKernelGGL((eri_row_kernel<LA, LB, LC, LD, TR>), grid, dim3(row_threads<LA, LB, LC, LD>()), (unsigned)lds,
-                       st, cd, ba);
+    if (cd.threads != kRowThreads[0] && cd.threads != kRowThreads[1]) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((eri_row_kernel<LA, LB, LC, LD, TR>), grid, dim3((unsigned)cd.threads), (unsigned)lds, st, cd, ba);
   } else if constexpr (SplitShape<LA, LB, LC, LD>::exists) {
     // (its dynamic LDS limit was raised by prepare_class at setup)
     hipLaunchKernelGGL((eri_split_kernel<LA, LB, LC, LD, TR>), grid, dim3(SplitShape<LA, LB, LC, LD>::NT),
@@ -4135,7 +4144,7 @@ int64_t class_row_lds(int c, int transposed, const int32_t *ncol, double xswitch
 template <int LA, int LB, int LC, int LD>
 static int row_quartets() {
   using P = SplitShape<LA, LB, LC, LD>;
-  return P::exists ? 64 * P::NBAT : row_threads<LA, LB, LC, LD>();
+  return P::exists ? 64 * P::NBAT : kRowThreads[0];
 }
 
 // Instruction counts of a primitive quartet and of the rest of a quartet (with

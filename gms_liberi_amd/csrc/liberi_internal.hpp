@@ -68,12 +68,15 @@ struct alignas(64) PrimRec {
 };
 
 // One workgroup of a row-tiled kernel: the quartets [q0, q0 + n) of one row,
-// starting in segment seg; in the lane-per-quartet kernels `team` adjacent
+// in the segments seg to last; in the lane-per-quartet kernels `team` adjacent
 // lanes share a quartet (a power of two up to 64).
 struct RowTile {
   int64_t q0;
-  int32_t n, seg, team, pad;
+  int32_t n, seg, team, last;
 };
+
+// workgroup sizes of the lane row-tiled kernels
+constexpr int kRowThreads[2] = {256, 512};
 
 // Device view of one class's quartet enumeration.  Kept pair lists are sorted
 // by (primitive count, Schwarz value descending); a segment is one kept bra
@@ -95,6 +98,7 @@ struct ClassDev {
   const RowTile *tiles;
   int32_t ntile;
   int32_t row_mode;
+  int32_t threads;  // of a workgroup of the lane row-tiled kernel
   // 0: rows run over the class's bra pairs, segments over its kets (as
   // above); 1: the roles are swapped -- seg_bra holds ket pairs and seg_ket0
   // bra pairs -- so that a row tile fixes the ket pair (non-diagonal classes)

@@ -1413,11 +1413,11 @@ __device__ __forceinline__ void split_integrals(const PairRec &bra, const PairRe
 
 constexpr int64_t kSplitLdsBytes = 160 * 1024;
 
-// Quartets of one part (slice PART) of a wave-split row tile: the run of 64
-// quartets qb + bat*64 + lane of every step of NBAT runs.
+// One part (slice PART) of a run of a wave-split row tile: the lane's quartet
+// q, of the segments [seg0, seg1] (none where q < q0).
 template <int LA, int LB, int LC, int LD, bool TR, int PART>
 __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &ba, const PairRec &fix, int32_t ifix,
-                                           int64_t q0, int64_t q1, int seg0, int bat, double *jfix_s,
+                                           int64_t q0, int64_t q, int seg0, int seg1, double *jfix_s,
                                            const double *dfix_s, double *rows, int ncols, int off2,
                                            const double *tab) {
   using P = SplitShape<LA, LB, LC, LD>;
@@ -1439,15 +1439,12 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
   constexpr Range<R::L2, R::L2> r2{};
   (void)ra, (void)rb, (void)rc, (void)rd;
   const double sfix = fix.sameAB ? 0.5 : 1.0;
-  const int lane = threadIdx.x & 63;
-  int sg = seg0;
-  for (int64_t qb = q0; qb < q1; qb += P::NBAT * 64) {
-    const int64_t q = qb + bat * 64 + lane;
+  {
     double jf[NJ];
 #pragma unroll
     for (int k = 0; k < NJ; ++k) jf[k] = 0.0;
-    if (q < q1) {
-      while (sg + 1 < cd.nseg && cd.seg_start[sg + 1] <= q) ++sg;
+    if (q >= q0) {
+      const int sg = find_segment(cd, q, seg0, seg1 + 1);
       const int32_t imov = cd.seg_ket0[sg] + (int32_t)(q - cd.seg_start[sg]);
       const PairRec mov = ba.pairs[imov];
       const PairRec &bra = TR ? mov : fix;
@@ -1620,19 +1617,19 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
   }
 }
 
-// the parts of wave slice wpart (S / W consecutive parts), one after the other
+// part `part` of a run
 template <int LA, int LB, int LC, int LD, bool TR, int PART>
-__device__ __forceinline__ void split_dispatch(int wpart, const ClassDev &cd, const BuildArgs &ba,
-                                               const PairRec &fix, int32_t ifix, int64_t q0, int64_t q1, int seg0,
-                                               int bat, double *jfix_s, const double *dfix_s, double *rows,
-                                               int ncols, int off2, const double *tab) {
-  using P = SplitShape<LA, LB, LC, LD>;
-  if constexpr (PART < P::S) {
-    if (PART / (P::S / P::W) == wpart)
-      split_part<LA, LB, LC, LD, TR, PART>(cd, ba, fix, ifix, q0, q1, seg0, bat, jfix_s, dfix_s, rows, ncols, off2,
+__device__ __forceinline__ void split_dispatch(int part, const ClassDev &cd, const BuildArgs &ba, const PairRec &fix,
+                                               int32_t ifix, int64_t q0, int64_t q, int seg0, int seg1, double *jfix_s,
+                                               const double *dfix_s, double *rows, int ncols, int off2,
+                                               const double *tab) {
+  if constexpr (PART < SplitShape<LA, LB, LC, LD>::S) {
+    if (PART == part)
+      split_part<LA, LB, LC, LD, TR, PART>(cd, ba, fix, ifix, q0, q, seg0, seg1, jfix_s, dfix_s, rows, ncols, off2,
                                            tab);
-    split_dispatch<LA, LB, LC, LD, TR, PART + 1>(wpart, cd, ba, fix, ifix, q0, q1, seg0, bat, jfix_s, dfix_s, rows,
-                                                 ncols, off2, tab);
+    else
+      split_dispatch<LA, LB, LC, LD, TR, PART + 1>(part, cd, ba, fix, ifix, q0, q, seg0, seg1, jfix_s, dfix_s, rows,
+                                                   ncols, off2, tab);
   }
 }
 
@@ -1641,40 +1638,51 @@ __device__ __forceinline__ void split_dispatch(int wpart, const ClassDev &cd, co
 template <int LA, int LB, int LC, int LD, bool TR>
 int64_t split_lds(const int32_t *ncol, double xswitch) {
   using R = RowShape<LA, LB, LC, LD, TR>;
-  return (int64_t)sizeof(double) * (2 * R::NFIX + R::NROW * row_columns<LA, LB, LC, LD, TR>(ncol) +
+  return (int64_t)sizeof(double) * (1 + 2 * R::NFIX + R::NROW * row_columns<LA, LB, LC, LD, TR>(ncol) +
                                     rys_table_used(SplitShape<LA, LB, LC, LD>::NR, xswitch));
 }
 
 // Wave-split row-tiled kernel: one workgroup owns one row tile (a run of
-// quartets sharing the fixed pair); wave w takes the parts of wave slice
-// w % W of the quartets of run w / W of each step.
+// quartets sharing the fixed pair).  Its work items are the parts of each run
+// of 64 quartets, part by part (the waves then share a part's code) and from
+// the end of the tile, the most primitives, to its start; a wave takes the next
+// one when it is done with one, so that rows of few runs keep all waves busy
+// (dealt out in turn, (dd|pp) of a 41-atom cluster, 3 runs a row, kept 3 of 8
+// waves busy: 0.52 -> 0.19 ms; C60 (dp|pp) 4.48 -> 3.67, (dd|pp) 3.12 -> 2.54).
 template <int LA, int LB, int LC, int LD, bool TR>
 __global__ __launch_bounds__((SplitShape<LA, LB, LC, LD>::NT)) void eri_split_kernel(ClassDev cd, BuildArgs ba) {
   using P = SplitShape<LA, LB, LC, LD>;
   using R = RowShape<LA, LB, LC, LD, TR>;
   constexpr int N1 = R::N1, NFIX = R::NFIX, NROW = R::NROW;
   extern __shared__ double lds[];
-  double *jfix_s = lds, *dfix_s = lds + NFIX, *rows = lds + 2 * NFIX;
+  int *next_item = (int *)lds;
+  double *jfix_s = lds + 1, *dfix_s = jfix_s + NFIX, *rows = dfix_s + NFIX;
   const int ncols = (int)row_columns<LA, LB, LC, LD, TR>(ba.ncol);
   const int off2 = R::M1 == R::M2 ? 0 : ba.ncol[R::M1];
   double *tab = rows + NROW * ncols;
   stage_rys_table<P::NR>(tab, cd.xswitch);
   const RowTile tl = cd.tiles[blockIdx.x];
   const int64_t q0 = tl.q0, q1 = q0 + tl.n;
-  const int seg0 = tl.seg;
-  const int32_t ifix = cd.seg_bra[seg0];
+  const int32_t ifix = cd.seg_bra[tl.seg];
   const PairRec fix = load_rec(const_view(ba.pairs), ifix);
   for (int i = threadIdx.x; i < NFIX; i += blockDim.x) {
     jfix_s[i] = 0.0;
     dfix_s[i] = ba.Dp[cd.fix_base + (int64_t)i * cd.fix_n + ifix];
   }
   for (int i = threadIdx.x; i < NROW * ncols; i += blockDim.x) rows[i] = 0.0;
+  if (threadIdx.x == 0) *next_item = 0;
   __syncthreads();
 
-  // slice and run of this wave (uniform over the wave)
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  split_dispatch<LA, LB, LC, LD, TR, 0>(wave % P::W, cd, ba, fix, ifix, q0, q1, seg0, wave / P::W, jfix_s, dfix_s,
-                                        rows, ncols, off2, tab);
+  const int lane = (int)__lane_id(), runs = (tl.n + 63) / 64;
+  for (;;) {
+    int it = 0;
+    if (lane == 0) it = __hip_atomic_fetch_add(next_item, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    it = __builtin_amdgcn_readfirstlane(it);
+    if (it >= P::S * runs) break;
+    const int part = it / runs, run = it - part * runs;
+    split_dispatch<LA, LB, LC, LD, TR, 0>(part, cd, ba, fix, ifix, q0, q1 - 64 * (int64_t)(run + 1) + lane, tl.seg,
+                                          tl.last, jfix_s, dfix_s, rows, ncols, off2, tab);
+  }
   __syncthreads();
 
   for (int i = threadIdx.x; i < NFIX; i += blockDim.x) {

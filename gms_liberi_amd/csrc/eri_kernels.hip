@@ -1175,8 +1175,7 @@ __global__ __launch_bounds__(kRowThreads[1], 2) void eri_row_kernel(ClassDev cd,
 // keeps its slice, its HRR and its part of the digestion in registers: no
 // LDS traffic in the primitive loop.  The exchange blocks land in the
 // workgroup's LDS rows as in eri_row_kernel; a block summed over the split
-// index gets one LDS add per part.  A wave runs S / W of the parts one after
-// the other over its quartets, so that W waves serve one run of 64 quartets.
+// index gets one LDS add per part.
 
 enum SplitSide { SPLIT_NONE = 0, SPLIT_COLS = 1, SPLIT_ROWS = 2, SPLIT_CONE = 3 };
 
@@ -1197,9 +1196,8 @@ __host__ __device__ constexpr int split_buffer(int LA, int LB, int LC, int LD, i
   return m;
 }
 
-// Parts S and waves per run W of the split form of a class (S = 0: none),
-// and for the ket cone the directions of D per part (3: all; 1: one, the
-// part is a (c, direction) pair).  Chosen so that the slice, the tables and
+// Parts S of the split form of a class (S = 0: none), and for the ket cone the
+// directions of D per part (3: all; 1: one, the part is a (c, direction) pair).  Chosen so that the slice, the tables and
 // the HRR levels of a part fit the registers of two waves per SIMD (8-wave
 // workgroups) or three (12 waves).
 template <int LA, int LB, int LC, int LD>
@@ -1228,22 +1226,15 @@ constexpr int split_parts() {
   if constexpr (LA == 3 && LB == 1 && LC == 3 && LD == 1) return 30;  // (fp|fp): one f of C, one direction
   return 0;
 }
+// waves of a workgroup: two per SIMD, or three where a part fits 168 VGPRs
 template <int LA, int LB, int LC, int LD>
 constexpr int split_waves() {
-  constexpr int S = split_parts<LA, LB, LC, LD>();
-  if constexpr (LA == 2 && LB == 1 && LC == 1 && LD == 1) return 1;  // (dp|pp): the 3 parts in turn
-  if constexpr (LA == 2 && LB == 1 && LC == 2 && LD == 1) return 2;  // (dp|dp): 3 parts per wave
-  if constexpr (LA == 2 && LB == 2 && LC == 2 && LD == 1) return 2;  // (dd|dp): 9 parts per wave
-  if constexpr (LA == 2 && LB == 2 && LC == 1 && LD == 1) return 1;  // (dd|pp): 9 parts per wave
-  if constexpr (LA == 3 && LB == 1 && LC == 1 && LD == 1) return 1;  // (fp|pp): 9 parts per wave
-  if constexpr ((LA == 3 || LC == 3) && S % 2 == 0) return 2;  // f classes: S/2 parts per wave
-  return S;
+  return (LA == 2 && LB == 2 && LC == 2 && LD == 0) || (LA == 1 && LB == 0 && LC == 2 && LD == 2) ? 12 : 8;
 }
 
 template <int LA, int LB, int LC, int LD>
 struct SplitShape {
   static constexpr int S = split_parts<LA, LB, LC, LD>();
-  static constexpr int W = split_waves<LA, LB, LC, LD>();
   static constexpr int NE = nrange(LA, LA + LB), NF = nrange(LC, LC + LD);
   static constexpr int SIDE = S == 0 ? SPLIT_NONE
                               : LD == 0 ? SPLIT_COLS
@@ -1253,17 +1244,14 @@ struct SplitShape {
   // ket cone: directions of D per part, parts per component c
   static constexpr int NDI = SIDE == SPLIT_CONE ? split_cone_dirs<LA, LB, LC, LD>() : ncart(LD);
   static constexpr int PPC = 3 / (NDI > 0 ? NDI : 1);
-  static constexpr bool exists = SIDE != SPLIT_NONE && W > 0 && S % W == 0 &&
+  static constexpr bool exists = SIDE != SPLIT_NONE &&
                                  (SIDE == SPLIT_COLS   ? NF % S == 0
                                   : SIDE == SPLIT_ROWS ? NE % S == 0
                                                        : (NDI == 1 || NDI == 3) && S == ncart(LC) * PPC);
   // rows e and columns f of (e0|f0) one part accumulates
   static constexpr int NEP = SIDE == SPLIT_ROWS ? NE / S : NE;
   static constexpr int NFP = SIDE == SPLIT_COLS ? NF / S : (SIDE == SPLIT_CONE ? 1 + NDI : NF);
-  // waves per workgroup: W per run of 64 quartets, NBAT runs; 8 waves when W
-  // divides it, else 12 (two or three waves per SIMD)
-  static constexpr int NBAT = !exists ? 1 : (8 % W == 0 ? 8 / W : 12 / W);
-  static constexpr int NT = 64 * W * NBAT;
+  static constexpr int NT = 64 * split_waves<LA, LB, LC, LD>();
   static constexpr int NR = (LA + LB + LC + LD) / 2 + 1;
   // slice of the block after the HRR: rows a (all but in the rows split),
   // columns c (one per part in the cone, all in the rows split), columns d
@@ -4152,7 +4140,8 @@ int64_t class_row_lds(int c, int transposed, const int32_t *ncol, double xswitch
 template <int LA, int LB, int LC, int LD>
 static int row_quartets() {
   using P = SplitShape<LA, LB, LC, LD>;
-  return P::exists ? 64 * P::NBAT : kRowThreads[0];
+  // (wave-split: runs enough for an item per wave)
+  return P::exists ? 64 * ((P::NT / 64 + P::S - 1) / P::S) : kRowThreads[0];
 }
 
 // Instruction counts of a primitive quartet and of the rest of a quartet (with

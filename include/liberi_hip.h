@@ -151,7 +151,9 @@ const char *liberi_c_last_error(void);
                                        row-tiled digestion per class and keeps the faster; 0: fixed
                                        choice (row tiles for the lane-per-quartet classes and the
                                        wave-split row tiles for the d classes that have them).
-                                       Setting it makes the next build decide again. */
+                                       Setting it makes the next build decide again.  With 1, and no
+                                       form, tile length, FP32 switch or diagnostic asked for, classes
+                                       of few quartets run several to a launch. */
 #define LIBERI_OPT_GRAPH 10         /* 1 (default): batched form -- the build's class launches run on
                                        four branches of a graph (largest first onto the least-loaded
                                        stream), captured once into a HIP graph that later builds on

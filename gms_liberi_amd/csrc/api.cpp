@@ -1804,6 +1804,11 @@ int liberi_c_fock_build_uhf_device(liberi_ctx *h, const double *dDa, const doubl
   double *dt = (double *)h->dens_t.p;
   int rcu = LIBERI_OK;
   if (!build_uhf_graph(h, dt, dDa, dDb, dFa, dFb, st, &rcu)) return rcu;
+  // Da + Db is written where a build on another stream may still read it
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  if (cap == hipStreamCaptureStatusNone && h->last_stream && h->last_stream != st)
+    HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
   if (int e = launch_add(dDa, dDb, dt, ntri, st))
     return fail(LIBERI_EDEVICE, std::string("Da + Db: ") + hipGetErrorString((hipError_t)e));
   if (int rc = build_on_device(h, dt, dFa, st, dDa, 2.0)) return rc;

@@ -863,7 +863,8 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
         for (int32_t j = 0; j < n; ++j) {
           const int32_t p = list[g0 + j];
           sorted.push_back(pairs[p]);
-          sorted.back().prim_off = off + j;
+          // (a pair without primitives has no record: an offset in the array all the same)
+          sorted.back().prim_off = np > 0 ? off + j : 0;
           sorted.back().prim_stride = n;
           sorted_x.push_back(pair_x[p]);
           list[g0 + j] = (int32_t)sorted.size() - 1;

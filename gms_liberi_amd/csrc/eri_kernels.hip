@@ -583,7 +583,8 @@ __device__ __forceinline__ void small_integrals(const PairRec &bra, const PairRe
       // classes the extra registers cost more occupancy than the latency it
       // hides)
       constexpr bool ahead = LA + LB + LC + LD == 0;
-      PrimRec Qn = prims[ket.prim_off];
+      PrimRec Qn{};
+      if (ahead && ket.nprim > 0) Qn = prims[ket.prim_off];
       for (int iq = 0; iq < ket.nprim; ++iq) {
         const PrimRec Q = ahead ? Qn : prims[ket.prim_off + iq * ket.prim_stride];
         if (ahead && iq + 1 < ket.nprim) Qn = prims[ket.prim_off + (iq + 1) * ket.prim_stride];

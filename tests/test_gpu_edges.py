@@ -82,3 +82,23 @@ def test_zero_density(handle, oracle):
     handle.setup(case.basis)
     f = handle.fock_build(np.zeros(case.basis.ntri))
     assert not np.any(f)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("row_tiles", [0, 2])
+def test_pairs_without_primitives(row_tiles, oracle):
+    """Kept shell pairs whose primitive pairs were all dropped, twelve times as
+    many as there are records: they add nothing, in the direct form of (ss|ss)
+    (which loads a ket's first record ahead) and in row tiles."""
+    from tests.test_host_calls import row_of_s
+
+    b = row_of_s(100)
+    d = np.random.default_rng(9).uniform(-1.0, 1.0, b.ntri)
+    h = liberi.Handle()
+    h.set_option(liberi.OPT_ROW_TILES, row_tiles)
+    h.set_option(liberi.OPT_AUTOTUNE, 0)
+    h.setup(b)
+    f = h.fock_build(d)
+    assert h.stats()["prim_pairs"] * 12 <= 5050
+    h.destroy()
+    assert np.max(np.abs(f - oracle.fock(b, d)[0])) <= FOCK_TOL

@@ -1,0 +1,120 @@
+"""What the host code of the built library allocates, launches, orders and
+frees, on the HIP calls of hip_host.cpp in place of the runtime (no GPU).
+
+Each scenario runs in a process of its own, in which those calls come before
+the runtime's."""
+import ctypes as C
+import re
+import subprocess
+import sys
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+if str(ROOT) not in sys.path:
+    sys.path.insert(0, str(ROOT))
+
+
+@pytest.fixture(scope="session")
+def host_lib(tmp_path_factory):
+    so = tmp_path_factory.mktemp("hip_host") / "hip_host.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-I/opt/rocm/include", "-o", str(so),
+                    str(ROOT / "tests" / "hip_host.cpp"), "-ldl"], check=True)
+    return so
+
+
+def run(scenario, host_lib):
+    p = subprocess.run([sys.executable, __file__, str(host_lib), scenario], capture_output=True, text=True, timeout=300,
+                       cwd=ROOT)
+    assert p.returncode == 0, f"{scenario}: exit {p.returncode}\n{p.stdout[-2000:]}\n{p.stderr[-4000:]}"
+
+
+class Host:
+    """The calls of hip_host.cpp, loaded before the library."""
+
+    def __init__(self, so):
+        self.c = C.CDLL(so, C.RTLD_GLOBAL)
+        self.c.host_log.restype = C.c_char_p
+        for f in ("host_bytes", "host_peak"):
+            getattr(self.c, f).restype = C.c_size_t
+        self.c.host_fail.argtypes = [C.c_size_t]
+        vp = C.c_void_p
+        for f in ("host_id", "host_in_flight"):
+            getattr(self.c, f).argtypes = [vp]
+        self.c.host_before.argtypes = [vp, vp]
+        self.c.hipStreamBeginCapture.argtypes = [vp, C.c_int]
+        self.c.hipStreamEndCapture.argtypes = [vp, C.POINTER(vp)]
+
+    def stream(self):
+        s = C.c_void_p()
+        assert self.c.hipStreamCreateWithFlags(C.byref(s), 0) == 0
+        return s
+
+    def array(self, values):
+        """A device array (host memory here)."""
+        values = np.ascontiguousarray(values, dtype=np.float64)
+        p = C.c_void_p()
+        assert self.c.hipMalloc(C.byref(p), C.c_size_t(values.nbytes)) == 0
+        C.memmove(p, values.ctypes.data, values.nbytes)
+        return p
+
+    def begin_capture(self, s):
+        assert self.c.hipStreamBeginCapture(s, 0) == 0
+
+    def end_capture(self, s):
+        g = C.c_void_p()
+        assert self.c.hipStreamEndCapture(s, C.byref(g)) == 0
+
+    def log(self):
+        """The lines since the last call."""
+        lines = self.c.host_log().decode().splitlines()
+        self.c.host_clear()
+        return lines
+
+
+def field(line, name):
+    m = re.search(rf"\b{name}=(\S+)", line)
+    return m and (int(m.group(1)) if m.group(1).isdigit() else m.group(1))
+
+
+def row_of_s(n):
+    """n atoms in a row, one tight s primitive each; Schwarz values of 1 keep
+    every pair, and most pairs have no primitive pair left."""
+    from gms_liberi_amd.caseio import Basis
+
+    one = np.arange(n) + 1
+    coef = np.zeros((4, n))
+    coef[0] = 1.0
+    xyz = np.zeros((n, 3))
+    xyz[:, 0] = 1.4 * np.arange(n)
+    return Basis(n, n, n, 1, np.ones(n, int), np.ones(n, int), one, one, one, one, one, np.full(n, 3.4), *coef, xyz.ravel(),
+                 np.ones(n * (n + 1) // 2))
+
+
+# ------------------------------------------------------------- scenarios
+def scenario_pairs_without_primitives(host):
+    """A kernel may read the first record of any pair it is given: those of a
+    pair without primitives lie inside the array as well."""
+    from gms_liberi_amd import liberi
+
+    h = liberi.Handle()
+    h.setup(row_of_s(100))
+    h.fock_build(np.zeros(100 * 101 // 2))
+    begin = [x for x in host.log() if "build_begin" in x]
+    assert begin and field(begin[0], "empty") > 3000
+    assert field(begin[0], "past") == 0, begin[0]
+    h.destroy()
+
+
+SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
+
+
+@pytest.mark.parametrize("scenario", SCENARIOS)
+def test_host_calls(scenario, host_lib):
+    run(scenario, host_lib)
+
+
+if __name__ == "__main__":
+    globals()["scenario_" + sys.argv[2]](Host(sys.argv[1]))

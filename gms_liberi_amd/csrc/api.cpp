@@ -121,10 +121,11 @@ struct liberi_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // builds share the handle's workspace (Dp, Jp, Dsq): one on another stream
-  // than the last waits for its end (ev1; last_stream is NULL after a build
-  // under a caller's capture, whose events cannot be waited for)
-  hipStream_t last_stream = nullptr;
+  // builds share the handle's workspace (Dp, Jp, Dsq): each waits for the end
+  // of the last one, on whatever stream that was.  ev1 is that end (built: it
+  // has been recorded); a build under a caller's capture, which does not run
+  // then, records neither event.
+  bool built = false;
   std::vector<DevBuf> owned;
   DevBuf pairs, prims, dens, fock;
   DevBuf tables;  // segments and row tiles of every class
@@ -175,7 +176,7 @@ struct liberi_ctx {
 // fold the events of the last build into the statistics (waits for it)
 static void collect_timing(liberi_ctx *h) {
   if (h->build_pending) {
-    if (hipEventSynchronize(h->ev1) == hipSuccess) {
+    if (h->built && hipEventSynchronize(h->ev1) == hipSuccess) {
       float ms = 0.f;
       if (hipEventElapsedTime(&ms, h->ev0, h->ev1) == hipSuccess) h->stats.last_build_ms = ms;
     }
@@ -1679,8 +1680,8 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   const BuildArgs ba = build_args(h, dD, dK ? dK : dD, dF, k_scale);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cap));
-  if (cap == hipStreamCaptureStatusNone && h->last_stream && h->last_stream != st)
-    HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
+  const bool runs = cap == hipStreamCaptureStatusNone;
+  if (runs && h->built) HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
   // the autotuner's timed launches see this build's max |D| (mixed form)
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
@@ -1699,14 +1700,16 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     h->g_dD = dD;
     h->g_dF = dF;
   }
-  HIP_TRY(hipEventRecord(h->ev0, st));
+  if (runs) HIP_TRY(hipEventRecord(h->ev0, st));
   if (graph) {
     HIP_TRY(hipGraphLaunch(h->gexec, st));
   } else if (int rc = enqueue_build(h, &ba, 1, dD, st, 1)) {
     return rc;
   }
-  HIP_TRY(hipEventRecord(h->ev1, st));
-  h->last_stream = cap == hipStreamCaptureStatusNone ? st : nullptr;
+  if (runs) {
+    HIP_TRY(hipEventRecord(h->ev1, st));
+    h->built = true;
+  }
   h->build_pending = true;
   h->fp32_pending = h->fp32_tau > 0.0;
   if (!h->fp32_pending) h->stats.fp32_quartets = 0;
@@ -1774,7 +1777,7 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
     if ((*rc = capture_build(h, bas, 2, &h->ugraph, &h->uexec))) return 0;
     std::copy(arrays, arrays + 4, h->ug_arrays);
   }
-  hipError_t e = h->last_stream && h->last_stream != st ? hipStreamWaitEvent(st, h->ev1, 0) : hipSuccess;
+  hipError_t e = h->built ? hipStreamWaitEvent(st, h->ev1, 0) : hipSuccess;
   if (e == hipSuccess) e = (hipError_t)launch_add(dDa, dDb, const_cast<double *>(dt), (int64_t)h->num_bas * (h->num_bas + 1) / 2, st);
   if (e == hipSuccess) e = hipEventRecord(h->ev0, st);
   if (e == hipSuccess) e = hipGraphLaunch(h->uexec, st);
@@ -1783,7 +1786,7 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
     *rc = fail(LIBERI_EDEVICE, std::string("UHF build: ") + hipGetErrorString(e));
     return 0;
   }
-  h->last_stream = st;
+  h->built = true;
   h->build_pending = true;
   h->fp32_pending = h->timing_pending = false;
   h->stats.fp32_quartets = 0;
@@ -1808,8 +1811,7 @@ int liberi_c_fock_build_uhf_device(liberi_ctx *h, const double *dDa, const doubl
   // Da + Db is written where a build on another stream may still read it
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cap));
-  if (cap == hipStreamCaptureStatusNone && h->last_stream && h->last_stream != st)
-    HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
+  if (cap == hipStreamCaptureStatusNone && h->built) HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
   if (int e = launch_add(dDa, dDb, dt, ntri, st))
     return fail(LIBERI_EDEVICE, std::string("Da + Db: ") + hipGetErrorString((hipError_t)e));
   if (int rc = build_on_device(h, dt, dFa, st, dDa, 2.0)) return rc;

@@ -102,3 +102,57 @@ def test_uhf_graph_matches_builds_one_after_the_other(name):
     got = h.fock_build_uhf(*pairs[1])
     assert np.max(np.abs(got[0] - want[1][0])) <= 1e-12 * max(1.0, float(np.max(np.abs(want[1][0]))))
     h.destroy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["cfg_water.npz", "cfg_ethane.npz", "cfg_cn_chain.npz"])
+def test_unrestricted_builds_on_device_arrays_and_streams(name):
+    """Unrestricted builds on two sets of device arrays, A on one stream and B
+    on another, with a restricted build among them and nothing waited for
+    on the host: first calls, calls that capture the graph of both spins, replays,
+    and an eager one at the end.  Each equals the build of a handle of its own
+    without graphs, to summation order (1e-12 of the largest element)."""
+    from gms_liberi_amd import hipmem
+
+    case = Case.load_npz(GOLD / name)
+    n = case.basis.ntri
+    rng = np.random.default_rng(6)
+    dens = {"A": (0.6 * case.density, 0.5 * rng.permutation(case.density)), "B": (0.3 * case.density, 0.9 * case.density)}
+    ref = liberi.Handle()
+    ref.set_option(liberi.OPT_GRAPH, 0)
+    ref.setup(case.basis)
+    want = {k: [f.copy() for f in ref.fock_build_uhf(*d)] for k, d in dens.items()}
+    want["R"] = [ref.fock_build(case.density).copy()]
+    ref.destroy()
+
+    h = liberi.Handle()
+    h.setup(case.basis)
+    arrays = {k: [hipmem.DeviceArray.from_host(x) for x in d] + [hipmem.DeviceArray(n), hipmem.DeviceArray(n)]
+              for k, d in dens.items()}
+    arrays["R"] = [hipmem.DeviceArray.from_host(case.density), hipmem.DeviceArray(n)]
+    streams = [hipmem.Stream(), hipmem.Stream()]
+    got = []
+
+    def build(k, s):
+        a = arrays[k]
+        if k == "R":
+            h.fock_build_device(a[0].address, a[1].address, n, s.address)
+        else:
+            assert h._lib.liberi_c_fock_build_uhf_device(h._h, *[x.ptr for x in a], n, s.ptr) == 0
+        for f, w in zip(a[len(a) // 2:], want[k]):
+            p = hipmem.PinnedArray(n)
+            f.copy_to_async(p, s)
+            got.append((k, p, w))
+
+    for k in "AABBAARBAB":
+        build(k, streams[k != "A"])
+    for s in streams:
+        s.synchronize()
+    h.set_option(liberi.OPT_GRAPH, 0)
+    build("A", streams[1])
+    streams[1].synchronize()
+    for i, (k, p, w) in enumerate(got):
+        assert np.max(np.abs(p.array - w)) <= 1e-12 * max(1.0, float(np.max(np.abs(w)))), (i, k)
+    h.destroy()
+    for s in streams:
+        s.destroy()

@@ -79,6 +79,12 @@ def field(line, name):
     return m and (int(m.group(1)) if m.group(1).isdigit() else m.group(1))
 
 
+def golden(name):
+    from gms_liberi_amd.caseio import Case
+
+    return Case.load_npz(ROOT / "tests" / "golden" / name).basis
+
+
 def row_of_s(n):
     """n atoms in a row, one tight s primitive each; Schwarz values of 1 keep
     every pair, and most pairs have no primitive pair left."""
@@ -105,6 +111,42 @@ def scenario_pairs_without_primitives(host):
     begin = [x for x in host.log() if "build_begin" in x]
     assert begin and field(begin[0], "empty") > 3000
     assert field(begin[0], "past") == 0, begin[0]
+    h.destroy()
+
+
+def scenario_builds_on_other_streams_wait(host):
+    """Every build of a handle comes after the last one that runs, whatever
+    its stream, restricted or not, also where one was captured in between."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_water.npz")
+    n = b.ntri
+    streams = [host.stream() for _ in range(4)]
+    D, F, Da, Db, Fa, Fb = (host.array(np.zeros(n)) for _ in range(6))
+    h = liberi.Handle()
+    h.setup(b)
+
+    def rhf(s):
+        h.fock_build_device(D.value, F.value, n, s.value)
+
+    def uhf(s):
+        assert h._lib.liberi_c_fock_build_uhf_device(h._h, Da, Db, Fa, Fb, n, s) == 0
+
+    uhf(streams[0])
+    for first in (rhf, uhf):
+        for second in (rhf, uhf):
+            for captured in (None, rhf, uhf):
+                a, x, c, d = streams
+                first(a)
+                if captured:
+                    host.begin_capture(x)
+                    captured(x)
+                    host.end_capture(x)
+                second(c)
+                assert host.c.host_before(a, c), (first.__name__, captured and captured.__name__, second.__name__)
+                second(d)  # (the unrestricted graph from its second call on)
+                assert host.c.host_before(c, d)
+    assert h.stats()["last_build_ms"] > 0
     h.destroy()
 
 

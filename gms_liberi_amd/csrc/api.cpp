@@ -164,6 +164,7 @@ struct liberi_ctx {
   hipGraphExec_t uexec = nullptr;
   const void *ug_arrays[4] = {}, *u_arrays[4] = {};
   DevBuf uhf_work;
+  bool uhf_refused = false;  // no memory for it: the spins' builds run one after the other
   bool fp32_pending = false;
   ClassState cls[kNumClasses];
   liberi_stats stats{};
@@ -214,6 +215,9 @@ static int dev_alloc_charged(DevBuf &b, size_t bytes) {
   if (bytes == 0) return LIBERI_OK;
   const hipError_t e = hipMalloc(&b.p, bytes);
   if (e != hipSuccess) {
+    // (a caller may go on without the memory: the launches after it return the
+    // thread's last error, which later successful calls leave as it is)
+    (void)hipGetLastError();
     b.p = nullptr;
     return fail(e == hipErrorOutOfMemory ? LIBERI_ENOMEM : LIBERI_EDEVICE,
                 "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
@@ -266,6 +270,7 @@ static void release_device(liberi_ctx *h) {
   drop_graph(h);
   std::fill(h->u_arrays, h->u_arrays + 4, nullptr);
   dev_free(h->uhf_work);
+  h->uhf_refused = false;
   for (auto &c : h->cls) {
     c = ClassState{};
   }
@@ -396,7 +401,10 @@ int liberi_c_set_option(liberi_ctx *h, int32_t opt, double v) {
       h->row_tiles = (int)v;
       break;
     case LIBERI_OPT_GRAPH: h->use_graph = v != 0.0; break;
-    case LIBERI_OPT_MAX_DEVICE_BYTES: h->max_device_bytes = v; break;
+    case LIBERI_OPT_MAX_DEVICE_BYTES:
+      h->max_device_bytes = v;
+      h->uhf_refused = false;
+      break;
     case LIBERI_OPT_RANK_SPLIT:
       if (v != 0.0 && v != 1.0) return fail(LIBERI_EARG, "liberi_c_set_option: RANK_SPLIT must be 0 or 1");
       h->rank_split = (int)v;
@@ -1759,13 +1767,20 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
   const bool again = std::equal(arrays, arrays + 4, h->u_arrays);
   std::copy(arrays, arrays + 4, h->u_arrays);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (!again || !h->use_graph || h->class_timing || h->only_class >= 0 || h->fused || h->fp32_tau > 0.0 ||
+  if (!again || h->uhf_refused || !h->use_graph || h->class_timing || h->only_class >= 0 || h->fused || h->fp32_tau > 0.0 ||
       choices_open(h) || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
     return 1;
   if (!h->uexec || !std::equal(arrays, arrays + 4, h->ug_arrays)) {
     drop_uhf_graph(h);
     const size_t npl = (size_t)h->layout.off[kNumPairClasses], nsq = (size_t)h->num_bas * h->num_bas;
-    if (!h->uhf_work.p && dev_alloc(h, h->uhf_work, (4 * npl + 2 * nsq) * sizeof(double)) != LIBERI_OK) return 1;
+    if (!h->uhf_work.p) {
+      const std::string msg = g_last_error;
+      if (dev_alloc(h, h->uhf_work, (4 * npl + 2 * nsq) * sizeof(double)) != LIBERI_OK) {
+        h->uhf_refused = true;
+        g_last_error = msg;
+        return 1;
+      }
+    }
     BuildArgs bas[2] = {build_args(h, dt, dDa, dFa, 2.0), build_args(h, dt, dDb, dFb, 2.0)};
     double *w = (double *)h->uhf_work.p;
     bas[1].Dp = w;
@@ -1902,9 +1917,11 @@ int liberi_c_schwarz(int32_t nsh, int32_t natoms, int32_t num_bas, int32_t mxgto
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (st) (void)hipStreamDestroy(st);
   if (buf) (void)hipFree(buf);
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
     return fail(e == hipErrorOutOfMemory ? LIBERI_ENOMEM : LIBERI_EDEVICE,
                 std::string("liberi_c_schwarz: ") + hipGetErrorString(e));
+  }
   schwarz_scatter(s, out.data(), schwrz_int);
   return LIBERI_OK;
 }

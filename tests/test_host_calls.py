@@ -150,6 +150,61 @@ def scenario_builds_on_other_streams_wait(host):
     h.destroy()
 
 
+def scenario_unrestricted_builds_without_a_second_workspace(host):
+    """Where the second workspace of the side-by-side unrestricted build is
+    refused, by the device or by the handle's budget, the builds run one
+    after the other; it is asked for once."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_water.npz")
+    n = b.ntri
+    s = host.stream()
+    arrays = [host.array(np.zeros(n)) for _ in range(4)]
+
+    def build(h):
+        host.log()
+        rc = h._lib.liberi_c_fock_build_uhf_device(h._h, *arrays, n, s)
+        return rc, host.log()
+
+    h = liberi.Handle()
+    h.setup(b)
+    assert build(h)[0] == 0
+    rc, lines = build(h)
+    size = [field(x.replace("malloc ", "malloc="), "malloc") for x in lines if x.startswith("malloc")]
+    assert rc == 0 and len(size) == 1 and any("replay" in x for x in lines)
+    with pytest.raises(liberi.LiberiError):
+        h.fock_build(np.zeros(n + 1))
+    message = h._lib.liberi_c_last_error()
+    h.destroy()
+    for budgeted in (False, True):
+        h = liberi.Handle()
+        h.setup(b)
+        assert build(h)[0] == 0
+        h.set_option(liberi.OPT_MAX_DEVICE_BYTES, h.stats()["device_bytes"] + size[0] - 1 if budgeted else 0)
+        host.c.host_fail(0 if budgeted else size[0])
+        refused = 0
+        for _ in range(3):
+            rc, lines = build(h)
+            assert rc == 0, h._lib.liberi_c_last_error()
+            refused += sum("malloc failed" in x for x in lines)
+            assert sum("build_begin" in x for x in lines) == 2 and not any("replay" in x for x in lines)
+        assert refused == (0 if budgeted else 1) and h._lib.liberi_c_last_error() == message
+        host.c.host_fail(0)
+        h.set_option(liberi.OPT_MAX_DEVICE_BYTES, 0)  # asked for again
+        assert any("replay" in x for x in build(h)[1])
+        h.destroy()
+    # a failed setup, or Schwarz call, leaves nothing behind for the next
+    h = liberi.Handle()
+    host.c.host_fail(1 << 10)
+    for call in (lambda: h.setup(b), lambda: liberi.schwarz(b)):
+        with pytest.raises(liberi.LiberiError) as e:
+            call()
+        assert e.value.code == 5
+    host.c.host_fail(0)
+    h.setup(b)
+    h.destroy()
+
+
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
 
 

@@ -249,24 +249,48 @@ static void dev_free(DevBuf &b) {
   b.bytes = 0;
 }
 
-static void drop_uhf_graph(liberi_ctx *h) {
-  if (h->uexec) (void)hipGraphExecDestroy(h->uexec);
-  if (h->ugraph) (void)hipGraphDestroy(h->ugraph);
-  h->uexec = nullptr;
-  h->ugraph = nullptr;
+// Waits on the host for the last build that ran, on whatever stream (a
+// thread that captures may call it: it waits for nothing captured).
+static void wait_last_build(liberi_ctx *h) {
+  if (!h->built) return;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  (void)hipEventSynchronize(h->ev1);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
+// A graph taken from the handle, destroyed once its replays are over.
+struct OldGraph {
+  liberi_ctx *h;
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  OldGraph(liberi_ctx *h_, hipGraph_t &g, hipGraphExec_t &e) : h(h_) {
+    std::swap(graph, g);
+    std::swap(exec, e);
+  }
+  OldGraph(const OldGraph &) = delete;
+  OldGraph &operator=(const OldGraph &) = delete;
+  ~OldGraph() { end(); }
+  void end() {
+    if (exec) {
+      wait_last_build(h);
+      (void)hipGraphExecDestroy(exec);
+    }
+    if (graph) (void)hipGraphDestroy(graph);
+    exec = nullptr;
+    graph = nullptr;
+  }
+};
+
 static void drop_graph(liberi_ctx *h) {
-  drop_uhf_graph(h);
-  if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
-  if (h->graph) (void)hipGraphDestroy(h->graph);
-  h->gexec = nullptr;
-  h->graph = nullptr;
+  OldGraph(h, h->ugraph, h->uexec);
+  OldGraph(h, h->graph, h->gexec);
   h->g_dD = nullptr;
   h->g_dF = nullptr;
 }
 
 static void release_device(liberi_ctx *h) {
+  wait_last_build(h);
   drop_graph(h);
   std::fill(h->u_arrays, h->u_arrays + 4, nullptr);
   dev_free(h->uhf_work);
@@ -1702,8 +1726,12 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   // the batched form: capture once (per D, F), replay afterwards.  Per-class
   // timing and single-class diagnostics run eagerly on st.
   const bool graph = h->use_graph && !h->class_timing && h->only_class < 0 && ba.DK == dD && k_scale == 1.0;
-  if (graph && (!h->gexec || h->g_dD != dD || h->g_dF != dF)) {
-    drop_graph(h);
+  // (a graph of other arrays may still run: it goes after the launch of the new one)
+  hipGraph_t no_graph = nullptr;
+  hipGraphExec_t no_exec = nullptr;
+  const bool recapture = graph && (!h->gexec || h->g_dD != dD || h->g_dF != dF);
+  OldGraph old(h, recapture ? h->graph : no_graph, recapture ? h->gexec : no_exec);
+  if (recapture) {
     if (int rc = capture_build(h, &ba, 1, &h->graph, &h->gexec)) return rc;
     h->g_dD = dD;
     h->g_dF = dF;
@@ -1714,6 +1742,7 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   } else if (int rc = enqueue_build(h, &ba, 1, dD, st, 1)) {
     return rc;
   }
+  old.end();
   if (runs) {
     HIP_TRY(hipEventRecord(h->ev1, st));
     h->built = true;
@@ -1770,8 +1799,11 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
   if (!again || h->uhf_refused || !h->use_graph || h->class_timing || h->only_class >= 0 || h->fused || h->fp32_tau > 0.0 ||
       choices_open(h) || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
     return 1;
-  if (!h->uexec || !std::equal(arrays, arrays + 4, h->ug_arrays)) {
-    drop_uhf_graph(h);
+  hipGraph_t no_graph = nullptr;
+  hipGraphExec_t no_exec = nullptr;
+  const bool recapture = !h->uexec || !std::equal(arrays, arrays + 4, h->ug_arrays);
+  OldGraph old(h, recapture ? h->ugraph : no_graph, recapture ? h->uexec : no_exec);
+  if (recapture) {
     const size_t npl = (size_t)h->layout.off[kNumPairClasses], nsq = (size_t)h->num_bas * h->num_bas;
     if (!h->uhf_work.p) {
       const std::string msg = g_last_error;
@@ -1796,6 +1828,7 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
   if (e == hipSuccess) e = (hipError_t)launch_add(dDa, dDb, const_cast<double *>(dt), (int64_t)h->num_bas * (h->num_bas + 1) / 2, st);
   if (e == hipSuccess) e = hipEventRecord(h->ev0, st);
   if (e == hipSuccess) e = hipGraphLaunch(h->uexec, st);
+  old.end();
   if (e == hipSuccess) e = hipEventRecord(h->ev1, st);
   if (e != hipSuccess) {
     *rc = fail(LIBERI_EDEVICE, std::string("UHF build: ") + hipGetErrorString(e));

@@ -205,6 +205,55 @@ def scenario_unrestricted_builds_without_a_second_workspace(host):
     h.destroy()
 
 
+def scenario_graphs_end_after_their_replays(host):
+    """A captured build is destroyed, whatever drops it, only after its replays
+    on the caller's stream; builds on other arrays are launched before that wait."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_water.npz")
+    n = b.ntri
+    s = host.stream()
+    a = [host.array(np.zeros(n)) for _ in range(4)]
+    c = [host.array(np.zeros(n)) for _ in range(4)]
+
+    def rhf(h, x):
+        h.fock_build_device(x[0].value, x[1].value, n, s.value)
+
+    def uhf(h, x):
+        for _ in range(2):
+            assert h._lib.liberi_c_fock_build_uhf_device(h._h, *x, n, s) == 0
+
+    def destroyed():
+        return [field(x, "in_flight") for x in host.log() if x.startswith("destroy")]
+
+    drops = [lambda h, build: h.set_option(liberi.OPT_VALUE_CUTOFF, 1e-12), lambda h, build: h.cleanup(),
+             lambda h, build: h.setup(b), lambda h, build: h.destroy(), lambda h, build: build(h, c)]
+    for build in (rhf, uhf):
+        for drop in drops:
+            h = liberi.Handle()
+            h.setup(b)
+            build(h, a)
+            build(h, a)
+            host.log()
+            assert host.c.host_in_flight(s)
+            drop(h, build)
+            assert destroyed() == [0], (build.__name__, drops.index(drop))
+            if drop is drops[-1]:
+                assert host.c.host_in_flight(s)  # the build on the other arrays
+            h.destroy()
+    # one that a capture of the caller's holds back
+    h = liberi.Handle()
+    h.setup(b)
+    rhf(h, a)
+    x = host.stream()
+    host.begin_capture(x)
+    host.log()
+    h.set_option(liberi.OPT_VALUE_CUTOFF, 1e-12)
+    host.end_capture(x)
+    assert destroyed() == [0]
+    h.destroy()
+
+
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
 
 

@@ -164,6 +164,10 @@ struct liberi_ctx {
   hipGraphExec_t uexec = nullptr;
   const void *ug_arrays[4] = {}, *u_arrays[4] = {};
   DevBuf uhf_work;
+  // workspaces of the builds in graphs of the caller's, one per Fock array: two
+  // builds into one array cannot run side by side anyway, those into others
+  // may, and beside the builds of the handle
+  std::vector<std::pair<const double *, DevBuf>> captured;
   bool uhf_refused = false;  // no memory for it: the spins' builds run one after the other
   bool fp32_pending = false;
   ClassState cls[kNumClasses];
@@ -295,6 +299,8 @@ static void release_device(liberi_ctx *h) {
   std::fill(h->u_arrays, h->u_arrays + 4, nullptr);
   dev_free(h->uhf_work);
   h->uhf_refused = false;
+  for (auto &w : h->captured) dev_free(w.second);
+  h->captured.clear();
   for (auto &c : h->cls) {
     c = ClassState{};
   }
@@ -1679,6 +1685,36 @@ static BuildArgs build_args(liberi_ctx *h, const double *dD, const double *dK, d
   return ba;
 }
 
+// doubles of a build's workspace beside the handle's own, and its arrays in `w`
+static size_t work_doubles(const liberi_ctx *h) {
+  return 4 * (size_t)h->layout.off[kNumPairClasses] + 2 * (size_t)h->num_bas * h->num_bas;
+}
+static void use_work(const liberi_ctx *h, BuildArgs &ba, double *w) {
+  const size_t npl = (size_t)h->layout.off[kNumPairClasses], nsq = (size_t)h->num_bas * h->num_bas;
+  ba.Dp = w;
+  ba.Dq = w + npl;
+  ba.Jp = w + 2 * npl;
+  ba.Jq = w + 3 * npl;
+  ba.Dsq = w + 4 * npl;
+  ba.Ksq = w + 4 * npl + nsq;
+}
+
+// The workspace of a build into ba.F under a caller's capture.
+static int use_captured_work(liberi_ctx *h, BuildArgs &ba) {
+  for (const auto &[F, buf] : h->captured)
+    if (F == ba.F) return use_work(h, ba, (double *)buf.p), LIBERI_OK;
+  DevBuf buf;
+  // (an allocation is no work of the stream's)
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  const int rc = dev_alloc(h, buf, work_doubles(h) * sizeof(double));
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  if (rc) return rc;
+  h->captured.push_back({ba.F, buf});
+  use_work(h, ba, (double *)buf.p);
+  return LIBERI_OK;
+}
+
 // whether the next build has to choose forms, tile lengths or times first
 static bool choices_open(const liberi_ctx *h) {
   for (int k = 0; k < kNumClasses; ++k) {
@@ -1709,11 +1745,14 @@ static int capture_build(liberi_ctx *h, const BuildArgs *bas, int spins, hipGrap
 
 static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStream_t st, const double *dK = nullptr,
                            double k_scale = 1.0) {
-  const BuildArgs ba = build_args(h, dD, dK ? dK : dD, dF, k_scale);
+  BuildArgs ba = build_args(h, dD, dK ? dK : dD, dF, k_scale);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cap));
   const bool runs = cap == hipStreamCaptureStatusNone;
   if (runs && h->built) HIP_TRY(hipStreamWaitEvent(st, h->ev1, 0));
+  // (the caller may replay what is captured here beside other builds)
+  if (!runs)
+    if (int rc = use_captured_work(h, ba)) return rc;
   // the autotuner's timed launches see this build's max |D| (mixed form)
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
@@ -1723,9 +1762,11 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
       return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
     if (int rc = choose_variants(h, ba, st)) return rc;
   }
-  // the batched form: capture once (per D, F), replay afterwards.  Per-class
+  // the batched form: capture once (per D, F), replay afterwards; under a
+  // caller's capture, its branches straight into the caller's graph.  Per-class
   // timing and single-class diagnostics run eagerly on st.
-  const bool graph = h->use_graph && !h->class_timing && h->only_class < 0 && ba.DK == dD && k_scale == 1.0;
+  const bool batched = h->use_graph && !h->class_timing && h->only_class < 0 && ba.DK == dD && k_scale == 1.0;
+  const bool graph = batched && runs;
   // (a graph of other arrays may still run: it goes after the launch of the new one)
   hipGraph_t no_graph = nullptr;
   hipGraphExec_t no_exec = nullptr;
@@ -1739,7 +1780,7 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   if (runs) HIP_TRY(hipEventRecord(h->ev0, st));
   if (graph) {
     HIP_TRY(hipGraphLaunch(h->gexec, st));
-  } else if (int rc = enqueue_build(h, &ba, 1, dD, st, 1)) {
+  } else if (int rc = enqueue_build(h, &ba, 1, dD, st, batched ? kBranches : 1)) {
     return rc;
   }
   old.end();
@@ -1804,23 +1845,16 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
   const bool recapture = !h->uexec || !std::equal(arrays, arrays + 4, h->ug_arrays);
   OldGraph old(h, recapture ? h->ugraph : no_graph, recapture ? h->uexec : no_exec);
   if (recapture) {
-    const size_t npl = (size_t)h->layout.off[kNumPairClasses], nsq = (size_t)h->num_bas * h->num_bas;
     if (!h->uhf_work.p) {
       const std::string msg = g_last_error;
-      if (dev_alloc(h, h->uhf_work, (4 * npl + 2 * nsq) * sizeof(double)) != LIBERI_OK) {
+      if (dev_alloc(h, h->uhf_work, work_doubles(h) * sizeof(double)) != LIBERI_OK) {
         h->uhf_refused = true;
         g_last_error = msg;
         return 1;
       }
     }
     BuildArgs bas[2] = {build_args(h, dt, dDa, dFa, 2.0), build_args(h, dt, dDb, dFb, 2.0)};
-    double *w = (double *)h->uhf_work.p;
-    bas[1].Dp = w;
-    bas[1].Dq = w + npl;
-    bas[1].Jp = w + 2 * npl;
-    bas[1].Jq = w + 3 * npl;
-    bas[1].Dsq = w + 4 * npl;
-    bas[1].Ksq = w + 4 * npl + nsq;
+    use_work(h, bas[1], (double *)h->uhf_work.p);
     if ((*rc = capture_build(h, bas, 2, &h->ugraph, &h->uexec))) return 0;
     std::copy(arrays, arrays + 4, h->ug_arrays);
   }

@@ -96,9 +96,11 @@ int liberi_c_fock_build(liberi_ctx *ctx, const double *density, double *fock, in
  * enqueueing.  No counterpart in the reference (which maps D/F per call,
  * src/liberi_driver.F90:66,163); for callers that keep D and F in HBM.
  * Builds of one handle share its device workspace: one enqueued on another
- * stream than the last waits for it (a build that the caller has captured
- * into a graph of its own must not be replayed beside another build of the
- * same handle; other handles are independent). */
+ * stream than the last waits for it.  A build that the caller captures into a
+ * graph of its own gets a workspace of its own (per Fock array, kept until the
+ * next setup or cleanup), so that its replays may run beside other builds of
+ * the handle; those of the mixed form, of the fused launch and of an
+ * unrestricted build share a few values besides and may not. */
 int liberi_c_fock_build_device(liberi_ctx *ctx, const double *d_density, double *d_fock, int64_t n,
                                void *stream);
 

@@ -499,3 +499,62 @@ def test_shared_launches_match_launches_per_class(mol, natoms, ranks):
     whole = h.fock_build(case.density)
     h.destroy()
     assert np.max(np.abs(total["shared"] - whole)) <= 1e-12 * max(1.0, float(np.max(np.abs(whole))))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,graph", [("cfg_water.npz", 1), ("cfg_ethane.npz", 1), ("cfg_ethane.npz", 0),
+                                        ("cfg_cn_chain.npz", 1)])
+def test_builds_in_graphs_of_the_callers(name, graph):
+    """Two builds of one handle captured by the caller, each into its own graph
+    and Fock array, replayed side by side and beside the handle's own builds on
+    a third stream: each replay equals the eager build of its density to
+    summation order (1e-12 of the largest element), over several replays with
+    new densities."""
+    import ctypes as C
+
+    from gms_liberi_amd import hipmem
+
+    case = Case.load_npz(GOLD / name)
+    n = case.basis.ntri
+    rng = np.random.default_rng(3)
+    ref = liberi.Handle()
+    ref.set_option(liberi.OPT_GRAPH, 0)
+    ref.setup(case.basis)
+    h = liberi.Handle()
+    h.set_option(liberi.OPT_GRAPH, graph)
+    h.setup(case.basis)
+    rt = hipmem.runtime()
+    streams = [hipmem.Stream() for _ in range(3)]
+    D = [hipmem.DeviceArray.from_host(case.density) for _ in range(3)]
+    F = [hipmem.DeviceArray(n) for _ in range(3)]
+    h.fock_build_device(D[2].address, F[2].address, n, streams[2].address)
+    execs = []
+    for k in range(2):
+        s, g, e = streams[k], C.c_void_p(), C.c_void_p()
+        assert rt.hipStreamBeginCapture(s.ptr, 2 * k) == 0  # global and relaxed mode
+        h.fock_build_device(D[k].address, F[k].address, n, s.address)
+        assert rt.hipStreamEndCapture(s.ptr, C.byref(g)) == 0
+        assert rt.hipGraphInstantiate(C.byref(e), g, None, None, C.c_size_t(0)) == 0
+        assert rt.hipGraphDestroy(g) == 0
+        execs.append(e)
+    h.fock_build_device(D[2].address, F[2].address, n, streams[2].address)
+    streams[2].synchronize()
+    for step in range(4):
+        dens = [np.ascontiguousarray(x * case.density) for x in rng.uniform(0.2, 1.0, 3)]
+        for d, a in zip(dens, D):
+            assert rt.hipMemcpy(a.ptr, d.ctypes.data, d.nbytes, 1) == 0
+        for _ in range(3):  # (nothing waited for between them)
+            for k in range(2):
+                assert rt.hipGraphLaunch(execs[k], streams[k].ptr) == 0
+            h.fock_build_device(D[2].address, F[2].address, n, streams[2].address)
+        for s in streams:
+            s.synchronize()
+        for k in range(3):
+            want = ref.fock_build(dens[k])
+            assert np.max(np.abs(F[k].to_host() - want)) <= 1e-12 * max(1.0, float(np.max(np.abs(want)))), (step, k)
+    for e in execs:
+        assert rt.hipGraphExecDestroy(e) == 0
+    h.destroy()
+    ref.destroy()
+    for s in streams:
+        s.destroy()

@@ -254,6 +254,58 @@ def scenario_graphs_end_after_their_replays(host):
     h.destroy()
 
 
+def scenario_captured_builds_have_their_own_workspace(host):
+    """A build under a caller's capture (which may be replayed beside others)
+    gets a workspace per Fock array, and gives it back with the handle's data."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_water.npz")
+    n = b.ntri
+    run, x = host.stream(), host.stream()
+    D = host.array(np.zeros(n))
+    F = [host.array(np.zeros(n)) for _ in range(3)]
+    h = liberi.Handle()
+    h.setup(b)
+    held = h.stats()["device_bytes"]
+
+    def build(f, s):
+        host.log()
+        h.fock_build_device(D.value, f.value, n, s.value)
+        lines = host.log()
+        assert not any("capture stream" in k or "replay" in k for k in lines) or s is run
+        return {field(k, "Jp") for k in lines if "build_begin" in k}
+
+    own = build(F[0], run)
+    h.stats()
+    for graph in (1, 0):
+        h.set_option(liberi.OPT_GRAPH, graph)
+        work = []
+        host.begin_capture(x)
+        for f in (F[0], F[1], F[2], F[1]):
+            work.append(build(f, x))
+        host.end_capture(x)
+        assert all(len(w) == 1 for w in work) and work[3] == work[1]
+        assert len(set.union(own, *work)) == 4
+        assert build(F[0], run) <= own
+    assert h.stats()["device_bytes"] > held
+    before = host.c.host_bytes()
+    h.cleanup()
+    assert h.stats()["device_bytes"] == 0 and host.c.host_bytes() < before
+    h.setup(b)
+    assert h.stats()["device_bytes"] == held
+    # no memory for it: refused, and the handle goes on
+    h.fock_build(np.zeros(n))
+    host.begin_capture(x)
+    host.c.host_fail(1 << 10)
+    with pytest.raises(liberi.LiberiError) as e:
+        build(F[1], x)
+    assert e.value.code == 5
+    host.c.host_fail(0)
+    host.end_capture(x)
+    h.fock_build(np.zeros(n))
+    h.destroy()
+
+
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
 
 

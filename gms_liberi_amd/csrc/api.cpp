@@ -94,8 +94,10 @@ struct ClassState {
   const RowTile *tiles[kNumTileLens] = {};
   int32_t ntile[kNumTileLens] = {};
   ClassDev dev{};
-  // shared launch the class runs in (-1: none), its workgroups there and, in a
-  // row-tiled one, its tiles
+  // form of the last build, as in liberi_stats (-1: not built)
+  int32_t ran = -1, ran_tile = 0, ran_fp32 = 0;
+  // shared launch the class has a place in (-1: none), its workgroups there and,
+  // in a row-tiled one, its tiles; the choices above are those of its own launch
   int shared = -1;
   int32_t shared_groups = 0;
   const RowTile *shared_tiles = nullptr;
@@ -146,7 +148,6 @@ struct liberi_ctx {
   bool fused = false;      // LIBERI_OPT_FUSED
   int row_orient = 0;      // LIBERI_OPT_ROW_ORIENT
   int tile_len = -1;       // LIBERI_OPT_TILE_LEN as an index into kTileLens; -1 chosen per class
-  bool last_fused = false; // the last build ran the fused launch
   DevBuf tune_F;        // autotuner's scratch Fock matrix
   DevBuf dens_t, dens_b, fock_b;  // UHF: Da + Db, and the beta density / Fock of the host entry point
   hipEvent_t tev[2] = {};
@@ -493,17 +494,9 @@ int liberi_c_get_stats(liberi_ctx *h, liberi_stats *out) {
   collect_timing(h);
   *out = h->stats;
   for (int c = 0; c < kNumClasses; ++c) {
-    const ClassState &cs_ = h->cls[c];
-    const bool row = cs_.row_ok && (h->row_tiles == 2 || (h->row_tiles == 1 && cs_.variant == 1));
-    out->class_variant[c] = !cs_.active || cs_.variant < 0       ? -1
-                            : h->last_fused && class_fused_nq(c) > 0 ? 4
-                            : row                                 ? 1 + cs_.dev.transposed
-                            : cs_.variant == 3 || class_kernel_kind(c) == 2 ? 3
-                                                                  : 0;
-    out->class_fp32[c] = cs_.active && h->fp32_tau > 0.0 && cs_.fp32 == 1;
-    out->class_tile[c] = cs_.active && row && cs_.tile >= 0 && !(h->last_fused && class_fused_nq(c) > 0)
-                             ? (int32_t)kTileLens[cs_.tile]
-                             : 0;
+    out->class_variant[c] = h->cls[c].ran;
+    out->class_fp32[c] = h->cls[c].ran_fp32;
+    out->class_tile[c] = h->cls[c].ran_tile;
   }
   return LIBERI_OK;
 }
@@ -1360,15 +1353,13 @@ static bool class_shared(const liberi_ctx *h, int c) {
          !h->fused && !h->class_timing && h->only_class < 0;
 }
 
-static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
+// Forms, tile lengths and times of the classes with launches of their own.
+// Without `timed` (under a caller's capture, where nothing runs) those of
+// earlier handles and the untimed ones.
+static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st, bool timed) {
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
-    if (!cs_.active || cs_.variant >= 0) continue;
-    if (class_shared(h, c)) {  // the form of its shared launch
-      cs_.dev.coop = cs_.shared > kSharedGroupLaunch && class_has_coop(c);
-      cs_.variant = cs_.shared < kSharedRowLaunches ? 1 : cs_.dev.coop ? 3 : 0;
-      continue;
-    }
+    if (!cs_.active || cs_.variant >= 0 || class_shared(h, c)) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
     // untimed choice: row tiles for the lane classes, and for the group
     // classes with a wave-split form unless the class is too small to time
@@ -1389,6 +1380,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
         cs_.dev.coop = prev == 3;
         continue;
       }
+      if (!timed) continue;
       const int forms[3] = {0, 3, 1};  // group, cooperative, wave-split rows
       float best[3] = {1e30f, 1e30f, 1e30f};
       for (int rep = 0; rep < 6; ++rep) {
@@ -1411,8 +1403,8 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
       cs_.variant = dflt;
       continue;
     }
-    if (const int prev = tuned_choice(c, nq, -1.0); prev >= 0) {
-      cs_.variant = prev;
+    if (const int prev = tuned_choice(c, nq, -1.0); prev >= 0 || !timed) {
+      cs_.variant = prev >= 0 ? prev : dflt;
       continue;
     }
     float best[2] = {1e30f, 1e30f};
@@ -1431,11 +1423,11 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
   // workgroups (rows longer than a tile are split)
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
-    if (!cs_.active || cs_.tile >= 0) continue;
+    if (!cs_.active || cs_.tile >= 0 || class_shared(h, c)) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
     cs_.tile = h->tile_len >= 0 ? h->tile_len : kDefaultTile;
     cs_.dev.threads = kRowThreads[0];
-    if (h->tile_len >= 0 || !h->autotune || !class_row_mode(h, c) || nq < kTuneMinQuartets || class_shared(h, c) ||
+    if (h->tile_len >= 0 || !h->autotune || !class_row_mode(h, c) || nq < kTuneMinQuartets ||
         (h->only_class >= 0 && c != h->only_class)) {
       use_tiles(cs_, cs_.tile);
       continue;
@@ -1444,6 +1436,10 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
       cs_.tile = prev;
       use_tiles(cs_, cs_.tile);
       if (tuned_choice(c, nq, -4.0) == 1) cs_.dev.threads = kRowThreads[1];
+      continue;
+    }
+    if (!timed) {
+      use_tiles(cs_, cs_.tile);
       continue;
     }
     float best[kNumTileLens];
@@ -1488,9 +1484,10 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
   constexpr float kFp32Gain = 0.02f;
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
-    if (!cs_.active || cs_.fp32 >= 0) continue;
+    if (!cs_.active || cs_.fp32 >= 0 || class_shared(h, c)) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
-    if (!(h->fp32_tau > 0.0) || class_kernel_kind(c) != 0) {
+    // (the cooperative form, (fs|fs)'s choice, has no FP32 path either)
+    if (!(h->fp32_tau > 0.0) || class_kernel_kind(c) != 0 || (cs_.dev.coop && !class_row_mode(h, c))) {
       cs_.fp32 = h->fp32_tau > 0.0 ? 0 : -1;
       continue;
     }
@@ -1498,8 +1495,8 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
       cs_.fp32 = 1;  // untimed: the form as asked for
       continue;
     }
-    if (const int prev = tuned_choice(c, nq, h->fp32_tau); prev >= 0) {
-      cs_.fp32 = prev;
+    if (const int prev = tuned_choice(c, nq, h->fp32_tau); prev >= 0 || !timed) {
+      cs_.fp32 = prev >= 0 ? prev : 1;
       continue;
     }
     float best[2] = {1e30f, 1e30f};
@@ -1512,6 +1509,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st) {
     cs_.fp32 = best[1] < (1.f - kFp32Gain) * best[0] ? 1 : 0;
     set_tuned_choice(c, nq, h->fp32_tau, cs_.fp32);
   }
+  if (!timed) return LIBERI_OK;
   // the time of every class not timed above, which spreads the classes over
   // the branches: from an earlier handle, or the second of two launches
   // (the first one of a kernel in the process loads its code, up to
@@ -1559,9 +1557,18 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs *bas, int spins, const d
       return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
+  // (nothing to time under a caller's capture)
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  const bool timing = h->class_timing && cap == hipStreamCaptureStatusNone;
   // the fused group launch, where on: its classes leave the per-class launches
   const bool fused = h->fused && h->fused_n > 0 && !h->class_timing && h->only_class < 0;
-  h->last_fused = fused;
+  auto ran = [&](int c, int variant, int64_t tile, bool fp32) {
+    ClassState &cs_ = h->cls[c];
+    cs_.ran = variant;
+    cs_.ran_tile = (int32_t)tile;
+    cs_.ran_fp32 = fp32;
+  };
   // launches of the build, by cost (ms): a class (its measured time, else the
   // proxy), or kNumClasses + k for shared launch k
   auto cost = [&](int c) { return h->cls[c].ms >= 0.f ? (double)h->cls[c].ms : class_cost_proxy(h, c); };
@@ -1570,11 +1577,21 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs *bas, int spins, const d
   double fused_cost = 0.0;
   for (int c = 0; c < kNumClasses; ++c)
     if (h->cls[c].active && (h->only_class < 0 || c == h->only_class)) {
-      if (fused && class_fused_nq(c) > 0) continue;
-      if (class_shared(h, c))
-        shared_cost[h->cls[c].shared] += class_cost_proxy(h, c);
-      else
+      const ClassState &cs_ = h->cls[c];
+      if (fused && class_fused_nq(c) > 0) {
+        ran(c, 4, 0, false);
+      } else if (class_shared(h, c)) {
+        shared_cost[cs_.shared] += class_cost_proxy(h, c);
+        if (cs_.shared < kSharedRowLaunches)
+          ran(c, 1 + cs_.dev.transposed, kSharedRowThreads, false);
+        else
+          ran(c, cs_.shared > kSharedGroupLaunch ? 3 : 0, 0, false);
+      } else {
         order.push_back({cost(c), c});
+        const bool row = class_row_mode(h, c), coop = !row && (cs_.dev.coop || class_kernel_kind(c) == 2);
+        ran(c, row ? 1 + cs_.dev.transposed : coop ? 3 : 0, row ? kTileLens[cs_.tile] : 0,
+            h->fp32_tau > 0.0 && cs_.fp32 == 1 && !coop);
+      }
     }
   for (int k = 0; k < kSharedLaunches; ++k)
     if (shared_cost[k] > 0.0) order.push_back({kSharedMs[k] + shared_cost[k], kNumClasses + k});
@@ -1627,7 +1644,7 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs *bas, int spins, const d
         if (int e = launch_shared(c - kNumClasses, h->shared[c - kNumClasses], (const ClassDev *)h->shared_cds.p, ba, st))
           return fail(LIBERI_EDEVICE, std::string("shared launch: ") + hipGetErrorString((hipError_t)e));
       } else {
-        if (h->class_timing && ns == 1) {
+        if (timing) {
           if (!h->cev0[c]) HIP_TRY(hipEventCreate(&h->cev0[c]));
           if (!h->cev1[c]) HIP_TRY(hipEventCreate(&h->cev1[c]));
           HIP_TRY(hipEventRecord(h->cev0[c], st));
@@ -1639,7 +1656,7 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs *bas, int spins, const d
         if (e != hipSuccess)
           return fail(LIBERI_EDEVICE,
                       std::string("launch ") + kClasses[c].name + ": " + hipGetErrorString((hipError_t)e));
-        if (h->class_timing && ns == 1) HIP_TRY(hipEventRecord(h->cev1[c], st));
+        if (timing) HIP_TRY(hipEventRecord(h->cev1[c], st));
       }
       if (ns > 1) HIP_TRY(captured(branch[k]));
     }
@@ -1719,9 +1736,9 @@ static int use_captured_work(liberi_ctx *h, BuildArgs &ba) {
 static bool choices_open(const liberi_ctx *h) {
   for (int k = 0; k < kNumClasses; ++k) {
     const ClassState &c = h->cls[k];
-    if (c.active && (c.variant < 0 || c.tile < 0 || (c.ms < 0.f && !class_shared(h, k)) ||
-                     (h->fp32_tau > 0.0 && c.fp32 < 0)))
-      return true;
+    if (!c.active || class_shared(h, k)) continue;
+    const bool runs = h->only_class < 0 || k == h->only_class;
+    if (c.variant < 0 || c.tile < 0 || (c.ms < 0.f && runs) || (h->fp32_tau > 0.0 && c.fp32 < 0)) return true;
   }
   return false;
 }
@@ -1757,10 +1774,25 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   if (h->fp32_tau > 0.0)
     if (int rc = enqueue_dmax(h, dD, st)) return rc;
   // (they also run before any build: Dp and Dsq from this build's density)
+  // (choices made under a caller's capture are untimed, and for that build only)
+  struct Choices {
+    liberi_ctx *h;
+    std::vector<ClassState> cls;
+    ~Choices() {
+      for (size_t c = 0; c < cls.size(); ++c) {
+        const ClassState &now = h->cls[c];
+        cls[c].ran = now.ran, cls[c].ran_tile = now.ran_tile, cls[c].ran_fp32 = now.ran_fp32;
+        h->cls[c] = cls[c];
+      }
+    }
+  } choices{h, {}};
   if (choices_open(h)) {
-    if (int e = launch_build_begin(ba, h->layout, build_work(ba), st))
+    if (!runs) {
+      choices.cls.assign(h->cls, h->cls + kNumClasses);
+    } else if (int e = launch_build_begin(ba, h->layout, build_work(ba), st)) {
       return fail(LIBERI_EDEVICE, std::string("start of the build: ") + hipGetErrorString((hipError_t)e));
-    if (int rc = choose_variants(h, ba, st)) return rc;
+    }
+    if (int rc = choose_variants(h, ba, st, runs)) return rc;
   }
   // the batched form: capture once (per D, F), replay afterwards; under a
   // caller's capture, its branches straight into the caller's graph.  Per-class
@@ -1791,7 +1823,7 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
   h->build_pending = true;
   h->fp32_pending = h->fp32_tau > 0.0;
   if (!h->fp32_pending) h->stats.fp32_quartets = 0;
-  h->timing_pending = h->class_timing && !graph;
+  h->timing_pending = h->class_timing && !graph && runs;
   if (!h->timing_pending)
     for (double &v : h->stats.class_ms) v = 0.0;
   return LIBERI_OK;

@@ -202,20 +202,22 @@ typedef struct {
                                            LIBERI_OPT_CLASS_TIMING is on (else 0) */
   int64_t prim_pairs;                   /* primitive pairs kept on the device */
   int64_t prim_pairs_dropped;           /* primitive pairs removed by LIBERI_OPT_PRIM_CUTOFF */
-  int32_t class_variant[LIBERI_NCLASS]; /* kernel form used per class in the last build: 0 its own
-                                           launch with direct atomics, 1 row tiles over bra pairs,
-                                           2 row tiles over ket pairs, 3 the cooperative form with a lane
-                                           per row of the block ((dd|dd), (fs|fs) and the group classes
-                                           with an f shell, timed against the other forms at the first
-                                           build; the only form of
+  int32_t class_variant[LIBERI_NCLASS]; /* kernel form of the class the last time it was built, in a
+                                           launch of its own or one shared with others: 0 a lane or a
+                                           group of lanes per quartet, without row tiles, 1 row tiles
+                                           over bra pairs, 2 row tiles over ket pairs, 3 the cooperative
+                                           form with a lane per row of the block ((dd|dd), (fs|fs) and the
+                                           group classes with an f shell, in their own launches timed
+                                           against the other forms at the first build; the only form of
                                            (ff|dd), (ff|fd), (ff|ff)), 4 inside the fused group
                                            launch (LIBERI_OPT_FUSED); -1 class inactive or not yet built */
   int32_t class_fp32[LIBERI_NCLASS];    /* 1: the mixed form (LIBERI_OPT_FP32_TAU > 0) evaluates this
                                            class's qualifying quartets in FP32, chosen per class from
                                            measured time at the first build under that tau; 0: FP64 */
-  int32_t class_tile[LIBERI_NCLASS];    /* row-tile length (quartets of one row per workgroup: 512,
-                                           1024, 4096 or 16384) of a row-tiled class, timed per class at the
-                                           first build after setup (LIBERI_OPT_AUTOTUNE) or 4096;
+  int32_t class_tile[LIBERI_NCLASS];    /* row-tile length of that build (quartets of one row per
+                                           workgroup: 512, 1024, 4096 or 16384, timed per class at the
+                                           first build after setup (LIBERI_OPT_AUTOTUNE) or 4096; 256 in
+                                           a launch shared with other classes);
                                            0 where the class is not row-tiled */
 } liberi_stats;
 int liberi_c_get_stats(liberi_ctx *ctx, liberi_stats *out);

@@ -57,7 +57,7 @@ std::string g_log;
 hipGraphNode_t g_deps[64];
 
 void log(const char *fmt, ...) {
-  char b[512];
+  char b[8192];
   va_list a;
   va_start(a, fmt);
   vsnprintf(b, sizeof b, fmt, a);
@@ -220,11 +220,13 @@ hipError_t hipEventQuery(hipEvent_t ev) {
   if (e->captured) return err(hipErrorCapturedEvent);
   return in_flight(e->clock) ? hipErrorNotReady : hipSuccess;
 }
-// row forms take half the time of the others
+// row forms take half the time of the others, lane row forms of 512 threads a
+// tenth less
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t b) {
   const std::string &k = ((Event *)b)->last;
   if (((Event *)b)->captured) return err(hipErrorCapturedEvent);
   *ms = k.find("eri_row") != k.npos || k.find("eri_split") != k.npos ? 0.01f : 0.02f;
+  if (k.find("eri_row") != k.npos && k.find(" 512") != k.npos) *ms *= 0.9f;
   return hipSuccess;
 }
 static thread_local struct {
@@ -240,7 +242,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
   *g = g_call.grid, *b = g_call.block, *lds = g_call.lds, *st = g_call.st;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t st) {
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t, hipStream_t st) {
   Dl_info info{};
   dladdr(f, &info);
   const std::string name = info.dli_sname ? info.dli_sname : "?";
@@ -256,9 +258,13 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, 
   if (name.find("eri_shared_") != name.npos) {
     const SharedArgs &sa = *(const SharedArgs *)args[0];
     const ClassDev *cds = *(const ClassDev **)args[1];
-    more = " classes=" + std::to_string(sa.n);
-    if (name.find("eri_shared_0") != name.npos)
-      for (int k = 0; k < sa.n; ++k) more += " [" + tile_lengths(cds[sa.cls[k]]) + "]";
+    const char launch = name[name.find("eri_shared_") + 11];
+    more = std::string(" launch=") + launch;
+    for (int k = 0; k < sa.n; ++k) {
+      more += " [class=" + std::to_string(sa.cls[k]) + " transposed=" + std::to_string(cds[sa.cls[k]].transposed);
+      if (launch < '0' + kSharedRowLaunches) more += " " + tile_lengths(cds[sa.cls[k]]);
+      more += "]";
+    }
   }
   if (name.find("build_begin") != name.npos) {
     // records of the primitive pairs that a kernel reads of a pair: at least the
@@ -277,12 +283,13 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, 
              (void *)ba.Jp);
     more = b;
   }
-  log("launch %s stream=%d captured=%d grid=%u%s", name.c_str(), s->id, s->capturing, grid.x, more.c_str());
+  log("launch %s stream=%d captured=%d grid=%u block=%u%s", name.c_str(), s->id, s->capturing, grid.x, block.x,
+      more.c_str());
   if (s->capturing)
     s->deps = {++g_node};
   else
     work(s);
-  s->last = name;
+  s->last = name + " " + std::to_string(block.x);
   return hipSuccess;
 }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {

@@ -306,6 +306,124 @@ def scenario_captured_builds_have_their_own_workspace(host):
     h.destroy()
 
 
+def launched_forms(lines):
+    """Class index -> (form, longest row tile, whether shared) of a build's launches."""
+    from gms_liberi_amd.census import CLASS_L
+
+    ids = {tuple(l): k for k, l in enumerate(CLASS_L)}
+    forms = {}
+    for x in lines:
+        m = re.search(r"eri_(small|row|split|group|coop)_kernelI((?:Li\d)+)(?:Lb([01]))?", x.replace("E", ""))
+        if m:
+            c = ids[tuple(int(v) for v in re.findall(r"Li(\d)", m.group(2)))]
+            form = {"small": 0, "group": 0, "coop": 3}.get(m.group(1), 1 + int(m.group(3) or 0))
+            forms[c] = (form, field(x, "longest") or 0, False)
+        for c, tr, tiles in re.findall(r"\[class=(\d+) transposed=(\d)(.*?)\]", x):
+            launch = field(x, "launch")
+            forms[int(c)] = (1 + int(tr), field(tiles, "longest"), True) if launch < 3 else (0 if launch == 3 else 3, 0, True)
+    return forms
+
+
+def cluster(n, seed):
+    from gms_liberi_amd import configs
+    from tests.oracle_ctypes import Oracle
+
+    b = configs.cluster(n, seed).basis
+    return b.with_schwarz(Oracle().schwarz(b))
+
+
+def scenario_statistics_name_the_launches(host):
+    """class_variant and class_tile are those of the launches of the last build,
+    shared or not, also after a build that chose other forms."""
+    from gms_liberi_amd import liberi
+
+    for b in (golden("cfg_ethane.npz"), golden("cfg_cn_chain.npz"), cluster(12, 21)):
+        d = np.zeros(b.ntri)
+        for options in ([], [(liberi.OPT_CLASS_TIMING, 1), (liberi.OPT_CLASS_TIMING, 0)], [(liberi.OPT_FP32_TAU, 1e-6)],
+                        [(liberi.OPT_FP32_TAU, 1e-6), (liberi.OPT_FP32_TAU, 0)], [(liberi.OPT_ROW_TILES, 2)],
+                        [(liberi.OPT_ROW_TILES, 0), (liberi.OPT_ROW_TILES, 1)], [(liberi.OPT_AUTOTUNE, 0)]):
+            h = liberi.Handle()
+            h.setup(b)
+            assert np.all(h.stats()["class_variant"] == -1)
+            for opt, value in options or [(liberi.OPT_GRAPH, 1)]:
+                h.set_option(opt, value)
+                h.fock_build(d)
+            h.set_option(liberi.OPT_GRAPH, 0)
+            host.log()
+            h.fock_build(d)
+            forms = launched_forms(host.log())
+            st = h.stats()
+            assert {c for c in range(55) if st["quartets"][c]} == set(forms)
+            for c in range(55):
+                form, longest, shared = forms.get(c, (-1, 0, False))
+                assert st["class_variant"][c] == form, (options, c)
+                assert (st["class_tile"][c] > 0) == (form in (1, 2)) and longest <= st["class_tile"][c], (options, c)
+                assert st["class_tile"][c] in ((256, 0) if shared else (512, 1024, 4096, 16384, 0)), (options, c)
+            h.destroy()
+
+
+def scenario_forms_do_not_depend_on_when_an_option_is_set(host):
+    """An option that takes classes out of their shared launch gives them the
+    forms and tile lengths that they would have had from the start."""
+    from gms_liberi_amd import liberi
+
+    b = cluster(12, 21)
+    d = np.zeros(b.ntri)
+    for opt, value in ((liberi.OPT_FP32_TAU, 1e-6), (liberi.OPT_CLASS_TIMING, 1), (liberi.OPT_FUSED, 1),
+                       (liberi.OPT_TILE_LEN, 1024), (liberi.OPT_ROW_TILES, 0), (liberi.OPT_ROW_TILES, 2)):
+        seen = []
+        for first in (True, False):
+            h = liberi.Handle()
+            h.setup(b)
+            if first:
+                h.fock_build(d)
+            h.set_option(liberi.OPT_GRAPH, 0)
+            h.set_option(opt, value)
+            h.fock_build(d)
+            host.log()
+            h.fock_build(d)
+            seen.append(sorted(re.sub(r"(stream|Jp)=\S+", "", x) for x in host.log() if x.startswith("launch")))
+            liberi.Handle().set_option(liberi.OPT_AUTOTUNE, 1)  # forgets the timed choices
+            h.destroy()
+        assert seen[0] == seen[1], (opt, value)
+
+
+def scenario_builds_under_a_capture_time_nothing(host):
+    """A build under a caller's capture chooses forms without running any:
+    after an option that changes them, and as the first one of a handle.  The
+    next build that runs chooses as ever."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_ethane.npz")
+    n = b.ntri
+    run, x = host.stream(), host.stream()
+    D, F = host.array(np.zeros(n)), host.array(np.zeros(n))
+
+    def build(h, s):
+        host.log()
+        h.fock_build_device(D.value, F.value, n, s.value)
+        return host.log()
+
+    for opt, value in ((liberi.OPT_GRAPH, 0), (liberi.OPT_CLASS_TIMING, 1), (liberi.OPT_TILE_LEN, 512),
+                       (liberi.OPT_ROW_TILES, 2), (liberi.OPT_ROW_TILES, 0), (liberi.OPT_FUSED, 1),
+                       (liberi.OPT_FP32_TAU, 1e-6), (liberi.OPT_AUTOTUNE, 0), (liberi.OPT_AUTOTUNE, 1)):
+        for first in (True, False):
+            h = liberi.Handle()
+            h.setup(b)
+            if first:
+                build(h, run)
+            h.set_option(opt, value)
+            host.begin_capture(x)
+            captured = build(h, x)
+            host.end_capture(x)
+            assert all(field(k, "captured") == 1 for k in captured if k.startswith("launch"))
+            counts = h.stats()["quartets"]
+            assert sum(v in launched_forms(captured) for v in np.flatnonzero(counts)) + (
+                7 if any("eri_group_fused" in k for k in captured) else 0) >= np.count_nonzero(counts)
+            build(h, run)
+            h.destroy()
+
+
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
 
 

@@ -89,10 +89,12 @@ struct ClassState {
   float ms = -1.f;      // device time of the class's launch, measured at the first build
   int64_t nquart = 0, nprimq = 0;
   int32_t nseg = 0;
-  int tile = -1;        // row-tile length chosen for the class, index into kTileLens (-1: not yet)
-  // the row tiles of this rank's share, for each tile length
-  const RowTile *tiles[kNumTileLens] = {};
-  int32_t ntile[kNumTileLens] = {};
+  int tile = -1;        // row tiles chosen for the class, index into `tiles` (-1: not yet)
+  // the row tiles of this rank's share, for each tile length and, for a class of
+  // few quartets (`small`), of one workgroup step each (kStepTile)
+  const RowTile *tiles[kNumTileLens + 1] = {};
+  int32_t ntile[kNumTileLens + 1] = {};
+  bool small = false;
   ClassDev dev{};
   // form of the last build, as in liberi_stats (-1: not built)
   int32_t ran = -1, ran_tile = 0, ran_fp32 = 0;
@@ -103,7 +105,16 @@ struct ClassState {
   const RowTile *shared_tiles = nullptr;
 };
 
-// Point the class's launch arguments at its row tiles of length kTileLens[k].
+// index of the tiles of one workgroup step
+constexpr int kStepTile = kNumTileLens;
+
+// the row tiles where none are timed or asked for
+static int default_tile(const ClassState &cs_) { return cs_.small ? kStepTile : kDefaultTile; }
+
+// length of tiles k of class c
+static int64_t tile_length(int c, int k) { return k == kStepTile ? class_row_quartets(c) : kTileLens[k]; }
+
+// Point the class's launch arguments at its row tiles k.
 static void use_tiles(ClassState &cs_, int k) {
   cs_.dev.tiles = cs_.tiles[k];
   cs_.dev.ntile = cs_.ntile[k];
@@ -691,12 +702,13 @@ static int setup_shared(liberi_ctx *h) {
 // rows of the fixed pairs with the most primitives first (the kept rows run
 // from few to many), the longest rows first among those.  Consecutive
 // segments of a row whose quartets are shared by the same number of lanes are
-// cut into tiles of `len` quartets at one lane each, fewer at more, or of what
-// one step of the workgroup (`hold`) holds where the class has few tiles.
-static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int64_t primq, int64_t len, int64_t hold,
+// cut into tiles of `len` quartets at one lane each, fewer at more.  `cut`: some
+// were longer, so that a larger `len` gives other tiles.
+static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int64_t primq, int64_t len, bool &cut,
                                       const std::vector<int64_t> &sstart, const std::vector<int32_t> &sbra,
                                       const std::vector<int32_t> &sket0, const std::vector<PairRec> &pairs) {
   std::vector<RowTile> tiles;
+  cut = false;
   if (q_begin >= q_end) return tiles;
   const size_t s0 = (size_t)(std::upper_bound(sstart.begin(), sstart.end(), q_begin) - sstart.begin()) - 1;
   const size_t s1 = (size_t)(std::lower_bound(sstart.begin(), sstart.end(), q_end) - sstart.begin());
@@ -706,7 +718,6 @@ static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int
     for (b = a; b < s1 && sbra[b] == sbra[a];) ++b;
     rows.push_back({a, b});
   }
-  if (q_end - q_begin <= hold * kRowSteps) len = std::min(len, hold);
   const double chain = class_row_chain(c, primq);
   auto team_of = [&](size_t s) {
     int32_t t = 1;
@@ -723,8 +734,9 @@ static std::vector<RowTile> row_tiles(int c, int64_t q_begin, int64_t q_end, int
       for (e = s + 1; e < b && team_of(e) == team;) ++e;
       const int64_t cap = std::max<int64_t>(1, len / team);
       size_t sg = s;
-      const int64_t q1 = std::min(sstart[e], q_end);
-      for (int64_t q = std::max(sstart[s], q_begin); q < q1; q += cap) {
+      const int64_t q1 = std::min(sstart[e], q_end), qs = std::max(sstart[s], q_begin);
+      cut |= q1 - qs > cap;
+      for (int64_t q = qs; q < q1; q += cap) {
         while (sstart[sg + 1] <= q) ++sg;
         const int64_t n = std::min(cap, q1 - q);
         size_t last = sg;
@@ -1041,13 +1053,27 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
       }
       primq = pq;
     }
-    for (int k = 0; k < kNumTileLens; ++k) {
-      std::vector<RowTile> tiles;
-      if (cs_.row_ok) tiles = row_tiles(c, d.q_begin, d.q_end, primq, kTileLens[k], class_row_quartets(c), sstart, sbra,
-                                        sket0, pairs);
-      cs_.ntile[k] = (int32_t)tiles.size();
-      if ((rc = put_table(tiles, cs_.tiles[k]))) return rc;
+    // (a class of at most kRowSteps workgroup steps takes one step a tile, and
+    // the timed lengths where one is asked for)
+    const int64_t nq = d.q_end - d.q_begin;
+    cs_.small = cs_.row_ok && nq <= class_row_quartets(c) * kRowSteps;
+    bool cut = true;
+    auto tiles_of = [&](int64_t len, const RowTile *&p, int32_t &n) -> int {
+      const std::vector<RowTile> tiles = row_tiles(c, d.q_begin, d.q_end, primq, len, cut, sstart, sbra, sket0, pairs);
+      if (tiles.size() > (size_t)INT32_MAX)
+        return fail(LIBERI_ESIZE, std::string("class ") + def.name + ": too many row tiles");
+      n = (int32_t)tiles.size();
+      return put_table(tiles, p);
+    };
+    for (int k = 0; cs_.row_ok && k < kNumTileLens; ++k) {
+      if (!cut) {  // no row is longer than the last length
+        cs_.tiles[k] = cs_.tiles[k - 1];
+        cs_.ntile[k] = cs_.ntile[k - 1];
+      } else if ((rc = tiles_of(kTileLens[k], cs_.tiles[k], cs_.ntile[k]))) {
+        return rc;
+      }
     }
+    if (cs_.small && (rc = tiles_of(class_row_quartets(c), cs_.tiles[kStepTile], cs_.ntile[kStepTile]))) return rc;
     d.row_mode = 0;
     d.threads = kRowThreads[0];
     d.transposed = p.transposed;
@@ -1070,15 +1096,16 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     h->stats.total_quartets += d.q_end - d.q_begin;
     // a place in a shared launch, where the class is small
     const int sl = class_shared_launch(c, p.transposed);
-    const int64_t nq = d.q_end - d.q_begin;
     if (sl >= 0 && nq > 0) {
       int64_t groups = 0;
       if (sl < kSharedRowLaunches) {
-        if (cs_.row_ok && nq <= kSharedRowThreads * kSharedRowGroups) {
-          const std::vector<RowTile> tiles =
-              row_tiles(c, d.q_begin, d.q_end, primq, kSharedRowThreads, kSharedRowThreads, sstart, sbra, sket0, pairs);
-          groups = (int64_t)tiles.size();
-          if (groups <= kSharedRowGroups && (rc = put_table(tiles, cs_.shared_tiles))) return rc;
+        if (cs_.small && class_row_quartets(c) == kSharedRowThreads) {
+          groups = cs_.ntile[kStepTile];
+          cs_.shared_tiles = cs_.tiles[kStepTile];
+        } else if (cs_.row_ok && nq <= kSharedRowThreads * kSharedRowGroups) {
+          int32_t n = 0;
+          if ((rc = tiles_of(kSharedRowThreads, cs_.shared_tiles, n))) return rc;
+          groups = n;
         }
       } else {
         groups = (nq + class_round_quartets(c) - 1) / class_round_quartets(c);
@@ -1217,7 +1244,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     at(cs_.dev.seg_ket0);
     for (auto &t : cs_.tiles) at(t);
     at(cs_.shared_tiles);
-    use_tiles(cs_, kDefaultTile);
+    use_tiles(cs_, default_tile(cs_));
   }
   if ((rc = setup_fused(h)) || (rc = setup_shared(h))) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
@@ -1418,14 +1445,15 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st, b
     cs_.ms = std::min(best[0], best[1]);
     set_tuned_choice(c, nq, -1.0, cs_.variant);
   }
-  // row-tile length of the row-tiled classes: shorter tiles give more
+  // row-tile length of the row-tiled classes (of those of few quartets only the
+  // time and the threads): shorter tiles give more
   // workgroups and more flushes of the exchange rows, longer ones fewer
   // workgroups (rows longer than a tile are split)
   for (int c = 0; c < kNumClasses; ++c) {
     ClassState &cs_ = h->cls[c];
     if (!cs_.active || cs_.tile >= 0 || class_shared(h, c)) continue;
     const int64_t nq = cs_.dev.q_end - cs_.dev.q_begin;
-    cs_.tile = h->tile_len >= 0 ? h->tile_len : kDefaultTile;
+    cs_.tile = h->tile_len >= 0 ? h->tile_len : default_tile(cs_);
     cs_.dev.threads = kRowThreads[0];
     if (h->tile_len >= 0 || !h->autotune || !class_row_mode(h, c) || nq < kTuneMinQuartets ||
         (h->only_class >= 0 && c != h->only_class)) {
@@ -1433,7 +1461,7 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st, b
       continue;
     }
     if (const int prev = tuned_choice(c, nq, -2.0); prev >= 0) {
-      cs_.tile = prev;
+      cs_.tile = cs_.small ? kStepTile : std::min(prev, kNumTileLens - 1);
       use_tiles(cs_, cs_.tile);
       if (tuned_choice(c, nq, -4.0) == 1) cs_.dev.threads = kRowThreads[1];
       continue;
@@ -1442,10 +1470,11 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st, b
       use_tiles(cs_, cs_.tile);
       continue;
     }
-    float best[kNumTileLens];
-    for (int k = 0; k < kNumTileLens; ++k) best[k] = 1e30f;
+    float best[kNumTileLens + 1];
+    const int k0 = cs_.small ? kStepTile : 0, k1 = cs_.small ? kStepTile : kNumTileLens - 1;
+    for (int k = k0; k <= k1; ++k) best[k] = 1e30f;
     for (int rep = 0; rep < 2; ++rep)
-      for (int k = 0; k < kNumTileLens; ++k) {
+      for (int k = k0; k <= k1; ++k) {
         if (cs_.ntile[k] <= 0) continue;
         use_tiles(cs_, k);
         float ms = 0.f;
@@ -1456,8 +1485,8 @@ static int choose_variants(liberi_ctx *h, const BuildArgs &ba, hipStream_t st, b
     // fill the tail of a class, but in a build the other classes do that, and
     // each tile costs a flush (one of 8 rank shares of C60: 4096 for every
     // class 10.6 ms, 512 12.2, the fastest of each class alone 10.7)
-    cs_.tile = kNumTileLens - 1;
-    for (int k = kNumTileLens - 2; k >= 0; --k)
+    cs_.tile = k1;
+    for (int k = k1 - 1; k >= k0; --k)
       if (best[k] < (1.f - kTileGain) * best[cs_.tile]) cs_.tile = k;
     use_tiles(cs_, cs_.tile);
     cs_.ms = best[cs_.tile];
@@ -1589,7 +1618,7 @@ static int enqueue_build(liberi_ctx *h, const BuildArgs *bas, int spins, const d
       } else {
         order.push_back({cost(c), c});
         const bool row = class_row_mode(h, c), coop = !row && (cs_.dev.coop || class_kernel_kind(c) == 2);
-        ran(c, row ? 1 + cs_.dev.transposed : coop ? 3 : 0, row ? kTileLens[cs_.tile] : 0,
+        ran(c, row ? 1 + cs_.dev.transposed : coop ? 3 : 0, row ? tile_length(c, cs_.tile) : 0,
             h->fp32_tau > 0.0 && cs_.fp32 == 1 && !coop);
       }
     }

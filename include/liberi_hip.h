@@ -173,9 +173,11 @@ const char *liberi_c_last_error(void);
                                         workloads measured).  Per-class timing and ONLY_CLASS builds
                                         launch per class.  Read at each build. */
 #define LIBERI_OPT_TILE_LEN 14       /* row-tile length of the row-tiled classes, in quartets of one row
-                                        per workgroup: 0 (default) timed per class at the first build
-                                        (LIBERI_OPT_AUTOTUNE; 4096 where untimed), or 512, 1024, 4096, 16384
-                                        for every class.  Read at each build. */
+                                        per workgroup (a quartet that several lanes share counts once a
+                                        lane): 0 (default) timed per class at the first build
+                                        (LIBERI_OPT_AUTOTUNE; 4096 where untimed), in classes of few
+                                        quartets what a workgroup holds at a time; or 512, 1024, 4096,
+                                        16384 for every class.  Read at each build. */
 #define LIBERI_OPT_ROW_ORIENT 15     /* orientation of the row tiles of a non-diagonal class: 0 (default)
                                         rows over the pair whose Coulomb block is larger, among the
                                         orientations whose accumulators fit; 1 rows over the bra pairs,
@@ -216,8 +218,9 @@ typedef struct {
                                            measured time at the first build under that tau; 0: FP64 */
   int32_t class_tile[LIBERI_NCLASS];    /* row-tile length of that build (quartets of one row per
                                            workgroup: 512, 1024, 4096 or 16384, timed per class at the
-                                           first build after setup (LIBERI_OPT_AUTOTUNE) or 4096; 256 in
-                                           a launch shared with other classes);
+                                           first build after setup (LIBERI_OPT_AUTOTUNE) or 4096; 64 to
+                                           512, what a workgroup holds at a time, in a class of few quartets,
+                                           256 in a launch shared with other classes);
                                            0 where the class is not row-tiled */
 } liberi_stats;
 int liberi_c_get_stats(liberi_ctx *ctx, liberi_stats *out);

@@ -558,3 +558,29 @@ def test_builds_in_graphs_of_the_callers(name, graph):
     ref.destroy()
     for s in streams:
         s.destroy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("natoms", [5, 17])
+def test_asked_tile_lengths_in_small_classes(natoms):
+    """LIBERI_OPT_TILE_LEN in classes of few quartets, which run one workgroup
+    step a tile where none is asked for: the same Fock matrix to summation order
+    (1e-12 of the largest element), and the statistics give the length."""
+    from gms_liberi_amd import configs
+
+    case = configs.cluster(natoms, 5)
+    h = liberi.Handle()
+    h.setup(case.basis.with_schwarz(liberi.schwarz(case.basis)))
+    ref = h.fock_build(case.density).copy()
+    for length in (512, 1024, 4096, 16384, 0):
+        h.set_option(liberi.OPT_TILE_LEN, length)
+        f = h.fock_build(case.density)
+        assert np.max(np.abs(f - ref)) <= 1e-12 * max(1.0, float(np.max(np.abs(ref)))), length
+        st = h.stats()
+        row = (st["class_variant"] == 1) | (st["class_variant"] == 2)
+        assert row.any() and np.all(st["class_tile"][~row] == 0)
+        if length:
+            assert np.all(st["class_tile"][row] == length)
+        else:
+            assert np.all(st["class_tile"][row] <= 512)
+    h.destroy()

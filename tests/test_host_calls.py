@@ -358,7 +358,7 @@ def scenario_statistics_name_the_launches(host):
                 form, longest, shared = forms.get(c, (-1, 0, False))
                 assert st["class_variant"][c] == form, (options, c)
                 assert (st["class_tile"][c] > 0) == (form in (1, 2)) and longest <= st["class_tile"][c], (options, c)
-                assert st["class_tile"][c] in ((256, 0) if shared else (512, 1024, 4096, 16384, 0)), (options, c)
+                assert not shared or st["class_tile"][c] in (256, 0), (options, c)
             h.destroy()
 
 
@@ -422,6 +422,43 @@ def scenario_builds_under_a_capture_time_nothing(host):
                 7 if any("eri_group_fused" in k for k in captured) else 0) >= np.count_nonzero(counts)
             build(h, run)
             h.destroy()
+
+
+def scenario_asked_tile_lengths_hold(host):
+    """LIBERI_OPT_TILE_LEN: every row-tiled class has tiles of that length, also
+    the classes of few quartets, which otherwise run one workgroup step a tile;
+    the statistics give the length of either."""
+    from gms_liberi_amd import liberi
+
+    b = cluster(17, 5)
+    d = np.zeros(b.ntri)
+    h = liberi.Handle()
+    h.setup(b)
+    h.set_option(liberi.OPT_GRAPH, 0)
+    longest = {}
+    for length in (0, 512, 1024, 4096, 16384, 0):
+        h.set_option(liberi.OPT_TILE_LEN, length)
+        for lines in (1, 2):
+            h.set_option(liberi.OPT_ROW_TILES, 2)  # (no shared launches)
+            host.log()
+            h.fock_build(d)
+        lines = [x for x in host.log() if x.startswith("launch")]
+        assert not any("GRID" in x for x in lines)
+        forms = launched_forms(lines)
+        tile = h.stats()["class_tile"]
+        rows = [c for c in forms if forms[c][0] in (1, 2)]
+        assert len(rows) >= 12
+        assert all(field(x, "quartets") == field(x, "share") for x in lines if "tiles=" in x)
+        for c in rows:
+            assert forms[c][1] <= tile[c], (length, c)
+            assert tile[c] == length if length else tile[c] <= 512, (length, c)
+        longest[length] = {c: forms[c][1] for c in rows}
+    # rows of up to 647 quartets: whole where the length allows
+    assert max(longest[512].values()) == 512 < max(longest[1024].values())
+    for c, n in longest[16384].items():
+        for length in (512, 1024, 4096):
+            assert longest[length][c] == min(n, length), (length, c)
+    h.destroy()
 
 
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]

@@ -975,9 +975,9 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
   };
   // (pointers into the tables are offsets until they are uploaded)
   auto put_table = [&](const auto &v, auto *&p) -> int {
-    if (int e = charge(h, v.size() * sizeof(v[0]))) return e;
+    const size_t before = tab.size();
     p = (std::remove_reference_t<decltype(p)>)put(tab, v);
-    return LIBERI_OK;
+    return charge(h, tab.size() - before);
   };
   // segments, share and tiles of a class from its segment lengths
   auto finish_class = [&](const Plan &p, const int32_t *len) -> int {
@@ -1122,7 +1122,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     const size_t o_jobs = put(up, jobs), o_len = (up.size() + 15) / 16 * 16;
     std::vector<int32_t> len(nlen);
     DevBuf buf;
-    if (int r = dev_alloc_charged(buf, o_len + nlen * sizeof(int32_t))) return r;
+    if (int r = dev_alloc(h, buf, o_len + nlen * sizeof(int32_t))) return r;
     auto *base = (unsigned char *)buf.p;
     hipError_t e = hipMemcpyAsync(base, up.data(), up.size(), hipMemcpyHostToDevice, h->stream);
     if (e == hipSuccess)
@@ -1131,6 +1131,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     if (e == hipSuccess)
       e = hipMemcpyAsync(len.data(), base + o_len, nlen * sizeof(int32_t), hipMemcpyDeviceToHost, h->stream);
     const hipError_t es = hipStreamSynchronize(h->stream);
+    h->stats.device_bytes -= (int64_t)buf.bytes;
     dev_free(buf);
     if (e == hipSuccess) e = es;
     if (e != hipSuccess) return fail(LIBERI_EDEVICE, std::string("segment generation: ") + hipGetErrorString(e));
@@ -1213,6 +1214,14 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
                         2 * ng * sizeof(int32_t) + nsegc * sizeof(int64_t);
     if ((rc = charge(h, work))) return rc;
     h->stats.device_bytes -= (int64_t)work;
+    // a batch holds at most 64 MB and what the budget leaves, or one class
+    // (sixteen bytes of padding an array)
+    const size_t add = kb.size() * (sizeof(double) + sizeof(int32_t)) + kk.size() * sizeof(double) +
+                       2 * ng * sizeof(int32_t) + nsegc * sizeof(int32_t) + sizeof(SegJob) + 7 * 16;
+    const size_t batch = up.size() + (jobs.size() * sizeof(SegJob)) + nlen * sizeof(int32_t) + add;
+    const double left = h->max_device_bytes > 0.0 ? h->max_device_bytes - (double)h->stats.device_bytes : INFINITY;
+    if (!plans.empty() && (batch > (size_t)64 << 20 || (double)batch > left))
+      if ((rc = finish_batch())) return rc;
     SegJob j;
     j.bra_x = (int64_t)put(up, bx);
     j.bra_group = (int64_t)put(up, bgroup);
@@ -1229,9 +1238,6 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     plans.push_back(Plan{c, transposed, diag, std::move(kb), std::move(kk), std::move(gbeg), nlen});
     nlen += nsegc;
     nblock += (nsegc + kSegThreads - 1) / kSegThreads;
-    // (a batch holds at most about 64 MB, or one class)
-    if (up.size() + nlen * sizeof(int32_t) > (size_t)64 << 20)
-      if ((rc = finish_batch())) return rc;
   }
   if ((rc = finish_batch())) return rc;
   if ((rc = dev_alloc_charged(h->tables, tab.size()))) return rc;

@@ -461,6 +461,38 @@ def scenario_asked_tile_lengths_hold(host):
     h.destroy()
 
 
+def scenario_setup_keeps_to_the_device_budget(host):
+    """LIBERI_OPT_MAX_DEVICE_BYTES: no moment of a setup holds more than the
+    budget, whether it succeeds or not, and the handle's resident bytes are
+    enough of a budget."""
+    from gms_liberi_amd import liberi
+
+    for b in (golden("cfg_water.npz"), golden("cfg_ethane.npz"), golden("cfg_cn_chain.npz"), cluster(12, 21)):
+        h = liberi.Handle()
+        before = host.c.host_bytes()
+        h.setup(b)
+        full = h.stats()["device_bytes"]
+        assert full >= host.c.host_bytes() - before  # all that is held is counted
+        quartets = h.stats()["quartets"]
+        h.cleanup()
+        for budget in [full + x for x in (1 << 20, 1 << 16, 1 << 12, 0, -1, -1000)] + [int(full * x / 40) for x in
+                                                                                     range(4, 40)]:
+            h.set_option(liberi.OPT_MAX_DEVICE_BYTES, budget)
+            before = host.c.host_bytes()
+            host.c.host_clear_peak()
+            try:
+                h.setup(b)
+            except liberi.LiberiError as e:
+                assert e.code == 5 and budget < full, budget - full
+                assert host.c.host_bytes() == before
+            else:
+                assert budget >= full and np.array_equal(h.stats()["quartets"], quartets)
+                h.cleanup()
+            assert host.c.host_peak() - before <= budget, (budget - full, host.c.host_peak() - before - budget)
+        h.set_option(liberi.OPT_MAX_DEVICE_BYTES, 0)
+        h.destroy()
+
+
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
 
 

@@ -1058,12 +1058,13 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     const int64_t nq = d.q_end - d.q_begin;
     cs_.small = cs_.row_ok && nq <= class_row_quartets(c) * kRowSteps;
     bool cut = true;
-    auto tiles_of = [&](int64_t len, const RowTile *&p, int32_t &n) -> int {
+    // (tiles above `most` are counted, not kept)
+    auto tiles_of = [&](int64_t len, const RowTile *&p, int32_t &n, size_t most = INT32_MAX) -> int {
       const std::vector<RowTile> tiles = row_tiles(c, d.q_begin, d.q_end, primq, len, cut, sstart, sbra, sket0, pairs);
       if (tiles.size() > (size_t)INT32_MAX)
         return fail(LIBERI_ESIZE, std::string("class ") + def.name + ": too many row tiles");
       n = (int32_t)tiles.size();
-      return put_table(tiles, p);
+      return tiles.size() <= most ? put_table(tiles, p) : LIBERI_OK;
     };
     for (int k = 0; cs_.row_ok && k < kNumTileLens; ++k) {
       if (!cut) {  // no row is longer than the last length
@@ -1104,7 +1105,7 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
           cs_.shared_tiles = cs_.tiles[kStepTile];
         } else if (cs_.row_ok && nq <= kSharedRowThreads * kSharedRowGroups) {
           int32_t n = 0;
-          if ((rc = tiles_of(kSharedRowThreads, cs_.shared_tiles, n))) return rc;
+          if ((rc = tiles_of(kSharedRowThreads, cs_.shared_tiles, n, kSharedRowGroups))) return rc;
           groups = n;
         }
       } else {

@@ -338,6 +338,8 @@ static void release_device(liberi_ctx *h) {
   dev_free(h->fock_b);
   for (auto &b : h->col_bf) dev_free(b);
   for (auto &n : h->ncol) n = 0;
+  // (nothing is left of the last build to report: its counter is gone)
+  h->build_pending = h->fp32_pending = h->timing_pending = false;
   h->stats = liberi_stats{};
   h->initialized = false;
 }

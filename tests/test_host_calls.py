@@ -493,6 +493,29 @@ def scenario_setup_keeps_to_the_device_budget(host):
         h.destroy()
 
 
+def scenario_statistics_after_a_cleanup(host):
+    """A build whose statistics were not read leaves nothing to read once the
+    handle's data is gone."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_water.npz")
+    n = b.ntri
+    s = host.stream()
+    D, F = host.array(np.zeros(n)), host.array(np.zeros(n))
+    for opt, value in ((liberi.OPT_FP32_TAU, 1e-6), (liberi.OPT_CLASS_TIMING, 1)):
+        h = liberi.Handle()
+        h.setup(b)
+        h.set_option(opt, value)
+        for end in (h.cleanup, lambda: h.setup(b)):
+            if not h.is_initialized:
+                h.setup(b)
+            h.fock_build_device(D.value, F.value, n, s.value)
+            end()
+            st = h.stats()
+            assert st["last_build_ms"] == 0 and st["fp32_quartets"] == 0 and not st["class_ms"].any()
+        h.destroy()
+
+
 SCENARIOS = [k[len("scenario_"):] for k in list(globals()) if k.startswith("scenario_")]
 
 

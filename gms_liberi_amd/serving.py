@@ -55,6 +55,32 @@ class Result:
         return self.done - self.arrival
 
 
+def _quartet_bounds(basis: Basis) -> tuple[int, int]:
+    """Upper bounds of the quartets that survive screening, all of them and those
+    with a (pd| or (dd| pair: every quartet of a small basis, else those whose
+    pairs' Gaussian decay exp(-ab/(a+b) R^2), at the smallest exponents, leaves
+    more than exp(-40) = 4e-18 of 5e-11 (a margin of 1e7 for what stands before
+    the exponentials)."""
+    nsh = basis.nsh
+    npairs = nsh * (nsh + 1) // 2
+    if npairs <= 4096:
+        return npairs * (npairs + 1) // 2, npairs * (npairs + 1) // 2
+    loc = np.asarray(basis.sh_loc, dtype=np.int64) - 1
+    e = np.array([np.min(basis.exponents[i:i + k]) for i, k in zip(loc, basis.contr_num)])
+    xyz = np.asarray(basis.coords).reshape(-1, 3)
+    atom = np.asarray(basis.atom_num) - 1
+    sq = np.sum(xyz * xyz, axis=1)
+    r2 = np.maximum(sq[:, None] + sq - 2.0 * xyz @ xyz.T, 0.0)[np.ix_(atom, atom)]
+    # ordered pairs by decay, in steps of 0.1 rounded down
+    step = np.minimum(10.0 * e[:, None] * e / (e[:, None] + e) * r2, 401.0).astype(np.int64)
+    L = np.asarray(basis.ang_mom) - 1
+    hi, lo = np.maximum(L[:, None], L), np.minimum(L[:, None], L)
+    every = np.bincount(step.ravel(), minlength=402)[:401]
+    pd = np.bincount(step[(hi == 2) & (lo >= 1)], minlength=402)[:401]
+    partners = np.cumsum(every)[::-1]
+    return int(every @ partners) // 8 + npairs * nsh, int(pd @ partners) // 4 + npairs * nsh
+
+
 def estimate_device_bytes(basis: Basis) -> int:
     """Upper estimate of the HBM a handle holds for this basis (bytes)."""
     L = np.asarray(basis.ang_mom) - 1
@@ -67,10 +93,15 @@ def estimate_device_bytes(basis: Basis) -> int:
     # pairs of each pair class (la >= lb)
     pcount = {(a, b): (per_l[a] * (per_l[a] + 1) // 2 if a == b else per_l[a] * per_l[b])
               for a in range(4) for b in range(a + 1)}
-    # each class keeps its two lists (4 B per pair) and, per kept row, up to a
-    # few segments (16 B) and tiles (12 B); a pair class serves as the rows of at
-    # most ~10 classes
-    tables = sum(10 * 60 * n for n in pcount.values())
+    # each class keeps, per kept row, a few segments (16 B) and a tile (24 B) in
+    # each of up to five tables; a pair class serves as the rows of at most 10
+    # classes.  Long rows have a tile every 512, 1024, 4096 and 16384 quartets
+    # (more where lanes share quartets, in classes of few), and classes of few
+    # quartets 2048 of one workgroup step at most; the work items of the fused
+    # launch (24 B) hold at least 32 quartets.
+    quartets, fused = _quartet_bounds(basis)
+    tables = (10 * (6 * 16 + 5 * 24) * npairs + 24 * min(quartets // 64, 55 * 2048)
+              + 24 * quartets * (1 / 512 + 1 / 1024 + 1 / 4096 + 1 / 16384) + 24 * fused / 32)
     # the density and the Coulomb sums by shell pair (twice each), the square
     # density and exchange sums
     ncart = [1, 3, 6, 10]
@@ -164,7 +195,8 @@ class Server:
         while pending or queue or active:
             now = time.perf_counter() - t0
             while pending and pending[0].arrival <= now:
-                queue.append(pending.popleft())
+                req = pending.popleft()
+                queue.append((req, estimate_device_bytes(req.basis)))
             progressed = False
             # retire finished requests first: their memory and slots go to the queue
             for s in list(active):
@@ -178,10 +210,10 @@ class Server:
                     progressed = True
             # admit while a slot and the memory allow (a lone request is always admitted)
             while queue and len(active) < self.max_active:
-                need = estimate_device_bytes(queue[0].basis)
+                req, need = queue[0]
                 if active and used + need > self.hbm_budget:
                     break
-                req = queue.popleft()
+                queue.popleft()
                 active.append(_Slot(req, time.perf_counter() - t0, need))
                 used += need
                 self.peak_active = max(self.peak_active, len(active))

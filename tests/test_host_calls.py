@@ -85,16 +85,16 @@ def golden(name):
     return Case.load_npz(ROOT / "tests" / "golden" / name).basis
 
 
-def row_of_s(n):
+def row_of_s(n, spacing=1.4):
     """n atoms in a row, one tight s primitive each; Schwarz values of 1 keep
-    every pair, and most pairs have no primitive pair left."""
+    every pair, and most pairs have no primitive pair left (at 1.4 bohr)."""
     from gms_liberi_amd.caseio import Basis
 
     one = np.arange(n) + 1
     coef = np.zeros((4, n))
     coef[0] = 1.0
     xyz = np.zeros((n, 3))
-    xyz[:, 0] = 1.4 * np.arange(n)
+    xyz[:, 0] = spacing * np.arange(n)
     return Basis(n, n, n, 1, np.ones(n, int), np.ones(n, int), one, one, one, one, one, np.full(n, 3.4), *coef, xyz.ravel(),
                  np.ones(n * (n + 1) // 2))
 
@@ -513,6 +513,22 @@ def scenario_statistics_after_a_cleanup(host):
             end()
             st = h.stats()
             assert st["last_build_ms"] == 0 and st["fp32_quartets"] == 0 and not st["class_ms"].any()
+        h.destroy()
+
+
+def scenario_footprint_estimate_is_an_upper_bound(host):
+    """The bytes that admit a request cover what its handle holds after a build,
+    from a few quartets to many for the number of pairs."""
+    from gms_liberi_amd import liberi, serving
+
+    for b in (golden("cfg_water.npz"), golden("cfg_ethane.npz"), golden("cfg_cn_chain.npz"), golden("cfg_c60.npz"),
+              cluster(17, 5), cluster(30, 6), row_of_s(100), row_of_s(300, 0.02)):
+        h = liberi.Handle()
+        before = host.c.host_bytes()
+        h.setup(b)
+        h.fock_build(np.zeros(b.ntri))
+        held = host.c.host_bytes() - before
+        assert held <= h.stats()["device_bytes"] <= serving.estimate_device_bytes(b), b.num_bas
         h.destroy()
 
 

@@ -289,19 +289,6 @@ __device__ __forceinline__ void quartet_of_segment(const ClassDev &cd, int s, in
   ket = cd.transposed ? row : col;
 }
 
-// quartet index -> (bra pair, ket pair) through the class's segment table
-__device__ __forceinline__ void decode_quartet(const ClassDev &cd, int64_t q, int32_t &bra, int32_t &ket) {
-  int lo = 0, hi = cd.nseg;  // seg_start[lo] <= q < seg_start[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (cd.seg_start[mid] <= q)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  quartet_of_segment(cd, lo, q, bra, ket);
-}
-
 __device__ __forceinline__ void fock_add(double *F, uint32_t i, uint32_t j, double v) {
   unsafeAtomicAdd(F + tri(i, j), v);
 }
@@ -906,11 +893,12 @@ __device__ __forceinline__ void wave_sum_to_lds(const double (&x)[K], double *ds
 
 // Row-tiled lane-per-quartet kernel.  One workgroup owns one tile: a run of
 // quartets that share the fixed pair.  Four of the six digestion blocks --
-// the exchange blocks K(AC), K(AD), K(BC), K(BD) -- land in Fock rows of the
-// fixed pair's shells; they are accumulated in LDS, rows[r][column], and
-// added to F once per tile.  The Coulomb block of the fixed pair is summed in
-// registers over the tile and reduced across the workgroup at the end.  Only
-// the Coulomb block of the moving pair goes to F per quartet.
+// the exchange blocks K(AC), K(AD), K(BC), K(BD) -- land in rows of the fixed
+// pair's shells; they are accumulated in LDS, rows[r][column], and added to the
+// exchange sums (BuildArgs::Ksq) once per tile.  The Coulomb block of the fixed
+// pair is summed in registers over the tile and reduced across the workgroup at
+// the end.  Only the Coulomb block of the moving pair goes to memory per
+// quartet, to the sums by pair (Jp), where the lanes' pairs are neighbours.
 // A workgroup of the kernel has 256 or 512 threads, timed per class
 // (ClassDev::threads): one copy of the tile's LDS rows and Rys table serves all
 // of them, so that 512 hold more waves per CU where the LDS limits them or the
@@ -1007,7 +995,7 @@ __device__ __forceinline__ void row_run(const ClassDev &cd, const BuildArgs &ba,
 #pragma unroll
     for (int i = 0; i < R::NM2; ++i) cm2[i] = off2 + mov.cB + gamess_pos(rm2.lx[i], rm2.ly[i], rm2.lz[i]);
 
-    // Coulomb: the fixed pair's block in registers, the moving pair's to F
+    // Coulomb: the fixed pair's block in registers, the moving pair's to the sums by pair
     if constexpr (!TR) {
       double dcd[NC * ND];
 #pragma unroll
@@ -1179,7 +1167,6 @@ __global__ __launch_bounds__(kRowThreads[1], 2) void eri_row_kernel(ClassDev cd,
 
 enum SplitSide { SPLIT_NONE = 0, SPLIT_COLS = 1, SPLIT_ROWS = 2, SPLIT_CONE = 3 };
 
-
 // largest HRR intermediate of a slice: NEP rows e and NFP columns f of
 // (e0|f0), bra levels on the NFP columns, ket levels on the slice's rows ab
 __host__ __device__ constexpr int split_buffer(int LA, int LB, int LC, int LD, int NEP, int NFP) {
@@ -1197,9 +1184,9 @@ __host__ __device__ constexpr int split_buffer(int LA, int LB, int LC, int LD, i
 }
 
 // Parts S of the split form of a class (S = 0: none), and for the ket cone the
-// directions of D per part (3: all; 1: one, the part is a (c, direction) pair).  Chosen so that the slice, the tables and
-// the HRR levels of a part fit the registers of two waves per SIMD (8-wave
-// workgroups) or three (12 waves).
+// directions of D per part (3: all; 1: one, the part is a (c, direction) pair).
+// Chosen so that the slice, the tables and the HRR levels of a part fit the
+// registers of two waves per SIMD (8-wave workgroups) or three (12 waves).
 template <int LA, int LB, int LC, int LD>
 constexpr int split_cone_dirs() {
   // (dp|pp), (dp|dp): 16 rows e, four columns per part; the others (25 or
@@ -1477,13 +1464,13 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
       for (int i = 0; i < NM2; ++i) cm2[i] = off2 + mov.cB + gamess_pos(rm2.lx[M20 + i], rm2.ly[M20 + i], rm2.lz[M20 + i]);
       auto V = [&](int a, int b, int c, int d) -> double { return v[((a * NB + b) * NCP + c) * NDP + d]; };
 
-      // Coulomb: the fixed pair's block summed over the wave, the moving pair's to F
+      // Coulomb: the fixed pair's block summed over the wave, the moving pair's to the sums by pair
       if constexpr (!TR) {
         double dcd[NCP * NDP];
 #pragma unroll
         for (int c = 0; c < NCP; ++c)
 #pragma unroll
-          for (int d = 0; d < NDP; ++d) 
+          for (int d = 0; d < NDP; ++d)
             dcd[c * NDP + d] = ba.Dp[cd.mov_base + (int64_t)((C0 + c) * ND + D0 + d) * cd.mov_n + imov];
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
@@ -1512,7 +1499,7 @@ __device__ __forceinline__ void split_part(const ClassDev &cd, const BuildArgs &
 #pragma unroll
         for (int a = 0; a < NAP; ++a)
 #pragma unroll
-          for (int b = 0; b < NB; ++b) 
+          for (int b = 0; b < NB; ++b)
             dab[a * NB + b] = ba.Dp[cd.mov_base + (int64_t)((A0 + a) * NB + b) * cd.mov_n + imov];
 #pragma unroll
         for (int c = 0; c < NCP; ++c)
@@ -2732,20 +2719,20 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
         rec[r] = ur;
         rec[NR + r] = wr * pref;
         if (r == 0) {
-        rec[2 * NR] = ipq;
-        rec[2 * NR + 1] = Q.p * ipq;
-        rec[2 * NR + 2] = P.p * ipq;
-        rec[2 * NR + 3] = 0.5 * nr_rcp(P.p);
-        rec[2 * NR + 4] = 0.5 * nr_rcp(Q.p);
-        rec[2 * NR + 5] = pqx;
-        rec[2 * NR + 6] = pqy;
-        rec[2 * NR + 7] = pqz;
-        rec[2 * NR + 8] = P.PAx;
-        rec[2 * NR + 9] = P.PAy;
-        rec[2 * NR + 10] = P.PAz;
-        rec[2 * NR + 11] = Q.PAx;
-        rec[2 * NR + 12] = Q.PAy;
-        rec[2 * NR + 13] = Q.PAz;
+          rec[2 * NR] = ipq;
+          rec[2 * NR + 1] = Q.p * ipq;
+          rec[2 * NR + 2] = P.p * ipq;
+          rec[2 * NR + 3] = 0.5 * nr_rcp(P.p);
+          rec[2 * NR + 4] = 0.5 * nr_rcp(Q.p);
+          rec[2 * NR + 5] = pqx;
+          rec[2 * NR + 6] = pqy;
+          rec[2 * NR + 7] = pqz;
+          rec[2 * NR + 8] = P.PAx;
+          rec[2 * NR + 9] = P.PAy;
+          rec[2 * NR + 10] = P.PAz;
+          rec[2 * NR + 11] = Q.PAx;
+          rec[2 * NR + 12] = Q.PAy;
+          rec[2 * NR + 13] = Q.PAz;
         }
       }
     };
@@ -2958,8 +2945,8 @@ __device__ __forceinline__ void grp_run(const ClassDev &cd, const BuildArgs &ba,
       if (valid) {
         const double sk = s * ba.k_scale;
         auto put = [&](double *dst, double x) {
-        if (x != 0.0) unsafeAtomicAdd(dst, x);
-      };
+          if (x != 0.0) unsafeAtomicAdd(dst, x);
+        };
         for (int i = gl; i < NCD; i += G) {
           double t = 0.0;
 #pragma unroll
@@ -3284,9 +3271,8 @@ __global__ __launch_bounds__(kSegThreads) void segment_lengths_kernel(const unsi
 // quartets; (ij|kl) and (kl|ij) of the one pair are equal, so that only those
 // with ij >= kl are formed, the others counted twice.  A lane alone walked up
 // to 1296 quartets: 20-atom C-N chain, (ss| 566 -> 27 us, all groups 1190 ->
-// 197 us;
-// the 2-D Rys integrals G(i, k) of each root (i on A, k on C = A) are moved
-// to the diagonal (a b | a b) in one step with the binomial form of the
+// 197 us.  The 2-D Rys integrals G(i, k) of each root (i on A, k on C = A) are
+// moved to the diagonal (a b | a b) in one step with the binomial form of the
 // transfer relation, I(a,b,a,b) = sum_t sum_u C(b,t) C(b,u) AB^(2b-t-u)
 // G(a+t, a+u), since the ket pair is the bra pair (CD = AB).
 __host__ __device__ constexpr int binom(int n, int k) {
@@ -3453,8 +3439,8 @@ int launch_schwarz(int la, int lb, const SchwarzPair *pairs, const SchwarzShell 
 }
 
 // Calls f(element, element in pair-major order, pair, class, a, b) for this
-// thread's elements of the pair layout: workgroup blk covers a run of pairs of one class and one component (a, b),
-// so nothing of the decoding is per lane.
+// thread's elements of the pair layout: workgroup blk covers a run of pairs of
+// one class and one component (a, b), so nothing of the decoding is per lane.
 template <class Body>
 __device__ __forceinline__ void for_pair_layout(const PairLayout &pl, int blk, Body f) {
   int c = 0;
@@ -3598,8 +3584,6 @@ constexpr bool use_small() {
   return nrange(LA, LA + LB) * nrange(LC, LC + LD) <= 100 && hrr_max_buffer(LA, LB, LC, LD) <= 100;
 }
 
-// LDS bytes of the row-tiled kernel of the class in orientation TR, or -1
-// when the class has no such kernel
 // (dynamic) LDS bytes of the row accumulators of the class in orientation TR
 template <int LA, int LB, int LC, int LD, bool TR>
 int64_t row_acc_bytes(const int32_t *ncol) {

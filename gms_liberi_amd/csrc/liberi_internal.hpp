@@ -58,11 +58,11 @@ struct PairRec {
   double x;          // Schwarz value of the pair
 };
 
-// One primitive pair (a in A, b in B): p = a + b, P, P - A, and
-// K = c_a c_b exp(-ab/p |A-B|^2) / p.
 // largest basis: n(n+1) stays below 2^32, so packed indices fit 32 bits
 constexpr int32_t kMaxBasis = 65535;
 
+// One primitive pair (a in A, b in B): p = a + b, P, P - A, and
+// K = c_a c_b exp(-ab/p |A-B|^2) / p.
 struct alignas(64) PrimRec {
   double p, Px, Py, Pz, PAx, PAy, PAz, K;
 };
@@ -225,7 +225,6 @@ int class_shared_launch(int c, int transposed);
 int class_round_quartets(int c);
 int launch_shared(int launch, const SharedArgs &sa, const ClassDev *cds, const BuildArgs &ba, void *stream);
 
-// longest row tile, quartets
 // row-tile lengths (quartets of one row per workgroup) the autotuner times
 // per row-tiled class; kDefaultTile where it does not time
 constexpr int kNumTileLens = 4;

@@ -1,10 +1,11 @@
 // Schwarz integrals without any device allocation: liberi_c_schwarz_noalloc.
 //
 // liberi_c_schwarz allocates a device buffer (pair list, shells, primitive-pair
-// records, results) and a stream per call, and frees them again; hipFree synchronises the whole device, which stalls every other
-// build in flight, and neither call is allowed under HIP graph capture.  This
-// variant stages the same data in one library-owned device array, `scratch`,
-// and runs on the caller's stream.
+// records, results) and a stream per call, and frees them again; hipFree
+// synchronises the whole device, which stalls every other build in flight, and
+// neither call is allowed under HIP graph capture.  This variant stages the same
+// data in one library-owned device array, `scratch`, and runs on the caller's
+// stream.
 //
 // The array lives as long as the process, once per GPU the library runs on.
 // Host code never passes its name to the runtime or to a kernel: its device

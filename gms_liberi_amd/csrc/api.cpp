@@ -139,6 +139,10 @@ struct liberi_ctx {
   // has been recorded); a build under a caller's capture, which does not run
   // then, records neither event.
   bool built = false;
+  // the end of every kPace-th build, in turn: at most 2 kPace are outstanding
+  hipEvent_t paced[2] = {};
+  bool paced_set[2] = {};
+  int pace_slot = 0, pace_count = 0;
   std::vector<DevBuf> owned;
   DevBuf pairs, prims, dens, fock;
   DevBuf tables;  // segments and row tiles of every class
@@ -265,14 +269,37 @@ static void dev_free(DevBuf &b) {
   b.bytes = 0;
 }
 
-// Waits on the host for the last build that ran, on whatever stream (a
-// thread that captures may call it: it waits for nothing captured).
-static void wait_last_build(liberi_ctx *h) {
-  if (!h->built) return;
+// Waits on the host for an event of builds that run (a thread that captures
+// may call it: it waits for nothing captured).
+static hipError_t wait_event(hipEvent_t e) {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   (void)hipThreadExchangeStreamCaptureMode(&mode);
-  (void)hipEventSynchronize(h->ev1);
+  const hipError_t rc = hipEventSynchronize(e);
   (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return rc;
+}
+
+// Waits on the host for the last build that ran, on whatever stream.
+static void wait_last_build(liberi_ctx *h) {
+  if (h->built) (void)wait_event(h->ev1);
+}
+
+// The end of a build on st.  A caller that enqueues builds without ever
+// waiting gets ahead of the device without bound, thousands of graph launches
+// for a small molecule; here it waits for the build kPace to 2 kPace before, so
+// that the device always has some to go on with.
+constexpr int kPace = 8;
+static hipError_t end_build(liberi_ctx *h, hipStream_t st) {
+  hipError_t e = hipEventRecord(h->ev1, st);
+  if (e != hipSuccess) return e;
+  h->built = true;
+  if (++h->pace_count < kPace) return hipSuccess;
+  h->pace_count = 0;
+  const int k = h->pace_slot;
+  if ((e = hipEventRecord(h->paced[k], st)) != hipSuccess) return e;
+  h->paced_set[k] = true;
+  h->pace_slot = k ^ 1;
+  return h->paced_set[k ^ 1] ? wait_event(h->paced[k ^ 1]) : hipSuccess;
 }
 
 // A graph taken from the handle, destroyed once its replays are over.
@@ -387,6 +414,7 @@ int liberi_c_create(liberi_ctx **ctx) {
   HIP_TRY(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
   HIP_TRY(hipEventCreate(&h->ev0));
   HIP_TRY(hipEventCreate(&h->ev1));
+  for (hipEvent_t &e : h->paced) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   *ctx = h;
   return LIBERI_OK;
 }
@@ -408,6 +436,8 @@ int liberi_c_destroy(liberi_ctx **ctx) {
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   for (hipEvent_t e : h->tev)
+    if (e) (void)hipEventDestroy(e);
+  for (hipEvent_t e : h->paced)
     if (e) (void)hipEventDestroy(e);
   for (int c = 0; c < kNumClasses; ++c) {
     if (h->cev0[c]) (void)hipEventDestroy(h->cev0[c]);
@@ -1854,10 +1884,7 @@ static int build_on_device(liberi_ctx *h, const double *dD, double *dF, hipStrea
     return rc;
   }
   old.end();
-  if (runs) {
-    HIP_TRY(hipEventRecord(h->ev1, st));
-    h->built = true;
-  }
+  if (runs) HIP_TRY(end_build(h, st));
   h->build_pending = true;
   h->fp32_pending = h->fp32_tau > 0.0;
   if (!h->fp32_pending) h->stats.fp32_quartets = 0;
@@ -1933,12 +1960,11 @@ static int build_uhf_graph(liberi_ctx *h, const double *dt, const double *dDa, c
   if (e == hipSuccess) e = hipEventRecord(h->ev0, st);
   if (e == hipSuccess) e = hipGraphLaunch(h->uexec, st);
   old.end();
-  if (e == hipSuccess) e = hipEventRecord(h->ev1, st);
+  if (e == hipSuccess) e = end_build(h, st);
   if (e != hipSuccess) {
     *rc = fail(LIBERI_EDEVICE, std::string("UHF build: ") + hipGetErrorString(e));
     return 0;
   }
-  h->built = true;
   h->build_pending = true;
   h->fp32_pending = h->timing_pending = false;
   h->stats.fp32_quartets = 0;

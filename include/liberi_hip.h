@@ -93,7 +93,8 @@ int liberi_c_fock_build(liberi_ctx *ctx, const double *density, double *fock, in
 
 /* Same build on device-resident arrays (hipMalloc'd, n doubles each) on the
  * given hipStream_t (NULL = the handle's stream).  Asynchronous: returns after
- * enqueueing.  No counterpart in the reference (which maps D/F per call,
+ * enqueueing, unless more than 8 builds of the handle are outstanding, when it
+ * may wait for the oldest of them (at most 16 are).  No counterpart in the reference (which maps D/F per call,
  * src/liberi_driver.F90:66,163); for callers that keep D and F in HBM.
  * Builds of one handle share its device workspace: one enqueued on another
  * stream than the last waits for it.  A build that the caller captures into a

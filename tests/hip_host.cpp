@@ -128,6 +128,8 @@ int host_id(Stream *s) { return s->id; }
 // whether the work issued so far on a comes before what b issues next
 int host_before(Stream *a, Stream *b) { return b->clock[a->id] >= a->clock[a->id]; }
 int host_in_flight(Stream *s) { return in_flight(s->clock); }
+// work items of s that nothing has waited for
+long host_outstanding(Stream *s) { return s->clock[s->id] - g_done[s->id]; }
 
 // ---- the runtime
 hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }

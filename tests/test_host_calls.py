@@ -41,8 +41,9 @@ class Host:
             getattr(self.c, f).restype = C.c_size_t
         self.c.host_fail.argtypes = [C.c_size_t]
         vp = C.c_void_p
-        for f in ("host_id", "host_in_flight"):
+        for f in ("host_id", "host_in_flight", "host_outstanding"):
             getattr(self.c, f).argtypes = [vp]
+        self.c.host_outstanding.restype = C.c_long
         self.c.host_before.argtypes = [vp, vp]
         self.c.hipStreamBeginCapture.argtypes = [vp, C.c_int]
         self.c.hipStreamEndCapture.argtypes = [vp, C.POINTER(vp)]
@@ -529,6 +530,37 @@ def scenario_footprint_estimate_is_an_upper_bound(host):
         h.fock_build(np.zeros(b.ntri))
         held = host.c.host_bytes() - before
         assert held <= h.stats()["device_bytes"] <= serving.estimate_device_bytes(b), b.num_bas
+        h.destroy()
+
+
+def scenario_outstanding_builds_are_bounded(host):
+    """A caller that never waits has at most 16 builds of a handle outstanding,
+    and the device at least 8 to go on with after every wait."""
+    from gms_liberi_amd import liberi
+
+    b = golden("cfg_water.npz")
+    n = b.ntri
+    D, F, Da, Db, Fa, Fb = (host.array(np.zeros(n)) for _ in range(6))
+    for graph in (1, 0):
+        h = liberi.Handle()
+        h.setup(b)
+        h.set_option(liberi.OPT_GRAPH, graph)
+        s = host.stream()
+        h.fock_build_device(D.value, F.value, n, s.value)
+        first = host.c.host_outstanding(s)
+        h.fock_build_device(D.value, F.value, n, s.value)
+        per = host.c.host_outstanding(s) - first  # work items of a build
+        most, least = 0, 10 ** 9
+        for k in range(1, 200):
+            h.fock_build_device(D.value, F.value, n, s.value)
+            now = host.c.host_outstanding(s)
+            most = max(most, now)
+            if k > 20:
+                least = min(least, now)
+        assert most <= 16 * per + first and least >= 8 * per, (graph, most, least, per)
+        for _ in range(100):
+            assert h._lib.liberi_c_fock_build_uhf_device(h._h, Da, Db, Fa, Fb, n, s) == 0
+            assert host.c.host_outstanding(s) <= 16 * (2 * per + 1) + 2 * first
         h.destroy()
 
 

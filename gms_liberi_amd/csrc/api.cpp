@@ -1052,8 +1052,8 @@ static int setup_basis(liberi_ctx *h, int32_t nsh, int32_t natoms, int32_t num_b
     // costs its primitive quartets plus kQuartetCost for its HRR and
     // digestion, and the kept lists run from few to many primitives, so equal
     // counts leave the last ranks the most work (C60 in 8 shares, time of the
-    // slowest over the mean: equal counts 1.39; kQuartetCost 4: 1.26,
-    // 8: 1.08, 16: 1.08, 32: 1.16).
+    // slowest over the mean: equal counts 1.47 to 1.50, this split 1.09 to
+    // 1.11; the constant was fitted on earlier kernels, 1.08 then).
     if (h->rank_split == 1 || num_procs == 1) {
       d.q_begin = total * my_rank / num_procs;
       d.q_end = total * (my_rank + 1) / num_procs;

@@ -159,7 +159,7 @@ const char *liberi_c_last_error(void);
                                        of few quartets run several to a launch. */
 #define LIBERI_OPT_GRAPH 10         /* 1 (default): batched form -- the build's class launches run on
                                        four branches of a graph (largest first onto the least-loaded
-                                       stream), captured once into a HIP graph that later builds on
+                                       branch), captured once into a HIP graph that later builds on
                                        the same D and F replay; 0: one stream, launched eagerly.
                                        Per-class timing and ONLY_CLASS builds run eagerly.  Read at
                                        each build; any option change drops the captured graph. */

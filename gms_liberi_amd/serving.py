@@ -63,22 +63,30 @@ def _quartet_bounds(basis: Basis) -> tuple[int, int]:
     the exponentials)."""
     nsh = basis.nsh
     npairs = nsh * (nsh + 1) // 2
-    if npairs <= 4096:
-        return npairs * (npairs + 1) // 2, npairs * (npairs + 1) // 2
-    loc = np.asarray(basis.sh_loc, dtype=np.int64) - 1
-    e = np.array([np.min(basis.exponents[i:i + k]) for i, k in zip(loc, basis.contr_num)])
-    xyz = np.asarray(basis.coords).reshape(-1, 3)
+    loc, k = np.asarray(basis.sh_loc, dtype=np.int64) - 1, np.asarray(basis.contr_num, dtype=np.int64)
+    expo, xyz = np.asarray(basis.exponents), np.asarray(basis.coords).reshape(-1, 3)
     atom = np.asarray(basis.atom_num) - 1
-    sq = np.sum(xyz * xyz, axis=1)
-    r2 = np.maximum(sq[:, None] + sq - 2.0 * xyz @ xyz.T, 0.0)[np.ix_(atom, atom)]
-    # ordered pairs by decay, in steps of 0.1 rounded down
-    step = np.minimum(10.0 * e[:, None] * e / (e[:, None] + e) * r2, 401.0).astype(np.int64)
+    every_quartet = npairs * (npairs + 1) // 2
+    # (a basis out of its arrays is the setup's to refuse)
+    if npairs <= 4096 or np.any((k < 1) | (loc < 0) | (loc + k > expo.size) | (atom < 0) | (atom >= len(xyz))):
+        return every_quartet, every_quartet
+    e = np.array([np.min(expo[i:i + n]) for i, n in zip(loc, k)])
+    if not (np.all(np.isfinite(e) & (e > 0)) and np.all(np.isfinite(xyz))):
+        return every_quartet, every_quartet
+    # ordered pairs by decay, in steps of 0.1 rounded down, some rows at a time
     L = np.asarray(basis.ang_mom) - 1
-    hi, lo = np.maximum(L[:, None], L), np.minimum(L[:, None], L)
-    every = np.bincount(step.ravel(), minlength=402)[:401]
-    pd = np.bincount(step[(hi == 2) & (lo >= 1)], minlength=402)[:401]
-    partners = np.cumsum(every)[::-1]
-    return int(every @ partners) // 8 + npairs * nsh, int(pd @ partners) // 4 + npairs * nsh
+    centre = xyz[atom]
+    sq = np.sum(centre * centre, axis=1)
+    every, pd = np.zeros(402), np.zeros(402)
+    for i in range(0, nsh, 512):
+        r = slice(i, i + 512)
+        r2 = np.maximum(sq[r, None] + sq - 2.0 * centre[r] @ centre.T, 0.0)
+        step = np.minimum(10.0 * e[r, None] * e / (e[r, None] + e) * r2, 401.0).astype(np.int64)
+        hi, lo = np.maximum(L[r, None], L), np.minimum(L[r, None], L)
+        every += np.bincount(step.ravel(), minlength=402)
+        pd += np.bincount(step[(hi == 2) & (lo >= 1)], minlength=402)
+    partners = np.cumsum(every[:401])[::-1]
+    return int(every[:401] @ partners / 8) + npairs * nsh, int(pd[:401] @ partners / 4) + npairs * nsh
 
 
 def estimate_device_bytes(basis: Basis) -> int:

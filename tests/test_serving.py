@@ -46,3 +46,19 @@ def test_footprint_estimate_grows_with_the_molecule():
     small = serving.request_stream(1, 1.0, seed=1, iterations=1, atoms=(10, 10))[0].basis
     large = serving.request_stream(1, 1.0, seed=1, iterations=1, atoms=(60, 60))[0].basis
     assert serving.estimate_device_bytes(large) > 4 * serving.estimate_device_bytes(small)
+
+
+def test_estimate_leaves_an_unsound_basis_to_the_setup():
+    """A basis that setup refuses still gets an estimate (of every quartet), and
+    a far larger one than the sound basis."""
+    import dataclasses
+
+    from gms_liberi_amd import configs
+
+    b = configs.cluster(24, 5).basis
+    good = serving.estimate_device_bytes(b)
+    for name, value in (("sh_loc", 10 ** 6), ("contr_num", 0), ("atom_num", 99), ("exponents", np.nan), ("exponents", -1.0),
+                        ("coords", np.inf)):
+        a = np.array(getattr(b, name), copy=True)
+        a[0] = value
+        assert serving.estimate_device_bytes(dataclasses.replace(b, **{name: a})) > good, name

@@ -168,7 +168,8 @@ const char *liberi_c_last_error(void);
                                         a per-quartet term); 1 equal quartet counts, the reference's split
                                         (e.g. src/rhf/rot_axis/int0001.F90:100-104).  Either way the ranks'
                                         partial Fock matrices sum to the full one.  Read at setup. */
-#define LIBERI_OPT_FUSED 13          /* 0 (default): one launch per class; 1: the seven s, p, d classes
+#define LIBERI_OPT_FUSED 13          /* 0 (default): launches of one class, small classes several to
+                                        a launch; 1: the seven s, p, d classes
                                         of the group path with the smallest LDS slots run in one
                                         persistent launch fed from a device work queue (slower on the
                                         workloads measured).  Per-class timing and ONLY_CLASS builds
